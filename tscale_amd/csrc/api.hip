@@ -18,6 +18,7 @@ struct tsattn_ctx {
     float *part_acc;
     float *part_ml;
     int32_t *seq_done;
+    void *head; // records of the softmax and sampling launches
 };
 
 // Scratch of the entry point that allocates nothing (tsattn_decode_static): split partials [pair][split][d] f32, their
@@ -183,18 +184,22 @@ int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
     c->part_acc = nullptr;
     c->part_ml = nullptr;
     c->seq_done = nullptr;
+    c->head = nullptr;
+    e = hipMalloc(&c->head, tsattn::HEAD_SCRATCH_BYTES);
+    if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc(row records)"); }
     size_t parts = (size_t)c->max_seqs * c->max_heads * c->max_splits;
     if (parts > 0 && c->max_head_dim > 0) {
         e = hipMalloc((void **)&c->part_acc, parts * c->max_head_dim * sizeof(float));
-        if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc(split partials)"); }
+        if (e != hipSuccess) { (void)hipFree(c->head); delete c; return hip_fail(e, "hipMalloc(split partials)"); }
         e = hipMalloc((void **)&c->part_ml, parts * 2 * sizeof(float));
-        if (e != hipSuccess) { (void)hipFree(c->part_acc); delete c; return hip_fail(e, "hipMalloc(split max/sum)"); }
+        if (e != hipSuccess) { (void)hipFree(c->head); (void)hipFree(c->part_acc); delete c; return hip_fail(e, "hipMalloc(split max/sum)"); }
     }
     if (c->max_seqs > 0) {
         // arrival counters of the single-split fused append: zero here, and left at zero by every launch
         e = hipMalloc((void **)&c->seq_done, (size_t)c->max_seqs * sizeof(int32_t));
         if (e == hipSuccess) e = hipMemset(c->seq_done, 0, (size_t)c->max_seqs * sizeof(int32_t));
         if (e != hipSuccess) {
+            (void)hipFree(c->head);
             if (c->seq_done) (void)hipFree(c->seq_done);
             if (c->part_acc) (void)hipFree(c->part_acc);
             if (c->part_ml) (void)hipFree(c->part_ml);
@@ -212,6 +217,7 @@ int tsattn_destroy(tsattn_handle_t h)
     if (h->part_acc) (void)hipFree(h->part_acc);
     if (h->part_ml) (void)hipFree(h->part_ml);
     if (h->seq_done) (void)hipFree(h->seq_done);
+    if (h->head) (void)hipFree(h->head);
     delete h;
     return TSATTN_OK;
 }
@@ -600,6 +606,7 @@ int tsattn_softmax_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const int3
     tsattn::HeadParams p = {};
     p.n_rows = n_rows; p.n = n; p.src = src; p.src_planes = src_planes > 1 ? src_planes : 1; p.src_plane_stride = src_plane_stride;
     p.src_pitch = src_pitch; p.scale = scale; p.bias = bias; p.prob = prob; p.prob_pitch = prob_pitch; p.argmax = argmax;
+    p.scratch = h->head;
     hipError_t e = tsattn::launch_softmax_rows(p, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "softmax launch");
     return TSATTN_OK;
@@ -617,6 +624,7 @@ int tsattn_sample_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const float
     tsattn::HeadParams p = {};
     p.n_rows = n_rows; p.n = n; p.prob = const_cast<float *>(prob); p.prob_pitch = prob_pitch; p.temperature = temperature;
     p.rnd = rnd; p.rnd_pitch = rnd_pitch; p.seed = seed; p.offset = offset; p.argmax = choice;
+    p.scratch = h->head;
     hipError_t e = tsattn::launch_sample_rows(p, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sampling launch");
     return TSATTN_OK;

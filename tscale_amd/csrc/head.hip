@@ -9,40 +9,35 @@ namespace tsattn {
 #pragma clang fp contract(off)
 
 // state[row][x] = sum over the row's labels of embed[label][x] * scale, added in label order starting from 0
-// (cpu_infer.cpp:559-565).  One thread per 16 consecutive x.
+// (cpu_infer.cpp:559-565).  One thread per four consecutive x, so that a wave stores 1 KiB of consecutive floats (bound by
+// those stores: 65536 rows of 2048, 184 us with sixteen x per thread, whose stores leave 64-byte gaps).
 __global__ __launch_bounds__(256) void embed_rows_kernel(HeadParams p)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int chunks = p.dim / 16;
-    if (i >= p.n_rows * chunks) return;
-    const int64_t row = i / chunks;
-    const int x0 = (int)(i - row * chunks) * 16;
-    float acc[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
+    const unsigned blocks_per_row = (p.dim / 4 + 255) / 256;
+    const int64_t row = blockIdx.x / blocks_per_row;
+    const int x0 = (int)((blockIdx.x % blocks_per_row) * 256 + threadIdx.x) * 4;
+    if (x0 >= p.dim) return;
+    v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     for (int l = 0; l < p.labels_per_row; ++l) {
         const int label = p.labels[row * p.labels_per_row + l];
         if (label < 0 || label >= p.n_labels) continue; // an empty slot
-        const v4i w = *(const v4i *)(p.embed + (int64_t)label * p.embed_pitch + x0);
-        const int ww[4] = {w.x, w.y, w.z, w.w};
+        const int w = *(const int *)(p.embed + (int64_t)label * p.embed_pitch + x0);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int8_t e = (int8_t)((ww[j / 4] >> (8 * (j % 4))) & 0xff);
-            acc[j] = acc[j] + (float)e * p.embed_scale;
-        }
+        for (int j = 0; j < 4; ++j) acc[j] = acc[j] + (float)(int8_t)((w >> (8 * j)) & 0xff) * p.embed_scale;
     }
-    float *o = p.state + row * p.state_pitch + x0;
-#pragma unroll
-    for (int j = 0; j < 16; j += 4) *(v4f *)(o + j) = v4f{acc[j], acc[j + 1], acc[j + 2], acc[j + 3]};
+    *(v4f *)(p.state + row * p.state_pitch + x0) = acc;
 }
 
-// One workgroup per row.  w[k] = vec[k] * scale + bias[k]; M = max(0, max w) (the buffer's maximum starts at 0,
-// cpu_infer.cpp:226-244); p[k] = 2^(w[k] - M) / sum (base 2: the scale carries 1/ln 2).  The choice is the first k of
-// the largest w.  A row is 200 KB of sums and as much bias for one CU, and what a CU gets per microsecond is what it
-// has in flight: 1024 threads, four requests of 16 bytes (rows start at any multiple of 4 bytes) per thread and round,
-// so that a pass is two rounds of memory latency and not two hundred.
-constexpr int SM_THREADS = 1024;
+// w[k] = vec[k] * scale + bias[k]; M = max(0, max w) (the buffer's maximum starts at 0, cpu_infer.cpp:226-244);
+// p[k] = 2^(w[k] - M) / sum (base 2: the scale carries 1/ln 2).  The choice is the first k of the largest w.
+//
+// A row is cut into chunks, one workgroup each, so that few rows still fill the chip: a vocabulary row of 200 KB for one
+// compute unit is bound by what that unit can have in flight.  Two launches: every chunk's largest value, where it is
+// first reached and the sum of its weights go to the handle's scratch, then every chunk reads all of its row's records
+// and writes its probabilities.  32 x 50257: 25.6 us with one workgroup per row walking it three times, 9 us like this.
+constexpr int SM_THREADS = 256;
 constexpr int SM_U = 4;
+constexpr int SM_CHUNK = 4 * SM_U * SM_THREADS; // values a workgroup takes per round
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -67,74 +62,133 @@ __device__ inline v4f softmax_logit4(const HeadParams &p, int64_t row, int64_t k
     return w;
 }
 
-// Walks a row: groups of four from the front, SM_U requests per thread out before the first is used (none under a
-// branch: a group past the end asks for the last whole group again), then the up to three values that are left.
+// Walks the values [begin, end) of a row (begin a multiple of 4): groups of four from the front, SM_U requests per thread
+// out before the first is used (none under a branch: a group past the end asks for the last whole group again), then the
+// up to three values that are left.  A thread sees its k in ascending order.
 template <typename F>
-__device__ inline void softmax_walk(const HeadParams &p, int64_t row, int tid, F &&f)
+__device__ inline void softmax_walk(const HeadParams &p, int64_t row, int64_t begin, int64_t end, int tid, F &&f)
 {
-    const int64_t n4 = p.n & ~(int64_t)3;
-    for (int64_t base = 0; base < n4; base += 4 * SM_THREADS * SM_U) {
+    const int64_t n4 = begin + ((end - begin) & ~(int64_t)3);
+    for (int64_t base = begin; base < n4; base += SM_CHUNK) {
         v4f w[SM_U];
 #pragma unroll
         for (int u = 0; u < SM_U; ++u) {
-            const int64_t k = base + 4 * (tid + (int64_t)u * SM_THREADS);
+            const int64_t k = base + 4 * (tid + u * SM_THREADS);
             w[u] = softmax_logit4(p, row, k < n4 ? k : n4 - 4);
         }
 #pragma unroll
         for (int u = 0; u < SM_U; ++u) {
-            const int64_t k = base + 4 * (tid + (int64_t)u * SM_THREADS);
-            if (k < n4) { f(k, w[u].x); f(k + 1, w[u].y); f(k + 2, w[u].z); f(k + 3, w[u].w); }
+            const int64_t k = base + 4 * (tid + u * SM_THREADS);
+            if (k < n4) f(k, w[u], 4);
         }
     }
-    if (n4 + tid < p.n) f(n4 + tid, softmax_logit(p, row, n4 + tid));
+    if (n4 + tid < end) {
+        const float w = softmax_logit(p, row, n4 + tid);
+        f(n4 + tid, v4f{w, w, w, w}, 1);
+    }
 }
 
-__global__ __launch_bounds__(SM_THREADS) void softmax_rows_kernel(HeadParams p)
+// largest value and the first index of it over the workgroup; every thread gets both
+__device__ inline void first_max(float &best, int &arg, float *s_max, int *s_arg, int tid)
 {
-    __shared__ float s_max[SM_THREADS / WAVE];
-    __shared__ int s_arg[SM_THREADS / WAVE];
-    __shared__ float s_sum[SM_THREADS / WAVE];
-    const int64_t row = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
-    // pass 1: maximum and where it is first reached (a thread sees its k in ascending order)
-    float best = -INFINITY;
-    int arg = 0x7fffffff;
-    softmax_walk(p, row, tid, [&](int64_t k, float w) {
-        if (w > best) { best = w; arg = (int)k; }
-    });
     for (int o = 32; o > 0; o >>= 1) {
         const float ob = __shfl_xor(best, o, WAVE);
         const int oa = __shfl_xor(arg, o, WAVE);
         if (ob > best || (ob == best && oa < arg)) { best = ob; arg = oa; }
     }
-    if (lane == 0) { s_max[wave] = best; s_arg[wave] = arg; }
+    if ((tid & (WAVE - 1)) == 0) { s_max[tid / WAVE] = best; s_arg[tid / WAVE] = arg; }
     __syncthreads();
     best = s_max[0]; arg = s_arg[0];
     for (int w = 1; w < SM_THREADS / WAVE; ++w) {
         if (s_max[w] > best || (s_max[w] == best && s_arg[w] < arg)) { best = s_max[w]; arg = s_arg[w]; }
     }
-    if (tid == 0 && p.argmax) p.argmax[row] = arg;
-    if (!p.prob) return;
-    const float M = fmaxf(0.0f, best);
-    // pass 2: sum of the weights
-    float sum = 0.0f;
-    softmax_walk(p, row, tid, [&](int64_t, float w) { sum += fast_exp2(fmaxf(w - M, -127.0f)); });
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, WAVE);
-    if (lane == 0) s_sum[wave] = sum;
-    __syncthreads();
-    sum = 0.0f;
-    for (int w = 0; w < SM_THREADS / WAVE; ++w) sum += s_sum[w];
-    const float inv = 1.0f / sum;
-    // pass 3: the probabilities
-    float *const prob = p.prob + row * p.prob_pitch;
-    softmax_walk(p, row, tid, [&](int64_t k, float w) { prob[k] = fast_exp2(fmaxf(w - M, -127.0f)) * inv; });
 }
 
+// What a chunk leaves for the second launch.  `sum`: weights against max(0, best), so that a row whose values are all far
+// below the floor of 0 adds up the clamped weights as one pass over it would.
+struct HeadRecord {
+    float best;
+    int arg;
+    float sum;
+    float pad;
+};
 
-// SampleFromDistr (cpu_infer.cpp:585-599), the Gumbel-max choice, one workgroup per row:
+__global__ __launch_bounds__(SM_THREADS) void softmax_stats_kernel(HeadParams p)
+{
+    __shared__ float s_max[SM_THREADS / WAVE], s_sum[SM_THREADS / WAVE];
+    __shared__ int s_arg[SM_THREADS / WAVE];
+    const int64_t row = p.row0 + blockIdx.y;
+    const int tid = threadIdx.x;
+    const int64_t begin = (int64_t)blockIdx.x * p.chunk, end = begin + p.chunk < p.n ? begin + p.chunk : p.n;
+    float best = -INFINITY;
+    int arg = 0x7fffffff;
+    softmax_walk(p, row, begin, end, tid, [&](int64_t k, v4f w, int) { // (a single value four times changes nothing)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (w[j] > best) { best = w[j]; arg = (int)k + j; }
+    });
+    first_max(best, arg, s_max, s_arg, tid);
+    float sum = 0.0f;
+    if (p.prob) { // the chunk again, from the nearest cache (one round of it where the rows are few)
+        const float M = fmaxf(0.0f, best);
+        softmax_walk(p, row, begin, end, tid, [&](int64_t, v4f w, int count) {
+            sum += fast_exp2(fmaxf(w.x - M, -127.0f));
+            if (count == 4) sum += fast_exp2(fmaxf(w.y - M, -127.0f)) + fast_exp2(fmaxf(w.z - M, -127.0f)) + fast_exp2(fmaxf(w.w - M, -127.0f));
+        });
+        sum = wave_sum(sum);
+        if ((tid & (WAVE - 1)) == 0) s_sum[tid / WAVE] = sum;
+        __syncthreads();
+        sum = 0.0f;
+        for (int w = 0; w < SM_THREADS / WAVE; ++w) sum += s_sum[w];
+    }
+    if (tid == 0) ((HeadRecord *)p.scratch)[blockIdx.y * gridDim.x + blockIdx.x] = HeadRecord{best, arg, sum, 0.0f};
+}
+
+__global__ __launch_bounds__(SM_THREADS) void softmax_write_kernel(HeadParams p, int n_chunks)
+{
+    const int64_t row = p.row0 + blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+    // every wave merges the row's records for itself
+    const HeadRecord *const rec = (const HeadRecord *)p.scratch + blockIdx.y * n_chunks;
+    float best = -INFINITY, top = 0.0f, sum = 0.0f;
+    int arg = 0x7fffffff;
+    for (int i = lane; i < n_chunks; i += WAVE) {
+        const HeadRecord r = rec[i];
+        if (r.best > best) { best = r.best; arg = r.arg; }
+        const float m = fmaxf(top, r.best);
+        sum = sum * fast_exp2(top - m) + r.sum * fast_exp2(fmaxf(0.0f, r.best) - m);
+        top = m;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const float ob = __shfl_xor(best, o, WAVE), ot = __shfl_xor(top, o, WAVE), os = __shfl_xor(sum, o, WAVE);
+        const int oa = __shfl_xor(arg, o, WAVE);
+        if (ob > best || (ob == best && oa < arg)) { best = ob; arg = oa; }
+        const float m = fmaxf(top, ot);
+        sum = sum * fast_exp2(top - m) + os * fast_exp2(ot - m);
+        top = m;
+    }
+    if (blockIdx.x == 0 && tid == 0 && p.argmax) p.argmax[row] = arg;
+    if (!p.prob) return;
+    const float inv = 1.0f / sum;
+    float *const prob = p.prob + row * p.prob_pitch;
+    const int64_t begin = (int64_t)blockIdx.x * p.chunk, end = begin + p.chunk < p.n ? begin + p.chunk : p.n;
+    softmax_walk(p, row, begin, end, tid, [&](int64_t k, v4f w, int count) {
+        v4f q;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = fast_exp2(fmaxf(w[j] - top, -127.0f)) * inv;
+        if (count == 4) *(v4f_any *)(prob + k) = q;
+        else prob[k] = q.x;
+    });
+}
+
+// SampleFromDistr (cpu_infer.cpp:585-599), the Gumbel-max choice:
 // score[k] = (float)(logf(prob[k]) / temperature - log(-log(u))), u = (r + 0.5) / 2^32 in double (GenRandReal3 of the
 // reference's 32-bit generator); the first k of the largest score above -1e38, else 0.  r: the caller's words, or a
 // 64-bit mix of (seed, offset + row * n + k), the output function of splitmix64 on a counter.
+//
+// Two logarithms in double per value were 80 us for 32 x 50257 values.  Only values that can win need them: a wave scores
+// 1024 values with the single-precision logarithm first, and evaluates exactly those that come within the error of that
+// score of the best so far -- one or two of the 1024.  Rows are cut into chunks as for the softmax.
 __device__ inline uint32_t mix32(uint64_t seed, uint64_t index)
 {
     uint64_t z = seed + (index + 1) * 0x9E3779B97F4A7C15ull;
@@ -144,82 +198,136 @@ __device__ inline uint32_t mix32(uint64_t seed, uint64_t index)
     return (uint32_t)(z >> 32);
 }
 
-__global__ __launch_bounds__(SM_THREADS) void sample_rows_kernel(HeadParams p)
+// The score to within 1e-3 + 1e-5 |log(prob) / temperature|.  -log(u): from u where u is below 1 - 2^-6 (its rounding to
+// float moves log(u) by 4e-6 of itself at most), from the series in 1 - u above (three terms leave 2^-24 of it).
+__device__ inline float rough_score(float prob, uint32_t r, float inv_temperature)
+{
+    const float LN2 = 0.69314718f;
+    const float u = ((float)r + 0.5f) * (1.0f / 4294967296.0f), v = ((float)(~r) + 0.5f) * (1.0f / 4294967296.0f);
+    const float near_one = v * (1.0f + v * (0.5f + v * 0.33333333f)), far = -LN2 * __builtin_amdgcn_logf(u);
+    const float e = v < 0.015625f ? near_one : far;
+    // (the logarithm instruction takes a denormal for zero)
+    const float lp = prob < 1e-30f ? __builtin_amdgcn_logf(prob * 4294967296.0f) - 32.0f : __builtin_amdgcn_logf(prob);
+    return LN2 * (lp * inv_temperature - __builtin_amdgcn_logf(e));
+}
+
+__global__ __launch_bounds__(SM_THREADS) void sample_rows_kernel(HeadParams p, int n_chunks)
 {
     __shared__ float s_max[SM_THREADS / WAVE];
     __shared__ int s_arg[SM_THREADS / WAVE];
-    const int64_t row = blockIdx.x;
+    const int64_t row = p.row0 + blockIdx.y;
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
-    float best = -1e38f;
-    int arg = 0x7fffffff;
-    auto take = [&](int64_t k, float prob, uint32_t r) {
-        const double u = ((double)r + 0.5) * (1.0 / 4294967296.0);
-        const float score = (float)((double)(logf(prob) / p.temperature) - log(-log(u)));
-        if (score > best) { best = score; arg = (int)k; }
-    };
-    // groups of four from the front (16-byte requests, all of a round out before the first is used; a thread sees its k
-    // in ascending order), then the up to three values that are left
+    const int64_t begin = (int64_t)blockIdx.x * p.chunk, end = begin + p.chunk < p.n ? begin + p.chunk : p.n;
     const float *const prob = p.prob + row * p.prob_pitch;
     const uint32_t *const rnd = p.rnd ? p.rnd + row * p.rnd_pitch : nullptr;
-    const int64_t n4 = p.n & ~(int64_t)3;
-    for (int64_t base = 0; base < n4; base += 4 * SM_THREADS * SM_U) {
-        v4f q[SM_U];
-        v4i r[SM_U];
+    const uint64_t counter = p.offset + (uint64_t)(row * p.n);
+    const float inv_t = fminf(1.0f / p.temperature, 3e38f);
+    float best = -1e38f;
+    int arg = 0x7fffffff;
+    constexpr int PER_WAVE = 16 * WAVE;
+    for (int64_t base = begin + wave * PER_WAVE; base < end; base += PER_WAVE * (SM_THREADS / WAVE)) {
+        float q[16];
+        uint32_t r[16];
 #pragma unroll
-        for (int u = 0; u < SM_U; ++u) {
-            const int64_t k = base + 4 * (tid + (int64_t)u * SM_THREADS), kc = k < n4 ? k : n4 - 4;
-            q[u] = *(const v4f_any *)(prob + kc);
-            r[u] = rnd ? (v4i)*(const v4i_any *)(rnd + kc) : v4i{0, 0, 0, 0};
+        for (int j = 0; j < 16; ++j) { // (past the end: the last value again, which changes no maximum)
+            const int64_t k = base + j * WAVE + lane, kc = k < end ? k : end - 1;
+            q[j] = prob[kc];
+            r[j] = rnd ? rnd[kc] : mix32(p.seed, counter + (uint64_t)kc);
         }
+        float top = -INFINITY;
 #pragma unroll
-        for (int u = 0; u < SM_U; ++u) {
-            const int64_t k = base + 4 * (tid + (int64_t)u * SM_THREADS);
-            if (k >= n4) continue;
-            const float qq[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
-            const int rr[4] = {r[u].x, r[u].y, r[u].z, r[u].w};
+        for (int j = 0; j < 16; ++j) {
+            q[j] = rough_score(q[j], r[j], inv_t);
+            top = fmaxf(top, q[j]);
+        }
+        // the best of the wave so far, exact or rough, less the error both may have
+        top = wave_max(fmaxf(top, best));
+        const float bound = top - (2e-3f + 2e-5f * (fminf(fabsf(top), 1e30f) + 64.0f));
+        uint32_t todo = 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                take(k + j, qq[j], rnd ? (uint32_t)rr[j] : mix32(p.seed, p.offset + (uint64_t)(row * p.n + k + j)));
+        for (int j = 0; j < 16; ++j)
+            if (q[j] >= bound && base + j * WAVE + lane < end) todo |= 1u << j;
+        while (todo) {
+            const int j = __ffs(todo) - 1;
+            todo &= todo - 1;
+            const int64_t k = base + j * WAVE + lane;
+            const uint32_t word = rnd ? rnd[k] : mix32(p.seed, counter + (uint64_t)k);
+            const double u = ((double)word + 0.5) * (1.0 / 4294967296.0);
+            const float score = (float)((double)(logf(prob[k]) / p.temperature) - log(-log(u)));
+            if (score > best) { best = score; arg = (int)k; } // (a thread's k ascend)
         }
     }
-    if (n4 + tid < p.n) {
-        const int64_t k = n4 + tid;
-        take(k, prob[k], rnd ? rnd[k] : mix32(p.seed, p.offset + (uint64_t)(row * p.n + k)));
+    first_max(best, arg, s_max, s_arg, tid);
+    if (tid != 0) return;
+    if (n_chunks > 1) ((HeadRecord *)p.scratch)[blockIdx.y * n_chunks + blockIdx.x] = HeadRecord{best, arg, 0.0f, 0.0f};
+    else p.argmax[row] = arg == 0x7fffffff ? 0 : arg;
+}
+
+// one wave per row: the chunks' choices
+__global__ __launch_bounds__(WAVE) void sample_merge_kernel(HeadParams p, int n_chunks)
+{
+    const int64_t row = p.row0 + blockIdx.x;
+    const int lane = threadIdx.x;
+    const HeadRecord *const rec = (const HeadRecord *)p.scratch + (int64_t)blockIdx.x * n_chunks;
+    float best = -1e38f;
+    int arg = 0x7fffffff;
+    for (int i = lane; i < n_chunks; i += WAVE) {
+        const HeadRecord r = rec[i];
+        if (r.best > best) { best = r.best; arg = r.arg; }
     }
     for (int o = 32; o > 0; o >>= 1) {
         const float ob = __shfl_xor(best, o, WAVE);
         const int oa = __shfl_xor(arg, o, WAVE);
         if (ob > best || (ob == best && oa < arg)) { best = ob; arg = oa; }
     }
-    if (lane == 0) { s_max[wave] = best; s_arg[wave] = arg; }
-    __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < SM_THREADS / WAVE; ++w) {
-            if (s_max[w] > best || (s_max[w] == best && s_arg[w] < arg)) { best = s_max[w]; arg = s_arg[w]; }
-        }
-        p.argmax[row] = arg == 0x7fffffff ? 0 : arg;
-    }
+    if (lane == 0) p.argmax[row] = arg == 0x7fffffff ? 0 : arg;
 }
+
+// How many workgroups share each of `rows` rows, and the values each takes: one round's worth each as long as the rows
+// are few, at most about four workgroups per compute unit in all and no more records than the scratch holds.  A row of
+// one chunk needs no second launch to sample.
+static int head_chunks(HeadParams &p, int64_t rows)
+{
+    int64_t chunks = (p.n + SM_CHUNK - 1) / SM_CHUNK;
+    chunks = chunks < 1024 / rows ? chunks : 1024 / rows;
+    chunks = chunks < 1 ? 1 : chunks;
+    p.chunk = ((p.n + chunks - 1) / chunks + 3) & ~(int64_t)3;
+    return (int)((p.n + p.chunk - 1) / p.chunk);
+}
+static_assert(HEAD_SCRATCH_BYTES >= 1024 * (int)sizeof(HeadRecord), "a record per workgroup");
+constexpr int64_t HEAD_ROWS = HEAD_SCRATCH_BYTES / (int64_t)sizeof(HeadRecord); // rows per launch
 
 hipError_t launch_embed_rows(const HeadParams &p, hipStream_t st)
 {
-    const int64_t n = p.n_rows * (p.dim / 16);
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(embed_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
-    return hipGetLastError();
-}
-
-hipError_t launch_softmax_rows(const HeadParams &p, hipStream_t st)
-{
-    if (p.n_rows == 0 || p.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(softmax_rows_kernel, dim3((unsigned)p.n_rows), dim3(SM_THREADS), 0, st, p);
-    return hipGetLastError();
-}
-
-hipError_t launch_sample_rows(const HeadParams &p, hipStream_t st)
-{
     if (p.n_rows == 0) return hipSuccess;
-    hipLaunchKernelGGL(sample_rows_kernel, dim3((unsigned)p.n_rows), dim3(SM_THREADS), 0, st, p);
+    const int64_t blocks = p.n_rows * ((p.dim / 4 + 255) / 256);
+    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(embed_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_softmax_rows(const HeadParams &params, hipStream_t st)
+{
+    HeadParams p = params;
+    if (p.n == 0) return hipSuccess;
+    for (p.row0 = 0; p.row0 < p.n_rows; p.row0 += HEAD_ROWS) {
+        const int64_t rows = p.n_rows - p.row0 < HEAD_ROWS ? p.n_rows - p.row0 : HEAD_ROWS;
+        const int chunks = head_chunks(p, rows);
+        hipLaunchKernelGGL(softmax_stats_kernel, dim3((unsigned)chunks, (unsigned)rows), dim3(SM_THREADS), 0, st, p);
+        hipLaunchKernelGGL(softmax_write_kernel, dim3(p.prob ? (unsigned)chunks : 1, (unsigned)rows), dim3(SM_THREADS), 0, st, p, chunks);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_sample_rows(const HeadParams &params, hipStream_t st)
+{
+    HeadParams p = params;
+    for (p.row0 = 0; p.row0 < p.n_rows; p.row0 += HEAD_ROWS) {
+        const int64_t rows = p.n_rows - p.row0 < HEAD_ROWS ? p.n_rows - p.row0 : HEAD_ROWS;
+        const int chunks = head_chunks(p, rows);
+        hipLaunchKernelGGL(sample_rows_kernel, dim3((unsigned)chunks, (unsigned)rows), dim3(SM_THREADS), 0, st, p, chunks);
+        if (chunks > 1) hipLaunchKernelGGL(sample_merge_kernel, dim3((unsigned)rows), dim3(WAVE), 0, st, p, chunks);
+    }
     return hipGetLastError();
 }
 
