@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/tsattn.h"
+#include "kernels.hpp"
 
 namespace tsattn {
 
@@ -95,6 +96,50 @@ __device__ inline int dpp_xor1(int v) { return dpp_mov<0xB1>(v); }        // qua
 __device__ inline int dpp_xor2(int v) { return dpp_mov<0x4E>(v); }        // quad_perm [2,3,0,1]
 __device__ inline int dpp_half_mirror(int v) { return dpp_mov<0x141>(v); } // lane i <-> 7-i in each 8
 __device__ inline int dpp_mirror(int v) { return dpp_mov<0x140>(v); }      // lane i <-> 15-i in each 16
+
+// A thread's share of a residual update: groups of four, `threads` apart; the first is requested before and stored after
+// whatever the kernel does in between.  delta * scale is rounded before it is added (two statements in the reference).
+struct ResidUpdate {
+    v4f st;
+    v4i part[4];
+    int first, step;
+    __device__ __forceinline__ void load(const UpdateParams &u, int j)
+    {
+        const int per_row = u.dim / 4, row = j / per_row, x = (j - row * per_row) * 4;
+        st = *(const v4f *)(u.state + row * u.state_pitch + x);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) // (planes that are not there: the last one again)
+            part[i] = *(const v4i *)(u.src + (i < u.planes ? i : u.planes - 1) * u.src_stride + (int64_t)row * u.dim + x);
+    }
+    __device__ __forceinline__ void store(const UpdateParams &u, int j)
+    {
+#pragma clang fp contract(off)
+        const int per_row = u.dim / 4, row = j / per_row, x = (j - row * per_row) * 4;
+        v4i a = part[0];
+#pragma unroll
+        for (int i = 1; i < 4; ++i)
+            if (i < u.planes) a += part[i];
+        v4f d = v4f{(float)a.x, (float)a.y, (float)a.z, (float)a.w};
+        d = v4f{d.x * u.scale, d.y * u.scale, d.z * u.scale, d.w * u.scale};
+        *(v4f *)(u.state + row * u.state_pitch + x) = v4f{st.x + d.x, st.y + d.y, st.z + d.z, st.w + d.w};
+    }
+    __device__ __forceinline__ void request(const UpdateParams &u, int index, int threads)
+    {
+        first = index;
+        step = threads;
+        if (u.state && first < u.rows * u.dim / 4) load(u, first);
+    }
+    __device__ __forceinline__ void finish(const UpdateParams &u)
+    {
+        if (!u.state) return;
+        const int total = u.rows * u.dim / 4;
+        if (first < total) store(u, first);
+        for (int j = first + step; j < total; j += step) {
+            load(u, j);
+            store(u, j);
+        }
+    }
+};
 
 __device__ inline float wave_max(float v)
 {

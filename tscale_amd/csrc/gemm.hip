@@ -3,9 +3,8 @@
 // MulForward (gpt/train/cpu_infer.cpp:294-305: one weight row per output, exact int32 sums, result as int32 or
 // converted to float) and AddScaled (:308-316: state += delta * scale).
 //
-// Two kernels.  Many rows (a prompt): 128 x 128 output tiles, K in steps of 64 bytes through LDS, four waves of
-// 64 x 64 each, v_mfma_i32_32x32x32_i8; bound by the matrix cores.  Few rows (one token per sequence): the
-// weights are read once from HBM, 32 weight rows per workgroup with K split over its four waves; bound by HBM.
+// Many rows (a prompt): 128 x 128 or 256 x 256 output tiles, K in steps of 64 bytes through LDS,
+// v_mfma_i32_32x32x32_i8; bound by the matrix cores.  Few rows (one token per sequence): gemm_few.hpp.
 // Integer sums are exact, so every decomposition gives the same bits.
 #include <type_traits>
 #include "common.hpp"
@@ -488,121 +487,6 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
     }
 }
 
-// ---- few rows ---------------------------------------------------------------------------------------------------
-// One workgroup per 32 weight rows and part of K.  K is walked in slabs of 1024 bytes: every wave instruction asks
-// for 1 KiB of consecutive memory of one row (the weights are read once, so what matters is that HBM sees long
-// consecutive requests and that many are in flight), the slab goes through LDS, and there the rows are read back the
-// way the MFMA wants them (32 bytes of a row per lane and step).  The four waves each take a quarter of the slab
-// and add their sums up in LDS.
-constexpr int GS_THREADS = 256;
-constexpr int GS_WAVES = GS_THREADS / WAVE;
-constexpr int GS_BN = 32;      // weight rows per workgroup
-constexpr int GS_MB = 4;       // blocks of 32 activation rows handled by this kernel
-constexpr int GS_SLAB = 1024;  // bytes of K per slab
-constexpr int GS_PITCH = GS_SLAB + 16;
-constexpr int GS_LD = 32 * GS_SLAB / 16 / GS_THREADS; // 16-byte chunks per thread and slab: 8
-
-template <int MODE>
-__global__ __launch_bounds__(GS_THREADS) void gemm_skinny_kernel(GemmParams p)
-{
-    __shared__ __attribute__((aligned(16))) uint8_t w_lds[32 * GS_PITCH];
-    __shared__ __attribute__((aligned(16))) uint8_t x_lds[32 * GS_PITCH];
-    static_assert(GS_MB * 16 * WAVE * 4 <= 32 * GS_PITCH, "the waves' sums are added up in the activations' slab");
-    int(*red)[16 * WAVE] = (int(*)[16 * WAVE]) x_lds;
-    const int tid = threadIdx.x;
-    const int lane = tid & (WAVE - 1);
-    const int wave = tid / WAVE;
-    const int li = lane & 31, g = lane >> 5;
-    const int64_t n0 = (int64_t)blockIdx.x * GS_BN;
-
-    // this workgroup's part of K (blockIdx.y of gridDim.y parts, in whole steps of 64 bytes); with more than one
-    // part the sums go to this part's plane of the workspace
-    const int all_steps = (int)(p.k / 64);
-    const int split_steps = (all_steps + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int k_begin = (int)blockIdx.y * split_steps * 64, k_end = min(all_steps, ((int)blockIdx.y + 1) * split_steps) * 64;
-    p.out = (uint8_t *)p.out + (int64_t)blockIdx.y * p.split_stride * 4;
-
-    const int n_mb = (int)((p.m + 31) / 32);
-    const __amdgpu_buffer_rsrc_t wr = rows_rsrc(p.w + n0 * p.w_pitch, p.n - n0 < GS_BN ? p.n - n0 : GS_BN, p.w_pitch, p.k);
-    const __amdgpu_buffer_rsrc_t ar = rows_rsrc(p.a, p.m, p.a_pitch, p.k);
-    // chunk i of this thread: row 4*i + wave, bytes 16*lane.. of the slab: one wave instruction = one row's KiB
-    v16i acc[GS_MB];
-#pragma unroll
-    for (int j = 0; j < GS_MB; ++j) acc[j] = v16i{0};
-
-    // the weights of a slab are requested while the slab before it is being multiplied
-    auto request_w = [&](int kb, v4i (&dst)[GS_LD]) __attribute__((always_inline)) {
-        const bool in_slab = 16 * lane < min(GS_SLAB, k_end - kb);
-#pragma unroll
-        for (int i = 0; i < GS_LD; ++i) {
-            const int row = 4 * i + wave;
-            dst[i] = in_slab ? __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, row * (int)p.w_pitch + 16 * lane, kb, 0)) : v4i{0, 0, 0, 0};
-        }
-    };
-    v4i rw[GS_LD], rw_next[GS_LD];
-    if (k_begin < k_end) request_w(k_begin, rw);
-    for (int kb = k_begin; kb < k_end; kb += GS_SLAB) {
-        const int slab = min(GS_SLAB, k_end - kb); // bytes of K in this slab, a multiple of 64
-        const bool in_slab = 16 * lane < slab;
-        const bool more = kb + GS_SLAB < k_end;
-#pragma unroll
-        for (int j = 0; j < GS_MB; ++j) {
-            if (j < n_mb) { // uniform
-                v4i rx[GS_LD];
-#pragma unroll
-                for (int i = 0; i < GS_LD; ++i) {
-                    const int row = 32 * j + 4 * i + wave;
-                    rx[i] = in_slab ? __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ar, row * (int)p.a_pitch + 16 * lane, kb, 0)) : v4i{0, 0, 0, 0};
-                }
-                if (j == 0 && more) request_w(kb + GS_SLAB, rw_next);
-                __syncthreads(); // the previous block's reads of x_lds (and, for j == 0, of w_lds) are done
-                if (j == 0) {
-#pragma unroll
-                    for (int i = 0; i < GS_LD; ++i) *(v4i *)(w_lds + (4 * i + wave) * GS_PITCH + 16 * lane) = rw[i];
-                }
-#pragma unroll
-                for (int i = 0; i < GS_LD; ++i) *(v4i *)(x_lds + (4 * i + wave) * GS_PITCH + 16 * lane) = rx[i];
-                __syncthreads();
-                // this wave's quarter of the slab: steps 4*wave .. 4*wave+3 (those inside the slab)
-                const uint8_t *wb = w_lds + li * GS_PITCH + 32 * g, *xb = x_lds + li * GS_PITCH + 32 * g;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int off = (4 * wave + u) * 64;
-                    if (off < slab) { // uniform
-                        const v4i w0 = *(const v4i *)(wb + off), w1 = *(const v4i *)(wb + off + 16);
-                        const v4i x0 = *(const v4i *)(xb + off), x1 = *(const v4i *)(xb + off + 16);
-                        acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w0, x0, acc[j], 0, 0, 0);
-                        acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w1, x1, acc[j], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < GS_LD; ++i) rw[i] = rw_next[i];
-        }
-    }
-    // sum the waves' shares in LDS; register r of block j: weight row n0 + 8*(r/4) + 4*g + r%4, activation row 32*j + li
-    __syncthreads(); // the slab has been read
-    for (int i = tid; i < GS_MB * 16 * WAVE; i += GS_THREADS) (&red[0][0])[i] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < GS_MB; ++j) {
-        if (j < n_mb) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) atomicAdd(&red[j][r * WAVE + lane], acc[j][r]);
-        }
-    }
-    __syncthreads();
-    for (int r = wave; r < 16; r += GS_WAVES) {
-        const int64_t n = n0 + 8 * (r / 4) + 4 * g + (r & 3);
-        for (int j = 0; j < n_mb; ++j) {
-            const int64_t m = 32 * j + li;
-            if (n < p.n && m < p.m) store_out<MODE>(p, m, n, red[j][r * WAVE + lane]);
-        }
-    }
-}
-
 // sums the planes of the workspace and applies the epilogue: one thread per output element
 template <int MODE>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p, const int32_t *ws, int n_split)
@@ -617,29 +501,20 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p, const in
 template <int MODE>
 void launch_mode(const GemmParams &p, hipStream_t st)
 {
-    if (p.m > 32 * GS_MB) {
-        // wide tiles when there are two rounds of them for every compute unit, 128 x 128 tiles otherwise
-        const int64_t tiles_n = (p.n + GT_BN - 1) / GT_BN;
-        const int64_t wide = ((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN);
-        if (wide >= 512) hipLaunchKernelGGL((gemm_wide_kernel<MODE, 0>), dim3((unsigned)wide), dim3(GW_THREADS), GW_LDS_BYTES, st, p);
-        else hipLaunchKernelGGL((gemm_tiled_kernel<MODE, 2>), dim3((unsigned)(((p.m + 127) / 128) * tiles_n)), dim3(GT_THREADS), 0, st, p);
-        return;
-    }
-    hipLaunchKernelGGL((gemm_skinny_kernel<MODE>), dim3((unsigned)((p.n + GS_BN - 1) / GS_BN), 1), dim3(GS_THREADS), 0, st, p);
+    // wide tiles when there are two rounds of them for every compute unit, 128 x 128 tiles otherwise
+    const int64_t tiles_n = (p.n + GT_BN - 1) / GT_BN;
+    const int64_t wide = ((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN);
+    if (wide >= 512) hipLaunchKernelGGL((gemm_wide_kernel<MODE, 0>), dim3((unsigned)wide), dim3(GW_THREADS), GW_LDS_BYTES, st, p);
+    else hipLaunchKernelGGL((gemm_tiled_kernel<MODE, 2>), dim3((unsigned)(((p.m + 127) / 128) * tiles_n)), dim3(GT_THREADS), 0, st, p);
 }
 
-// Few rows: the weights are streamed once and every compute unit has to help.  With 32 weight rows per workgroup
-// there are too few workgroups unless K is split as well, which needs room for the parts' sums.  A workgroup walks
-// its slabs with the next one's weights on their way, so parts of two and more slabs cost little more than parts of
-// one: about one workgroup per compute unit (measured: 1.86 ms per token step of 24 layers against 1.89 with twice as
-// many parts and 1.92 with half as many).
-int split_for(const GemmParams &p, int64_t room_bytes)
+FewParams few_params(const GemmParams &p)
 {
-    if (p.m > 32 * GS_MB) return 1;
-    const int64_t n_tiles = (p.n + GS_BN - 1) / GS_BN;
-    int split = 1;
-    while (split < 16 && n_tiles * split < 256 && p.k / (split * 2) >= GS_SLAB && (int64_t)(split * 2) * p.m * p.n * 4 <= room_bytes) split *= 2;
-    return split;
+    FewParams f = {};
+    f.w = p.w; f.w_pitch = p.w_pitch; f.m = p.m; f.n = p.n; f.k = p.k; f.a = p.a; f.a_pitch = p.a_pitch;
+    f.mode = p.mode == TSATTN_MM_I32_PLANES ? TSATTN_MM_I32 : p.mode;
+    f.scale = p.scale; f.out = p.out; f.out_pitch = p.out_pitch; f.parts = 1;
+    return f;
 }
 
 } // namespace
@@ -659,7 +534,7 @@ hipError_t prepare_matmul_i8()
         const hipError_t e = hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds);
         if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    return prepare_gemm_few();
 }
 
 hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out)
@@ -668,51 +543,58 @@ hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out
         if (planes_out) *planes_out = 1;
         return hipSuccess;
     }
+    const bool few = p.m <= FEW_ROWS;
     if (p.mode == TSATTN_MM_I32_PLANES) {
-        // the parts' sums straight into the caller's planes (16 * m * n ints of room by contract)
-        const int split = split_for(p, (int64_t)16 * p.m * p.n * 4);
+        // the parts' sums straight into the caller's planes (with few rows 16 * m * n ints of room by contract)
+        FewParams f = few_params(p);
+        if (few) f.parts = few_parts(f, 16);
+        f.out_stride = p.m * p.n;
+        *planes_out = f.parts;
         GemmParams q = p;
-        q.split_stride = p.m * p.n;
         if (p.ep_head_dim) {
             // the producer on the result: in the product's own kernel where the wide tiles are used, else after it
             q.ep.src = p.out; q.ep.src_pitch = p.n; q.ep.n_rows = p.m; q.ep.n_heads = (int)(p.n / p.ep_head_dim);
-            q.ep.src_planes = split; q.ep.src_plane_stride = p.m * p.n;
-            *planes_out = split;
+            q.ep.src_planes = f.parts; q.ep.src_plane_stride = p.m * p.n;
             const int64_t wide = ((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN);
             // (the epilogue addresses a tile's rows with 32-bit offsets)
             const bool offsets_fit = q.ep.dst_pitch < (1 << 23) && (!q.ep.resid || q.ep.resid_pitch < (1 << 21)) &&
                                      (!q.ep.pos || q.ep.rope_len * p.ep_head_dim * 4 < ((int64_t)1 << 31));
             const bool one_operand = !(q.ep.resid && q.ep.pos); // (registers for the old state or for cos and sin)
             const bool head_group = p.ep_head_dim == 64 || p.ep_head_dim == 128; // (wider groups: the producer's own launch)
-            if (p.m > 32 * GS_MB && wide >= 512 && p.ep_dst_dtype == TSATTN_I8 && offsets_fit && one_operand && head_group) {
+            if (!few && wide >= 512 && p.ep_dst_dtype == TSATTN_I8 && offsets_fit && one_operand && head_group) {
                 if (p.ep_head_dim == 128) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 128>), dim3((unsigned)wide), dim3(GW_THREADS), gw_lds_bytes(128), st, q);
                 else hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 64>), dim3((unsigned)wide), dim3(GW_THREADS), gw_lds_bytes(64), st, q);
                 return hipGetLastError();
             }
-            if (split == 1) launch_mode<TSATTN_MM_I32>(q, st);
-            else hipLaunchKernelGGL((gemm_skinny_kernel<TSATTN_MM_I32>), dim3((unsigned)((p.n + GS_BN - 1) / GS_BN), (unsigned)split), dim3(GS_THREADS), 0, st, q);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-            return launch_rope_normalize(q.ep, p.ep_dst_dtype, p.ep_head_dim, true, st);
         }
-        if (split == 1) launch_mode<TSATTN_MM_I32>(q, st);
-        else hipLaunchKernelGGL((gemm_skinny_kernel<TSATTN_MM_I32>), dim3((unsigned)((p.n + GS_BN - 1) / GS_BN), (unsigned)split), dim3(GS_THREADS), 0, st, q);
-        *planes_out = split;
-        return hipGetLastError();
+        hipError_t e = hipSuccess;
+        if (few) {
+            e = launch_gemm_few(f, st);
+        } else {
+            launch_mode<TSATTN_MM_I32>(q, st);
+            e = hipGetLastError();
+        }
+        if (e != hipSuccess || !p.ep_head_dim) return e;
+        return launch_rope_normalize(q.ep, p.ep_dst_dtype, p.ep_head_dim, true, st);
     }
-    const int split = split_for(p, p.workspace ? p.workspace_bytes : 0);
-    if (split > 1) {
-        GemmParams q = p;
-        q.out = p.workspace;
-        q.out_pitch = p.n;
-        q.split_stride = p.m * p.n;
-        hipLaunchKernelGGL((gemm_skinny_kernel<TSATTN_MM_I32>), dim3((unsigned)((p.n + GS_BN - 1) / GS_BN), (unsigned)split), dim3(GS_THREADS), 0, st, q);
+    if (few) {
+        FewParams f = few_params(p);
+        // Parts through the caller's workspace and a second launch that adds them up: where the weights would otherwise
+        // come in through a few compute units only (an eighth of them).
+        const int64_t room = p.workspace ? p.workspace_bytes / (p.m * p.n * 4) : 0;
+        if (room < 2 || (p.n + 15) / 16 >= 32) return launch_gemm_few(f, st);
+        f.mode = TSATTN_MM_I32;
+        f.parts = few_parts(f, room >= 16 ? 16 : room >= 8 ? 8 : room >= 4 ? 4 : 2);
+        if (f.parts == 1) return launch_gemm_few(few_params(p), st);
+        f.out = p.workspace; f.out_pitch = p.n; f.out_stride = p.m * p.n;
+        const hipError_t e = launch_gemm_few(f, st);
+        if (e != hipSuccess) return e;
         GemmParams r = p;
         r.split_stride = p.m * p.n;
         const dim3 grid((unsigned)((p.m * p.n + 255) / 256));
-        if (p.mode == TSATTN_MM_I32) hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_I32>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, split);
-        else if (p.mode == TSATTN_MM_F32) hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_F32>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, split);
-        else hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_ADD_SCALED>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, split);
+        if (p.mode == TSATTN_MM_I32) hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_I32>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, f.parts);
+        else if (p.mode == TSATTN_MM_F32) hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_F32>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, f.parts);
+        else hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_ADD_SCALED>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, f.parts);
         return hipGetLastError();
     }
     if (p.mode == TSATTN_MM_I32) launch_mode<TSATTN_MM_I32>(p, st);

@@ -8,6 +8,31 @@
 
 namespace tsattn {
 
+// A residual update that rides along in a launch: state += sum of the planes * scale, dim columns of rows rows
+struct UpdateParams {
+    float *state; // null: none
+    int64_t state_pitch;
+    const int32_t *src;
+    int planes; // 1..4, [rows][dim], src_stride apart
+    int64_t src_stride;
+    int rows, dim;
+    float scale;
+};
+
+// The step that makes a token's attention operands, done by the attention launch itself: q, the new key and value rows
+// and the key of KVProduct are heads of the projections' int32 planes [n_seqs][4 n_heads d] (qk, qv, k, v one after the other)
+struct FrontParams {
+    const int32_t *src; // null: the operands are in memory
+    int planes;         // 1..4
+    int64_t src_stride;
+    const int32_t *pos;
+    const float *rope;
+    int64_t rope_len;
+    float key_mult, vec_scale;
+    uint8_t *k_row; // [n_seqs][n_heads d]: the key of KVProduct for the merge launch
+    UpdateParams upd;
+};
+
 struct DecodeParams {
     const uint8_t *q;
     int64_t q_pitch;
@@ -43,6 +68,7 @@ struct DecodeParams {
     int64_t kv_out_pitch;
     int kv_rep;
     float kv_mult;
+    FrontParams front;
 };
 
 hipError_t launch_decode(const DecodeParams &p, int dtype, int head_dim, bool qbf16, int n_seqs, float *out, hipStream_t st);
@@ -195,6 +221,37 @@ struct GemmParams {
     ProduceParams ep;
     int ep_head_dim, ep_dst_dtype;
 };
+
+// The product with at most FEW_ROWS activation rows (gemm_few.hpp); the launcher fills in everything below `parts`.
+constexpr int FEW_ROWS = 128;
+constexpr int FEW_NORM_ROWS = 16; // ... when the kernel normalises the activations itself (see gemm_few.hip)
+struct FewParams {
+    const uint8_t *w;
+    int64_t w_pitch;
+    int64_t m, n, k;
+    int mode; // TSATTN_MM_I32 (planes, out_stride apart), _F32 or _ADD_SCALED (one part)
+    float scale;
+    void *out;
+    int64_t out_pitch, out_stride;
+    // activations: int8 rows, or (a null) the normalisation of src_planes int32 planes [m][k], src_stride apart, and / or
+    // the f32 state they update by resid_scale, in groups of `group` values
+    const uint8_t *a;
+    int64_t a_pitch;
+    const int32_t *src;
+    int src_planes;
+    int64_t src_stride;
+    const float *state;
+    int64_t state_pitch;
+    float resid_scale, vec_scale;
+    int group, relu;
+    UpdateParams upd; // (sources of planes alone)
+    int parts; // parts of K, one plane of the result each
+    int wn, wn_log, wk, wk_log, k_part, k_chunk, groups, walk, group_log;
+};
+bool few_source_ok(const FewParams &p);              // whether the kernel can normalise this source itself
+int few_parts(const FewParams &p, int max_parts);    // how many parts K is best cut into, at most max_parts
+hipError_t launch_gemm_few(const FewParams &p, hipStream_t st);
+hipError_t prepare_gemm_few(); // once per device
 
 hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out);
 hipError_t prepare_matmul_i8(); // once per device, before the first product

@@ -4,10 +4,10 @@
 // operation: the same float products, the sum of squares taken in index order, no fused multiply-adds, so the
 // bytes and scales are identical to a CPU evaluation in that order.
 //
-// A workgroup takes 32 (8 in a small launch) consecutive (row, head) pairs.  The rotated values go to LDS (row pitch d+1 floats, so
+// A workgroup takes 32 consecutive (row, head) pairs.  The rotated values go to LDS (row pitch d+1 floats, so
 // that 32 lanes walking 32 different pairs in step hit 32 different banks); then lane j of the first wave sums
 // pair j's squares one after the other, which keeps the summation order while 32 sums advance together; then
-// all threads convert and write the bytes out, sixteen per thread, consecutively.
+// all threads convert and write the bytes out, sixteen per thread, consecutively.  Few pairs: see normalize_few_kernel.
 #include <math.h>
 
 #include "common.hpp"
@@ -16,7 +16,7 @@
 namespace tsattn {
 
 constexpr int PR_PAIRS = 32;       // (row, head) pairs per workgroup
-constexpr int PR_PAIRS_FEW = 8;    // ... of a small launch: more workgroups, each with less to wait for
+constexpr int64_t PR_FEW = 4096;   // up to this many pairs one wave each takes a few
 
 // every float operation below is meant as written: no fused multiply-adds
 #pragma clang fp contract(off)
@@ -169,19 +169,150 @@ __global__ __launch_bounds__(256) void rope_normalize_kernel(ProduceParams p)
     }
 }
 
+// The same for few pairs (one token per sequence), where a launch is a chain of waits: one wave per 64 / (D / 8) pairs, a
+// lane holds eight values (four couples x, x + 32), squares go through the wave's LDS to the lane that adds its pair's up in
+// index order -- additions only, one instruction per value -- and the multiplier comes back through a lane exchange: no
+// barrier, no second pass over the values.  32 x 2048, two planes and the residual update: 5.6 us with workgroups of 256
+// threads and three barriers.
+template <int D, int DST, bool SRC_I32>
+__global__ __launch_bounds__(WAVE) void normalize_few_kernel(ProduceParams p)
+{
+    constexpr int LPP = D / 8, PAIRS = WAVE / LPP; // lanes per pair, pairs per wave
+    constexpr int PITCH = D + 4;
+    __shared__ __attribute__((aligned(16))) float squares[PAIRS * PITCH];
+    const int lane = threadIdx.x;
+    const int pr = lane / LPP, c = lane % LPP;
+    const uint32_t pair = blockIdx.x * PAIRS + pr, n_pairs = (uint32_t)p.n_rows * (uint32_t)p.n_heads;
+    const bool mine = pr < PAIRS && pair < n_pairs;
+    const uint32_t pc = mine ? pair : n_pairs - 1;
+    const int64_t row = pc / (uint32_t)p.n_heads;
+    const int head = (int)(pc % (uint32_t)p.n_heads);
+    const int x0 = (c / 8) * 64 + (c % 8) * 4;
+    v4f v0, v1;
+    v4f u0, u1, cs, sn;
+    const int64_t e = row * p.src_pitch + (int64_t)head * D + x0;
+    float *const resid = p.resid + row * p.resid_pitch + (int64_t)head * D + x0;
+    if (SRC_I32) {
+        constexpr int PL = 4; // planes asked for together (those that are not there: the last one again)
+        const int32_t *const src = (const int32_t *)p.src + e;
+        v4i a = v4i{0, 0, 0, 0}, b = v4i{0, 0, 0, 0};
+        for (int p0 = 0; p0 < p.src_planes; p0 += PL) {
+            v4i qa[PL], qb[PL];
+#pragma unroll
+            for (int i = 0; i < PL; ++i) {
+                const int32_t *const q = src + (p0 + i < p.src_planes ? p0 + i : p.src_planes - 1) * p.src_plane_stride;
+                qa[i] = *(const v4i *)q;
+                qb[i] = *(const v4i *)(q + 32);
+            }
+            if (p0 == 0 && p.resid) {
+                u0 = *(const v4f *)resid;
+                u1 = *(const v4f *)(resid + 32);
+            }
+#pragma unroll
+            for (int i = 0; i < PL; ++i)
+                if (p0 + i < p.src_planes) { a += qa[i]; b += qb[i]; }
+        }
+        v0 = v4f{(float)a.x, (float)a.y, (float)a.z, (float)a.w};
+        v1 = v4f{(float)b.x, (float)b.y, (float)b.z, (float)b.w};
+    } else {
+        v0 = *(const v4f *)((const float *)p.src + e);
+        v1 = *(const v4f *)((const float *)p.src + e + 32);
+        if (p.resid) {
+            u0 = *(const v4f *)resid;
+            u1 = *(const v4f *)(resid + 32);
+        }
+    }
+    if (p.resid) {
+        v0 = u0 + v0 * p.resid_scale;
+        v1 = u1 + v1 * p.resid_scale;
+        if (mine) {
+            *(v4f *)resid = v0;
+            *(v4f *)(resid + 32) = v1;
+        }
+    }
+    if (p.pos) {
+        int t = p.pos[row];
+        t = t < 0 ? 0 : (t >= p.rope_len ? (int)p.rope_len - 1 : t);
+        const float *const rr = p.rope + (int64_t)t * D + x0;
+        cs = *(const v4f *)rr;
+        sn = *(const v4f *)(rr + 32);
+        const bool turn = head < p.rope_heads; // (the other heads turn by the identity)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float cos_value = turn ? cs[i] : 1.0f;
+            const float sin_value = turn ? sn[i] * p.rotate_dir : 0.0f;
+            const float r0 = v0[i] * cos_value - v1[i] * sin_value;
+            const float r1 = v0[i] * sin_value + v1[i] * cos_value;
+            v0[i] = r0;
+            v1[i] = r1;
+        }
+    }
+    if (pr < PAIRS) {
+        *(v4f *)(squares + pr * PITCH + x0) = v0 * v0;
+        *(v4f *)(squares + pr * PITCH + x0 + 32) = v1 * v1;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (one wave: its LDS accesses are in order)
+    float mult = 0.0f;
+    if (lane < PAIRS) {
+        const float *const v = squares + lane * PITCH;
+        float sum2 = 0.0f;
+#pragma unroll 4
+        for (int x = 0; x < D; x += 32) {
+            v4f q[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) q[i] = *(const v4f *)(v + x + 4 * i);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                sum2 = sum2 + q[i].x;
+                sum2 = sum2 + q[i].y;
+                sum2 = sum2 + q[i].z;
+                sum2 = sum2 + q[i].w;
+            }
+        }
+        float discr = 0.0f;
+        if (sum2 != 0.0f) { // the root: see rope_normalize_kernel
+            discr = (float)sqrt((double)(sum2 / (float)D)) * p.vec_scale;
+            mult = 1.0f / discr;
+        }
+        const uint32_t q = blockIdx.x * PAIRS + lane;
+        if (p.scale && q < n_pairs) {
+            const int sh = (int)(q % (uint32_t)p.n_heads) - p.scale_head_begin;
+            if (sh >= 0 && sh < p.scale_head_count) p.scale[sh * p.scale_pitch + (int64_t)(q / (uint32_t)p.n_heads) * p.scale_row_stride] = discr * p.scale_mult;
+        }
+    }
+    mult = __shfl(mult, pr < PAIRS ? pr : 0, WAVE);
+    if (!mine) return;
+    uint32_t w0, w1;
+    if (DST == TSATTN_I8) {
+        const float low = p.relu ? 0.0f : -127.0f;
+        w0 = pack_i8x4(v0.x * mult, v0.y * mult, v0.z * mult, v0.w * mult, low);
+        w1 = pack_i8x4(v1.x * mult, v1.y * mult, v1.z * mult, v1.w * mult, low);
+    } else {
+        w0 = w1 = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { // (a head of zeros is zero bytes whatever the signs of its zeros)
+            w0 |= (mult == 0.0f ? 0u : (uint32_t)float_to_e4m3(v0[i] * mult)) << (8 * i);
+            w1 |= (mult == 0.0f ? 0u : (uint32_t)float_to_e4m3(v1[i] * mult)) << (8 * i);
+        }
+    }
+    uint8_t *const dst = p.dst + row * p.dst_pitch + (int64_t)head * D + x0;
+    *(uint32_t *)dst = w0;
+    *(uint32_t *)(dst + 32) = w1;
+}
+
 hipError_t launch_rope_normalize(const ProduceParams &p, int dst_dtype, int head_dim, bool src_i32, hipStream_t st)
 {
     const int64_t n_pairs = p.n_rows * p.n_heads;
     if (n_pairs == 0) return hipSuccess;
-    // a small launch (one token per sequence) is a chain of waits -- positions, rows, the ordered sums -- that more,
-    // smaller workgroups get through sooner; a large one is bound by memory and takes 32 pairs per workgroup
-    // (groups wider than a head -- the feed-forward groups of 128 * ReluMult -- always: 32 of them would not fit in LDS)
-    const bool few = n_pairs <= 4096 || head_dim > 128;
-    const int per_wg = few ? PR_PAIRS_FEW : PR_PAIRS;
-    dim3 grid((unsigned)((n_pairs + per_wg - 1) / per_wg)), block(256);
+    // Groups wider than a head (the feed-forward groups of 128 * ReluMult) are taken by one wave each whatever their number:
+    // 32 of them would not fit in LDS.
+    const bool few = n_pairs <= PR_FEW || head_dim > 128;
+    if (few && p.n_rows > 0xffffffffll / p.n_heads) return hipErrorInvalidValue;
+    const int per_wg = few ? WAVE / (head_dim / 8) : PR_PAIRS;
+    dim3 grid((unsigned)((n_pairs + per_wg - 1) / per_wg)), block(few ? WAVE : 256);
 #define TSATTN_PR(D_, DST_, I32_)                                                                                   \
     do {                                                                                                            \
-        if (few) hipLaunchKernelGGL((rope_normalize_kernel<D_, DST_, I32_, PR_PAIRS_FEW>), grid, block, 0, st, p);  \
+        if (few) hipLaunchKernelGGL((normalize_few_kernel<D_, DST_, I32_>), grid, block, 0, st, p);                 \
         else hipLaunchKernelGGL((rope_normalize_kernel<D_, DST_, I32_, PR_PAIRS>), grid, block, 0, st, p);          \
     } while (0)
     if (head_dim == 128 && dst_dtype == TSATTN_I8 && !src_i32) TSATTN_PR(128, TSATTN_I8, false);
@@ -194,9 +325,9 @@ hipError_t launch_rope_normalize(const ProduceParams &p, int dst_dtype, int head
     else if (head_dim == 64 && dst_dtype == TSATTN_E4M3 && src_i32) TSATTN_PR(64, TSATTN_E4M3, true);
 #define TSATTN_PR_WIDE(D_)                                                                                          \
     else if (head_dim == D_ && dst_dtype == TSATTN_I8 && !src_i32)                                                  \
-        hipLaunchKernelGGL((rope_normalize_kernel<D_, TSATTN_I8, false, PR_PAIRS_FEW>), grid, block, 0, st, p);     \
+        hipLaunchKernelGGL((normalize_few_kernel<D_, TSATTN_I8, false>), grid, block, 0, st, p);                    \
     else if (head_dim == D_ && dst_dtype == TSATTN_I8 && src_i32)                                                   \
-        hipLaunchKernelGGL((rope_normalize_kernel<D_, TSATTN_I8, true, PR_PAIRS_FEW>), grid, block, 0, st, p);
+        hipLaunchKernelGGL((normalize_few_kernel<D_, TSATTN_I8, true>), grid, block, 0, st, p);
     TSATTN_PR_WIDE(256)
     TSATTN_PR_WIDE(384)
     TSATTN_PR_WIDE(512)
