@@ -403,6 +403,58 @@ typedef struct tsattn_matmul_args {
 
 int tsattn_matmul_i8(tsattn_handle_t h, const tsattn_matmul_args *a, void *stream);
 
+/* One layer of the int8 inference path for one new token per sequence (AddLookupProduct, gpt/train/cpu_infer.cpp:465-527) in
+ * five launches with up to 16 sequences, eight with more (one more where the attention splits the cache): what the calls
+ * above make as a chain -- state normalisation, the four projections, RoPE and normalisation of their heads, cache append,
+ * attention with KVProduct, combiner, residual update and normalisation, the two feed-forward products -- with the
+ * normalisations done by the launches that consume them (with more sequences only the heads': by the attention).
+ * The bytes and sums are those of the chain; the attention's output is that of tsattn_decode.
+ *
+ * The contract product of the layer before may come in as planes that are still to be added to the state (pending ...), and
+ * this layer's is left as such planes (parts ...): the state holds everything up to and including the combiner's update
+ * when the call's work is done.  parts and pending may be the same array.
+ *
+ * Served (tsattn_layer_token_scratch_bytes > 0): up to 128 sequences, heads of 64 or 128, dim a multiple of 128, relu_dim =
+ * 64 or 128 per head, window > 0; TSATTN_ERR_UNSUPPORTED otherwise.  The cache is int8 with scale planes for keys; where it
+ * has them for values, VEC_SCALE (vec_scale) is written.  All matrices int8, one row per output, rows of w_pitch = their K
+ * bytes, 16-byte aligned.  cache_len counts the rows before this token and is raised by the call. */
+typedef struct tsattn_layer_args {
+    int n_seqs, n_heads, head_dim;
+    int64_t dim, relu_dim;
+    const void *proj;          /* [4*n_heads*head_dim][dim]: the QK, QV, K and V matrices one after the other */
+    const void *combiner;      /* [dim][4*n_heads*head_dim] */
+    const void *expand;        /* [relu_dim][dim] */
+    const void *contract;      /* [dim][relu_dim] */
+    float vec_scale;           /* the reference's VEC_SCALE = 1/24; also the scale of queries */
+    float key_mult;            /* what the key scales are multiplied by: QVScale * VEC_SCALE * CalcDotScale(dim) */
+    float combiner_scale;      /* state += combiner product * combiner_scale */
+    const int32_t *pos;        /* device [n_seqs] */
+    const float *rope;         /* device [rope_len][head_dim] */
+    int64_t rope_len;
+    void *k_cache, *v_cache;   /* strides as in tsattn_decode_args */
+    int64_t seq_stride, head_stride, tok_stride;
+    float *k_scale, *v_scale;  /* v_scale NULL: the constant below */
+    int64_t s_seq_stride, s_head_stride;
+    float v_scale_const;
+    int32_t *cache_len;
+    int max_len;
+    int64_t window;
+    float alibi_slope;
+    float *state;              /* [n_seqs][state_pitch], dim wide */
+    int64_t state_pitch;
+    float *val;                /* [n_seqs][n_heads*head_dim]: the attention output */
+    const int32_t *pending;    /* NULL, or 1, 2 or 4 planes [n_seqs][dim]: state += sum * pending_scale first */
+    int pending_planes;
+    float pending_scale;
+    int32_t *parts;            /* room for 4 planes [n_seqs][dim]: the contract product */
+    int *n_parts;              /* host: how many of them are in use */
+    void *scratch;             /* 16-byte aligned; holds nothing between calls */
+    int64_t scratch_bytes;
+} tsattn_layer_args;
+
+size_t tsattn_layer_token_scratch_bytes(int n_seqs, int n_heads, int head_dim, int64_t dim, int64_t relu_dim);
+int tsattn_layer_token(tsattn_handle_t h, const tsattn_layer_args *a, void *stream);
+
 /* The two ends of ComputePrediction (gpt/train/cpu_infer.cpp:552-582) around the layers.
  *
  * tsattn_embed_rows: state[row][x] = sum over the row's labels of embed[label][x] * embed_scale, added in label order

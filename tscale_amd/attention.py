@@ -452,6 +452,12 @@ def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratc
     groups = dim // STATE_NORM_TILE
     f32 = np.float32
     sc = scratch if scratch is not None else {}
+    fused = _layer_token(ctx, layer, cache, t, rope, state, sc, pending)
+    if fused is not None:
+        if defer:
+            return fused
+        flush_state(ctx, fused[1], state)
+        return fused[0]
     if "planes" not in sc:
         sc["planes"] = torch.empty((16, B, max(4 * qsum, dim, layer["expand"].shape[0])), dtype=torch.int32, device=state.device)
         sc["v_scale"] = torch.full((B, H), VEC_SCALE, dtype=torch.float32, device=state.device)
@@ -490,6 +496,55 @@ def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratc
         return val, (parts, contract_scale)
     ctx.matmul_i8(relu, layer["contract"], mode=capi.MM_ADD_SCALED, out=state, workspace=workspace, scale=contract_scale)
     return val
+
+
+def _layer_token(ctx, layer, cache, t, rope, state, sc, pending):
+    """The layer in one library call (tsattn_layer_token: five launches instead of nine), where it serves the shape: returns
+    (attention output, pending), or None."""
+    B, dim = state.shape
+    H, d = cache.n_heads, cache.head_dim
+    proj, combiner, expand, contract = layer["proj"], layer["combiner"], layer["expand"], layer["contract"]
+    relu_dim = expand.shape[0]
+    qsum = H * d
+    if (layer["width"] <= 0 or cache.dtype != capi.I8 or not isinstance(cache.k_scale, torch.Tensor) or not isinstance(cache.v_scale, torch.Tensor)
+            or state.stride(1) != 1 or (pending is not None and pending[0].shape[0] not in (1, 2, 4))
+            or not (proj.is_contiguous() and combiner.is_contiguous() and expand.is_contiguous() and contract.is_contiguous())):
+        return None
+    room = sc.get("fused")
+    if room is None or sc.get("fused_shape") != (B, H, d, dim, relu_dim):
+        need = int(ctx.lib.tsattn_layer_token_scratch_bytes(B, H, d, dim, relu_dim))
+        if need == 0:
+            return None
+        room = sc["fused"] = torch.empty(need, dtype=torch.uint8, device=state.device)
+        sc["fused_shape"] = (B, H, d, dim, relu_dim)
+        sc["parts"] = torch.empty((4, B, dim), dtype=torch.int32, device=state.device)
+        sc["val"] = torch.empty((B, qsum), dtype=torch.float32, device=state.device)
+    assert proj.shape == (4 * qsum, dim) and combiner.shape == (dim, 4 * qsum) and expand.shape == (relu_dim, dim) and contract.shape == (dim, relu_dim)
+    assert t.dtype == torch.int32 and state.dtype == torch.float32 and cache.n_seqs == B
+    f32 = np.float32
+    a = capi.LayerArgs()
+    a.n_seqs, a.n_heads, a.head_dim, a.dim, a.relu_dim = B, H, d, dim, relu_dim
+    a.proj, a.combiner, a.expand, a.contract = proj.data_ptr(), combiner.data_ptr(), expand.data_ptr(), contract.data_ptr()
+    a.vec_scale = VEC_SCALE
+    a.key_mult = float(f32(layer["qv_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(dim))))
+    a.combiner_scale = float(f32(layer["combiner_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(qsum * COMBINER_REP))))
+    a.pos, a.rope, a.rope_len = t.data_ptr(), rope.data_ptr(), rope.shape[0]
+    a.k_cache, a.v_cache = cache.k.data_ptr(), cache.v.data_ptr()
+    a.seq_stride, a.head_stride, a.tok_stride, _ = cache.k.stride()
+    a.k_scale, a.v_scale = cache.k_scale.data_ptr(), cache.v_scale.data_ptr()
+    a.s_seq_stride, a.s_head_stride, _ = cache.k_scale.stride()
+    a.cache_len, a.max_len = cache.cache_len.data_ptr(), cache.max_len
+    a.window, a.alibi_slope = int(layer["width"]), float(layer["slope"])
+    a.state, a.state_pitch = state.data_ptr(), state.stride(0)
+    parts, val = sc["parts"], sc["val"]
+    a.val, a.parts = val.data_ptr(), parts.data_ptr()
+    if pending is not None:
+        a.pending, a.pending_planes, a.pending_scale = pending[0].data_ptr(), pending[0].shape[0], pending[1]
+    n_parts = ctypes.c_int(0)
+    a.n_parts = ctypes.pointer(n_parts)
+    a.scratch, a.scratch_bytes = room.data_ptr(), room.numel()
+    capi.check(ctx.lib.tsattn_layer_token(ctx.handle, ctypes.byref(a), _stream_ptr()))
+    return val, (parts[:n_parts.value], float(f32(layer["contract_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(relu_dim)))))
 
 
 def flush_state(ctx, pending, state):

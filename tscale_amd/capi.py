@@ -120,8 +120,23 @@ class MergeArgs(_c.Structure):
     ]
 
 
+class LayerArgs(_c.Structure):
+    _fields_ = [
+        ("n_seqs", _c.c_int), ("n_heads", _c.c_int), ("head_dim", _c.c_int), ("dim", _c.c_int64), ("relu_dim", _c.c_int64),
+        ("proj", _c.c_void_p), ("combiner", _c.c_void_p), ("expand", _c.c_void_p), ("contract", _c.c_void_p),
+        ("vec_scale", _c.c_float), ("key_mult", _c.c_float), ("combiner_scale", _c.c_float),
+        ("pos", _c.c_void_p), ("rope", _c.c_void_p), ("rope_len", _c.c_int64),
+        ("k_cache", _c.c_void_p), ("v_cache", _c.c_void_p), ("seq_stride", _c.c_int64), ("head_stride", _c.c_int64),
+        ("tok_stride", _c.c_int64), ("k_scale", _c.c_void_p), ("v_scale", _c.c_void_p), ("s_seq_stride", _c.c_int64),
+        ("s_head_stride", _c.c_int64), ("v_scale_const", _c.c_float), ("cache_len", _c.c_void_p), ("max_len", _c.c_int),
+        ("window", _c.c_int64), ("alibi_slope", _c.c_float), ("state", _c.c_void_p), ("state_pitch", _c.c_int64),
+        ("val", _c.c_void_p), ("pending", _c.c_void_p), ("pending_planes", _c.c_int), ("pending_scale", _c.c_float),
+        ("parts", _c.c_void_p), ("n_parts", _c.POINTER(_c.c_int)), ("scratch", _c.c_void_p), ("scratch_bytes", _c.c_int64),
+    ]
+
+
 EXPORTS = ["tsattn_scratch_bytes", "tsattn_create", "tsattn_destroy", "tsattn_last_error", "tsattn_prefill", "tsattn_prefill_workspace_bytes",
-           "tsattn_decode", "tsattn_decode_static", "tsattn_cache_append", "tsattn_cache_fill", "tsattn_merge_lookups", "tsattn_span_tiles_count", "tsattn_build_span_tiles", "tsattn_rope_normalize_rows", "tsattn_fill_rope_table", "tsattn_kv_product", "tsattn_matmul_i8", "tsattn_embed_rows", "tsattn_softmax_rows", "tsattn_sample_rows", "tsattn_quantize_rows", "tsattn_build_spans", "tsattn_debug_read_counters", "tsattn_version"]
+           "tsattn_decode", "tsattn_decode_static", "tsattn_cache_append", "tsattn_cache_fill", "tsattn_merge_lookups", "tsattn_span_tiles_count", "tsattn_build_span_tiles", "tsattn_rope_normalize_rows", "tsattn_fill_rope_table", "tsattn_kv_product", "tsattn_matmul_i8", "tsattn_layer_token_scratch_bytes", "tsattn_layer_token", "tsattn_embed_rows", "tsattn_softmax_rows", "tsattn_sample_rows", "tsattn_quantize_rows", "tsattn_build_spans", "tsattn_debug_read_counters", "tsattn_version"]
 
 _lib = None
 
@@ -172,6 +187,10 @@ def load():
                                         _c.c_void_p, _c.c_int64, _c.c_float, _c.c_void_p, _c.c_int64, _c.c_void_p]
         L.tsattn_matmul_i8.restype = _c.c_int
         L.tsattn_matmul_i8.argtypes = [_c.c_void_p, _c.POINTER(MatmulArgs), _c.c_void_p]
+        L.tsattn_layer_token_scratch_bytes.restype = _c.c_size_t
+        L.tsattn_layer_token_scratch_bytes.argtypes = [_c.c_int, _c.c_int, _c.c_int, _c.c_int64, _c.c_int64]
+        L.tsattn_layer_token.restype = _c.c_int
+        L.tsattn_layer_token.argtypes = [_c.c_void_p, _c.POINTER(LayerArgs), _c.c_void_p]
         L.tsattn_embed_rows.restype = _c.c_int
         L.tsattn_embed_rows.argtypes = [_c.c_void_p, _c.c_int64, _c.c_int, _c.c_void_p, _c.c_int, _c.c_void_p, _c.c_int64, _c.c_int64,
                                         _c.c_float, _c.c_void_p, _c.c_int64, _c.c_void_p]

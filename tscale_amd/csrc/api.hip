@@ -68,16 +68,17 @@ bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0; }
 } // namespace
 
 // The body of both decode entry points; `lim` says what the scratch behind part_acc / part_ml / seq_done was sized for.
-static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_args *a, void *stream)
+// With `front` the queries, the new row and KVProduct's key are made by the launch itself (tsattn_layer_token).
+static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_args *a, void *stream, const tsattn::FrontParams *front = nullptr)
 {
     if (!dtype_ok(a->dtype)) return fail(TSATTN_ERR_UNSUPPORTED, "tsattn_decode: dtype %d", a->dtype);
     if (a->q_dtype != TSATTN_Q_8BIT && a->q_dtype != TSATTN_Q_BF16) return fail(TSATTN_ERR_UNSUPPORTED, "tsattn_decode: q_dtype %d", a->q_dtype);
     if (!head_dim_ok(a->head_dim)) return fail(TSATTN_ERR_UNSUPPORTED, "tsattn_decode: head_dim %d (64 or 128 supported)", a->head_dim);
     if (a->n_seqs < 0 || a->n_heads <= 0 || a->max_len < 0 || a->window < 0) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: negative size");
     if (a->n_seqs == 0) return TSATTN_OK;
-    if (!a->q || !a->k_cache || !a->v_cache || !a->cache_len || !a->out) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: null data pointer");
+    if ((!a->q && !front) || !a->k_cache || !a->v_cache || !a->cache_len || !a->out) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: null data pointer");
     const int qbytes = a->q_dtype == TSATTN_Q_BF16 ? 2 : 1;
-    if (a->q_pitch < (int64_t)a->n_heads * a->head_dim * qbytes || a->q_pitch % 16) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: q_pitch");
+    if (!front && (a->q_pitch < (int64_t)a->n_heads * a->head_dim * qbytes || a->q_pitch % 16)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: q_pitch");
     if (a->tok_stride < a->head_dim || a->tok_stride % 16 || a->head_stride % 16 || a->seq_stride % 16)
         return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: cache strides must be multiples of 16 bytes, tok_stride >= head_dim");
     if (!aligned16(a->q) || !aligned16(a->k_cache) || !aligned16(a->v_cache)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: q and caches must be 16-byte aligned");
@@ -117,8 +118,9 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     p.ks_new = a->k_scale_new; p.vs_new = a->v_scale_new;
     p.cache_len_rw = const_cast<int32_t *>(a->cache_len); p.max_len = a->max_len;
     p.seq_done = lim.seq_done;
+    if (front) p.front = *front;
     if (a->kv_out) {
-        if (!a->kv_k) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: the fused KVProduct needs kv_k");
+        if (!a->kv_k && !front) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: the fused KVProduct needs kv_k");
         if (a->dtype != TSATTN_I8) return fail(TSATTN_ERR_UNSUPPORTED, "tsattn_decode: the fused KVProduct is defined for int8 keys");
         if (a->kv_rep < 1 || a->kv_rep > 4) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: kv_rep %d (1..4)", a->kv_rep);
         if (((uintptr_t)a->kv_k & 3) || a->kv_k_pitch % 4 || a->kv_k_pitch < (int64_t)a->n_heads * a->head_dim ||
@@ -134,7 +136,7 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
             return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: k_new/v_new must be 16-byte aligned with a pitch that covers a row");
         if ((a->k_scale_new && !a->k_scale) || (a->v_scale_new && !a->v_scale)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: new scales given without scale planes");
     }
-    if (lim.clear_counters && a->k_new) {
+    if (lim.clear_counters && (a->k_new || front)) {
         // the arrival counters of the single-split fused append start at zero: a launch leaves them so, but this scratch is
         // shared by every caller on the device (a fill kernel, not a memset: callers may be capturing a graph)
         hipError_t ez = tsattn::launch_zero_i32(lim.seq_done, a->n_seqs, (hipStream_t)stream);
@@ -145,6 +147,16 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     return TSATTN_OK;
 }
 
+static DecodeScratch decode_scratch(tsattn_handle_t h)
+{
+    DecodeScratch lim;
+    lim.max_seqs = h->max_seqs; lim.max_head_dim = h->max_head_dim; lim.max_splits = h->max_splits;
+    lim.max_pairs = (int64_t)h->max_seqs * h->max_heads;
+    lim.max_parts = lim.max_pairs * h->max_splits;
+    lim.part_acc = h->part_acc; lim.part_ml = h->part_ml; lim.seq_done = h->seq_done;
+    lim.clear_counters = false;
+    return lim;
+}
 
 extern "C" {
 
@@ -307,13 +319,7 @@ size_t tsattn_prefill_workspace_bytes(int64_t n_tokens, int n_heads, int head_di
 int tsattn_decode(tsattn_handle_t h, const tsattn_decode_args *a, void *stream)
 {
     if (!h || !a) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: null argument");
-    DecodeScratch lim;
-    lim.max_seqs = h->max_seqs; lim.max_head_dim = h->max_head_dim; lim.max_splits = h->max_splits;
-    lim.max_pairs = (int64_t)h->max_seqs * h->max_heads;
-    lim.max_parts = lim.max_pairs * h->max_splits;
-    lim.part_acc = h->part_acc; lim.part_ml = h->part_ml; lim.seq_done = h->seq_done;
-    lim.clear_counters = false;
-    return decode_with_scratch(lim, a, stream);
+    return decode_with_scratch(decode_scratch(h), a, stream);
 }
 
 int tsattn_debug_read_counters(tsattn_handle_t h, int32_t *dst, int n, void *stream)
@@ -572,6 +578,143 @@ int tsattn_matmul_i8(tsattn_handle_t h, const tsattn_matmul_args *a, void *strea
     p.workspace = ws_ok ? a->workspace : nullptr; p.workspace_bytes = ws_ok ? a->workspace_bytes : 0; p.split_stride = 0;
     hipError_t e = tsattn::launch_matmul_i8(p, (hipStream_t)stream, a->planes_out);
     if (e != hipSuccess) return hip_fail(e, "matmul launch");
+    return TSATTN_OK;
+}
+
+namespace {
+
+// scratch of a layer's token step: planes of the projections (the expand product's later), planes of the combiner, KVProduct's
+// bytes, the heads' keys for the merge launch, a product's normalised rows where a launch of its own makes them
+struct LayerScratch {
+    int64_t wide, combiner, kv, key, norm, total;
+};
+constexpr int LAYER_PARTS = 4;
+
+LayerScratch layer_scratch(int64_t n_seqs, int64_t qsum, int64_t dim, int64_t relu_dim)
+{
+    const auto up = [](int64_t b) { return (b + 255) & ~(int64_t)255; };
+    LayerScratch s;
+    s.wide = 0;
+    s.combiner = s.wide + up(LAYER_PARTS * n_seqs * std::max(4 * qsum, relu_dim) * 4);
+    s.kv = s.combiner + up(LAYER_PARTS * n_seqs * dim * 4);
+    s.key = s.kv + up(n_seqs * 4 * qsum);
+    s.norm = s.key + up(n_seqs * qsum);
+    s.total = s.norm + up(n_seqs * std::max(dim, relu_dim));
+    return s;
+}
+
+} // namespace
+
+size_t tsattn_layer_token_scratch_bytes(int n_seqs, int n_heads, int head_dim, int64_t dim, int64_t relu_dim)
+{
+    if (n_seqs < 1 || n_seqs > tsattn::FEW_ROWS || n_heads < 1 || !head_dim_ok(head_dim) || dim < 128 || dim % 128 || dim > (1 << 20) || relu_dim < 1 ||
+        (relu_dim != (int64_t)n_heads * 64 && relu_dim != (int64_t)n_heads * 128) || (int64_t)n_heads * head_dim > (1 << 20))
+        return 0;
+    return (size_t)layer_scratch(n_seqs, (int64_t)n_heads * head_dim, dim, relu_dim).total;
+}
+
+int tsattn_layer_token(tsattn_handle_t h, const tsattn_layer_args *a, void *stream)
+{
+    if (!h || !a) return fail(TSATTN_ERR_BAD_ARG, "tsattn_layer_token: null argument");
+    const size_t need = tsattn_layer_token_scratch_bytes(a->n_seqs, a->n_heads, a->head_dim, a->dim, a->relu_dim);
+    if (need == 0 || a->window <= 0)
+        return fail(TSATTN_ERR_UNSUPPORTED, "tsattn_layer_token: %d sequences, %d heads of %d, dim %lld, relu_dim %lld, window %lld", a->n_seqs, a->n_heads,
+                    a->head_dim, (long long)a->dim, (long long)a->relu_dim, (long long)a->window);
+    if (!a->proj || !a->combiner || !a->expand || !a->contract || !a->pos || !a->rope || a->rope_len <= 0 || !a->k_scale || !a->state || !a->val || !a->parts ||
+        !a->n_parts || !a->scratch)
+        return fail(TSATTN_ERR_BAD_ARG, "tsattn_layer_token: null data pointer");
+    if (!aligned16(a->proj) || !aligned16(a->combiner) || !aligned16(a->expand) || !aligned16(a->contract) || !aligned16(a->rope) || !aligned16(a->state) ||
+        !aligned16(a->parts) || !aligned16(a->pending) || !aligned16(a->scratch) || a->state_pitch < a->dim || a->state_pitch % 4)
+        return fail(TSATTN_ERR_BAD_ARG, "tsattn_layer_token: matrices, rope, state and planes must be 16-byte aligned, state_pitch a multiple of 4 that covers a row");
+    if (a->scratch_bytes < (int64_t)need) return fail(TSATTN_ERR_SCRATCH, "tsattn_layer_token: %lld bytes of scratch, %lld needed", (long long)a->scratch_bytes, (long long)need);
+    if (a->pending && a->pending_planes != 1 && a->pending_planes != 2 && a->pending_planes != 4)
+        return fail(TSATTN_ERR_UNSUPPORTED, "tsattn_layer_token: %d pending planes (1, 2 or 4)", a->pending_planes);
+    const int64_t B = a->n_seqs, qsum = (int64_t)a->n_heads * a->head_dim;
+    const LayerScratch at = layer_scratch(B, qsum, a->dim, a->relu_dim);
+    uint8_t *const room = (uint8_t *)a->scratch;
+    int32_t *const wide = (int32_t *)(room + at.wide), *const combined = (int32_t *)(room + at.combiner);
+    const hipStream_t st = (hipStream_t)stream;
+
+    const auto launch = [&](tsattn::FewParams &f) {
+        f.parts = tsattn::few_parts(f, LAYER_PARTS);
+        return tsattn::launch_gemm_few(f, st);
+    };
+    // w [n][k] times the rows that normalisation of `source` gives -- int32 planes, the state, or the state with the planes'
+    // residual update -- which the product's launch makes itself (and leaves the state alone), or with more rows a launch
+    // before it (which stores the updated state).
+    const bool own = B <= tsattn::FEW_NORM_ROWS;
+    const auto norm_product = [&](const void *w, int64_t n, int64_t k, int32_t *out, int group, const int32_t *source, int planes, float *state, float scale,
+                                  int relu, const tsattn::UpdateParams *update, int *parts) {
+        tsattn::FewParams f = {};
+        f.w = (const uint8_t *)w; f.w_pitch = k; f.m = B; f.n = n; f.k = k; f.mode = TSATTN_MM_I32;
+        f.out = out; f.out_pitch = n; f.out_stride = B * n;
+        if (own) {
+            f.vec_scale = a->vec_scale; f.group = group; f.relu = relu;
+            f.state = state; f.state_pitch = a->state_pitch;
+            f.src = source; f.src_planes = planes; f.src_stride = B * k; f.resid_scale = scale;
+            if (update) f.upd = *update;
+        } else {
+            tsattn::ProduceParams q = {};
+            q.src = source ? (const void *)source : (const void *)state;
+            q.src_pitch = source ? k : a->state_pitch; q.src_planes = planes > 1 ? planes : 1; q.src_plane_stride = B * k;
+            q.n_rows = B; q.n_heads = (int)(k / group); q.vec_scale = a->vec_scale; q.relu = relu;
+            q.dst = room + at.norm; q.dst_pitch = k;
+            if (source && state) { q.resid = state; q.resid_pitch = a->state_pitch; q.resid_scale = scale; }
+            const hipError_t e = tsattn::launch_rope_normalize(q, TSATTN_I8, group, source != nullptr, st);
+            if (e != hipSuccess) return e;
+            f.a = room + at.norm; f.a_pitch = k;
+        }
+        const hipError_t e = launch(f);
+        *parts = f.parts;
+        return e;
+    };
+    const auto update_of = [&](const int32_t *src, int planes, float scale) {
+        tsattn::UpdateParams u = {};
+        if (own && src) {
+            u.state = a->state; u.state_pitch = a->state_pitch; u.src = src; u.planes = planes; u.src_stride = B * a->dim;
+            u.rows = a->n_seqs; u.dim = (int)a->dim; u.scale = scale;
+        }
+        return u;
+    };
+
+    // 1. normalised state (with the layer before's contract product added) times the four projections
+    int proj_parts = 1, expand_parts = 1;
+    hipError_t e = norm_product(a->proj, 4 * qsum, a->dim, wide, 128, a->pending, a->pending ? a->pending_planes : 0, a->state, a->pending_scale, 0, nullptr, &proj_parts);
+    if (e != hipSuccess) return hip_fail(e, "layer: projections launch");
+
+    // 2. attention: heads out of the projections, append, KVProduct; a pending update that the first launch has read past
+    // goes into the state
+    tsattn::FrontParams front = {};
+    front.src = wide; front.planes = proj_parts; front.src_stride = B * 4 * qsum;
+    front.pos = a->pos; front.rope = a->rope; front.rope_len = a->rope_len;
+    front.key_mult = a->key_mult; front.vec_scale = a->vec_scale; front.k_row = room + at.key;
+    front.upd = update_of(a->pending, a->pending_planes, a->pending_scale);
+    tsattn_decode_args d = {};
+    d.dtype = TSATTN_I8; d.q_dtype = TSATTN_Q_8BIT; d.n_seqs = a->n_seqs; d.n_heads = a->n_heads; d.head_dim = a->head_dim;
+    d.q_scale_const = a->vec_scale;
+    d.k_cache = a->k_cache; d.v_cache = a->v_cache; d.seq_stride = a->seq_stride; d.head_stride = a->head_stride; d.tok_stride = a->tok_stride;
+    d.k_scale = a->k_scale; d.v_scale = a->v_scale; d.s_seq_stride = a->s_seq_stride; d.s_head_stride = a->s_head_stride; d.v_scale_const = a->v_scale_const;
+    d.cache_len = a->cache_len; d.max_len = a->max_len; d.window = a->window; d.alibi_slope = a->alibi_slope; d.out = a->val;
+    d.kv_k = front.k_row; d.kv_k_pitch = qsum; d.kv_out = room + at.kv; d.kv_out_pitch = 4 * qsum; d.kv_rep = 4; d.kv_mult = 1.0f;
+    const int rc = decode_with_scratch(decode_scratch(h), &d, stream, &front);
+    if (rc != TSATTN_OK) return rc;
+
+    // 3. combiner
+    tsattn::FewParams comb = {};
+    comb.w = (const uint8_t *)a->combiner; comb.w_pitch = 4 * qsum; comb.m = B; comb.n = a->dim; comb.k = 4 * qsum; comb.mode = TSATTN_MM_I32;
+    comb.out = combined; comb.out_pitch = a->dim; comb.out_stride = B * a->dim;
+    comb.a = room + at.kv; comb.a_pitch = 4 * qsum;
+    e = launch(comb);
+    if (e != hipSuccess) return hip_fail(e, "layer: combiner launch");
+
+    // 4. updated and normalised state times the expand matrix
+    e = norm_product(a->expand, a->relu_dim, a->dim, wide, 128, combined, comb.parts, a->state, a->combiner_scale, 0, nullptr, &expand_parts);
+    if (e != hipSuccess) return hip_fail(e, "layer: expand launch");
+
+    // 5. its normalised positive part times the contract matrix; the combiner's update goes into the state
+    const tsattn::UpdateParams update = update_of(combined, comb.parts, a->combiner_scale);
+    e = norm_product(a->contract, a->dim, a->relu_dim, a->parts, (int)(a->relu_dim / a->n_heads), wide, expand_parts, nullptr, 1.0f, 1, &update, a->n_parts);
+    if (e != hipSuccess) return hip_fail(e, "layer: contract launch");
     return TSATTN_OK;
 }
 

@@ -21,7 +21,7 @@ namespace tsattn {
 
 constexpr int DEC_THREADS = 256;
 constexpr int DEC_WAVES = DEC_THREADS / WAVE;
-constexpr int DEC_U = 8; // cache rows per lane group kept in flight per step
+constexpr int DEC_LONG = 8, DEC_SHORT = 2; // cache rows per lane group and step (short: ranges of one step of four waves)
 
 template <int DTYPE>
 struct QFrag;
@@ -136,7 +136,11 @@ __device__ inline void kv_product_store(const uint8_t *kv_k, int64_t kv_k_pitch,
     }
 }
 
-template <int DTYPE, int D, bool QBF16, bool DUMP>
+// FRONT: what the launch before would have made -- q, the new key and value rows, the key of KVProduct, RoPE and
+// normalisation included -- is made by the first wave of every workgroup from the projections' planes of its own head, while
+// the other waves ask for their first cache rows (nothing is made twice but q by the splits of a head).  It saves a launch
+// of 5.7 us for 1.5 us; the bytes are those of rope_normalize_kernel, the same float operations in the same order.
+template <int DTYPE, int D, bool QBF16, bool DUMP, bool FRONT, int DEC_U>
 __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams p)
 {
     constexpr int LPK = D / 16;      // lanes per cache row
@@ -155,14 +159,44 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     __shared__ float sm_m[DEC_WAVES];
     __shared__ float sm_l[DEC_WAVES];
     __shared__ float sm_acc[DEC_WAVES][D];
+    __shared__ __attribute__((aligned(16))) float f_square[FRONT ? 4 * (D + 4) : 4];
+    __shared__ __attribute__((aligned(16))) uint8_t f_row[FRONT ? 4 * D : 16]; // q, new key, key of KVProduct, new value
+    __shared__ float f_key_scale;
+
+    ResidUpdate update;
+    v4i fa[FRONT ? 4 : 1], fb[FRONT ? 4 : 1];
+    v4f f_cos, f_sin;
+    const int f_part = lane / (D / 8), f_x = ((lane % (D / 8)) / 8) * 64 + (lane % 8) * 4; // values f_x.. and f_x + 32.. of a row
+    const bool f_mine = FRONT && wave == 0 && lane < D / 2;
+    if constexpr (FRONT) {
+        if (f_mine) {
+            const int32_t *const src = p.front.src + ((int64_t)seq * 4 + f_part) * p.n_heads * D + head * D + f_x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { // (planes that are not there: the last one again)
+                const int32_t *const q = src + (i < p.front.planes ? i : p.front.planes - 1) * p.front.src_stride;
+                fa[i] = *(const v4i *)q;
+                fb[i] = *(const v4i *)(q + 32);
+            }
+            int t = p.front.pos[seq];
+            t = t < 0 ? 0 : (t >= p.front.rope_len ? (int)p.front.rope_len - 1 : t);
+            const float *const rr = p.front.rope + (int64_t)t * D + f_x;
+            f_cos = *(const v4f *)rr;
+            f_sin = *(const v4f *)(rr + 32);
+        } else if (wave != 0) {
+            const int wg = (seq * p.n_heads + head) * p.n_splits + split;
+            update.request(p.front.upd, wg * (DEC_THREADS - WAVE) + tid - WAVE, (int)(gridDim.x * gridDim.y * gridDim.z) * (DEC_THREADS - WAVE));
+        }
+    }
 
     // ---- key range of this block --------------------------------------------------------------
     // With a fused append the cache holds cache_len rows and the new token's row is being added as row cache_len
     // by the first split's workgroup of each head (a full cache drops it, as the separate append does).
     int cur = p.cache_len[seq] - 1;
-    if (p.k_new && cur + 1 < p.max_len) {
+    const bool append = FRONT || p.k_new != nullptr;
+    const bool new_row = append && cur + 1 < p.max_len;
+    if (new_row) {
         cur += 1;
-        if (split == 0 && tid < 2 * LPK) {
+        if (!FRONT && split == 0 && tid < 2 * LPK) {
             const int pl = tid / LPK, ch = tid % LPK; // plane (K or V), 16-byte chunk
             const int64_t src = (int64_t)seq * p.new_pitch + head * D + ch * 16;
             const int64_t dst = (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + (int64_t)cur * p.tok_stride + ch * 16;
@@ -189,7 +223,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             }
         }
     };
-    const bool count_row = direct && p.k_new != nullptr;
+    const bool count_row = direct && append;
     int lo, n;
     if (cur < 0) {
         lo = 0; n = 0;
@@ -206,7 +240,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     if (s1 > lo + n) s1 = lo + n;
 
     const int64_t part = ((int64_t)seq * p.n_heads + head) * p.n_splits + split;
-    if (s0 >= s1) { // nothing to do: neutral partial (max 0, sum 0, zeros)
+    if (!FRONT && s0 >= s1) { // nothing to do: neutral partial (max 0, sum 0, zeros)
         if (direct) {
             if (tid < D) {
                 p.out[((int64_t)seq * p.n_heads + head) * D + tid] = 0.0f;
@@ -223,10 +257,109 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         return;
     }
 
+    const uint8_t *kbase = p.k + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + c * 16;
+    const uint8_t *vbase = p.v + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + c * 16;
+    const float *ksb = p.ks ? p.ks + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
+    const float *vsb = p.vs ? p.vs + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
+    v4i kreg[DEC_U], vreg[DEC_U];
+    float ksr[DEC_U], vsr[DEC_U];
+    auto request = [&](int base) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < DEC_U; ++u) {
+            const int r = base + u * KPL + g;
+            const int rc = (r < s1) ? r : s1 - 1; // clamp the address, mask the logit below
+            kreg[u] = __builtin_nontemporal_load((const v4i *)(kbase + (int64_t)rc * p.tok_stride));
+            ksr[u] = ksb ? ksb[rc] : p.ks_const;
+        }
+#pragma unroll
+        for (int u = 0; u < DEC_U; ++u) {
+            const int r = base + u * KPL + g;
+            const int rc = (r < s1) ? r : s1 - 1;
+            vreg[u] = __builtin_nontemporal_load((const v4i *)(vbase + (int64_t)rc * p.tok_stride));
+            vsr[u] = vsb ? vsb[rc] : p.vs_const;
+        }
+    };
+    int base = s0 + wave * ROWS_PER_STEP;
+    if (base < s1) request(base);
+
     // ---- query slice of this lane ----------------------------------------------------------------
     QFrag<DTYPE> qf;
     float qs;
-    {
+    if constexpr (FRONT) {
+#pragma clang fp contract(off)
+        if (wave == 0) {
+            float mult = 0.0f;
+            v4f v0, v1;
+            if (f_mine) {
+                v4i a = fa[0], b = fb[0];
+#pragma unroll
+                for (int i = 1; i < 4; ++i)
+                    if (i < p.front.planes) { a += fa[i]; b += fb[i]; }
+                v0 = v4f{(float)a.x, (float)a.y, (float)a.z, (float)a.w};
+                v1 = v4f{(float)b.x, (float)b.y, (float)b.z, (float)b.w};
+                const bool turn = f_part < 2; // (k and v turn by the identity, as in the producer)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float cos_value = turn ? f_cos[i] : 1.0f, sin_value = turn ? f_sin[i] : 0.0f;
+                    const float r0 = v0[i] * cos_value - v1[i] * sin_value;
+                    const float r1 = v0[i] * sin_value + v1[i] * cos_value;
+                    v0[i] = r0;
+                    v1[i] = r1;
+                }
+                *(v4f *)(f_square + f_part * (D + 4) + f_x) = v4f{v0.x * v0.x, v0.y * v0.y, v0.z * v0.z, v0.w * v0.w};
+                *(v4f *)(f_square + f_part * (D + 4) + f_x + 32) = v4f{v1.x * v1.x, v1.y * v1.y, v1.z * v1.z, v1.w * v1.w};
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (one wave: its LDS accesses are in order)
+            float discr = 0.0f;
+            if (lane < 4) { // squares added in index order
+                const float *const v = f_square + lane * (D + 4);
+                float sum2 = 0.0f;
+#pragma unroll
+                for (int x = 0; x < D; x += 32) {
+                    v4f q[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) q[i] = *(const v4f *)(v + x + 4 * i);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        sum2 = sum2 + q[i].x;
+                        sum2 = sum2 + q[i].y;
+                        sum2 = sum2 + q[i].z;
+                        sum2 = sum2 + q[i].w;
+                    }
+                }
+                if (sum2 != 0.0f) {
+                    discr = (float)sqrt((double)(sum2 / (float)D)) * p.front.vec_scale;
+                    mult = 1.0f / discr;
+                }
+                if (lane == 1) f_key_scale = discr * p.front.key_mult;
+            }
+            mult = __shfl(mult, f_part & 3, WAVE);
+            if (f_mine) {
+                *(uint32_t *)(f_row + f_part * D + f_x) = pack_i8x4(v0.x * mult, v0.y * mult, v0.z * mult, v0.w * mult, -127.0f);
+                *(uint32_t *)(f_row + f_part * D + f_x + 32) = pack_i8x4(v1.x * mult, v1.y * mult, v1.z * mult, v1.w * mult, -127.0f);
+            }
+        } else {
+            update.finish(p.front.upd);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (cache rows stay on their way over the barrier)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        qf.set(f_row + c * 16);
+        qs = p.q_scale_const;
+        if (split == 0) {
+            if (new_row && tid < 2 * LPK) {
+                const int pl = tid / LPK, ch = tid % LPK; // plane (K or V), 16-byte chunk
+                const int64_t dst = (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + (int64_t)cur * p.tok_stride + ch * 16;
+                *(v4i *)(const_cast<uint8_t *>(pl == 0 ? p.k : p.v) + dst) = *(const v4i *)(f_row + (pl == 0 ? 1 : 3) * D + ch * 16);
+                if (ch == 0) {
+                    const int64_t sd = (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride + cur;
+                    if (pl == 0 && p.ks) const_cast<float *>(p.ks)[sd] = f_key_scale;
+                    if (pl == 1 && p.vs) const_cast<float *>(p.vs)[sd] = p.front.vec_scale;
+                }
+            }
+            if (!direct && tid < LPK) *(v4i *)(p.front.k_row + ((int64_t)seq * p.n_heads + head) * D + tid * 16) = *(const v4i *)(f_row + 2 * D + tid * 16);
+        }
+    } else {
         __attribute__((aligned(16))) uint8_t qb[16];
         if (QBF16) {
             const uint16_t *src = (const uint16_t *)(p.q + (int64_t)seq * p.q_pitch) + head * D + c * 16;
@@ -258,34 +391,13 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         qf.set(qb);
     }
 
-    const uint8_t *kbase = p.k + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + c * 16;
-    const uint8_t *vbase = p.v + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + c * 16;
-    const float *ksb = p.ks ? p.ks + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
-    const float *vsb = p.vs ? p.vs + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
     const float ads = att_dot_scale(D);
 
     float m = 0.0f, l = 0.0f;
     float acc[16];
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 
-    for (int base = s0 + wave * ROWS_PER_STEP; base < s1; base += DEC_WAVES * ROWS_PER_STEP) {
-        v4i kreg[DEC_U], vreg[DEC_U];
-        float ksr[DEC_U], vsr[DEC_U];
-        int row[DEC_U];
-#pragma unroll
-        for (int u = 0; u < DEC_U; ++u) {
-            int r = base + u * KPL + g;
-            row[u] = r;
-            int rc = (r < s1) ? r : s1 - 1; // clamp the address, mask the logit below
-            kreg[u] = __builtin_nontemporal_load((const v4i *)(kbase + (int64_t)rc * p.tok_stride));
-            ksr[u] = ksb ? ksb[rc] : p.ks_const;
-        }
-#pragma unroll
-        for (int u = 0; u < DEC_U; ++u) {
-            int rc = (row[u] < s1) ? row[u] : s1 - 1;
-            vreg[u] = __builtin_nontemporal_load((const v4i *)(vbase + (int64_t)rc * p.tok_stride));
-            vsr[u] = vsb ? vsb[rc] : p.vs_const;
-        }
+    for (; base < s1; base += DEC_WAVES * ROWS_PER_STEP) {
         float s[DEC_U];
         float m_new = m;
 #pragma unroll
@@ -293,12 +405,12 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             float bits = group_sum_bits<DTYPE, LPK>(qf.dot_partial_as_bits(kreg[u]));
             float accf = (DTYPE == TSATTN_I8) ? (float)__float_as_int(bits) : bits;
             if (DUMP) {
-                if (c == 0 && row[u] < s1) {
-                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + row[u]] = bits;
+                if (c == 0 && (base + u * KPL + g) < s1) {
+                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + (base + u * KPL + g)] = bits;
                 }
             }
-            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - row[u]);
-            s[u] = (row[u] < s1) ? dp : -INFINITY;
+            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - (base + u * KPL + g));
+            s[u] = ((base + u * KPL + g) < s1) ? dp : -INFINITY;
             m_new = fmaxf(m_new, s[u]);
         }
         float alpha = fast_exp2(m - m_new);
@@ -312,6 +424,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             l += pu;
             accumulate_values<DTYPE>(pu * vsr[u], vreg[u], acc);
         }
+        if (base + DEC_WAVES * ROWS_PER_STEP < s1) request(base + DEC_WAVES * ROWS_PER_STEP);
     }
 
     // ---- merge the lane groups of this wave ---------------------------------------------------
@@ -349,7 +462,8 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             // the only split: add the zero vector's weight 2^-M (M >= 0 by construction) and normalise here
             const float res = o / (L + fast_exp2(-M));
             p.out[((int64_t)seq * p.n_heads + head) * D + tid] = res;
-            if (p.kv_out) kv_product_store<D>(p.kv_k, p.kv_k_pitch, p.kv_out, p.kv_out_pitch, p.kv_rep, p.kv_mult, seq, head, tid, res);
+            if (FRONT) kv_product_store<D>(f_row + 2 * D - (int64_t)head * D, 0, p.kv_out, p.kv_out_pitch, p.kv_rep, p.kv_mult, seq, head, tid, res);
+            else if (p.kv_out) kv_product_store<D>(p.kv_k, p.kv_k_pitch, p.kv_out, p.kv_out_pitch, p.kv_rep, p.kv_mult, seq, head, tid, res);
         } else {
             p.part_acc[part * D + tid] = o;
             if (tid == 0) { p.part_ml[part * 2] = M; p.part_ml[part * 2 + 1] = L; }
@@ -386,32 +500,51 @@ __global__ __launch_bounds__(D) void decode_merge_kernel(const float *part_acc, 
     if (kv_out) kv_product_store<D>(kv_k, kv_k_pitch, kv_out, kv_out_pitch, kv_rep, kv_mult, sh / n_heads, (int)(sh % n_heads), x, res);
 }
 
-template <int DTYPE, int D>
-static void launch_decode_dd(const DecodeParams &p, bool qbf16, bool dump, dim3 grid, hipStream_t st)
+template <int DTYPE, int D, int U>
+static hipError_t launch_decode_u(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
 {
-    if (qbf16) {
-        if (dump) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, true>), grid, dim3(DEC_THREADS), 0, st, p);
-        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, false>), grid, dim3(DEC_THREADS), 0, st, p);
+    const bool dump = p.dbg != nullptr;
+    if (p.front.src) {
+        if constexpr (DTYPE == TSATTN_I8) {
+            if (qbf16 || dump || !p.kv_out) return hipErrorInvalidValue;
+            hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, false, true, U>), grid, dim3(DEC_THREADS), 0, st, p);
+        } else {
+            return hipErrorInvalidValue;
+        }
+    } else if (qbf16) {
+        if (dump) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, true, false, DEC_LONG>), grid, dim3(DEC_THREADS), 0, st, p);
+        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, false, false, U>), grid, dim3(DEC_THREADS), 0, st, p);
     } else {
-        if (dump) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, true>), grid, dim3(DEC_THREADS), 0, st, p);
-        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, false>), grid, dim3(DEC_THREADS), 0, st, p);
+        if (dump) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, true, false, DEC_LONG>), grid, dim3(DEC_THREADS), 0, st, p);
+        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, false, false, U>), grid, dim3(DEC_THREADS), 0, st, p);
     }
+    return hipGetLastError();
+}
+
+template <int DTYPE, int D>
+static hipError_t launch_decode_dd(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
+{
+    // A range that four waves cover in one step of two rows per lane group (a 64-key window) is shared out in such steps:
+    // with steps of eight the first wave alone would compute all of it (W = 64, d = 128: 1.8 us of its instructions).
+    int64_t rows = p.max_len < p.window ? p.max_len : p.window;
+    rows = (rows + p.n_splits - 1) / p.n_splits;
+    if (rows <= (int64_t)DEC_WAVES * DEC_SHORT * (WAVE / (D / 16))) return launch_decode_u<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st);
+    return launch_decode_u<DTYPE, D, DEC_LONG>(p, qbf16, grid, st);
 }
 
 hipError_t launch_decode(const DecodeParams &p, int dtype, int head_dim, bool qbf16, int n_seqs, float *out, hipStream_t st)
 {
     dim3 grid(p.n_splits, p.n_heads, n_seqs);
-    const bool dump = p.dbg != nullptr;
-    if (dtype == TSATTN_I8 && head_dim == 128) launch_decode_dd<TSATTN_I8, 128>(p, qbf16, dump, grid, st);
-    else if (dtype == TSATTN_I8 && head_dim == 64) launch_decode_dd<TSATTN_I8, 64>(p, qbf16, dump, grid, st);
-    else if (dtype == TSATTN_E4M3 && head_dim == 128) launch_decode_dd<TSATTN_E4M3, 128>(p, qbf16, dump, grid, st);
-    else if (dtype == TSATTN_E4M3 && head_dim == 64) launch_decode_dd<TSATTN_E4M3, 64>(p, qbf16, dump, grid, st);
+    hipError_t e;
+    if (dtype == TSATTN_I8 && head_dim == 128) e = launch_decode_dd<TSATTN_I8, 128>(p, qbf16, grid, st);
+    else if (dtype == TSATTN_I8 && head_dim == 64) e = launch_decode_dd<TSATTN_I8, 64>(p, qbf16, grid, st);
+    else if (dtype == TSATTN_E4M3 && head_dim == 128) e = launch_decode_dd<TSATTN_E4M3, 128>(p, qbf16, grid, st);
+    else if (dtype == TSATTN_E4M3 && head_dim == 64) e = launch_decode_dd<TSATTN_E4M3, 64>(p, qbf16, grid, st);
     else return hipErrorInvalidValue;
-    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (p.n_splits == 1) return hipSuccess; // the split kernel wrote the output (and counted a fused append's row) itself
     dim3 mgrid((unsigned)(n_seqs * p.n_heads));
-    int32_t *bump = p.k_new ? p.cache_len_rw : nullptr;
+    int32_t *bump = p.k_new || p.front.src ? p.cache_len_rw : nullptr;
     if (head_dim == 128) hipLaunchKernelGGL((decode_merge_kernel<128>), mgrid, dim3(128), 0, st, p.part_acc, p.part_ml, p.n_splits, out, bump, p.n_heads, p.max_len, p.kv_k, p.kv_k_pitch, p.kv_out, p.kv_out_pitch, p.kv_rep, p.kv_mult);
     else hipLaunchKernelGGL((decode_merge_kernel<64>), mgrid, dim3(64), 0, st, p.part_acc, p.part_ml, p.n_splits, out, bump, p.n_heads, p.max_len, p.kv_k, p.kv_k_pitch, p.kv_out, p.kv_out_pitch, p.kv_rep, p.kv_mult);
     return hipGetLastError();
