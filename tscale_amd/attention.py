@@ -8,6 +8,7 @@ TAttentionVecHistory::AddVectors (:403-408).  torch tensors are used for device 
 arithmetic happens in libtsattn.so.  There is no fallback path: a missing library raises.
 """
 import ctypes
+import functools
 
 import numpy as np
 import torch
@@ -23,12 +24,21 @@ def _stream_ptr():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def _raw_stream():
+    """The current device's current stream, as an integer."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def _scale_arg(s):
-    """tensor -> (pointer, 0.0); python number -> (None, value)."""
+    """tensor -> (tensor, 0.0); python number -> (None, value)."""
     if isinstance(s, torch.Tensor):
         assert s.dtype == torch.float32 and s.is_cuda and s.is_contiguous()
-        return _ptr(s), 0.0
+        return s, 0.0
     return None, float(s)
+
+
+def _new(rows, cols, dtype, device):
+    return torch.empty_strided((rows, cols), (cols, 1), dtype=dtype, device=device)
 
 
 def alibi_layer_schedule(depth, wide_window):
@@ -58,13 +68,16 @@ class AttentionContext:
         h = ctypes.c_void_p()
         capi.check(self.lib.tsattn_create(ctypes.byref(cfg), ctypes.byref(h)))
         self.handle = h
+        self._h = h.value
+        self._count = ctypes.c_int(0)  # where calls write a number of planes
+        self._count_at = ctypes.addressof(self._count)
         self.device = torch.device("cuda", device)
         self._workspace = None  # scratch of the long-span prefill kernel, grown on demand
 
     def close(self):
         if self.handle:
             self.lib.tsattn_destroy(self.handle)
-            self.handle = None
+            self.handle = self._h = None
 
     def __del__(self):
         try:
@@ -79,11 +92,10 @@ class AttentionContext:
         n_rows, hd = x.shape
         src = capi.SRC_F32 if x.dtype == torch.float32 else capi.SRC_BF16
         assert x.dtype in (torch.float32, torch.bfloat16)
-        q = torch.empty((n_rows, hd), dtype=torch.uint8, device=x.device)
-        scale = torch.empty((n_heads, n_rows), dtype=torch.float32, device=x.device)
-        capi.check(self.lib.tsattn_quantize_rows(self.handle, src, dtype, _ptr(x), hd * x.element_size(), n_rows,
-                                                 n_heads, hd // n_heads, _ptr(q), hd, _ptr(scale), n_rows,
-                                                 _stream_ptr()))
+        q = _new(n_rows, hd, torch.uint8, x.device)
+        scale = _new(n_heads, n_rows, torch.float32, x.device)
+        capi.check(capi.native.quantize_rows(self._h, src, dtype, x, hd * (4 if src == capi.SRC_F32 else 2), n_rows, n_heads, hd // n_heads, q, hd, scale,
+                                             n_rows, _raw_stream()))
         return q, scale
 
     def fill_rope_table(self, head_dim, max_len):
@@ -93,28 +105,23 @@ class AttentionContext:
         return host.to(self.device)
 
     def _produce_args(self, n_rows, hd, device, n_heads, dtype, pos, rope, rotate_dir, vec_scale, scale_mult, row_major_scale, relu,
-                      rope_heads, scale_heads, resid, resid_scale):
-        """The producer's arguments (without its source) and its two results."""
-        q = torch.empty((n_rows, hd), dtype=torch.uint8, device=device)
+                      rope_heads, scale_heads, resid, resid_scale, source=(0, None, 0, 0, 0)):
+        """The fields of the producer's arguments (source: dtype, data, pitch, planes, plane stride) and its two results."""
+        q = _new(n_rows, hd, torch.uint8, device)
         n_scale = n_heads if scale_heads is None else scale_heads[1]
-        scale = torch.empty((n_rows, n_scale) if row_major_scale else (n_scale, n_rows), dtype=torch.float32, device=device)
-        a = capi.ProduceArgs()
-        a.dst_dtype = dtype
-        a.n_rows, a.n_heads, a.head_dim = n_rows, n_heads, hd // n_heads
-        a.pos, a.rope = _ptr(pos), _ptr(rope)
-        a.rope_len = 0 if rope is None else rope.shape[0]
-        a.rope_heads = int(rope_heads)
-        a.rotate_dir, a.vec_scale, a.scale_mult = float(rotate_dir), float(vec_scale), float(scale_mult)
-        a.dst, a.dst_pitch = _ptr(q), hd
-        a.scale, a.scale_pitch = _ptr(scale), (1 if row_major_scale else n_rows)
-        a.scale_row_stride = n_scale if row_major_scale else 1
-        if scale_heads is not None:
-            a.scale_head_begin, a.scale_head_count = int(scale_heads[0]), int(scale_heads[1])
-        a.relu = int(bool(relu))
+        if row_major_scale:
+            scale, pitch, stride = _new(n_rows, n_scale, torch.float32, device), 1, n_scale
+        else:
+            scale, pitch, stride = _new(n_scale, n_rows, torch.float32, device), n_rows, 1
+        first, count = (0, 0) if scale_heads is None else (int(scale_heads[0]), int(scale_heads[1]))
+        resid_pitch = 0
         if resid is not None:
             assert resid.dtype == torch.float32 and resid.shape == (n_rows, hd) and resid.stride(1) == 1
-            a.resid, a.resid_pitch, a.resid_scale = _ptr(resid), resid.stride(0), float(resid_scale)
-        return a, q, scale
+            resid_pitch = resid.stride(0)
+        src_dtype, src, src_pitch, planes, plane_stride = source
+        return (src_dtype, dtype, n_rows, n_heads, hd // n_heads, src, src_pitch, pos, rope, 0 if rope is None else rope.shape[0], rotate_dir, vec_scale,
+                scale_mult, q, hd, scale, pitch, stride, int(bool(relu)), planes, plane_stride, int(rope_heads), first, count, resid, resid_pitch,
+                resid_scale), q, scale
 
     def rope_normalize_rows(self, x, n_heads, dtype, pos=None, rope=None, rotate_dir=1.0, vec_scale=1.0 / 24,
                             scale_mult=1.0, row_major_scale=False, relu=False, rope_heads=0, scale_heads=None,
@@ -131,12 +138,10 @@ class AttentionContext:
             assert x.dtype == torch.int32
             planes = x.shape[0]
         n_rows, hd = x.shape[-2:]
-        a, q, scale = self._produce_args(n_rows, hd, x.device, n_heads, dtype, pos, rope, rotate_dir, vec_scale, scale_mult, row_major_scale,
-                                         relu, rope_heads, scale_heads, resid, resid_scale)
-        a.src_dtype = capi.SRC_F32 if x.dtype == torch.float32 else capi.SRC_I32
-        a.src, a.src_pitch = _ptr(x), hd
-        a.src_planes, a.src_plane_stride = planes, n_rows * hd
-        capi.check(self.lib.tsattn_rope_normalize_rows(self.handle, ctypes.byref(a), _stream_ptr()))
+        source = (capi.SRC_F32 if x.dtype == torch.float32 else capi.SRC_I32, x, hd, planes, n_rows * hd)
+        fields, q, scale = self._produce_args(n_rows, hd, x.device, n_heads, dtype, pos, rope, rotate_dir, vec_scale, scale_mult, row_major_scale,
+                                              relu, rope_heads, scale_heads, resid, resid_scale, source)
+        capi.check(capi.calls.rope_normalize_rows(self._h, _raw_stream(), *fields))
         return q, scale
 
     def matmul_normalize(self, a, w, n_heads, dtype, scratch=None, **producer):
@@ -157,26 +162,18 @@ class AttentionContext:
         kw.update(producer)
         ep, q, scale = self._produce_args(m, n, a.device, n_heads, dtype, kw["pos"], kw["rope"], kw["rotate_dir"], kw["vec_scale"], kw["scale_mult"],
                                           kw["row_major_scale"], kw["relu"], kw["rope_heads"], kw["scale_heads"], kw["resid"], kw["resid_scale"])
-        args = capi.MatmulArgs()
-        args.m, args.n, args.k = m, n, k
-        args.a, args.a_pitch = _ptr(a), a.stride(0)
-        args.w, args.w_pitch = _ptr(w), w.stride(0)
-        args.mode, args.scale = capi.MM_I32_PLANES, 1.0
-        args.out, args.out_pitch = _ptr(scratch), n
-        planes = ctypes.c_int(0)
-        args.planes_out = ctypes.pointer(planes)
-        args.epilogue = ctypes.cast(ctypes.pointer(ep), ctypes.c_void_p)
-        capi.check(self.lib.tsattn_matmul_i8(self.handle, ctypes.byref(args), _stream_ptr()))
+        capi.check(capi.calls.matmul_i8(self._h, _raw_stream(), m, n, k, a, a.stride(0), w, w.stride(0), capi.MM_I32_PLANES, 1.0, scratch, n, None, 0,
+                                        self._count_at, capi.calls.rope_normalize_rows.pack(*ep)))
         return q, scale
 
     def kv_product(self, k, value, n_heads, rep=4, mult=1.0):
         """KVProduct (cpu_infer.cpp:320-337): k uint8 (int8 bytes) [n, H*d], value f32/f16 [n, H*d] -> uint8 [n, H*d*rep]."""
         n, hd = k.shape
         assert value.shape == k.shape and value.is_contiguous() and k.stride(1) == 1
-        kv = torch.empty((n, hd * rep), dtype=torch.uint8, device=k.device)
+        kv = _new(n, hd * rep, torch.uint8, k.device)
         vdt = capi.OUT_F16 if value.dtype == torch.float16 else capi.OUT_F32
-        capi.check(self.lib.tsattn_kv_product(self.handle, n, n_heads, hd // n_heads, rep, _ptr(k), k.stride(0), vdt, _ptr(value), hd,
-                                              float(mult), _ptr(kv), hd * rep, _stream_ptr()))
+        capi.check(capi.native.kv_product(self._h, n, n_heads, hd // n_heads, rep, k, k.stride(0), vdt, value, hd, float(mult), kv, hd * rep,
+                                          _raw_stream()))
         return kv
 
     def matmul_i8(self, a, w, mode=capi.MM_I32, scale=1.0, out=None, workspace=None):
@@ -192,29 +189,16 @@ class AttentionContext:
             if out is None:
                 out = torch.empty(room, dtype=torch.int32, device=a.device)
             assert out.is_contiguous() and out.dtype == torch.int32 and out.numel() >= room
-            args = capi.MatmulArgs()
-            args.m, args.n, args.k = m, n, k
-            args.a, args.a_pitch = _ptr(a), a.stride(0)
-            args.w, args.w_pitch = _ptr(w), w.stride(0)
-            args.mode, args.scale = mode, 1.0
-            args.out, args.out_pitch = _ptr(out), n
-            planes = ctypes.c_int(0)
-            args.planes_out = ctypes.pointer(planes)
-            capi.check(self.lib.tsattn_matmul_i8(self.handle, ctypes.byref(args), _stream_ptr()))
-            return out.view(-1)[:planes.value * m * n].view(planes.value, m, n)
+            capi.check(capi.calls.matmul_i8(self._h, _raw_stream(), m, n, k, a, a.stride(0), w, w.stride(0), mode, 1.0, out, n, None, 0, self._count_at))
+            planes = self._count.value if m and n else 0
+            return out.view(-1)[:planes * m * n].view(planes, m, n)
         if out is None:
             assert mode != capi.MM_ADD_SCALED
-            out = torch.empty((m, n), dtype=torch.int32 if mode == capi.MM_I32 else torch.float32, device=a.device)
+            out = _new(m, n, torch.int32 if mode == capi.MM_I32 else torch.float32, a.device)
         assert out.stride(1) == 1 and out.dtype == (torch.int32 if mode == capi.MM_I32 else torch.float32)
-        args = capi.MatmulArgs()
-        args.m, args.n, args.k = m, n, k
-        args.a, args.a_pitch = _ptr(a), a.stride(0)
-        args.w, args.w_pitch = _ptr(w), w.stride(0)
-        args.mode, args.scale = mode, float(scale)
-        args.out, args.out_pitch = _ptr(out), out.stride(0)
-        if workspace is not None:   # a uint8 tensor the caller keeps: room for split-K partial sums when m is small
-            args.workspace, args.workspace_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
-        capi.check(self.lib.tsattn_matmul_i8(self.handle, ctypes.byref(args), _stream_ptr()))
+        # workspace: a uint8 tensor the caller keeps, room for split-K partial sums when m is small
+        room = 0 if workspace is None else workspace.numel() * workspace.element_size()
+        capi.check(capi.calls.matmul_i8(self._h, _raw_stream(), m, n, k, a, a.stride(0), w, w.stride(0), mode, float(scale), out, out.stride(0), workspace, room))
         return out
 
     def embed_rows(self, labels, embed, embed_scale, out=None):
@@ -225,10 +209,10 @@ class AttentionContext:
         n_rows, per_row = labels.shape
         n_labels, dim = embed.shape
         if out is None:
-            out = torch.empty((n_rows, dim), dtype=torch.float32, device=embed.device)
+            out = _new(n_rows, dim, torch.float32, embed.device)
         assert labels.dtype == torch.int32 and labels.is_contiguous() and embed.stride(1) == 1 and out.stride(1) == 1
-        capi.check(self.lib.tsattn_embed_rows(self.handle, n_rows, dim, _ptr(labels), per_row, _ptr(embed), embed.stride(0), n_labels,
-                                              float(embed_scale), _ptr(out), out.stride(0), _stream_ptr()))
+        capi.check(capi.native.embed_rows(self._h, n_rows, dim, labels, per_row, embed, embed.stride(0), n_labels, float(embed_scale), out, out.stride(0),
+                                          _raw_stream()))
         return out
 
     def softmax_rows(self, vec, scale, bias=None, want_prob=True, argmax=None):
@@ -237,11 +221,10 @@ class AttentionContext:
         planes = vec.shape[0] if vec.dim() == 3 else 1
         n_rows, n = vec.shape[-2:]
         assert vec.dtype == torch.int32 and vec.is_contiguous()
-        prob = torch.empty((n_rows, n), dtype=torch.float32, device=vec.device) if want_prob else None
+        prob = _new(n_rows, n, torch.float32, vec.device) if want_prob else None
         if argmax is None:
-            argmax = torch.empty(n_rows, dtype=torch.int32, device=vec.device)
-        capi.check(self.lib.tsattn_softmax_rows(self.handle, n_rows, n, _ptr(vec), planes, n_rows * n, n, float(scale), _ptr(bias),
-                                                _ptr(prob), n, _ptr(argmax), _stream_ptr()))
+            argmax = torch.empty_strided((n_rows,), (1,), dtype=torch.int32, device=vec.device)
+        capi.check(capi.native.softmax_rows(self._h, n_rows, n, vec, planes, n_rows * n, n, float(scale), bias, prob, n, argmax, _raw_stream()))
         return prob, argmax
 
     def sample_rows(self, prob, temperature, rnd=None, seed=0, offset=0, choice=None):
@@ -252,26 +235,23 @@ class AttentionContext:
         if rnd is not None:
             assert rnd.shape == prob.shape and rnd.element_size() == 4 and rnd.stride(1) == 1
         if choice is None:
-            choice = torch.empty(n_rows, dtype=torch.int32, device=prob.device)
-        capi.check(self.lib.tsattn_sample_rows(self.handle, n_rows, n, _ptr(prob), prob.stride(0), float(temperature), _ptr(rnd),
-                                               rnd.stride(0) if rnd is not None else 0, int(seed), int(offset), _ptr(choice),
-                                               _stream_ptr()))
+            choice = torch.empty_strided((n_rows,), (1,), dtype=torch.int32, device=prob.device)
+        capi.check(capi.native.sample_rows(self._h, n_rows, n, prob, prob.stride(0), float(temperature), rnd, rnd.stride(0) if rnd is not None else 0,
+                                           int(seed), int(offset), choice, _raw_stream()))
         return choice
 
     def build_spans(self, seq_offset, n_tokens, window, doc_start_flag=None):
         """seq_offset: int32 [n_seqs+1] on the device.  Returns (span_start, span_finish) int32 [n_tokens]."""
-        st = torch.empty(n_tokens, dtype=torch.int32, device=self.device)
-        fi = torch.empty(n_tokens, dtype=torch.int32, device=self.device)
-        capi.check(self.lib.tsattn_build_spans(self.handle, seq_offset.numel() - 1, _ptr(seq_offset), n_tokens,
-                                               _ptr(doc_start_flag), int(window), _ptr(st), _ptr(fi), _stream_ptr()))
+        st = torch.empty_strided((n_tokens,), (1,), dtype=torch.int32, device=self.device)
+        fi = torch.empty_strided((n_tokens,), (1,), dtype=torch.int32, device=self.device)
+        capi.check(capi.native.build_spans(self._h, seq_offset.numel() - 1, seq_offset, n_tokens, doc_start_flag, int(window), st, fi, _raw_stream()))
         return st, fi
 
     def build_span_tiles(self, span_start, span_finish):
         """Per-128-row summary of a span list for compute_val_lookup(span_tiles=...); build once per batch and mask."""
         n = span_start.numel()
-        tiles = torch.empty((self.lib.tsattn_span_tiles_count(n), capi.SPAN_TILE_INTS), dtype=torch.int32, device=self.device)
-        capi.check(self.lib.tsattn_build_span_tiles(self.handle, n, _ptr(span_start), _ptr(span_finish), _ptr(tiles),
-                                                    _stream_ptr()))
+        tiles = _new((n + 127) // 128, capi.SPAN_TILE_INTS, torch.int32, self.device)
+        capi.check(capi.native.build_span_tiles(self._h, n, span_start, span_finish, tiles, _raw_stream()))
         return tiles
 
     # ---- prefill --------------------------------------------------------------------------------
@@ -292,40 +272,30 @@ class AttentionContext:
         d = hd // n_heads
         assert want_out or kv_product is not None
         if out is None and want_out:
-            out = torch.empty((n_tokens, hd), dtype=torch.float16 if out_f16 else torch.float32, device=q.device)
-        a = capi.PrefillArgs()
-        a.dtype = dtype
-        a.out_dtype = capi.OUT_F16 if (out is not None and out.dtype == torch.float16) else capi.OUT_F32
-        a.n_tokens, a.n_heads, a.head_dim = n_tokens, n_heads, d
-        a.q, a.k, a.v = _ptr(q), _ptr(k), _ptr(v)
-        a.q_pitch, a.k_pitch, a.v_pitch = q.stride(0), k.stride(0), v.stride(0)
-        a.q_scale, a.q_scale_const = _scale_arg(q_scale)
-        a.k_scale, a.k_scale_const = _scale_arg(k_scale)
-        a.v_scale, a.v_scale_const = _scale_arg(v_scale)
-        pitches = [s.stride(0) for s in (q_scale, k_scale, v_scale, sum_weight_log) if isinstance(s, torch.Tensor)]
-        assert len(set(pitches)) <= 1, "all scale planes must share one pitch"
-        a.scale_pitch = pitches[0] if pitches else n_tokens
-        a.k_global_scale = _ptr(k_global_scale)
-        a.span_start, a.span_finish = _ptr(span_start), _ptr(span_finish)
+            out = _new(n_tokens, hd, torch.float16 if out_f16 else torch.float32, q.device)
+        qs, qs_const = _scale_arg(q_scale)
+        ks, ks_const = _scale_arg(k_scale)
+        vs, vs_const = _scale_arg(v_scale)
+        pitch = None
+        for plane in (qs, ks, vs, sum_weight_log):
+            if plane is not None:
+                at = plane.stride(0)
+                assert pitch is None or at == pitch, "all scale planes must share one pitch"
+                pitch = at
+        parts = part_stride = 0
         if span_start.dim() == 2:      # rows with several spans: [n_parts, n_tokens], part i = every row's i-th span
             assert span_finish.shape == span_start.shape and span_start.stride(1) == 1 and span_finish.stride() == span_start.stride()
-            a.n_span_parts, a.span_part_stride = span_start.shape[0], span_start.stride(0)
+            parts, part_stride = span_start.shape[0], span_start.stride(0)
             assert span_tiles is None or (span_tiles.is_contiguous() and span_tiles.shape[0] == span_start.shape[0])
-        a.alibi_slope = float(alibi_slope)
-        if out is not None:
-            a.out, a.out_pitch = _ptr(out), out.stride(0) * out.element_size()
-        a.sum_weight_log = _ptr(sum_weight_log)
-        if debug_qk_acc is not None:
-            a.debug_qk_acc, a.debug_pitch = _ptr(debug_qk_acc), debug_qk_acc.stride(1)
+        out_f16 = out is not None and out.dtype == torch.float16
+        kv_k = kv_out = None
+        kv_k_pitch = kv_out_pitch = kv_rep = 0
+        kv_mult = 0.0
         if kv_product is not None:
             kv_k, kv_out, kv_rep, kv_mult = kv_product
             assert kv_k.stride(1) == 1 and kv_out.stride(1) == 1
-            a.kv_k, a.kv_k_pitch = _ptr(kv_k), kv_k.stride(0)
-            a.kv_out, a.kv_out_pitch = _ptr(kv_out), kv_out.stride(0)
-            a.kv_rep, a.kv_mult = int(kv_rep), float(kv_mult)
-        a.causal_period = int(causal_period)
-        a.span_tiles = _ptr(span_tiles)
-        a.span_len_hint = int(span_len_hint)
+            kv_k_pitch, kv_out_pitch = kv_k.stride(0), kv_out.stride(0)
+        room = 0
         if span_len_hint >= capi.PREFILL_LONG_SPAN:
             need = int(self.lib.tsattn_prefill_workspace_bytes(n_tokens, n_heads, d))
             if workspace is None and need > 0:
@@ -333,8 +303,15 @@ class AttentionContext:
                     self._workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
                 workspace = self._workspace
             if workspace is not None:
-                a.workspace, a.workspace_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
-        capi.check(self.lib.tsattn_prefill(self.handle, ctypes.byref(a), _stream_ptr()))
+                room = workspace.numel() * workspace.element_size()
+        else:
+            workspace = None
+        capi.check(capi.calls.prefill(
+            self._h, _raw_stream(), dtype, capi.OUT_F16 if out_f16 else capi.OUT_F32, n_tokens, n_heads, d, q, k, v, q.stride(0), k.stride(0), v.stride(0),
+            qs, ks, vs, n_tokens if pitch is None else pitch, qs_const, ks_const, vs_const, k_global_scale, span_start, span_finish, float(alibi_slope),
+            out, 0 if out is None else out.stride(0) * (2 if out_f16 else out.element_size()), sum_weight_log,
+            debug_qk_acc, 0 if debug_qk_acc is None else debug_qk_acc.stride(1), span_tiles, int(causal_period),
+            kv_k, kv_k_pitch, kv_out, kv_out_pitch, int(kv_rep), float(kv_mult), workspace, room, int(span_len_hint), parts, part_stride))
         return out
 
     def merge_lookups(self, part_out, part_swl, out=None, out_f16=False, sum_weight_log=None):
@@ -394,45 +371,39 @@ class AttentionContext:
         static_scratch: go through tsattn_decode_static, the entry point that needs no handle and allocates nothing."""
         B, H, d = cache.n_seqs, cache.n_heads, cache.head_dim
         if out is None:
-            out = torch.empty((B, H * d), dtype=torch.float32, device=q.device)
-        a = capi.DecodeArgs()
-        a.dtype = cache.dtype
-        a.q_dtype = capi.Q_BF16 if q.dtype == torch.bfloat16 else capi.Q_8BIT
-        a.n_seqs, a.n_heads, a.head_dim = B, H, d
-        a.q, a.q_pitch = _ptr(q), q.stride(0) * q.element_size()
-        a.q_scale, a.q_scale_const = _scale_arg(q_scale if q_scale is not None else 1.0)
-        a.k_cache, a.v_cache = _ptr(cache.k), _ptr(cache.v)
-        a.seq_stride, a.head_stride, a.tok_stride = cache.k.stride(0), cache.k.stride(1), cache.k.stride(2)
-        a.k_scale, a.k_scale_const = _scale_arg(cache.k_scale)
-        a.v_scale, a.v_scale_const = _scale_arg(cache.v_scale)
-        if isinstance(cache.k_scale, torch.Tensor):
-            a.s_seq_stride, a.s_head_stride = cache.k_scale.stride(0), cache.k_scale.stride(1)
-        a.cache_len = _ptr(cache.cache_len)
-        a.max_len = cache.max_len if max_len is None else int(max_len)
-        a.window = int(window)
-        a.alibi_slope = float(alibi_slope)
-        a.out = _ptr(out)
-        a.n_splits = int(n_splits)
-        if debug_qk_acc is not None:
-            a.debug_qk_acc, a.debug_pitch = _ptr(debug_qk_acc), debug_qk_acc.stride(1)
-        if append is not None:
-            k_new, ks_new, v_new, vs_new = append
-            a.k_new, a.v_new, a.new_pitch = _ptr(k_new), _ptr(v_new), k_new.stride(0)
-            a.k_scale_new, a.v_scale_new = _ptr(ks_new), _ptr(vs_new)
-        if kv_product is not None:
-            kk, kv_out, rep, mult = kv_product
-            a.kv_k, a.kv_k_pitch, a.kv_out, a.kv_out_pitch = _ptr(kk), kk.stride(0), _ptr(kv_out), kv_out.stride(0)
-            a.kv_rep, a.kv_mult = int(rep), float(mult)
+            out = _new(B, H * d, torch.float32, q.device)
+        bf16 = q.dtype == torch.bfloat16
+        qs, qs_const = _scale_arg(q_scale if q_scale is not None else 1.0)
+        ks, ks_const = _scale_arg(cache.k_scale)
+        vs, vs_const = _scale_arg(cache.v_scale)
+        seq_stride, head_stride, tok_stride, _ = cache.k.stride()
+        s_seq_stride, s_head_stride, _ = (0, 0, 0) if ks is None else ks.stride()
+        fields = (cache.dtype, capi.Q_BF16 if bf16 else capi.Q_8BIT, B, H, d, q, q.stride(0) * (2 if bf16 else q.element_size()), qs, qs_const,
+                  cache.k, cache.v, seq_stride, head_stride, tok_stride, ks, vs, s_seq_stride, s_head_stride, ks_const, vs_const, cache.cache_len,
+                  cache.max_len if max_len is None else int(max_len), int(window), float(alibi_slope), out, int(n_splits))
+        if debug_qk_acc is not None or append is not None or kv_product is not None:
+            k_new, ks_new, v_new, vs_new = append if append is not None else (None, None, None, None)
+            kk, kv_out, rep, mult = kv_product if kv_product is not None else (None, None, 0, 0.0)
+            fields += (debug_qk_acc, 0 if debug_qk_acc is None else debug_qk_acc.stride(1), k_new, v_new, 0 if k_new is None else k_new.stride(0),
+                       ks_new, vs_new, kk, 0 if kk is None else kk.stride(0), kv_out, 0 if kk is None else kv_out.stride(0), int(rep), float(mult))
         if static_scratch:
+            a = capi.DecodeArgs.from_buffer_copy(capi.calls.decode.pack(*fields))
             capi.check(self.lib.tsattn_decode_static(ctypes.byref(a), _stream_ptr()))
         else:
-            capi.check(self.lib.tsattn_decode(self.handle, ctypes.byref(a), _stream_ptr()))
+            capi.check(capi.calls.decode(self._h, _raw_stream(), *fields))
         return out
 
 
 VEC_SCALE = 1.0 / 24      # gpt/train/cpu_infer.cpp:16
 STATE_NORM_TILE = 128     # gpt/model_params/model_dim.h:22
 COMBINER_REP = 4          # gpt/model_params/model_dim.h:12
+
+
+@functools.lru_cache(maxsize=4096)
+def _product_scale(scale, width):
+    """A matrix's scale times VEC_SCALE * CalcDotScale(width), in single precision as the reference multiplies it up."""
+    f32 = np.float32
+    return float(f32(scale) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(width))))
 
 
 def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratch=None, pending=None, defer=False):
@@ -450,7 +421,6 @@ def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratc
     H, d = cache.n_heads, cache.head_dim
     qsum = H * d
     groups = dim // STATE_NORM_TILE
-    f32 = np.float32
     sc = scratch if scratch is not None else {}
     fused = _layer_token(ctx, layer, cache, t, rope, state, sc, pending)
     if fused is not None:
@@ -468,7 +438,7 @@ def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratc
         norm, _ = ctx.rope_normalize_rows(state, groups, capi.I8)
     # the four projections as one product; RoPE on the qk and qv heads, per-head normalisation of all four in one call
     proj = ctx.matmul_i8(norm, layer["proj"], mode=capi.MM_I32_PLANES, out=planes_buf)
-    key_mult = float(f32(layer["qv_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(dim))))
+    key_mult = _product_scale(layer["qv_scale"], dim)
     q4, qv_scale = ctx.rope_normalize_rows(proj, 4 * H, capi.I8, pos=t, rope=rope, scale_mult=key_mult, row_major_scale=True,
                                            rope_heads=2 * H, scale_heads=(H, H))
     qk, qv, k, v = q4[:, :qsum], q4[:, qsum:2 * qsum], q4[:, 2 * qsum:3 * qsum], q4[:, 3 * qsum:]
@@ -486,11 +456,11 @@ def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratc
     # combiner; its AddScaled is done by the normalisation that follows
     delta = ctx.matmul_i8(kv, layer["combiner"], mode=capi.MM_I32_PLANES, out=planes_buf)
     norm, _ = ctx.rope_normalize_rows(delta, groups, capi.I8, resid=state,
-                                      resid_scale=float(f32(layer["combiner_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(qsum * COMBINER_REP)))))
+                                      resid_scale=_product_scale(layer["combiner_scale"], qsum * COMBINER_REP))
     relu_src = ctx.matmul_i8(norm, layer["expand"], mode=capi.MM_I32_PLANES, out=planes_buf)
     relu, _ = ctx.rope_normalize_rows(relu_src, H, capi.I8, relu=True)
     relu_dim = relu_src.shape[-1]
-    contract_scale = float(f32(layer["contract_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(relu_dim))))
+    contract_scale = _product_scale(layer["contract_scale"], relu_dim)
     if defer:
         parts = ctx.matmul_i8(relu, layer["contract"], mode=capi.MM_I32_PLANES, out=planes_buf)
         return val, (parts, contract_scale)
@@ -517,34 +487,21 @@ def _layer_token(ctx, layer, cache, t, rope, state, sc, pending):
             return None
         room = sc["fused"] = torch.empty(need, dtype=torch.uint8, device=state.device)
         sc["fused_shape"] = (B, H, d, dim, relu_dim)
-        sc["parts"] = torch.empty((4, B, dim), dtype=torch.int32, device=state.device)
+        planes = torch.empty((4, B, dim), dtype=torch.int32, device=state.device)
+        sc["parts"] = {n: planes[:n] for n in (1, 2, 4)}
         sc["val"] = torch.empty((B, qsum), dtype=torch.float32, device=state.device)
     assert proj.shape == (4 * qsum, dim) and combiner.shape == (dim, 4 * qsum) and expand.shape == (relu_dim, dim) and contract.shape == (dim, relu_dim)
     assert t.dtype == torch.int32 and state.dtype == torch.float32 and cache.n_seqs == B
-    f32 = np.float32
-    a = capi.LayerArgs()
-    a.n_seqs, a.n_heads, a.head_dim, a.dim, a.relu_dim = B, H, d, dim, relu_dim
-    a.proj, a.combiner, a.expand, a.contract = proj.data_ptr(), combiner.data_ptr(), expand.data_ptr(), contract.data_ptr()
-    a.vec_scale = VEC_SCALE
-    a.key_mult = float(f32(layer["qv_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(dim))))
-    a.combiner_scale = float(f32(layer["combiner_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(qsum * COMBINER_REP))))
-    a.pos, a.rope, a.rope_len = t.data_ptr(), rope.data_ptr(), rope.shape[0]
-    a.k_cache, a.v_cache = cache.k.data_ptr(), cache.v.data_ptr()
-    a.seq_stride, a.head_stride, a.tok_stride, _ = cache.k.stride()
-    a.k_scale, a.v_scale = cache.k_scale.data_ptr(), cache.v_scale.data_ptr()
-    a.s_seq_stride, a.s_head_stride, _ = cache.k_scale.stride()
-    a.cache_len, a.max_len = cache.cache_len.data_ptr(), cache.max_len
-    a.window, a.alibi_slope = int(layer["width"]), float(layer["slope"])
-    a.state, a.state_pitch = state.data_ptr(), state.stride(0)
     parts, val = sc["parts"], sc["val"]
-    a.val, a.parts = val.data_ptr(), parts.data_ptr()
-    if pending is not None:
-        a.pending, a.pending_planes, a.pending_scale = pending[0].data_ptr(), pending[0].shape[0], pending[1]
-    n_parts = ctypes.c_int(0)
-    a.n_parts = ctypes.pointer(n_parts)
-    a.scratch, a.scratch_bytes = room.data_ptr(), room.numel()
-    capi.check(ctx.lib.tsattn_layer_token(ctx.handle, ctypes.byref(a), _stream_ptr()))
-    return val, (parts[:n_parts.value], float(f32(layer["contract_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(relu_dim)))))
+    seq_stride, head_stride, tok_stride, _ = cache.k.stride()
+    s_seq_stride, s_head_stride, _ = cache.k_scale.stride()
+    planes, planes_scale = (None, 0.0) if pending is None else pending
+    capi.check(capi.calls.layer_token(
+        ctx._h, _raw_stream(), B, H, d, dim, relu_dim, proj, combiner, expand, contract, VEC_SCALE, _product_scale(layer["qv_scale"], dim),
+        _product_scale(layer["combiner_scale"], qsum * COMBINER_REP), t, rope, rope.shape[0], cache.k, cache.v, seq_stride, head_stride, tok_stride,
+        cache.k_scale, cache.v_scale, s_seq_stride, s_head_stride, 0.0, cache.cache_len, cache.max_len, int(layer["width"]), float(layer["slope"]),
+        state, state.stride(0), val, planes, 0 if planes is None else planes.shape[0], planes_scale, parts[4], ctx._count_at, room, room.numel()))
+    return val, (parts[ctx._count.value], _product_scale(layer["contract_scale"], relu_dim))
 
 
 def flush_state(ctx, pending, state):
@@ -569,12 +526,11 @@ def add_lookup_product_prompt(ctx, layer, cache, seq_offset, pos, rope, state, s
     H, d = cache.n_heads, cache.head_dim
     qsum = H * d
     groups = dim // STATE_NORM_TILE
-    f32 = np.float32
     if norm is None:
         norm, _ = ctx.rope_normalize_rows(state, groups, capi.I8)
     # every product with its normalisation as epilogue (large products never write their int32 sums); one scratch
     # buffer for whichever falls back to two launches
-    key_mult = float(f32(layer["qv_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(dim))))
+    key_mult = _product_scale(layer["qv_scale"], dim)
     room = torch.empty((16 if n <= 128 else 1) * n * max(4 * qsum, dim, layer["expand"].shape[0]), dtype=torch.int32, device=state.device)
     q4, qv_scale = ctx.matmul_normalize(norm, layer["proj"], 4 * H, capi.I8, room, pos=pos, rope=rope, scale_mult=key_mult,
                                         rope_heads=2 * H, scale_heads=(H, H))      # scales as [head][token] planes
@@ -586,11 +542,11 @@ def add_lookup_product_prompt(ctx, layer, cache, seq_offset, pos, rope, state, s
                                  want_out=want_val)
     cache.fill_from_prefill(seq_offset, qv, qv_scale, v)       # value scales: the cache's constant VEC_SCALE
     norm, _ = ctx.matmul_normalize(kv, layer["combiner"], groups, capi.I8, room, resid=state,
-                                   resid_scale=float(f32(layer["combiner_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(qsum * COMBINER_REP)))))
+                                   resid_scale=_product_scale(layer["combiner_scale"], qsum * COMBINER_REP))
     del kv
     relu, _ = ctx.matmul_normalize(norm, layer["expand"], H, capi.I8, room, relu=True)
     relu_dim = relu.shape[-1]
-    contract_scale = float(f32(layer["contract_scale"]) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(relu_dim))))
+    contract_scale = _product_scale(layer["contract_scale"], relu_dim)
     if want_norm:   # state += product * scale, and the updated state normalised for whoever comes next
         norm_next, _ = ctx.matmul_normalize(relu, layer["contract"], groups, capi.I8, room, resid=state, resid_scale=contract_scale)
         return val, norm_next
@@ -618,35 +574,25 @@ class KVCache:
 
     def add_vectors(self, k_new, k_scale_new, v_new, v_scale_new=None):
         """k_new, v_new: uint8 [n_seqs, n_heads*d]; scales f32 [n_seqs, n_heads] (None with constant scales)."""
-        a = capi.AppendArgs()
-        a.n_seqs, a.n_heads, a.head_dim = self.n_seqs, self.n_heads, self.head_dim
-        a.k_new, a.v_new, a.new_pitch = _ptr(k_new), _ptr(v_new), k_new.stride(0)
-        a.k_scale_new, a.v_scale_new = _ptr(k_scale_new), _ptr(v_scale_new)
-        a.k_cache, a.v_cache = _ptr(self.k), _ptr(self.v)
-        a.seq_stride, a.head_stride, a.tok_stride = self.k.stride(0), self.k.stride(1), self.k.stride(2)
-        if isinstance(self.k_scale, torch.Tensor):
-            a.k_scale, a.v_scale = _ptr(self.k_scale), _ptr(self.v_scale)
-            a.s_seq_stride, a.s_head_stride = self.k_scale.stride(0), self.k_scale.stride(1)
-        a.cache_len, a.max_len = _ptr(self.cache_len), self.max_len
-        capi.check(self.ctx.lib.tsattn_cache_append(self.ctx.handle, ctypes.byref(a), _stream_ptr()))
+        seq_stride, head_stride, tok_stride, _ = self.k.stride()
+        planes = isinstance(self.k_scale, torch.Tensor)
+        s_seq_stride, s_head_stride, _ = self.k_scale.stride() if planes else (0, 0, 0)
+        capi.check(capi.calls.cache_append(
+            self.ctx._h, _raw_stream(), self.n_seqs, self.n_heads, self.head_dim, k_new, v_new, k_new.stride(0), k_scale_new, v_scale_new, self.k, self.v,
+            seq_stride, head_stride, tok_stride, self.k_scale if planes else None, self.v_scale if planes else None, s_seq_stride, s_head_stride,
+            self.cache_len, self.max_len))
 
     def fill_from_prefill(self, seq_offset, k, k_scale, v, v_scale=None):
         """Append a prefill batch: k, v uint8 [n_tokens, n_heads*d]; scales f32 [n_heads, n_tokens] planes (None
         with constant scales); seq_offset int32 [n_seqs+1] on the device.  Equals add_vectors once per token."""
-        a = capi.FillArgs()
-        a.n_seqs, a.n_heads, a.head_dim = self.n_seqs, self.n_heads, self.head_dim
-        a.n_tokens = k.shape[0]
-        a.seq_offset = _ptr(seq_offset)
-        a.k, a.v, a.pitch = _ptr(k), _ptr(v), k.stride(0)
+        n_tokens = k.shape[0]
         assert v.stride(0) == k.stride(0)
-        a.k_scale, a.v_scale = _ptr(k_scale), _ptr(v_scale)
-        pitches = [s.stride(0) for s in (k_scale, v_scale) if s is not None]
+        pitches = [p.stride(0) for p in (k_scale, v_scale) if p is not None]
         assert len(set(pitches)) <= 1
-        a.scale_pitch = pitches[0] if pitches else a.n_tokens
-        a.k_cache, a.v_cache = _ptr(self.k), _ptr(self.v)
-        a.seq_stride, a.head_stride, a.tok_stride = self.k.stride(0), self.k.stride(1), self.k.stride(2)
-        if isinstance(self.k_scale, torch.Tensor):
-            a.k_scale_cache, a.v_scale_cache = _ptr(self.k_scale), _ptr(self.v_scale)
-            a.s_seq_stride, a.s_head_stride = self.k_scale.stride(0), self.k_scale.stride(1)
-        a.cache_len, a.max_len = _ptr(self.cache_len), self.max_len
-        capi.check(self.ctx.lib.tsattn_cache_fill(self.ctx.handle, ctypes.byref(a), _stream_ptr()))
+        seq_stride, head_stride, tok_stride, _ = self.k.stride()
+        planes = isinstance(self.k_scale, torch.Tensor)
+        s_seq_stride, s_head_stride, _ = self.k_scale.stride() if planes else (0, 0, 0)
+        capi.check(capi.calls.cache_fill(
+            self.ctx._h, _raw_stream(), self.n_seqs, self.n_heads, self.head_dim, n_tokens, seq_offset, k, v, k.stride(0), k_scale, v_scale,
+            pitches[0] if pitches else n_tokens, self.k, self.v, seq_stride, head_stride, tok_stride, self.k_scale if planes else None,
+            self.v_scale if planes else None, s_seq_stride, s_head_stride, self.cache_len, self.max_len))

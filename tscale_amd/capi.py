@@ -5,6 +5,7 @@ no CPU fallback; if the library is missing or a call fails, it raises.
 """
 import ctypes
 import os
+import struct
 
 _c = ctypes
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -207,8 +208,35 @@ def load():
         L.tsattn_build_spans.restype = _c.c_int
         L.tsattn_build_spans.argtypes = [_c.c_void_p, _c.c_int, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64,
                                          _c.c_void_p, _c.c_void_p, _c.c_void_p]
+        _bind_native(L)
         _lib = L
     return _lib
+
+
+class _Calls:
+    """Entry points that take an argument struct, as callables (handle, stream, field values in the struct's order): filled in
+    when the library is loaded.  The flat entry points are functions of the extension itself (`native`)."""
+
+
+calls = _Calls()
+native = None
+
+
+def _bind_native(L):
+    global native
+    try:
+        from . import _native
+    except ImportError as e:
+        raise FileNotFoundError("tscale_amd/_native.so is missing: build it with `make -C tscale_amd/csrc`") from e
+    kinds = {_c.c_int: "i", _c.c_int64: "q", _c.c_float: "f"}
+    address = lambda name: _c.cast(getattr(L, name), _c.c_void_p).value
+    for name, cls in (("prefill", PrefillArgs), ("decode", DecodeArgs), ("cache_append", AppendArgs), ("cache_fill", FillArgs),
+                      ("rope_normalize_rows", ProduceArgs), ("matmul_i8", MatmulArgs), ("layer_token", LayerArgs)):
+        fields = b"".join(struct.pack("<HB", getattr(cls, f).offset, ord(kinds.get(t, "p"))) for f, t in cls._fields_)
+        setattr(calls, name, _native.Call(address("tsattn_" + name), _c.sizeof(cls), fields))
+    _native.bind(*(address("tsattn_" + n) for n in ("quantize_rows", "build_spans", "build_span_tiles", "embed_rows", "softmax_rows", "sample_rows",
+                                                    "kv_product")))
+    native = _native
 
 
 def check(code):

@@ -15,6 +15,7 @@
 struct tsattn_ctx {
     int device;
     int max_seqs, max_heads, max_head_dim, max_splits;
+    void *mem; // the handle's one allocation, in which:
     float *part_acc;
     float *part_ml;
     int32_t *seq_done;
@@ -184,41 +185,43 @@ int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
     if (cfg->device < 0 || cfg->device >= n_dev) return fail(TSATTN_ERR_BAD_ARG, "tsattn_create: device %d of %d", cfg->device, n_dev);
     e = hipSetDevice(cfg->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
-    e = tsattn::prepare_matmul_i8();
-    if (e == hipSuccess) e = tsattn::prepare_prefill_long();
-    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");
+    {
+        // the kernels' LDS limits: once per device and process, and not again for every handle (some 60 runtime calls)
+        static std::mutex prepared_mutex;
+        static bool prepared[STATIC_MAX_DEVICES];
+        std::lock_guard<std::mutex> lock(prepared_mutex);
+        if (cfg->device >= STATIC_MAX_DEVICES || !prepared[cfg->device]) {
+            e = tsattn::prepare_matmul_i8();
+            if (e == hipSuccess) e = tsattn::prepare_prefill_long();
+            if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute");
+            if (cfg->device < STATIC_MAX_DEVICES) prepared[cfg->device] = true;
+        }
+    }
     tsattn_ctx *c = new tsattn_ctx();
     c->device = cfg->device;
     c->max_seqs = cfg->max_seqs;
     c->max_heads = cfg->max_heads;
     c->max_head_dim = cfg->max_head_dim;
     c->max_splits = cfg_splits(cfg);
-    c->part_acc = nullptr;
-    c->part_ml = nullptr;
-    c->seq_done = nullptr;
-    c->head = nullptr;
-    e = hipMalloc(&c->head, tsattn::HEAD_SCRATCH_BYTES);
-    if (e != hipSuccess) { delete c; return hip_fail(e, "hipMalloc(row records)"); }
-    size_t parts = (size_t)c->max_seqs * c->max_heads * c->max_splits;
-    if (parts > 0 && c->max_head_dim > 0) {
-        e = hipMalloc((void **)&c->part_acc, parts * c->max_head_dim * sizeof(float));
-        if (e != hipSuccess) { (void)hipFree(c->head); delete c; return hip_fail(e, "hipMalloc(split partials)"); }
-        e = hipMalloc((void **)&c->part_ml, parts * 2 * sizeof(float));
-        if (e != hipSuccess) { (void)hipFree(c->head); (void)hipFree(c->part_acc); delete c; return hip_fail(e, "hipMalloc(split max/sum)"); }
+    // one allocation: row records, arrival counters of the single-split fused append (zero here, and left at zero by every
+    // launch), split maxima and sums, split partials
+    const size_t parts = c->max_head_dim > 0 ? (size_t)c->max_seqs * c->max_heads * c->max_splits : 0;
+    const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t cnt_at = up(tsattn::HEAD_SCRATCH_BYTES), ml_at = cnt_at + up((size_t)c->max_seqs * sizeof(int32_t)),
+                 acc_at = ml_at + up(parts * 2 * sizeof(float)), total = acc_at + parts * c->max_head_dim * sizeof(float);
+    uint8_t *mem = nullptr;
+    e = hipMalloc((void **)&mem, total);
+    if (e == hipSuccess && c->max_seqs > 0) e = hipMemset(mem + cnt_at, 0, (size_t)c->max_seqs * sizeof(int32_t));
+    if (e != hipSuccess) {
+        if (mem) (void)hipFree(mem);
+        delete c;
+        return hip_fail(e, "hipMalloc(handle scratch)");
     }
-    if (c->max_seqs > 0) {
-        // arrival counters of the single-split fused append: zero here, and left at zero by every launch
-        e = hipMalloc((void **)&c->seq_done, (size_t)c->max_seqs * sizeof(int32_t));
-        if (e == hipSuccess) e = hipMemset(c->seq_done, 0, (size_t)c->max_seqs * sizeof(int32_t));
-        if (e != hipSuccess) {
-            (void)hipFree(c->head);
-            if (c->seq_done) (void)hipFree(c->seq_done);
-            if (c->part_acc) (void)hipFree(c->part_acc);
-            if (c->part_ml) (void)hipFree(c->part_ml);
-            delete c;
-            return hip_fail(e, "hipMalloc(arrival counters)");
-        }
-    }
+    c->mem = mem;
+    c->head = mem;
+    c->seq_done = (int32_t *)(mem + cnt_at);
+    c->part_ml = (float *)(mem + ml_at);
+    c->part_acc = (float *)(mem + acc_at);
     *out = c;
     return TSATTN_OK;
 }
@@ -226,10 +229,7 @@ int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
 int tsattn_destroy(tsattn_handle_t h)
 {
     if (!h) return TSATTN_OK;
-    if (h->part_acc) (void)hipFree(h->part_acc);
-    if (h->part_ml) (void)hipFree(h->part_ml);
-    if (h->seq_done) (void)hipFree(h->seq_done);
-    if (h->head) (void)hipFree(h->head);
+    (void)hipFree(h->mem);
     delete h;
     return TSATTN_OK;
 }
