@@ -3,8 +3,8 @@
 // MulForward (gpt/train/cpu_infer.cpp:294-305: one weight row per output, exact int32 sums, result as int32 or
 // converted to float) and AddScaled (:308-316: state += delta * scale).
 //
-// Many rows (a prompt): 128 x 128 or 256 x 256 output tiles, K in steps of 64 bytes through LDS,
-// v_mfma_i32_32x32x32_i8; bound by the matrix cores.  Few rows (one token per sequence): gemm_few.hpp.
+// Here the largest products (256 x 256 output tiles; bound by the matrix cores) and the choice between the kernels; a few
+// hundred to a few thousand rows: gemm_mid.hip, few rows (one token per sequence): gemm_few.hpp.
 // Integer sums are exact, so every decomposition gives the same bits.
 #include <type_traits>
 #include "common.hpp"
@@ -13,10 +13,6 @@
 namespace tsattn {
 
 namespace {
-
-constexpr int GT_THREADS = 256;
-constexpr int GT_BN = 128, GT_BK = 64;
-constexpr int GT_PITCH = GT_BK + 16; // LDS row pitch: 16-lane phases of a 16-byte read hit distinct banks
 
 __device__ inline __amdgpu_buffer_rsrc_t rows_rsrc(const void *base, int64_t rows, int64_t pitch, int64_t row_bytes)
 {
@@ -38,137 +34,6 @@ __device__ inline void store_out(const GemmParams &p, int64_t m, int64_t n, int 
         float *o = (float *)p.out + m * p.out_pitch + n;
         *o += (float)acc * p.scale; // (*pRes)[k] += delta[k] * scale
     }
-}
-
-// ---- many rows --------------------------------------------------------------------------------------------------
-// Products too small for the wide tiles below: output tiles of 64 MT x 128 (MT = 2 in use), K in steps of 64 bytes
-// through LDS (two buffers), four waves as 2 x 2, each wave 32 MT x 64 = MT x 2 MFMA tiles.  One 32x32x32 MFMA takes 32
-// cycles and two KiB of operands, so operands have to be used several times from registers.
-template <int MODE, int MT>
-__global__ __launch_bounds__(GT_THREADS, 2) void gemm_tiled_kernel(GemmParams p)
-{
-    constexpr int BM = 64 * MT;
-    constexpr int A_CH = BM * GT_BK / 16 / GT_THREADS, W_CH = GT_BN * GT_BK / 16 / GT_THREADS; // 16-byte chunks per thread
-    __shared__ __attribute__((aligned(16))) uint8_t a_lds[2][BM * GT_PITCH];
-    __shared__ __attribute__((aligned(16))) uint8_t w_lds[2][GT_BN * GT_PITCH];
-    const int tid = threadIdx.x;
-    const int lane = tid & (WAVE - 1);
-    const int wave = tid / WAVE;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int li = lane & 31, g = lane >> 5;
-
-    // Which output tile.  The 8 XCDs take workgroups round-robin and each has its own L2; the 64 or so workgroups an
-    // XCD runs at a time walk through K at about the same pace, so its L2 only has to hold the current slices of the
-    // rows they use.  Give those 64 an 8 x 8 block of tiles: 8 tiles of activations and 8 of weights cross the fabric
-    // per 64 output tiles instead of up to 64 + 8.  Shapes that do not divide that way walk along rows of tiles.
-    const int64_t tiles_n = (p.n + GT_BN - 1) / GT_BN, tiles_m = (p.m + BM - 1) / BM;
-    int64_t tile_m, tile_n;
-    if (tiles_n % 8 == 0 && tiles_m % 8 == 0 && ((tiles_n >> 3) * (tiles_m >> 3)) % 8 == 0) { // whole blocks, eight at a time
-        const int64_t x = blockIdx.x & 7, l = blockIdx.x >> 3;
-        const int64_t sb = (l >> 6) * 8 + x, within = l & 63; // super-block of 8 x 8 tiles, tile inside it
-        const int64_t sb_per_row = tiles_n >> 3;
-        tile_m = (sb / sb_per_row) * 8 + (within >> 3);
-        tile_n = (sb % sb_per_row) * 8 + (within & 7);
-    } else {
-        tile_m = blockIdx.x / tiles_n;
-        tile_n = blockIdx.x % tiles_n;
-    }
-    const int64_t m0 = tile_m * BM, n0 = tile_n * GT_BN;
-
-    const __amdgpu_buffer_rsrc_t ar = rows_rsrc(p.a + m0 * p.a_pitch, p.m - m0 < BM ? p.m - m0 : BM, p.a_pitch, p.k);
-    const __amdgpu_buffer_rsrc_t wr = rows_rsrc(p.w + n0 * p.w_pitch, p.n - n0 < GT_BN ? p.n - n0 : GT_BN, p.w_pitch, p.k);
-    // staging: a row of 64 bytes is four chunks of 16
-    int a_off[A_CH], w_off[W_CH], a_dst[A_CH], w_dst[W_CH];
-#pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-        const int ch = tid + i * GT_THREADS, r = ch >> 2, c = ch & 3;
-        a_off[i] = r * (int)p.a_pitch + c * 16;
-        a_dst[i] = r * GT_PITCH + c * 16;
-    }
-#pragma unroll
-    for (int i = 0; i < W_CH; ++i) {
-        const int ch = tid + i * GT_THREADS, r = ch >> 2, c = ch & 3;
-        w_off[i] = r * (int)p.w_pitch + c * 16;
-        w_dst[i] = r * GT_PITCH + c * 16;
-    }
-    // two sets of staging registers: what is requested at the end of step s is the tile of step s + 3 and has two
-    // whole steps to arrive before it is written to LDS
-    v4i ra[2][A_CH], rw[2][W_CH];
-    auto load = [&](int set, int kb) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < A_CH; ++i) ra[set][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ar, a_off[i], kb, 0));
-#pragma unroll
-        for (int i = 0; i < W_CH; ++i) rw[set][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off[i], kb, 0));
-    };
-    auto stage = [&](int set, int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < A_CH; ++i) *(v4i *)(a_lds[buf] + a_dst[i]) = ra[set][i];
-#pragma unroll
-        for (int i = 0; i < W_CH; ++i) *(v4i *)(w_lds[buf] + w_dst[i]) = rw[set][i];
-    };
-
-    v16i acc[MT][2];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = v16i{0};
-
-    const int n_steps = (int)(p.k / GT_BK);
-    auto compute = [&](int buf) __attribute__((always_inline)) {
-        const uint8_t *ab = a_lds[buf] + (wm * (BM / 2) + li) * GT_PITCH + 16 * g;
-        const uint8_t *wb = w_lds[buf] + (wn * 64 + li) * GT_PITCH + 16 * g;
-        // all of the step's operands are asked for before the first MFMA: the LDS latency is paid once per step
-        v4i a[2][MT], w[2][2];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) w[ks][j] = *(const v4i *)(wb + j * 32 * GT_PITCH + 32 * ks);
-#pragma unroll
-            for (int i = 0; i < MT; ++i) a[ks][i] = *(const v4i *)(ab + i * 32 * GT_PITCH + 32 * ks);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[ks][i], w[ks][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // step s computes from LDS buffer s & 1, then writes the tile of step s + 1 (register set (s + 1) & 1) to the
-    // other buffer and asks for the tile of step s + 3 into the set just emptied
-    // (Requests and LDS writes are unconditional: past K a request reads zeros or other rows of the tile, never
-    // outside it, and nobody computes from what it leaves in LDS.  With branches around them the compiler loses track
-    // of which request is which and waits for all of them before every write.)
-    load(0, 0);
-    stage(0, 0);
-    load(1, GT_BK);
-    load(0, 2 * GT_BK);
-    __syncthreads();
-    for (int s = 0; s < n_steps; s += 2) {
-        compute(0);
-        stage(1, 1);
-        load(1, (s + 3) * GT_BK);
-        __syncthreads();
-        if (s + 1 < n_steps) compute(1);
-        stage(0, 0);
-        load(0, (s + 4) * GT_BK);
-        __syncthreads();
-    }
-
-    // accumulator register r of tile (i, j): row m0 + wm*(BM/2) + i*32 + 8*(r/4) + 4*g + r%4, column n0 + wn*64 + j*32 + li
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int64_t n = n0 + wn * 64 + j * 32 + li;
-            if (n >= p.n) continue;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int64_t m = m0 + wm * (BM / 2) + i * 32 + 8 * (r / 4) + 4 * g + (r & 3);
-                if (m < p.m) store_out<MODE>(p, m, n, acc[i][j][r]);
-            }
-        }
 }
 
 // Wide tiles for the largest products: 256 x 256 outputs by eight waves of 128 x 64, K in steps of 64 bytes, one
@@ -200,7 +65,10 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
     const int wm = wave >> 2, wn = wave & 3;
     const int li = lane & 31, g = lane >> 5;
 
-    // 8 x 8 blocks of tiles per XCD where the shape allows (see gemm_tiled_kernel)
+    // Which output tile.  The 8 XCDs take workgroups round-robin and each has its own L2; the workgroups an XCD runs at a
+    // time walk through K at about the same pace, so its L2 only has to hold the current slices of the rows they use.  8 x 8
+    // blocks of tiles per XCD where the shape allows: 8 tiles of activations and 8 of weights cross the fabric per 64
+    // output tiles instead of up to 64 + 8.  Shapes that do not divide that way walk along rows of tiles.
     const int64_t tiles_n = (p.n + GW_BN - 1) / GW_BN, tiles_m = (p.m + GW_BM - 1) / GW_BM;
     int64_t tile_m, tile_n;
     if (tiles_n % 8 == 0 && tiles_m % 8 == 0 && ((tiles_n >> 3) * (tiles_m >> 3)) % 8 == 0) {
@@ -498,14 +366,48 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p, const in
     store_out<MODE>(p, i / p.n, i % p.n, sum);
 }
 
-template <int MODE>
-void launch_mode(const GemmParams &p, hipStream_t st)
+// Which kernel, by about what each would take (microseconds): rounds of one workgroup per compute unit, each a fixed part --
+// launch, first stages, the last steps -- and a part per 128 bytes of K, both as measured on products of 40 to 8192 rows, 768 to
+// 8192 columns, K of 768 to 8192; with every compute unit at work the wide tiles' rounds take up to 1.6 times as long (the
+// clock), the others' 1.1 times.  Examples: 2048 x 8192 x 2048 wide 37, 128 rows 51, 64 rows 69; 550 x 8192 x 2048: 25, 25, 32;
+// 400 x 2048 x 2048: 24, 13, 10; 100 x 2048 x 8192 with the normalisation: 65, 32, 21, few-row kernel and its launch 20.
+enum class Tiles { WIDE, ROWS128, ROWS64, FEW };
+
+double rounds_us(int64_t tiles, double fixed, double per_stage, double full, int64_t k)
 {
-    // wide tiles when there are two rounds of them for every compute unit, 128 x 128 tiles otherwise
-    const int64_t tiles_n = (p.n + GT_BN - 1) / GT_BN;
-    const int64_t wide = ((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN);
-    if (wide >= 512) hipLaunchKernelGGL((gemm_wide_kernel<MODE, 0>), dim3((unsigned)wide), dim3(GW_THREADS), GW_LDS_BYTES, st, p);
-    else hipLaunchKernelGGL((gemm_tiled_kernel<MODE, 2>), dim3((unsigned)(((p.m + 127) / 128) * tiles_n)), dim3(GT_THREADS), 0, st, p);
+    const double rounds = (double)((tiles + 255) / 256);
+    return rounds * (fixed + per_stage * ((double)k / 128)) * (1.0 + full * (double)tiles / (256.0 * rounds));
+}
+
+FewParams few_params(const GemmParams &p);
+
+Tiles choose_tiles(const GemmParams &p, bool wide_ok, bool normalised)
+{
+    const int64_t n256 = (p.n + 255) / 256, n128 = (p.n + 127) / 128;
+    double best = rounds_us(n128 * ((p.m + 127) / 128), 6.7, 0.40, 0.1, p.k);
+    Tiles tiles = Tiles::ROWS128;
+    const auto consider = [&](Tiles t, double us) {
+        if (us < best) { best = us; tiles = t; }
+    };
+    consider(Tiles::ROWS64, rounds_us(n128 * ((p.m + 63) / 64), 5.8, 0.25, 0.1, p.k));
+    if (wide_ok) consider(Tiles::WIDE, rounds_us(n256 * ((p.m + 255) / 256), 10.0, 0.87, 0.6, p.k));
+    if (p.m <= FEW_ROWS) consider(Tiles::FEW, few_ns(few_params(p), p.mode == TSATTN_MM_I32_PLANES ? 16 : 1) * 1e-3 + (normalised ? 5.0 : 0.0));
+    return tiles;
+}
+
+template <int MODE>
+hipError_t launch_tiles(const GemmParams &p, Tiles tiles, int ep_d, hipStream_t st)
+{
+    if (tiles != Tiles::WIDE) {
+        GemmParams q = p;
+        q.mode = MODE;
+        return launch_gemm_mid(q, tiles == Tiles::ROWS64 ? 64 : 128, ep_d, st);
+    }
+    const dim3 grid((unsigned)(((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN)));
+    if (ep_d == 128) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 128>), grid, dim3(GW_THREADS), gw_lds_bytes(128), st, p);
+    else if (ep_d == 64) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 64>), grid, dim3(GW_THREADS), gw_lds_bytes(64), st, p);
+    else hipLaunchKernelGGL((gemm_wide_kernel<MODE, 0>), grid, dim3(GW_THREADS), GW_LDS_BYTES, st, p);
+    return hipGetLastError();
 }
 
 FewParams few_params(const GemmParams &p)
@@ -534,7 +436,8 @@ hipError_t prepare_matmul_i8()
         const hipError_t e = hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds);
         if (e != hipSuccess) return e;
     }
-    return prepare_gemm_few();
+    const hipError_t e = prepare_gemm_few();
+    return e != hipSuccess ? e : prepare_gemm_mid();
 }
 
 hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out)
@@ -543,41 +446,38 @@ hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out
         if (planes_out) *planes_out = 1;
         return hipSuccess;
     }
-    const bool few = p.m <= FEW_ROWS;
     if (p.mode == TSATTN_MM_I32_PLANES) {
-        // the parts' sums straight into the caller's planes (with few rows 16 * m * n ints of room by contract)
-        FewParams f = few_params(p);
-        if (few) f.parts = few_parts(f, 16);
-        f.out_stride = p.m * p.n;
-        *planes_out = f.parts;
         GemmParams q = p;
+        bool fused = false, offsets_fit = true;
         if (p.ep_head_dim) {
-            // the producer on the result: in the product's own kernel where the wide tiles are used, else after it
+            // the producer on the result: in the product's own kernel, or after it
             q.ep.src = p.out; q.ep.src_pitch = p.n; q.ep.n_rows = p.m; q.ep.n_heads = (int)(p.n / p.ep_head_dim);
-            q.ep.src_planes = f.parts; q.ep.src_plane_stride = p.m * p.n;
-            const int64_t wide = ((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN);
-            // (the epilogue addresses a tile's rows with 32-bit offsets)
-            const bool offsets_fit = q.ep.dst_pitch < (1 << 23) && (!q.ep.resid || q.ep.resid_pitch < (1 << 21)) &&
-                                     (!q.ep.pos || q.ep.rope_len * p.ep_head_dim * 4 < ((int64_t)1 << 31));
-            const bool one_operand = !(q.ep.resid && q.ep.pos); // (registers for the old state or for cos and sin)
-            const bool head_group = p.ep_head_dim == 64 || p.ep_head_dim == 128; // (wider groups: the producer's own launch)
-            if (!few && wide >= 512 && p.ep_dst_dtype == TSATTN_I8 && offsets_fit && one_operand && head_group) {
-                if (p.ep_head_dim == 128) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 128>), dim3((unsigned)wide), dim3(GW_THREADS), gw_lds_bytes(128), st, q);
-                else hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 64>), dim3((unsigned)wide), dim3(GW_THREADS), gw_lds_bytes(64), st, q);
-                return hipGetLastError();
-            }
+            q.ep.src_planes = 1; q.ep.src_plane_stride = p.m * p.n;
+            // (the wide kernel's epilogue addresses a tile's rows with 32-bit offsets)
+            offsets_fit = q.ep.dst_pitch < (1 << 23) && (!q.ep.resid || q.ep.resid_pitch < (1 << 21)) &&
+                          (!q.ep.pos || q.ep.rope_len * p.ep_head_dim * 4 < ((int64_t)1 << 31));
+            // one operand besides the product: the old state, or cos and sin; wider groups than a head have a launch of their own
+            fused = p.ep_dst_dtype == TSATTN_I8 && !(q.ep.resid && q.ep.pos) && (p.ep_head_dim == 64 || p.ep_head_dim == 128);
         }
-        hipError_t e = hipSuccess;
-        if (few) {
+        const Tiles tiles = choose_tiles(p, offsets_fit || !fused, p.ep_head_dim != 0);
+        *planes_out = 1;
+        if (tiles != Tiles::FEW && fused) return launch_tiles<TSATTN_MM_I32>(q, tiles, p.ep_head_dim, st);
+        hipError_t e;
+        if (tiles == Tiles::FEW) {
+            // the parts' sums straight into the caller's planes (with few rows 16 * m * n ints of room by contract)
+            FewParams f = few_params(p);
+            f.parts = few_parts(f, 16);
+            f.out_stride = p.m * p.n;
+            *planes_out = q.ep.src_planes = f.parts;
             e = launch_gemm_few(f, st);
         } else {
-            launch_mode<TSATTN_MM_I32>(q, st);
-            e = hipGetLastError();
+            e = launch_tiles<TSATTN_MM_I32>(q, tiles, 0, st);
         }
         if (e != hipSuccess || !p.ep_head_dim) return e;
         return launch_rope_normalize(q.ep, p.ep_dst_dtype, p.ep_head_dim, true, st);
     }
-    if (few) {
+    const Tiles tiles = choose_tiles(p, true, false);
+    if (tiles == Tiles::FEW) {
         FewParams f = few_params(p);
         // Parts through the caller's workspace and a second launch that adds them up: where the weights would otherwise
         // come in through a few compute units only (an eighth of them).
@@ -597,11 +497,10 @@ hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out
         else hipLaunchKernelGGL((gemm_reduce_kernel<TSATTN_MM_ADD_SCALED>), grid, dim3(256), 0, st, r, (const int32_t *)p.workspace, f.parts);
         return hipGetLastError();
     }
-    if (p.mode == TSATTN_MM_I32) launch_mode<TSATTN_MM_I32>(p, st);
-    else if (p.mode == TSATTN_MM_F32) launch_mode<TSATTN_MM_F32>(p, st);
-    else if (p.mode == TSATTN_MM_ADD_SCALED) launch_mode<TSATTN_MM_ADD_SCALED>(p, st);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (p.mode == TSATTN_MM_I32) return launch_tiles<TSATTN_MM_I32>(p, tiles, 0, st);
+    if (p.mode == TSATTN_MM_F32) return launch_tiles<TSATTN_MM_F32>(p, tiles, 0, st);
+    if (p.mode == TSATTN_MM_ADD_SCALED) return launch_tiles<TSATTN_MM_ADD_SCALED>(p, tiles, 0, st);
+    return hipErrorInvalidValue;
 }
 
 } // namespace tsattn

@@ -129,6 +129,8 @@ bool few_source_ok(const FewParams &p)
 
 int few_parts(const FewParams &p, int max_parts) { return few_best(p, 1, max_parts).parts; }
 
+double few_ns(const FewParams &p, int max_parts) { return few_best(p, 1, max_parts).ns; }
+
 hipError_t launch_gemm_few(const FewParams &params, hipStream_t st)
 {
     FewParams p = params;

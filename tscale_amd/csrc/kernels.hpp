@@ -250,9 +250,13 @@ struct FewParams {
 };
 bool few_source_ok(const FewParams &p);              // whether the kernel can normalise this source itself
 int few_parts(const FewParams &p, int max_parts);    // how many parts K is best cut into, at most max_parts
+double few_ns(const FewParams &p, int max_parts);    // about what the launch then takes, in nanoseconds
 hipError_t launch_gemm_few(const FewParams &p, hipStream_t st);
 hipError_t prepare_gemm_few(); // once per device
 
+// gemm_mid.hip: tiles of `rows` (64 or 128) x 128; ep_d: the head width of the producer as the last step (p.ep), 0 for none
+hipError_t launch_gemm_mid(const GemmParams &p, int rows, int ep_d, hipStream_t st);
+hipError_t prepare_gemm_mid(); // once per device
 hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out);
 hipError_t prepare_matmul_i8(); // once per device, before the first product
 
