@@ -128,3 +128,33 @@ def test_cache_fill_equals_token_by_token_append(ctx, d):
         assert torch.equal(a, b)
     assert torch.equal(bulk.k[0, 1, 16], k[16, d:2 * d]) and torch.equal(bulk.v[2, 2, 5], v[17, 2 * d:3 * d])
     assert not bulk.k[1].any()
+
+
+@pytest.mark.parametrize("d,H,n", [(64, 3, 1), (64, 5, 13), (128, 1, 31), (192, 3, 7), (256, 2, 5)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_quantize_rows_widths_and_alignment(ctx, d, H, n, offset):
+    """Numbers of (row, head) pairs that leave a workgroup part empty, and sources that wide requests cannot read."""
+    x = np.random.default_rng(d + n).standard_normal(n * H * d + 1).astype(np.float32)[:n * H * d].reshape(n, H * d)
+    want_q, want_s = orc.quantize_rows(orc.I8, x, H)
+    memory = torch.zeros(n * H * d + 1, device="cuda")
+    src = memory[offset:offset + n * H * d].view(n, H * d).copy_(torch.from_numpy(x))
+    q, s = ctx.quantize_rows(src, H, capi.I8)
+    assert np.array_equal(q.cpu().numpy(), want_q) and np.array_equal(s.cpu().numpy(), want_s)
+
+
+@pytest.mark.parametrize("n", [4095, 4097])
+def test_cache_fill_on_both_sides_of_the_small_batch(ctx, n):
+    from tscale_amd import KVCache
+    H, d = 2, 64
+    off = np.array([0, 2050, n], np.int32)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    k, v = (torch.randint(0, 256, (n, H * d), dtype=torch.uint8, device="cuda", generator=g) for _ in range(2))
+    ks, vs = (torch.rand((H, n), device="cuda", generator=g) for _ in range(2))
+    c = KVCache(ctx, capi.I8, 2, H, 2050, d)
+    c.fill_from_prefill(torch.from_numpy(off).cuda(), k, ks, v, vs)
+    assert c.cache_len.tolist() == [2050, n - 2050]
+    for b in range(2):
+        lo, hi = int(off[b]), int(off[b + 1])
+        for plane, rows in ((c.k, k), (c.v, v)):
+            assert torch.equal(plane[b, :, :hi - lo], rows[lo:hi].view(-1, H, d).transpose(0, 1))
+        assert torch.equal(c.k_scale[b, :, :hi - lo], ks[:, lo:hi]) and torch.equal(c.v_scale[b, :, :hi - lo], vs[:, lo:hi])

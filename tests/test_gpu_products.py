@@ -47,9 +47,10 @@ def test_products_with_the_producer_at_tile_edges(ctx, m, heads, d, k, variant):
     a, w = (dev(rng.integers(-127, 128, s).astype(np.int8).view(np.uint8)) for s in ((m, k), (n, k)))
     a[3] = 0                                       # a row of zeros: scale and bytes 0
     state = rng.standard_normal((m, n)).astype(np.float32)
+    pos = dev(rng.integers(-1, 70, m).astype(np.int32))
     outs = []
     for fused in (True, False):
-        kw = {"rope": dict(pos=dev(rng.integers(-1, 70, m).astype(np.int32)) if fused else kw["pos"], rope=dev(orc.fill_rope(d, 64)), scale_mult=0.4,
+        kw = {"rope": dict(pos=pos, rope=dev(orc.fill_rope(d, 64)), scale_mult=0.4,
                            rope_heads=max(1, heads - 1), scale_heads=(heads // 2, 1)),
               "resid": dict(resid=dev(state), resid_scale=0.01), "relu": dict(relu=True, row_major_scale=True)}[variant]
         if fused:

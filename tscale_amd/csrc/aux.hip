@@ -5,8 +5,67 @@
 
 namespace tsattn {
 
-// One wave per (row, head).  scale = absmax/127 (int8) or absmax/256 (e4m3); values times 1/scale,
+// scale = absmax/127 (int8) or absmax/256 (e4m3); values times 1/scale,
 // rounded to nearest even (lib/cuda/cuda_matmul.cuh:237-249, lib/cuda/cuda_util.cuh:286-297).
+__device__ inline void quantize_scale(int dst, float amax, float &discr, float &mult)
+{
+    discr = mult = 0.0f;
+    if (amax > 0) {
+        discr = dst == TSATTN_I8 ? amax / 127.0f : amax / 256.0f;
+        mult = 1.0f / discr;
+    }
+}
+
+// Rows of 64, 128 or 256 values in 16-byte aligned memory: a lane takes eight consecutive values, a wave 8, 4 or 2 (row, head)
+// pairs.  Bound by memory in large launches, by one round trip in small ones (2145 x 12 x 64 bf16: 8.7 us with one wave per pair and
+// a value per lane and request).
+template <int SRC, int DST, int D>
+__global__ __launch_bounds__(256) void quantize_aligned_kernel(const uint8_t *src, int64_t src_pitch, int64_t n_rows, int n_heads, uint8_t *dst, int64_t dst_pitch,
+                                                               float *scale, int64_t scale_pitch)
+{
+    constexpr int LPP = D / 8, PAIRS = 256 / LPP;
+    const int c = threadIdx.x % LPP;
+    const uint32_t pair = blockIdx.x * PAIRS + threadIdx.x / LPP, n_pairs = (uint32_t)n_rows * (uint32_t)n_heads;
+    const uint32_t pc = pair < n_pairs ? pair : n_pairs - 1;
+    const uint32_t row = pc / (uint32_t)n_heads, head = pc % (uint32_t)n_heads;
+    const uint8_t *const at = src + (int64_t)row * src_pitch + ((int64_t)head * D + c * 8) * (SRC == TSATTN_SRC_F32 ? 4 : 2);
+    float x[8];
+    if (SRC == TSATTN_SRC_F32) {
+        const v4f a = *(const v4f *)at, b = *(const v4f *)(at + 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { x[i] = a[i]; x[4 + i] = b[i]; }
+    } else {
+        const v4i a = *(const v4i *)at;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[2 * i] = __uint_as_float((uint32_t)a[i] << 16);
+            x[2 * i + 1] = __uint_as_float((uint32_t)a[i] & 0xffff0000u);
+        }
+    }
+    float amax = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[i]));
+#pragma unroll
+    for (int o = 1; o < LPP; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, WAVE));
+    float discr, mult;
+    quantize_scale(DST, amax, discr, mult);
+    if (pair >= n_pairs) return;
+    uint32_t w[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if (DST == TSATTN_I8) {
+            w[k] = pack_i8x4(x[4 * k] * mult, x[4 * k + 1] * mult, x[4 * k + 2] * mult, x[4 * k + 3] * mult, -127.0f);
+        } else {
+            w[k] = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[k] |= (uint32_t)float_to_e4m3(x[4 * k + i] * mult) << (8 * i);
+        }
+    }
+    *(v2i *)(dst + (int64_t)row * dst_pitch + (int64_t)head * D + c * 8) = v2i{(int)w[0], (int)w[1]};
+    if (c == 0) scale[(int64_t)head * scale_pitch + row] = discr;
+}
+
+// Any other width (a multiple of 64 up to 256) or alignment: one wave per (row, head).
 template <int SRC, int DST>
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint8_t *src, int64_t src_pitch, int64_t n_rows, int n_heads,
                                                             int head_dim, uint8_t *dst, int64_t dst_pitch, float *scale,
@@ -27,11 +86,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const uint8_t *src, 
         amax = fmaxf(amax, fabsf(x[i]));
     }
     amax = wave_max(amax);
-    float discr = 0, mult = 0;
-    if (amax > 0) {
-        discr = (DST == TSATTN_I8) ? amax / 127.0f : amax / 256.0f;
-        mult = 1.0f / discr;
-    }
+    float discr, mult;
+    quantize_scale(DST, amax, discr, mult);
     for (int i = 0; i < per; ++i) {
         float y = x[i] * mult;
         uint8_t b = (DST == TSATTN_I8) ? (uint8_t)float_to_i8(y) : float_to_e4m3(y);
@@ -47,15 +103,25 @@ hipError_t launch_quantize_rows(int src_dtype, int dst_dtype, const void *src, i
     int64_t jobs = n_rows * n_heads;
     if (jobs == 0) return hipSuccess;
     dim3 grid((unsigned)((jobs + 3) / 4)), block(256);
+    const bool aligned = (((uintptr_t)src | (uintptr_t)src_pitch) & 15) == 0 && (((uintptr_t)dst | (uintptr_t)dst_pitch) & 7) == 0 && jobs < ((int64_t)1 << 31);
+#define TSATTN_QA(S, D, W)                                                                                           \
+    hipLaunchKernelGGL((quantize_aligned_kernel<S, D, W>), dim3((unsigned)((jobs + 2048 / W - 1) / (2048 / W))), block, 0, st,      \
+                       (const uint8_t *)src, src_pitch, n_rows, n_heads, (uint8_t *)dst, dst_pitch, scale, scale_pitch)
 #define TSATTN_QR(S, D)                                                                                              \
-    hipLaunchKernelGGL((quantize_rows_kernel<S, D>), grid, block, 0, st, (const uint8_t *)src, src_pitch, n_rows,   \
-                       n_heads, head_dim, (uint8_t *)dst, dst_pitch, scale, scale_pitch)
+    do {                                                                                                             \
+        if (aligned && head_dim == 64) TSATTN_QA(S, D, 64);                                                          \
+        else if (aligned && head_dim == 128) TSATTN_QA(S, D, 128);                                                   \
+        else if (aligned && head_dim == 256) TSATTN_QA(S, D, 256);                                                   \
+        else hipLaunchKernelGGL((quantize_rows_kernel<S, D>), grid, block, 0, st, (const uint8_t *)src, src_pitch, n_rows,   \
+                                n_heads, head_dim, (uint8_t *)dst, dst_pitch, scale, scale_pitch);                   \
+    } while (0)
     if (src_dtype == TSATTN_SRC_F32 && dst_dtype == TSATTN_I8) TSATTN_QR(TSATTN_SRC_F32, TSATTN_I8);
     else if (src_dtype == TSATTN_SRC_F32 && dst_dtype == TSATTN_E4M3) TSATTN_QR(TSATTN_SRC_F32, TSATTN_E4M3);
     else if (src_dtype == TSATTN_SRC_BF16 && dst_dtype == TSATTN_I8) TSATTN_QR(TSATTN_SRC_BF16, TSATTN_I8);
     else if (src_dtype == TSATTN_SRC_BF16 && dst_dtype == TSATTN_E4M3) TSATTN_QR(TSATTN_SRC_BF16, TSATTN_E4M3);
     else return hipErrorInvalidValue;
 #undef TSATTN_QR
+#undef TSATTN_QA
     return hipGetLastError();
 }
 
@@ -204,11 +270,14 @@ hipError_t launch_cache_append(const AppendParams &p, int n_seqs, hipStream_t st
 }
 
 // Bulk form of the append: the K/V rows of a prefill batch ([token][head*d]) go to the planar cache.
-// A workgroup handles 16 consecutive tokens with all their heads: a wave reads 1 KiB of a row at a time, four
+// A workgroup handles 16 consecutive tokens with all their heads (4 up to 4096 tokens, for more workgroups: 531 tokens
+// of 16 x 128 take 8.5 us, with 16 per workgroup 10.4 us): a wave reads 1 KiB of a row at a time, four
 // requests of K and four of V per thread are out before the first store, and every token is looked up in the
 // sequence offsets once, not once per thread.
-constexpr int FILL_TOKENS = 16;
+constexpr int FILL_TOKENS = 16, FILL_TOKENS_FEW = 4;
+constexpr int64_t FILL_FEW = 4096; // tokens of a small batch
 
+template <int FILL_TOKENS>
 __global__ __launch_bounds__(256) void cache_fill_kernel(FillParams p)
 {
     __shared__ int s_seq[FILL_TOKENS];
@@ -283,7 +352,8 @@ __global__ void cache_len_add_kernel(int32_t *cache_len, const int32_t *seq_offs
 hipError_t launch_cache_fill(const FillParams &p, hipStream_t st)
 {
     if (p.n_seqs == 0 || p.n_tokens == 0) return hipSuccess;
-    hipLaunchKernelGGL(cache_fill_kernel, dim3((unsigned)((p.n_tokens + FILL_TOKENS - 1) / FILL_TOKENS)), dim3(256), 0, st, p);
+    if (p.n_tokens <= FILL_FEW) hipLaunchKernelGGL((cache_fill_kernel<FILL_TOKENS_FEW>), dim3((unsigned)((p.n_tokens + FILL_TOKENS_FEW - 1) / FILL_TOKENS_FEW)), dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((cache_fill_kernel<FILL_TOKENS>), dim3((unsigned)((p.n_tokens + FILL_TOKENS - 1) / FILL_TOKENS)), dim3(256), 0, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(cache_len_add_kernel, dim3((unsigned)((p.n_seqs + 255) / 256)), dim3(256), 0, st, p.cache_len, p.seq_offset,

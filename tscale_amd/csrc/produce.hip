@@ -4,10 +4,11 @@
 // operation: the same float products, the sum of squares taken in index order, no fused multiply-adds, so the
 // bytes and scales are identical to a CPU evaluation in that order.
 //
-// A workgroup takes 32 consecutive (row, head) pairs.  The rotated values go to LDS (row pitch d+1 floats, so
-// that 32 lanes walking 32 different pairs in step hit 32 different banks); then lane j of the first wave sums
-// pair j's squares one after the other, which keeps the summation order while 32 sums advance together; then
-// all threads convert and write the bytes out, sixteen per thread, consecutively.  Few pairs: see normalize_few_kernel.
+// One wave takes 64 / (D / 8) pairs: a lane holds eight values (four couples x, x + 32), squares go through the wave's LDS to
+// the lane that adds its pair's up in index order -- additions only, one instruction per value -- and the multiplier comes back
+// through a lane exchange: no barrier, no second pass over the values.  Bound by memory for large launches (65536 x 16 x 128 f32 ->
+// int8: 117 us, 5.8 TB/s; 121 us with workgroups of 32 pairs, 256 threads and three barriers), by its chain of waits for small
+// ones (531 x 16 x 128: 4.8 against 6.3 us; 32 x 16, two planes and the residual update: 4.5 against 5.6 us).
 #include <math.h>
 
 #include "common.hpp"
@@ -15,167 +16,11 @@
 
 namespace tsattn {
 
-constexpr int PR_PAIRS = 32;       // (row, head) pairs per workgroup
-constexpr int64_t PR_FEW = 4096;   // up to this many pairs one wave each takes a few
-
 // every float operation below is meant as written: no fused multiply-adds
 #pragma clang fp contract(off)
 
-template <int D, int DST, bool SRC_I32, int PAIRS>
-__global__ __launch_bounds__(256) void rope_normalize_kernel(ProduceParams p)
-{
-    constexpr int PITCH = D + 1;
-    __shared__ float vals[PAIRS * PITCH];
-    __shared__ float mults[PAIRS];
-    __shared__ int64_t s_row[PAIRS];
-    __shared__ int s_head[PAIRS], s_pos[PAIRS];
-    const int tid = threadIdx.x;
-    const int64_t pair0 = (int64_t)blockIdx.x * PAIRS;
-    const int64_t n_pairs = p.n_rows * p.n_heads;
-    const int n_here = (int)(n_pairs - pair0 < PAIRS ? n_pairs - pair0 : PAIRS);
-
-    if (tid < n_here) {
-        const int64_t pair = pair0 + tid;
-        const int64_t row = pair / p.n_heads;
-        s_row[tid] = row;
-        s_head[tid] = (int)(pair - row * p.n_heads);
-        int t = p.pos ? p.pos[row] : 0;
-        s_pos[tid] = t < 0 ? 0 : (t >= p.rope_len ? (int)p.rope_len - 1 : t);
-    }
-    __syncthreads();
-
-    // ---- load + rotate: four (k, k+32) couples per thread and step, 16-byte loads; all loads of a thread are
-    //      issued before the first is used ------------------------------------------------------------------
-    constexpr int PER_PAIR = D / 8;
-    constexpr int STEPS = (PAIRS * PER_PAIR + 255) / 256;
-    v4f v0[STEPS], v1[STEPS], cs[STEPS], sn[STEPS];
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) {
-        const int j = tid + st * 256;
-        const int pr = j / PER_PAIR, c = j % PER_PAIR;
-        if (pr >= n_here) continue;
-        const int x0 = (c / 8) * 64 + (c % 8) * 4, x1 = x0 + 32;
-        const int64_t e = s_row[pr] * p.src_pitch + (int64_t)s_head[pr] * D;
-        if (SRC_I32) {
-            v4i a = *(const v4i *)((const int32_t *)p.src + e + x0), b = *(const v4i *)((const int32_t *)p.src + e + x1);
-            for (int pl = 1; pl < p.src_planes; ++pl) { // the parts of a product whose K was split: exact integer sums
-                a += *(const v4i *)((const int32_t *)p.src + pl * p.src_plane_stride + e + x0);
-                b += *(const v4i *)((const int32_t *)p.src + pl * p.src_plane_stride + e + x1);
-            }
-            v0[st] = v4f{(float)a.x, (float)a.y, (float)a.z, (float)a.w};
-            v1[st] = v4f{(float)b.x, (float)b.y, (float)b.z, (float)b.w};
-        } else {
-            v0[st] = *(const v4f *)((const float *)p.src + e + x0);
-            v1[st] = *(const v4f *)((const float *)p.src + e + x1);
-        }
-        if (p.pos) { // heads that are not rotated read their row too and then turn by the identity: no divergent branch
-            const float *rr = p.rope + (int64_t)s_pos[pr] * D;
-            cs[st] = *(const v4f *)(rr + x0);
-            sn[st] = *(const v4f *)(rr + x1);
-        }
-    }
-    if (p.resid) {
-        // state += delta * scale, written back; the updated state is what gets normalised.  (In loops of their own, after
-        // every request above has been issued: a store in between would keep the compiler from issuing them together.)
-        v4f u0[STEPS], u1[STEPS];
-#pragma unroll
-        for (int st = 0; st < STEPS; ++st) {
-            const int j = tid + st * 256;
-            const int pr = j / PER_PAIR, c = j % PER_PAIR;
-            if (pr >= n_here) continue;
-            const int x0 = (c / 8) * 64 + (c % 8) * 4;
-            const float *r0 = p.resid + s_row[pr] * p.resid_pitch + (int64_t)s_head[pr] * D + x0;
-            u0[st] = *(const v4f *)r0;
-            u1[st] = *(const v4f *)(r0 + 32);
-        }
-#pragma unroll
-        for (int st = 0; st < STEPS; ++st) {
-            const int j = tid + st * 256;
-            const int pr = j / PER_PAIR, c = j % PER_PAIR;
-            if (pr >= n_here) continue;
-            const int x0 = (c / 8) * 64 + (c % 8) * 4;
-            float *r0 = p.resid + s_row[pr] * p.resid_pitch + (int64_t)s_head[pr] * D + x0;
-            v0[st] = u0[st] + v0[st] * p.resid_scale;
-            v1[st] = u1[st] + v1[st] * p.resid_scale;
-            *(v4f *)r0 = v0[st];
-            *(v4f *)(r0 + 32) = v1[st];
-        }
-    }
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) {
-        const int j = tid + st * 256;
-        const int pr = j / PER_PAIR, c = j % PER_PAIR;
-        if (pr >= n_here) continue;
-        const int x0 = (c / 8) * 64 + (c % 8) * 4, x1 = x0 + 32;
-        if (p.pos) {
-            const bool turn = s_head[pr] < p.rope_heads;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float cos_value = turn ? cs[st][i] : 1.0f;
-                const float sin_value = turn ? sn[st][i] * p.rotate_dir : 0.0f;
-                const float r0 = v0[st][i] * cos_value - v1[st][i] * sin_value;
-                const float r1 = v0[st][i] * sin_value + v1[st][i] * cos_value;
-                v0[st][i] = r0;
-                v1[st][i] = r1;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            vals[pr * PITCH + x0 + i] = v0[st][i];
-            vals[pr * PITCH + x1 + i] = v1[st][i];
-        }
-    }
-    __syncthreads();
-
-    // ---- per pair: sum of squares in index order, scale -----------------------------------------------------
-    if (tid < n_here) {
-        const float *v = vals + tid * PITCH;
-        float sum2 = 0.0f;
-#pragma unroll 8
-        for (int x = 0; x < D; ++x) sum2 = sum2 + v[x] * v[x];
-        float discr = 0.0f, mult = 0.0f;
-        if (sum2 != 0.0f) {
-            // the single-precision square root instruction is one ulp off now and then; the double-precision routine
-            // is exact to well below a float ulp, and rounding its result to float gives the correctly rounded root
-            const float sko = (float)sqrt((double)(sum2 / (float)D));
-            discr = sko * p.vec_scale;
-            mult = 1.0f / discr;
-        }
-        mults[tid] = mult;
-        const int sh = s_head[tid] - p.scale_head_begin;
-        if (p.scale && sh >= 0 && sh < p.scale_head_count) p.scale[sh * p.scale_pitch + s_row[tid] * p.scale_row_stride] = discr * p.scale_mult;
-    }
-    __syncthreads();
-
-    // ---- convert and store, 16 bytes per thread and step ------------------------------------------------------
-    constexpr int OUT_PER_PAIR = D / 16;
-    for (int j = tid; j < n_here * OUT_PER_PAIR; j += 256) {
-        const int pr = j / OUT_PER_PAIR, x = (j % OUT_PER_PAIR) * 16;
-        const float mult = mults[pr];
-        uint32_t w[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            w[k] = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float y = vals[pr * PITCH + x + 4 * k + i] * mult;
-                // a head of zeros is written as zero bytes whatever the signs of its (rotated) zeros
-                uint32_t b = mult == 0.0f ? 0u : ((DST == TSATTN_I8) ? (uint8_t)float_to_i8(y) : float_to_e4m3(y));
-                if (DST == TSATTN_I8 && p.relu && (b & 0x80u)) b = 0u; // x = max(0, x)
-                w[k] |= b << (8 * i);
-            }
-        }
-        *(v4i *)(p.dst + s_row[pr] * p.dst_pitch + (int64_t)s_head[pr] * D + x) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-    }
-}
-
-// The same for few pairs (one token per sequence), where a launch is a chain of waits: one wave per 64 / (D / 8) pairs, a
-// lane holds eight values (four couples x, x + 32), squares go through the wave's LDS to the lane that adds its pair's up in
-// index order -- additions only, one instruction per value -- and the multiplier comes back through a lane exchange: no
-// barrier, no second pass over the values.  32 x 2048, two planes and the residual update: 5.6 us with workgroups of 256
-// threads and three barriers.
 template <int D, int DST, bool SRC_I32>
-__global__ __launch_bounds__(WAVE) void normalize_few_kernel(ProduceParams p)
+__global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
 {
     constexpr int LPP = D / 8, PAIRS = WAVE / LPP; // lanes per pair, pairs per wave
     constexpr int PITCH = D + 4;
@@ -196,7 +41,15 @@ __global__ __launch_bounds__(WAVE) void normalize_few_kernel(ProduceParams p)
         constexpr int PL = 4; // planes asked for together (those that are not there: the last one again)
         const int32_t *const src = (const int32_t *)p.src + e;
         v4i a = v4i{0, 0, 0, 0}, b = v4i{0, 0, 0, 0};
-        for (int p0 = 0; p0 < p.src_planes; p0 += PL) {
+        if (p.src_planes == 1) {
+            a = *(const v4i *)src;
+            b = *(const v4i *)(src + 32);
+            if (p.resid) {
+                u0 = *(const v4f *)resid;
+                u1 = *(const v4f *)(resid + 32);
+            }
+        }
+        for (int p0 = 0; p0 < p.src_planes && p.src_planes > 1; p0 += PL) {
             v4i qa[PL], qb[PL];
 #pragma unroll
             for (int i = 0; i < PL; ++i) {
@@ -270,7 +123,9 @@ __global__ __launch_bounds__(WAVE) void normalize_few_kernel(ProduceParams p)
             }
         }
         float discr = 0.0f;
-        if (sum2 != 0.0f) { // the root: see rope_normalize_kernel
+        if (sum2 != 0.0f) {
+            // the single-precision square root instruction is one ulp off now and then; the double-precision routine
+            // is exact to well below a float ulp, and rounding its result to float gives the correctly rounded root
             discr = (float)sqrt((double)(sum2 / (float)D)) * p.vec_scale;
             mult = 1.0f / discr;
         }
@@ -304,17 +159,10 @@ hipError_t launch_rope_normalize(const ProduceParams &p, int dst_dtype, int head
 {
     const int64_t n_pairs = p.n_rows * p.n_heads;
     if (n_pairs == 0) return hipSuccess;
-    // Groups wider than a head (the feed-forward groups of 128 * ReluMult) are taken by one wave each whatever their number:
-    // 32 of them would not fit in LDS.
-    const bool few = n_pairs <= PR_FEW || head_dim > 128;
-    if (few && p.n_rows > 0xffffffffll / p.n_heads) return hipErrorInvalidValue;
-    const int per_wg = few ? WAVE / (head_dim / 8) : PR_PAIRS;
-    dim3 grid((unsigned)((n_pairs + per_wg - 1) / per_wg)), block(few ? WAVE : 256);
-#define TSATTN_PR(D_, DST_, I32_)                                                                                   \
-    do {                                                                                                            \
-        if (few) hipLaunchKernelGGL((normalize_few_kernel<D_, DST_, I32_>), grid, block, 0, st, p);                 \
-        else hipLaunchKernelGGL((rope_normalize_kernel<D_, DST_, I32_, PR_PAIRS>), grid, block, 0, st, p);          \
-    } while (0)
+    if (p.n_rows > 0xffffffffll / p.n_heads) return hipErrorInvalidValue; // (pairs are counted in 32 bits: 1 TB of values)
+    const int per_wave = WAVE / (head_dim / 8); // (one group of 384 or 512 values)
+    dim3 grid((unsigned)((n_pairs + per_wave - 1) / per_wave)), block(WAVE);
+#define TSATTN_PR(D_, DST_, I32_) hipLaunchKernelGGL((rope_normalize_kernel<D_, DST_, I32_>), grid, block, 0, st, p)
     if (head_dim == 128 && dst_dtype == TSATTN_I8 && !src_i32) TSATTN_PR(128, TSATTN_I8, false);
     else if (head_dim == 128 && dst_dtype == TSATTN_I8 && src_i32) TSATTN_PR(128, TSATTN_I8, true);
     else if (head_dim == 128 && dst_dtype == TSATTN_E4M3 && !src_i32) TSATTN_PR(128, TSATTN_E4M3, false);
@@ -323,11 +171,9 @@ hipError_t launch_rope_normalize(const ProduceParams &p, int dst_dtype, int head
     else if (head_dim == 64 && dst_dtype == TSATTN_I8 && src_i32) TSATTN_PR(64, TSATTN_I8, true);
     else if (head_dim == 64 && dst_dtype == TSATTN_E4M3 && !src_i32) TSATTN_PR(64, TSATTN_E4M3, false);
     else if (head_dim == 64 && dst_dtype == TSATTN_E4M3 && src_i32) TSATTN_PR(64, TSATTN_E4M3, true);
-#define TSATTN_PR_WIDE(D_)                                                                                          \
-    else if (head_dim == D_ && dst_dtype == TSATTN_I8 && !src_i32)                                                  \
-        hipLaunchKernelGGL((normalize_few_kernel<D_, TSATTN_I8, false>), grid, block, 0, st, p);                    \
-    else if (head_dim == D_ && dst_dtype == TSATTN_I8 && src_i32)                                                   \
-        hipLaunchKernelGGL((normalize_few_kernel<D_, TSATTN_I8, true>), grid, block, 0, st, p);
+#define TSATTN_PR_WIDE(D_)                                                                               \
+    else if (head_dim == D_ && dst_dtype == TSATTN_I8 && !src_i32) TSATTN_PR(D_, TSATTN_I8, false);      \
+    else if (head_dim == D_ && dst_dtype == TSATTN_I8 && src_i32) TSATTN_PR(D_, TSATTN_I8, true);
     TSATTN_PR_WIDE(256)
     TSATTN_PR_WIDE(384)
     TSATTN_PR_WIDE(512)
