@@ -587,3 +587,30 @@ def test_merge_lookups_argument_checks(ctx):
     a.n_parts, a.n_tokens, a.n_heads, a.head_dim = 0, 8, 1, 64
     with pytest.raises(capi.TsattnError):                  # no parts
         capi.check(ctx.lib.tsattn_merge_lookups(ctx.handle, ctypes.byref(a), None))
+
+
+@pytest.mark.parametrize("dtype,d,seq_lens,window,slope,constant", [
+    (capi.E4M3, 64, [1], 10 ** 6, 0.0, False), (capi.I8, 128, [33], 10 ** 6, 0.0, True), (capi.E4M3, 128, [127, 2], 10 ** 6, 0.5, False),
+    (capi.I8, 64, [31, 1, 97], 40, 0.5, True), (capi.E4M3, 64, [161, 300], 10 ** 6, 0.0, False), (capi.E4M3, 128, [700], 256, 0.25, True),
+    (capi.I8, 128, [5, 450, 64], 10 ** 6, 0.0, False), (capi.I8, 64, [515], 10 ** 6, 0.0, False)])
+def test_prefill_few_and_many_heads(ctx, dtype, d, seq_lens, window, slope, constant):
+    """The same heads alone, where the keys of 32 rows are shared out to the waves of a workgroup, and repeated until the chip
+    is full, where a workgroup owns 128 rows: both against the oracle, with rows without keys and a last group of rows that
+    is not whole."""
+    H, n = 2, sum(seq_lens)
+    q, qs, k, ks, v, vs = make_qkv(n + d, n, H, d, dtype)
+    if constant:
+        qs, vs = 0.01, 0.03
+    st, fi = orc.make_spans(seq_lens, window)
+    want = orc.prefill_q8(dtype, q, k, v, H, qs, ks, vs, st, fi, slope)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda() if isinstance(a, np.ndarray) else a
+    wide = lambda a, r: t(a).reshape(n, H, d).repeat(1, r, 1).reshape(n, r * H * d)
+    scales = lambda a, r: t(a).repeat(r, 1).contiguous() if isinstance(a, np.ndarray) else a
+    tiles = ctx.build_span_tiles(t(st), t(fi))
+    for r in (1, 2 + 512 // ((n + 127) // 128)):
+        out = ctx.compute_val_lookup(dtype, r * H, wide(q, r), wide(k, r), wide(v, r), scales(qs, r), scales(ks, r), scales(vs, r), t(st), t(fi), slope,
+                                     span_tiles=tiles, span_len_hint=min(window, max(seq_lens)))
+        out = out.reshape(n, r, H * d)
+        assert torch.equal(out, out[:, :1].expand_as(out))
+        assert_within_tolerance(out[:, 0].cpu().numpy(), want, "%d heads" % (r * H))
+        assert not out[fi < st].any()

@@ -298,6 +298,7 @@ int tsattn_prefill(tsattn_handle_t h, const tsattn_prefill_args *a, void *stream
     p.dbg = a->debug_qk_acc; p.dbg_pitch = a->debug_pitch;
     p.n_tokens = (int)a->n_tokens; p.n_heads = a->n_heads;
     p.period_tiles = (a->causal_period > 0 && a->causal_period % 128 == 0 && a->n_tokens % a->causal_period == 0) ? (int)(a->causal_period / 128) : 0;
+    p.span_len_hint = a->span_len_hint;
     // Long spans with room for the f16 copy of V: the kernel that streams K and that copy through LDS.  (It addresses
     // K and the copy with 31-bit byte offsets.)
     if (a->workspace && a->span_len_hint >= TSATTN_PREFILL_LONG_SPAN && a->head_dim == 128 && a->alibi_slope == 0.0f && !a->debug_qk_acc && !a->kv_out && a->n_span_parts <= 1) {

@@ -93,6 +93,7 @@ struct PrefillParams {
     int n_tokens;
     int n_heads;
     int period_tiles; // query tiles per period of equal span structure, 0 = unknown (launch order only)
+    int64_t span_len_hint; // about the longest row's keys, 0 = unknown (choice of kernel only)
     // optional fused consumer (kv_out != nullptr): KVProduct of the f32 result with the rows of kv_k; out may then be null
     const uint8_t *kv_k;
     int64_t kv_k_pitch;

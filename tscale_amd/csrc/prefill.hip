@@ -94,7 +94,8 @@ typedef __attribute__((address_space(3))) v4s *lds_v4s_ptr;
 // multiplied into the key scales as they are staged and a logit costs one multiply-add instead of a multiply and one.
 // CONSTS == 2: the value scale is one number too (cpu_infer.cpp:454): V is widened as it is -- exactly -- and the
 // result multiplied by the scale.
-template <int DTYPE, int D, bool OUT_F16, bool SLOPE, bool DUMP, bool MULTI, int CONSTS>
+// SPLIT: few query rows in all: a workgroup owns 32 rows and each of its waves a quarter of their keys (see below).
+template <int DTYPE, int D, bool OUT_F16, bool SLOPE, bool DUMP, bool MULTI, int CONSTS, bool SPLIT = false>
 __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefill_kernel(PrefillParams p, int n_qtiles)
 {
     typedef PfLayout<D> L;
@@ -110,10 +111,13 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
     // scale of the range at once.
     constexpr int LOOP_BYTES = 2 * L::K_BYTES + 2 * L::V_BYTES + 2 * PF_BN * 4;
     constexpr int SHORT_BYTES = PF_SHORT_KEYS * L::V_PITCH + PF_SHORT_KEYS * 4;
-    constexpr bool HAS_SHORT = (D == 64) && !DUMP;
+    constexpr int SPLIT_WAVE_BYTES = 32 * L::V_PITCH + 32 * 4, SUM_BYTES = DT * 16 * WAVE * 4; // (SUM_BYTES: a wave's accumulators)
+    constexpr int SPLIT_BYTES = PF_WAVES * SPLIT_WAVE_BYTES > (PF_WAVES - 1) * SUM_BYTES ? PF_WAVES * SPLIT_WAVE_BYTES : (PF_WAVES - 1) * SUM_BYTES;
+    constexpr bool HAS_SHORT = (D == 64) && !DUMP && !SPLIT;
+    static_assert(!SPLIT || (!DUMP && !MULTI), "the split form exists for one span per row");
     // the common-tile loop with ALiBi only where it fits into the registers without spilling
-    constexpr bool FAST_LOOP = !DUMP && (!SLOPE || (D == 128 && DTYPE == TSATTN_E4M3 && !MULTI)); // (with ALiBi and a loop over parts it would spill)
-    constexpr int LDS_BYTES = (HAS_SHORT && SHORT_BYTES > LOOP_BYTES) ? SHORT_BYTES : LOOP_BYTES;
+    constexpr bool FAST_LOOP = !DUMP && !SPLIT && (!SLOPE || (D == 128 && DTYPE == TSATTN_E4M3 && !MULTI)); // (with ALiBi and a loop over parts it would spill)
+    constexpr int LDS_BYTES = SPLIT ? SPLIT_BYTES : (HAS_SHORT && SHORT_BYTES > LOOP_BYTES) ? SHORT_BYTES : LOOP_BYTES;
     // the fused KVProduct exists where the reference has one: behind int8 attention with an f32 result (cpu_infer.cpp:509-511)
     constexpr bool KV_FUSED = DTYPE == TSATTN_I8 && !OUT_F16 && !DUMP;
     __shared__ __attribute__((aligned(16))) uint8_t lds_raw[LDS_BYTES];
@@ -135,14 +139,15 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
     PF_TOUCH(p.span_tiles); PF_TOUCH(p.n_tokens); PF_TOUCH(p.n_heads); PF_TOUCH(p.k_global_scale);
     PF_TOUCH(p.map.period_tiles); PF_TOUCH(p.map.period_group); PF_TOUCH(p.map.units_per_xcd); PF_TOUCH(p.map.hg_shift);
     PF_TOUCH(p.map.by_qtiles.d); PF_TOUCH(p.map.by_qtiles.m); PF_TOUCH(p.map.by_group_wgs.d); PF_TOUCH(p.map.by_group_wgs.m);
+    PF_TOUCH(n_qtiles); PF_TOUCH(gridDim.x); PF_TOUCH(p.map.resident); PF_TOUCH(p.map.by_units.d); PF_TOUCH(p.map.by_units.m);
     PF_TOUCH(p.map.by_group_units.d); PF_TOUCH(p.map.by_group_units.m); PF_TOUCH(p.map.by_seqs.d); PF_TOUCH(p.map.by_seqs.m);
     PF_TOUCH(p.qs_const); PF_TOUCH(p.ks_const); PF_TOUCH(p.vs_const); PF_TOUCH(p.slope); PF_TOUCH(p.out); PF_TOUCH(p.out_pitch);
 #undef PF_TOUCH
     // which (head, query tile) this workgroup computes: divisions by launch constants whose reciprocals the host
     // has prepared
     int head, tile;
-    wg_locate(p.map, blockIdx.x, gridDim.x, n_qtiles, head, tile);
-    const int q0 = tile * PF_BM + wave * 32;
+    wg_locate<SPLIT || !SLOPE>(p.map, blockIdx.x, gridDim.x, n_qtiles, head, tile);
+    const int q0 = SPLIT ? tile * 32 : tile * PF_BM + wave * 32;
     const int from = q0 + qi;
     const bool row_ok = from < p.n_tokens;
     const int64_t hoff = (int64_t)head * D;
@@ -183,23 +188,24 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
     const bool have_summary = p.span_tiles != nullptr;
     if (have_summary) {
         typedef __attribute__((address_space(4))) const int32_t *const_i32_ptr;
-        const const_i32_ptr t = (const_i32_ptr)(p.span_tiles + ((int64_t)part * n_qtiles + tile) * SPAN_TILE_INTS);
-        const const_i32_ptr w = t + SPAN_TILE_WAVE0 + __builtin_amdgcn_readfirstlane(wave) * SPAN_TILE_WAVE_INTS;
-        b_min_a = t[SPAN_TILE_MIN_A];
-        b_max_b = t[SPAN_TILE_MAX_B];
+        const int64_t summary = SPLIT ? tile / PF_WAVES : (int64_t)part * n_qtiles + tile;
+        const const_i32_ptr t = (const_i32_ptr)(p.span_tiles + summary * SPAN_TILE_INTS);
+        const const_i32_ptr w = t + SPAN_TILE_WAVE0 + (SPLIT ? tile % PF_WAVES : __builtin_amdgcn_readfirstlane(wave)) * SPAN_TILE_WAVE_INTS;
+        b_min_a = SPLIT ? w[0] : t[SPAN_TILE_MIN_A];
+        b_max_b = SPLIT ? w[3] : t[SPAN_TILE_MAX_B];
         w_min_a = w[0];
         w_max_a = w[1];
         w_min_b = w[2];
         w_max_b = w[3];
         w_all_have_keys = w[4] != 0;
     }
-    int sp_a = 1, sp_b = 0;
-    if (row_ok) {
-        sp_a = part_start[from];
-        sp_b = part_finish[from];
-    }
+    // Rows past the end stand for the last row (they have zero operands and are not stored): without spans of their own they
+    // would keep the wave with the longest rows of an odd number of tokens off the paths that need every row to have keys.
+    const int from_span = row_ok ? from : p.n_tokens - 1;
+    int sp_a = part_start[from_span], sp_b = part_finish[from_span];
+    const int rows_left = p.n_tokens - __builtin_amdgcn_readfirstlane(q0); // (of this wave's 32; the same in every lane)
     if (!have_summary) {
-        const bool hk = sp_b >= sp_a;
+        const bool hk = sp_b >= sp_a && rows_left > 0;
         w_all_have_keys = __all(hk);
         w_min_a = hk ? sp_a : 0x7fffffff, w_max_a = hk ? sp_a : -1;
         w_min_b = hk ? sp_b : 0x7fffffff, w_max_b = hk ? sp_b : -1;
@@ -209,21 +215,34 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
             w_min_b = min(w_min_b, __shfl_xor(w_min_b, o, WAVE));
             w_max_b = max(w_max_b, __shfl_xor(w_max_b, o, WAVE));
         }
-        if (lane == 0) {
-            red_lds[wave] = w_min_a;
-            red_lds[PF_WAVES + wave] = w_max_b;
-        }
-        __syncthreads();
-        b_min_a = red_lds[0], b_max_b = red_lds[PF_WAVES];
-        for (int w = 1; w < PF_WAVES; ++w) {
-            b_min_a = min(b_min_a, red_lds[w]);
-            b_max_b = max(b_max_b, red_lds[PF_WAVES + w]);
+        b_min_a = w_min_a, b_max_b = w_max_b;
+        if constexpr (!SPLIT) {
+            if (lane == 0) {
+                red_lds[wave] = w_min_a;
+                red_lds[PF_WAVES + wave] = w_max_b;
+            }
+            __syncthreads();
+            for (int w = 0; w < PF_WAVES; ++w) {
+                b_min_a = min(b_min_a, red_lds[w]);
+                b_max_b = max(b_max_b, red_lds[PF_WAVES + w]);
+            }
         }
     }
 
+    // A row without keys begins behind every key: "some span starts later" then holds for all of the wave's tiles.  (Done once
+    // K and V have been requested: nothing before needs it or the rows' own spans.)
+    auto settle_spans = [&]() __attribute__((always_inline)) {
+        if (have_summary && rows_left > 0 && rows_left < 32) w_all_have_keys = __all(sp_b >= sp_a); // (the summary counts rows past the end as rows without keys)
+        if (!w_all_have_keys) {
+            w_max_a = 0x7fffffff;
+            if (sp_b < sp_a) sp_a = sp_b = 0x7fffffff;
+        }
+    };
+
     if (b_max_b >= b_min_a) {
         // the same in every lane; said explicitly so that everything derived from them stays in scalar registers
-        const int kb_first = __builtin_amdgcn_readfirstlane((b_min_a / PF_BN) * PF_BN);
+        constexpr int FIRST = SPLIT ? 32 : PF_BN;
+        const int kb_first = __builtin_amdgcn_readfirstlane((b_min_a / FIRST) * FIRST);
         const int n_tiles = __builtin_amdgcn_readfirstlane((b_max_b - kb_first) / PF_BN + 1);
 
         // ---- staging: global -> registers -> LDS (K as is; V widened to f16 * row scale) -----------------
@@ -328,7 +347,6 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
         auto weights_general = [&](const typename Qk::acc_t &acc, const float *ksp, int key0, v2h (&pp)[8], float &s0, float &s1) __attribute__((always_inline)) {
             const int rel_a = sp_a - key0 - 4 * g;           // span start relative to this lane's first key
             const unsigned span_w = (unsigned)(sp_b - sp_a); // in-span <=> (unsigned)(off - rel_a) <= span_w
-            const bool has_keys = sp_b >= sp_a;
             const float dist0 = (float)(from - key0 - 4 * g);
             float t[16];
             float tmax = -INFINITY;
@@ -342,7 +360,7 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
                 for (int j = 0; j < 4; ++j) {
                     const int r = c4 * 4 + j;
                     const int off = 8 * c4 + j;
-                    const bool in_span = (unsigned)(off - rel_a) <= span_w && has_keys;
+                    const bool in_span = (unsigned)(off - rel_a) <= span_w;
                     if (DUMP) {
                         if (in_span) {
                             ((float *)p.dbg)[((int64_t)head * p.n_tokens + from) * p.dbg_pitch + key0 + off + 4 * g] = Qk::bits(acc, r);
@@ -379,7 +397,7 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
                 s1 += p1;
             }
         };
-        // Weights with fewer instructions for the usual edge cases: every row of the wave has keys and at most one
+        // Weights with fewer instructions for the usual edge cases: at most one
         // end of the spans cuts through the sub-tile (LOW: some span starts after its first key; HIGH: some span
         // ends before its last).  No maximum is computed; a masked weight is zeroed after the exponential (one
         // compare against a per-lane bound and one select).  The caller checks the weight sum.
@@ -422,7 +440,7 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
             v2h pp[8];
             float s0 = 0.0f, s1 = 0.0f;
             const bool low = w_max_a > key0, high = w_min_b < key0 + 31;
-            bool general = DUMP || !w_all_have_keys || (low && high);
+            bool general = DUMP || (low && high);
             if (!general) {
                 if (low) weights_quick(std::true_type{}, std::false_type{}, acc, ksp, key0, pp, s0, s1);
                 else if (high) weights_quick(std::false_type{}, std::true_type{}, acc, ksp, key0, pp, s0, s1);
@@ -615,7 +633,63 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
         // sequence) everything is requested at once: the V rows and key scales of the range (widened into LDS by
         // all threads) and each wave's K operands (straight into registers: a key's row slice is exactly what the
         // MFMA operand of that lane holds).  One round trip to memory and one barrier instead of one per tile.
-        bool short_done = false;
+        bool short_done = SPLIT;
+        if constexpr (SPLIT) {
+            // ---- few query rows in all: the keys of 32 rows shared out to the waves ---------------------------------
+            // The time of a launch that leaves the chip partly idle is the chain of tiles of its longest workgroup (1.2 to
+            // 1.6 us each).  Here a wave walks a quarter of the keys of 32 rows by itself, 32 keys at a time: K operands from
+            // memory into registers, V through a corner of LDS of its own, NB sub-tiles requested ahead (three: no faster, and
+            // for width 64 a wave less per SIMD) and no barrier until the waves' sums are merged.  K and V are read once per
+            // 32 rows instead of once per 128, out of L2.
+            const int n_sub = (b_max_b - kb_first) / 32 + 1, per = (n_sub + PF_WAVES - 1) / PF_WAVES;
+            const int j0 = __builtin_amdgcn_readfirstlane(wave * per), j1 = __builtin_amdgcn_readfirstlane(min(n_sub, wave * per + per));
+            uint8_t *const v_own = lds_raw + wave * SPLIT_WAVE_BYTES;
+            float *const ks_own = (float *)(v_own + 32 * L::V_PITCH);
+            constexpr int QS = Qk::STEPS, NV = 32 * CHUNKS / WAVE, NB = 2;
+            typename Qk::kop_t kk[NB][QS];
+            v4i vv[NB][NV];
+            float vvs[NB][NV], kks[NB];
+            auto ask = [&](int slot, int j) __attribute__((always_inline)) {
+#pragma unroll
+                for (int st = 0; st < QS; ++st) kk[slot][st] = Qk::load_k_global(kr, qi * (int)p.k_pitch, g, st, j * 32 * (int)p.k_pitch);
+#pragma unroll
+                for (int i = 0; i < NV; ++i) {
+                    const int r = (lane + i * WAVE) / CHUNKS, c = lane % CHUNKS;
+                    vv[slot][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(vr, r * (int)p.v_pitch + c * 16, j * 32 * (int)p.v_pitch, 0));
+                    vvs[slot][i] = vs_ptr ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(vsr, r * 4, j * 128, 0)) : p.vs_const;
+                }
+                kks[slot] = ks_ptr ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ksr, qi * 4, j * 128, 0)) : p.ks_const;
+            };
+#pragma unroll
+            for (int slot = 0; slot < NB; ++slot)
+                if (j0 + slot < j1) ask(slot, j0 + slot);
+            settle_spans();
+#pragma unroll 1
+            for (int jb = j0; jb < j1; jb += NB) {
+#pragma unroll
+                for (int slot = 0; slot < NB; ++slot) {
+                    const int j = jb + slot;
+                    if (j < j1) {
+                        typename Qk::acc_t acc = {0};
+#pragma unroll
+                        for (int st = 0; st < QS; ++st) acc = qk.step(kk[slot][st], st, acc);
+                        asm volatile("" ::: "memory"); // (a wave's LDS accesses stay in order: the last sub-tile has been read)
+#pragma unroll
+                        for (int i = 0; i < NV; ++i) {
+                            const int r = (lane + i * WAVE) / CHUNKS, c = lane % CHUNKS;
+                            v8h lo, hi;
+                            widen_v<DTYPE, !VS_CONST>(vv[slot][i], vvs[slot][i], lo, hi);
+                            *(v8h *)(v_own + r * L::V_PITCH + c * 32) = lo;
+                            *(v8h *)(v_own + r * L::V_PITCH + c * 32 + 16) = hi;
+                        }
+                        if (lane < 32) ks_own[lane] = kks[slot] * ads;
+                        if (j + NB < j1) ask(slot, j + NB);
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave's rows are in LDS (nobody else reads them)
+                        sub_tile(acc, ks_own, v_own, kb_first + 32 * j);
+                    }
+                }
+            }
+        }
         if constexpr (HAS_SHORT) {
             if (n_tiles * PF_BN <= PF_SHORT_KEYS) {
                 short_done = true;
@@ -663,6 +737,7 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
                     }
                 }
                 if (tid < n_keys) ks_short[tid] = sks * ads;
+                settle_spans();
                 __syncthreads();
 #pragma unroll 1
                 for (int j = 0; s_lo + j <= s_hi; ++j) {
@@ -686,6 +761,7 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
         load_tile();
         store_tile(0);
         if (n_tiles > 1) load_tile();
+        settle_spans();
         __syncthreads();
         // Tiles in key order are: not needed by this wave, partly inside its spans, fully inside, partly
         // inside (the diagonal), not needed.  The fully-inside run [f0, f1) takes the common-tile path (never
@@ -727,6 +803,50 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
     if (MULTI && part + 1 < n_parts) __syncthreads(); // the next part stages its tiles into the same LDS (and reduces into red_lds)
     } // parts
 
+    if constexpr (SPLIT) {
+        // Merge: every wave scales its sums to the common maximum; the first adds the others' up and goes on alone.
+        __shared__ float stats[PF_WAVES][2][32];
+        l += l2;
+        l += __shfl_xor(l, 32, WAVE);
+        if (g == 0) {
+            stats[wave][0][qi] = m_ref;
+            stats[wave][1][qi] = l;
+        }
+        __syncthreads();
+        float top = m_ref;
+#pragma unroll
+        for (int w = 0; w < PF_WAVES; ++w) top = fmaxf(top, stats[w][0][qi]);
+        l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < PF_WAVES; ++w) l += stats[w][1][qi] * fast_exp2(stats[w][0][qi] - top);
+        const float f = fast_exp2(m_ref - top);
+        v4f *const merge = (v4f *)lds_raw + lane;
+#pragma unroll
+        for (int i = 0; i < DT; ++i) o_acc[i] *= f;
+        if (wave != 0) {
+#pragma unroll
+            for (int i = 0; i < DT; ++i)
+#pragma unroll
+                for (int c4 = 0; c4 < 4; ++c4)
+                    merge[((wave - 1) * DT * 4 + i * 4 + c4) * WAVE] = v4f{o_acc[i][4 * c4], o_acc[i][4 * c4 + 1], o_acc[i][4 * c4 + 2], o_acc[i][4 * c4 + 3]};
+        }
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int w = 0; w < PF_WAVES - 1; ++w)
+#pragma unroll
+            for (int i = 0; i < DT; ++i)
+#pragma unroll
+                for (int c4 = 0; c4 < 4; ++c4) {
+                    const v4f x = merge[(w * DT * 4 + i * 4 + c4) * WAVE];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) o_acc[i][4 * c4 + k] += x[k];
+                }
+        m_ref = top;
+        l = g == 0 ? l : 0.0f;
+        l2 = 0.0f;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // read before results are staged in the same memory
+    }
     // ---- epilogue: add the zero vector's weight, normalise, store -----------------------------------
     l += l2;
     float l_all = l + __shfl_xor(l, 32, WAVE);
@@ -740,10 +860,10 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
         // 16 bytes per lane.
         constexpr int KV_PITCH = D + 16;
         static_assert(PF_WAVES * 2 * 32 * KV_PITCH <= LDS_BYTES, "the KVProduct rows of all waves fit into the tiles' LDS");
-        __syncthreads(); // every wave is done with the K and V tiles
+        if constexpr (!SPLIT) __syncthreads(); // every wave is done with the K and V tiles
         // (what follows is computed from these copies, which the compiler cannot trace back: nothing of it is
         // prepared before the tile loop and kept in registers through it)
-        int qi = lane & 31, g = lane >> 5, q0 = tile * PF_BM + wave * 32;
+        int qi = lane & 31, g = lane >> 5, q0 = SPLIT ? tile * 32 : tile * PF_BM + wave * 32;
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("" : "+v"(qi), "+v"(g), "+v"(q0));
 #endif
@@ -803,10 +923,10 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
             // instruction writes four whole rows of the head (16 bytes per lane, consecutive), half as many of them.
             constexpr int OUT_PITCH = D * 2 + 16;
             static_assert(PF_WAVES * 32 * OUT_PITCH <= LDS_BYTES, "the waves' result rows fit into the tiles' LDS");
-            __syncthreads(); // every wave is done with the K and V tiles
+            if constexpr (!SPLIT) __syncthreads(); // every wave is done with the K and V tiles
             // (computed from these copies, which the compiler cannot trace back: nothing of it is prepared before the
             // tile loop and kept in registers through it)
-            int qi = lane & 31, g = lane >> 5, q0 = tile * PF_BM + wave * 32;
+            int qi = lane & 31, g = lane >> 5, q0 = SPLIT ? tile * 32 : tile * PF_BM + wave * 32;
 #if defined(__HIP_DEVICE_COMPILE__)
             asm volatile("" : "+v"(qi), "+v"(g), "+v"(q0));
 #endif
@@ -835,8 +955,8 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
         // the same for an f32 result, half of the head's columns at a time (a wave's corner of LDS holds 32 half rows)
         constexpr int HALF = D / 2, OUT_PITCH = HALF * 4 + 16;
         static_assert(PF_WAVES * 32 * OUT_PITCH <= LDS_BYTES, "the waves' result rows fit into the tiles' LDS");
-        __syncthreads(); // every wave is done with the K and V tiles (and with the rows a fused KVProduct staged)
-        int qi = lane & 31, g = lane >> 5, q0 = tile * PF_BM + wave * 32;
+        if constexpr (!SPLIT) __syncthreads(); // every wave is done with the K and V tiles (and with the rows a fused KVProduct staged)
+        int qi = lane & 31, g = lane >> 5, q0 = SPLIT ? tile * 32 : tile * PF_BM + wave * 32;
 #if defined(__HIP_DEVICE_COMPILE__)
         asm volatile("" : "+v"(qi), "+v"(g), "+v"(q0));
 #endif
@@ -868,7 +988,7 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
         if (p.sum_weight_log) {
             // (the row's index from opaque copies again: kept in registers through the tile loops it costs the ALiBi
             // kernels a spill; the kernels with a loop over parts around the tile loops fare better as they are)
-            int qi_e = lane & 31, g_e = lane >> 5, q0_e = tile * PF_BM + wave * 32;
+            int qi_e = lane & 31, g_e = lane >> 5, q0_e = SPLIT ? tile * 32 : tile * PF_BM + wave * 32;
 #if defined(__HIP_DEVICE_COMPILE__)
             asm volatile("" : "+v"(qi_e), "+v"(g_e), "+v"(q0_e));
 #endif
@@ -880,6 +1000,18 @@ __global__ __launch_bounds__(PF_THREADS, (D == 64 && !MULTI) ? 3 : 2) void prefi
     }
 }
 
+// (ALiBi always compiled in: with slope 0 it adds zeros)
+template <int DTYPE, int D, bool OUT_F16>
+static void launch_prefill_split(const PrefillParams &p_in, hipStream_t st)
+{
+    PrefillParams p = p_in;
+    const int n_qtiles = (p.n_tokens + 31) / 32;
+    p.map = wg_plan(n_qtiles, p.n_heads, D, 32, p.period_tiles * (PF_BM / 32));
+    const dim3 grid((unsigned)n_qtiles * (unsigned)p.n_heads), block(PF_THREADS);
+    if (p.qs == nullptr && p.vs == nullptr) hipLaunchKernelGGL((prefill_kernel<DTYPE, D, OUT_F16, true, false, false, 2, true>), grid, block, 0, st, p, n_qtiles);
+    else hipLaunchKernelGGL((prefill_kernel<DTYPE, D, OUT_F16, true, false, false, 0, true>), grid, block, 0, st, p, n_qtiles);
+}
+
 template <int DTYPE, int D, bool OUT_F16>
 static void launch_prefill_do(const PrefillParams &p_in, dim3 grid2, hipStream_t st)
 {
@@ -887,6 +1019,15 @@ static void launch_prefill_do(const PrefillParams &p_in, dim3 grid2, hipStream_t
     dim3 grid(grid2.x * grid2.y);
     PrefillParams p = p_in;
     p.map = wg_plan(n_qtiles, p.n_heads, D, PF_BM, p.period_tiles);
+    // Few rows in all: the keys of 32 rows shared out to the waves of a workgroup.  From where the chip holds every workgroup of
+    // that form at once (two per compute unit for width 128, three for 64) it is never slower: one sequence of 700 tokens, 12 heads
+    // of width 64: 17.6 -> 9.3 us, of 2000 tokens, 8 heads of width 128: 38 -> 25 us, 20 of 100 tokens, 8 heads: 8.3 -> 6.4 us.
+    // Beyond that the longer chains of width 64 still gain (3 of 1300 tokens, 8 heads: 30 -> 19 us; 6 of 600, 12 heads: 22 -> 20 us;
+    // at 384 workgroups 4 of 1024 tokens lose 8 %).
+    const int64_t wgs = (int64_t)grid2.x * grid2.y, split_wgs = (int64_t)((p.n_tokens + 31) / 32) * p.n_heads;
+    const bool few = split_wgs <= 256 * (D == 64 ? 3 : 2) || (D == 64 && p.span_len_hint >= 512 && wgs <= 352);
+    if (few && !p.dbg && p.n_parts == 1 && (int64_t)p.n_tokens * (p.k_pitch > p.v_pitch ? p.k_pitch : p.v_pitch) < ((int64_t)1 << 31))
+        return launch_prefill_split<DTYPE, D, OUT_F16>(p, st);
     const bool dump = p.dbg != nullptr;
     const bool slope = p.slope != 0.0f;
     dim3 block(PF_THREADS);

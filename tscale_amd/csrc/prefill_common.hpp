@@ -58,10 +58,10 @@ struct QkMma<TSATTN_E4M3, D> {
     }
     __device__ acc_t step(kop_t kk, int s, acc_t acc) const { return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kk, q[s], acc, 0, 0, 0, 0, 0, 0); }
     // the same operand straight from global memory (row_off: byte offset of the key's row in the descriptor)
-    __device__ static kop_t load_k_global(__amdgpu_buffer_rsrc_t kr, int row_off, int g, int s)
+    __device__ static kop_t load_k_global(__amdgpu_buffer_rsrc_t kr, int row_off, int g, int s, int scalar_off = 0)
     {
-        const v4i a = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(kr, row_off + 64 * s + 32 * g, 0, 0));
-        const v4i b = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(kr, row_off + 64 * s + 32 * g + 16, 0, 0));
+        const v4i a = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(kr, row_off + 64 * s + 32 * g, scalar_off, 0));
+        const v4i b = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(kr, row_off + 64 * s + 32 * g + 16, scalar_off, 0));
         return v8i{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
     }
     __device__ static float to_float(const acc_t &a, int r) { return a[r]; }
@@ -94,9 +94,9 @@ struct QkMma<TSATTN_I8, D> {
     typedef v4i kop_t;
     __device__ static kop_t load_k(const uint8_t *krow, int g, int s) { return *(const v4i *)(krow + 32 * s + 16 * g); }
     __device__ acc_t step(kop_t kk, int s, acc_t acc) const { return __builtin_amdgcn_mfma_i32_32x32x32_i8(kk, q[s], acc, 0, 0, 0); }
-    __device__ static kop_t load_k_global(__amdgpu_buffer_rsrc_t kr, int row_off, int g, int s)
+    __device__ static kop_t load_k_global(__amdgpu_buffer_rsrc_t kr, int row_off, int g, int s, int scalar_off = 0)
     {
-        return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(kr, row_off + 32 * s + 16 * g, 0, 0));
+        return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(kr, row_off + 32 * s + 16 * g, scalar_off, 0));
     }
     __device__ static float to_float(const acc_t &a, int r) { return (float)a[r]; }
     __device__ static float bits(const acc_t &a, int r) { return __int_as_float(a[r]); }

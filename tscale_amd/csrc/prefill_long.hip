@@ -137,18 +137,16 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_long_kernel(PrefillPara
         w_max_b = w[3];
         w_all_have_keys = w[4] != 0;
     }
-    int sp_a = 1, sp_b = 0;
-    if (row_ok) {
-        sp_a = p.span_start[from];
-        sp_b = p.span_finish[from];
-    }
+    const int from_span = row_ok ? from : p.n_tokens - 1; // (rows past the end stand for the last row, as in prefill_kernel)
+    const int sp_a = p.span_start[from_span], sp_b = p.span_finish[from_span];
+    if (have_summary && q0 < p.n_tokens && q0 + 32 > p.n_tokens) w_all_have_keys = __all(sp_b >= sp_a);
     Qk qk;
     if (row_ok) qk.load_q(p.q + (int64_t)from * p.q_pitch + hoff, g);
     else qk.clear_q();
     float qs = row_ok ? (p.qs ? p.qs[(int64_t)head * p.scale_pitch + from] : p.qs_const) : 0.0f;
     int *const red = (int *)(pl_lds + PL_RED_OFF);
     if (!have_summary) {
-        const bool hk = sp_b >= sp_a;
+        const bool hk = sp_b >= sp_a && q0 < p.n_tokens;
         w_all_have_keys = __all(hk);
         w_min_a = hk ? sp_a : 0x7fffffff, w_max_a = hk ? sp_a : -1;
         w_min_b = hk ? sp_b : 0x7fffffff, w_max_b = hk ? sp_b : -1;

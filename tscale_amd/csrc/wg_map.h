@@ -43,8 +43,21 @@ struct WgMap {
     int period_group;  // G: units per group of the period-aware order, 0 = that order is not used
     int units_per_xcd; // R: (head group, sequence) units per XCD
     int hg_shift;      // log2 of the heads that share a cache line (d = 64 with an even head count: 1)
-    WgDiv by_qtiles, by_group_wgs, by_group_units, by_seqs;
+    int resident;      // workgroups per XCD if the chip holds all of them at once, 0 = it does not (or they are not shared out evenly)
+    WgDiv by_qtiles, by_group_wgs, by_group_units, by_seqs, by_units;
 };
+
+// A launch that the chip holds as a whole: an XCD's workgroups i, i + 32, i + 64 share a compute unit, and the launch lasts
+// as long as the fullest one.  Position i of `n` in such a launch -> which workgroup of the order "longest first" goes there:
+// the longest ones where the fewest others come, a short one next to a long one.  (One sequence of 4096 tokens, 16 heads of
+// width 128: 81 us longest first, the two longest on the same compute unit.)
+TSATTN_HD inline uint32_t wg_even(uint32_t i, uint32_t n)
+{
+    // compute unit c; n % 32 of them hold one more than the others
+    const uint32_t c = i & 31, first = (c - n) & (n < 32 ? 0u : 31u), few = n < 32 ? i : first;
+    const uint32_t later = (i < 64) & (n >= 64) ? 63 - first : n - 1 - c;
+    return i < 32 ? few : later;
+}
 
 // Plans the mapping of a launch of n_qtiles * n_heads workgroups.  The period-aware order is usable only if every
 // XCD's share of the grid is a whole number of (head group, sequence) units; units are then walked in groups whose
@@ -60,8 +73,10 @@ inline WgMap wg_plan(int n_qtiles, int n_heads, int head_dim, int rows_per_tile,
     m.hg_shift = hg == 2 ? 1 : 0;
     m.by_qtiles = wg_make_div((uint32_t)n_qtiles);
     m.by_group_wgs = m.by_group_units = m.by_seqs = wg_make_div(1);
+    m.by_units = wg_make_div((uint32_t)(n_heads / hg));
     const int T = period_tiles;
     const int64_t n_wg = (int64_t)n_qtiles * n_heads, per_xcd = n_wg / 8;
+    m.resident = n_wg % (8 * hg) == 0 && per_xcd <= 32 * (head_dim == 64 ? 3 : 2) ? (int)per_xcd : 0;
     if (T > 1 && n_wg % 8 == 0 && per_xcd % (T * hg) == 0 && n_qtiles % T == 0) {
         const int R = (int)(per_xcd / (T * hg));
         const int64_t unit_bytes = (int64_t)kv_bytes_per_value * T * rows_per_tile * head_dim * hg;
@@ -83,6 +98,10 @@ inline WgMap wg_plan(int n_qtiles, int n_heads, int head_dim, int rows_per_tile,
 // equal work per XCD, and the K/V rows a run shares stay in its L2.  With d = 64 one 128-byte line of K or V holds
 // the rows of two heads: consecutive workgroups then alternate between the two heads of a pair on the same query
 // tile, so the pair shares the line in L2.
+//
+// EVEN = false: without the order of resident launches, for kernels of short windows: their rows are all about as long, and its
+// instructions cost them 3 %.
+template <bool EVEN = true>
 TSATTN_HD inline void wg_locate(const WgMap &m, uint32_t block, uint32_t n_wg, int n_qtiles, int &head, int &tile)
 {
     const int hs = m.hg_shift, hg = 1 << hs;
@@ -92,7 +111,7 @@ TSATTN_HD inline void wg_locate(const WgMap &m, uint32_t block, uint32_t n_wg, i
         // of G units position by position from the end of the sequences to their start: the longest rows of every
         // unit first, the shortest last, so the launch does not end on a few long-running workgroups.
         const int T = m.period_tiles, G = m.period_group;
-        const uint32_t x = block & 7, i = block >> 3; // XCD and index inside its run
+        const uint32_t x = block & 7, i = EVEN && m.resident ? wg_even(block >> 3, (uint32_t)m.resident) : block >> 3; // XCD and index inside its run
         uint32_t j, rem, seq;
         const uint32_t grp = wg_divmod(i, m.by_group_wgs, j);          // / (G * T * hg)
         const uint32_t pos_rank = wg_divmod(j, m.by_group_units, rem); // / (G * hg)
@@ -101,10 +120,14 @@ TSATTN_HD inline void wg_locate(const WgMap &m, uint32_t block, uint32_t n_wg, i
         head = (int)((hgrp << hs) + (rem & (uint32_t)(hg - 1)));
         tile = (int)(seq * (uint32_t)T + ((uint32_t)T - 1 - pos_rank));
     } else {
-        uint32_t wg = block, t;
-        if ((n_wg & 7) == 0) wg = (block & 7) * (n_wg >> 3) + (block >> 3);
-        const uint32_t hgrp = wg_divmod(wg >> hs, m.by_qtiles, t);
-        head = (int)((hgrp << hs) + (wg & (uint32_t)(hg - 1)));
+        // Resident launch: all heads' longest rows first, an XCD sees every eighth head group.
+        const bool resident = EVEN && m.resident != 0;
+        const uint32_t x = block & 7, i = wg_even(block >> 3, (uint32_t)m.resident);
+        const uint32_t run = (n_wg & 7) == 0 ? x * (n_wg >> 3) + (block >> 3) : block;
+        uint32_t r;
+        const uint32_t q = wg_divmod(resident ? ((i >> hs) << 3) + x : run >> hs, resident ? m.by_units : m.by_qtiles, r);
+        const uint32_t hgrp = resident ? r : q, t = resident ? q : r;
+        head = (int)((hgrp << hs) + ((resident ? i : run) & (uint32_t)(hg - 1)));
         tile = n_qtiles - 1 - (int)t; // long rows first
     }
 }
