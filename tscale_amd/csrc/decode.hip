@@ -280,7 +280,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         }
     };
     int base = s0 + wave * ROWS_PER_STEP;
-    if (base < s1) request(base);
+    if (FRONT && base < s1) request(base);
 
     // ---- query slice of this lane ----------------------------------------------------------------
     QFrag<DTYPE> qf;
@@ -398,6 +398,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 
     for (; base < s1; base += DEC_WAVES * ROWS_PER_STEP) {
+        if constexpr (!FRONT) request(base); // (with nothing to wait for but the query a second copy of the requests only makes the code longer: 4 % of a short launch)
         float s[DEC_U];
         float m_new = m;
 #pragma unroll
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             l += pu;
             accumulate_values<DTYPE>(pu * vsr[u], vreg[u], acc);
         }
-        if (base + DEC_WAVES * ROWS_PER_STEP < s1) request(base + DEC_WAVES * ROWS_PER_STEP);
+        if (FRONT && base + DEC_WAVES * ROWS_PER_STEP < s1) request(base + DEC_WAVES * ROWS_PER_STEP);
     }
 
     // ---- merge the lane groups of this wave ---------------------------------------------------
