@@ -38,6 +38,12 @@ def test_products_at_tile_edges(ctx, m, n, k):
     assert np.array_equal(added.cpu().numpy(), orc.matmul_i8(a, w, mode=2, scale=0.003, out=state))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 313001, 64), (16, 104170, 192), (17, 31300, 640), (31, 19999, 1088), (32, 12003, 2048), (5, 6600, 3072)])
+def test_products_of_a_large_matrix_under_few_rows(ctx, m, n, k):
+    """Blocks of rows cut by the waves' shares, a last block that is not full, K that ends in half a stage; all result forms."""
+    test_products_at_tile_edges(ctx, m, n, k)
+
+
 @pytest.mark.parametrize("m,heads,d,k", [(40, 2, 128, 64), (129, 3, 64, 192), (190, 5, 128, 320), (1030, 33, 64, 128), (1300, 17, 128, 64)])
 @pytest.mark.parametrize("variant", ["rope", "resid", "relu"])
 def test_products_with_the_producer_at_tile_edges(ctx, m, heads, d, k, variant):

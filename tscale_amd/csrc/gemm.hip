@@ -6,6 +6,7 @@
 // Here the largest products (256 x 256 output tiles; bound by the matrix cores) and the choice between the kernels; a few
 // hundred to a few thousand rows: gemm_mid.hip, few rows (one token per sequence): gemm_few.hpp.
 // Integer sums are exact, so every decomposition gives the same bits.
+#include <algorithm>
 #include <type_traits>
 #include "common.hpp"
 #include "kernels.hpp"
@@ -384,12 +385,14 @@ FewParams few_params(const GemmParams &p);
 Tiles choose_tiles(const GemmParams &p, bool wide_ok, bool normalised)
 {
     const int64_t n256 = (p.n + 255) / 256, n128 = (p.n + 127) / 128;
-    double best = rounds_us(n128 * ((p.m + 127) / 128), 6.7, 0.40, 0.1, p.k);
+    // no tiles faster than memory brings them the matrix (32 x 50257 x 2048: 26.5 us, 3.9 TB/s)
+    const double memory = 4.0 + (double)p.n * p.k * 1e-6 / 4.6;
+    double best = std::max(memory, rounds_us(n128 * ((p.m + 127) / 128), 6.7, 0.40, 0.1, p.k));
     Tiles tiles = Tiles::ROWS128;
     const auto consider = [&](Tiles t, double us) {
         if (us < best) { best = us; tiles = t; }
     };
-    consider(Tiles::ROWS64, rounds_us(n128 * ((p.m + 63) / 64), 5.8, 0.25, 0.1, p.k));
+    consider(Tiles::ROWS64, std::max(memory, rounds_us(n128 * ((p.m + 63) / 64), 5.8, 0.25, 0.1, p.k)));
     if (wide_ok) consider(Tiles::WIDE, rounds_us(n256 * ((p.m + 255) / 256), 10.0, 0.87, 0.6, p.k));
     if (p.m <= FEW_ROWS) consider(Tiles::FEW, few_ns(few_params(p), p.mode == TSATTN_MM_I32_PLANES ? 16 : 1) * 1e-3 + (normalised ? 5.0 : 0.0));
     return tiles;

@@ -1,5 +1,5 @@
 // The int8 product with few activation rows (one token per sequence): plan and launches.  The kernel: gemm_few.hpp.
-#include "gemm_few.hpp"
+#include "gemm_stream.hpp"
 
 namespace tsattn {
 
@@ -119,6 +119,30 @@ hipError_t launch_norm(const FewParams &p, int planes, bool resid, hipStream_t s
     return launch_one<TSATTN_MM_I32, 1, 4, false>(p, st, prepare);
 }
 
+// The matrix through LDS (gemm_stream.hpp) from 20 MB on and up to 32 rows: 50257 x 2048 under 32 rows 27.8 -> 22.5 us, under
+// one 26.3 -> 20.4; 20000 x 1024: 8.3 -> 8.0 and 8.6 -> 7.7.  Below that its one long run of the matrix per compute unit is no
+// gain (8192 x 2048: 6.9 and 7.2 us); with 64 rows the activations leave little room for the waves' rings (20000 x 1024: 9.3
+// and 10.2 us), and so does a K of 5000 and more.
+bool stream_fits(const FewParams &p)
+{
+    return p.a && p.m <= 32 && p.n * p.k >= 20000000 && gs_lds_bytes(few_mt(p.m), p.k) <= GF_LDS_MAX;
+}
+
+template <int MODE>
+hipError_t launch_stream(FewParams p, hipStream_t st, bool prepare)
+{
+    if (prepare) {
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_stream_kernel<MODE, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, GF_LDS_MAX);
+        return e != hipSuccess ? e : hipFuncSetAttribute((const void *)gemm_stream_kernel<MODE, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, GF_LDS_MAX);
+    }
+    const int mt = few_mt(p.m);
+    const unsigned lds = (unsigned)gs_lds_bytes(mt, p.k);
+    p.k_chunk = (int)gs_rows_bytes(mt, p.k);
+    if (mt == 1) hipLaunchKernelGGL((gemm_stream_kernel<MODE, 1>), dim3(256), dim3(GS_THREADS), lds, st, p);
+    else hipLaunchKernelGGL((gemm_stream_kernel<MODE, 2>), dim3(256), dim3(GS_THREADS), lds, st, p);
+    return hipGetLastError();
+}
+
 } // namespace
 
 bool few_source_ok(const FewParams &p)
@@ -127,9 +151,13 @@ bool few_source_ok(const FewParams &p)
            (p.src_planes == 1 || p.src_planes == 2 || p.src_planes == 4 || (p.src_planes == 0 && p.state));
 }
 
-int few_parts(const FewParams &p, int max_parts) { return few_best(p, 1, max_parts).parts; }
+int few_parts(const FewParams &p, int max_parts) { return stream_fits(p) ? 1 : few_best(p, 1, max_parts).parts; }
 
-double few_ns(const FewParams &p, int max_parts) { return few_best(p, 1, max_parts).ns; }
+double few_ns(const FewParams &p, int max_parts)
+{
+    // (through LDS: the matrix, and the result; as measured between 16384 x 2048, 50257 x 512 and 50257 x 2048)
+    return stream_fits(p) ? 4000 + (double)p.n * p.k / 6100 + p.m * (15 + (double)p.n * 4 / 4500) : few_best(p, 1, max_parts).ns;
+}
 
 hipError_t launch_gemm_few(const FewParams &params, hipStream_t st)
 {
@@ -137,6 +165,11 @@ hipError_t launch_gemm_few(const FewParams &params, hipStream_t st)
     if (p.m < 1 || p.m > FEW_ROWS || p.k <= 0 || p.k % 64 || p.parts < 1 || (p.parts > 1 && p.mode != TSATTN_MM_I32) ||
         (!p.a && (p.mode != TSATTN_MM_I32 || !few_source_ok(p))))
         return hipErrorInvalidValue;
+    if (p.parts == 1 && stream_fits(p)) {
+        if (p.mode == TSATTN_MM_I32) return launch_stream<TSATTN_MM_I32>(p, st, false);
+        if (p.mode == TSATTN_MM_F32) return launch_stream<TSATTN_MM_F32>(p, st, false);
+        return launch_stream<TSATTN_MM_ADD_SCALED>(p, st, false);
+    }
     const FewPlan f = few_best(p, p.parts, p.parts);
     if (f.parts == 0) return hipErrorInvalidValue;
     p.wn_log = f.wn_log; p.wn = 1 << f.wn_log; p.wk = f.waves >> f.wn_log; p.wk_log = log2_of(p.wk); p.group_log = log2_of(p.group);
@@ -159,6 +192,9 @@ hipError_t prepare_gemm_few()
         if (e == hipSuccess) e = launch_rows<TSATTN_MM_F32>(p, mt, nullptr, true);
         if (e == hipSuccess) e = launch_rows<TSATTN_MM_ADD_SCALED>(p, mt, nullptr, true);
     }
+    if (e == hipSuccess) e = launch_stream<TSATTN_MM_I32>(p, nullptr, true);
+    if (e == hipSuccess) e = launch_stream<TSATTN_MM_F32>(p, nullptr, true);
+    if (e == hipSuccess) e = launch_stream<TSATTN_MM_ADD_SCALED>(p, nullptr, true);
     for (int planes = 0; planes <= 4 && e == hipSuccess; planes = planes ? planes * 2 : 1)
         for (int resid = planes ? 0 : 1; resid < 2 && e == hipSuccess; ++resid) e = launch_norm(p, planes, resid != 0, nullptr, true);
     return e;
