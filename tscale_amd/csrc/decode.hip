@@ -263,18 +263,18 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     const float *vsb = p.vs ? p.vs + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
     v4i kreg[DEC_U], vreg[DEC_U];
     float ksr[DEC_U], vsr[DEC_U];
+    int row[DEC_U];
     auto request = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < DEC_U; ++u) {
-            const int r = base + u * KPL + g;
-            const int rc = (r < s1) ? r : s1 - 1; // clamp the address, mask the logit below
+            row[u] = base + u * KPL + g;
+            const int rc = (row[u] < s1) ? row[u] : s1 - 1; // clamp the address, mask the logit below
             kreg[u] = __builtin_nontemporal_load((const v4i *)(kbase + (int64_t)rc * p.tok_stride));
             ksr[u] = ksb ? ksb[rc] : p.ks_const;
         }
 #pragma unroll
         for (int u = 0; u < DEC_U; ++u) {
-            const int r = base + u * KPL + g;
-            const int rc = (r < s1) ? r : s1 - 1;
+            const int rc = (row[u] < s1) ? row[u] : s1 - 1;
             vreg[u] = __builtin_nontemporal_load((const v4i *)(vbase + (int64_t)rc * p.tok_stride));
             vsr[u] = vsb ? vsb[rc] : p.vs_const;
         }
@@ -398,7 +398,15 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 
     for (; base < s1; base += DEC_WAVES * ROWS_PER_STEP) {
-        if constexpr (!FRONT) request(base); // (with nothing to wait for but the query a second copy of the requests only makes the code longer: 4 % of a short launch)
+        if constexpr (!FRONT) { // (with nothing to wait for but the query a second copy of the requests only makes the code longer: 4 % of a short launch)
+            request(base);
+            // Every request of the step before the first sum: left to itself the compiler moves the last value row's request
+            // behind the waits for the keys, and where one workgroup per compute unit is all there is nothing hides that row's
+            // latency (e4m3, width 128: 8 x 16 pairs of 1024 rows 13.2 us that way, 12.6 this way; 16 x 16 16.4 and 15.9; width 64,
+            // 13 x 12 pairs of 1500 rows 11.6 and 11.2).  With two workgroups per unit it can be the other way round (int8,
+            // width 128: 32 x 16 pairs of 512 rows 14.2 and 14.6 us, 24 x 16 of 2048 36.5 and 37.6), from three on they are equal.
+            __builtin_amdgcn_sched_barrier(0);
+        }
         float s[DEC_U];
         float m_new = m;
 #pragma unroll
@@ -406,12 +414,12 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             float bits = group_sum_bits<DTYPE, LPK>(qf.dot_partial_as_bits(kreg[u]));
             float accf = (DTYPE == TSATTN_I8) ? (float)__float_as_int(bits) : bits;
             if (DUMP) {
-                if (c == 0 && (base + u * KPL + g) < s1) {
-                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + (base + u * KPL + g)] = bits;
+                if (c == 0 && row[u] < s1) {
+                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + row[u]] = bits;
                 }
             }
-            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - (base + u * KPL + g));
-            s[u] = ((base + u * KPL + g) < s1) ? dp : -INFINITY;
+            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - row[u]);
+            s[u] = (row[u] < s1) ? dp : -INFINITY;
             m_new = fmaxf(m_new, s[u]);
         }
         float alpha = fast_exp2(m - m_new);
