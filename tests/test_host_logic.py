@@ -38,3 +38,13 @@ def test_prefill_workgroup_mapping_visits_every_head_and_tile_once(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout[-2000:]
     assert r.stdout.startswith("OK")
+
+
+def test_decode_splits(tmp_path):
+    """tests/cpp/test_decode_splits.cpp holds the choice of tscale_amd/csrc/decode_splits.h against measured launches."""
+    import subprocess
+    exe = tmp_path / "test_decode_splits"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", str(exe), os.path.join(ROOT, "tests", "cpp", "test_decode_splits.cpp")], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout[-2000:]
+    assert r.stdout.startswith("OK")

@@ -10,6 +10,7 @@
 
 #include "../../include/tsattn.h"
 #include "../../include/tsattn_test_hooks.h"
+#include "decode_splits.h"
 #include "kernels.hpp"
 
 struct tsattn_ctx {
@@ -91,22 +92,8 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     int splits = a->n_splits;
     if (splits < 0 || splits > max_splits) return fail(TSATTN_ERR_SCRATCH, "tsattn_decode: n_splits %d exceeds the scratch's %d for this batch", splits, max_splits);
     if (splits == 0) {
-        // The number of splits with the least time by a fit of measured ones: a workgroup streams its rows at 37 bytes per
-        // nanosecond or at its share of the memory's rate, and more than one split costs the merge launch.  One sequence of
-        // 12 heads of width 64, 1 or 8 splits: 6.9 or 8.4 us at 701 rows, 19 or 9.7 us at 4096; 13 such sequences of 1500
-        // rows 10.8 us with 1 and 13.1 us with 2; 8 of 16 heads of width 128 and 4096 rows 34 us with 1 and 28 us with 4;
-        // from 256 pairs up one split is best at any length.
-        const int64_t pairs = (int64_t)a->n_seqs * a->n_heads;
-        int64_t rows = a->max_len;   // rows one query can see
-        if (a->window < rows) rows = a->window > 0 ? a->window : 1;
-        const double bytes = (double)rows * (2 * a->head_dim + 8);
-        int64_t want = 1;
-        double best = bytes / std::min(37.0, 6800.0 / (double)pairs);
-        for (int64_t s = 2; s <= max_splits && s * pairs <= 1024 && rows / s >= 256; ++s) {
-            const double ns = bytes / (double)s / std::min(37.0, 6800.0 / (double)(pairs * s)) + 3500.0 + 40.0 * (double)s;
-            if (ns < best) { best = ns; want = s; }
-        }
-        splits = (int)want;
+        const int64_t rows = a->window < a->max_len ? std::max<int64_t>(a->window, 1) : a->max_len; // rows one query can see
+        splits = tsattn::decode_choose_splits(rows, a->head_dim, (int64_t)a->n_seqs * a->n_heads, max_splits);
     }
     tsattn::DecodeParams p = {};
     p.q = (const uint8_t *)a->q; p.q_pitch = a->q_pitch; p.q_scale = a->q_scale; p.q_scale_const = a->q_scale_const;

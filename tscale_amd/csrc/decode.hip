@@ -15,6 +15,7 @@
 // scale (:454).  The running max starts at 0 in every split, which is what the zero logit makes it
 // in the reference anyway, so no split ever needs a -inf state.
 #include "common.hpp"
+#include "decode_splits.h"
 #include "kernels.hpp"
 
 namespace tsattn {
@@ -22,6 +23,7 @@ namespace tsattn {
 constexpr int DEC_THREADS = 256;
 constexpr int DEC_WAVES = DEC_THREADS / WAVE;
 constexpr int DEC_LONG = 8, DEC_SHORT = 2; // cache rows per lane group and step (short: ranges of one step of four waves)
+static_assert(decode_step_rows(64) == DEC_WAVES * DEC_LONG * (WAVE / (64 / 16)) && decode_step_rows(128) == DEC_WAVES * DEC_LONG * (WAVE / (128 / 16)), "the split rule's step");
 
 template <int DTYPE>
 struct QFrag;
