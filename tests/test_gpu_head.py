@@ -1,5 +1,7 @@
 """GPU: the embedding sum, the final softmax with the greedy choice (ComputePrediction, gpt/train/cpu_infer.cpp:552-582) and
 the sampled choice (SampleFromDistr, :585-599) through the C ABI against the oracle."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -99,3 +101,65 @@ def test_sample_rows_argument_checks(ctx):
         ctx.sample_rows(prob, 0.0)
     with pytest.raises(capi.TsattnError):
         ctx.sample_rows(prob, -1.0)
+
+
+@pytest.mark.parametrize("n_rows,n", [(1, 4096), (3, 4097), (2, 8193), (32, 50257), (513, 4099), (1030, 4101), (1, 1100000), (4097, 3)])
+def test_softmax_and_choices_at_chunk_edges(ctx, n_rows, n):
+    """The library's forms -- records in lent scratch, records in the probabilities' place or choices exchanged between chunks,
+    one workgroup per row over its own input -- against each other and float64, with ties over chunk boundaries."""
+    from tscale_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(n)
+    src = (torch.randn((n_rows, n), device="cuda", generator=g) * 3000).to(torch.int32)
+    top = int(src.max()) + 5
+    for at in (n - 1, n // 2, (n // 2 + 4096) % n):
+        src[::2, at] = top
+    bias = -torch.randn(n, device="cuda", generator=g).abs() * (src.amax(0) < top)   # (ties stay ties, and the largest)
+    w = src.double() * float(np.float32(1e-3)) + bias.double()
+    want = torch.softmax(w * math.log(2.0), 1)
+    # the reference's exponent of 2 takes w = vec * scale + bias in float: three roundings of up to 2^-24 |w|, the subtraction's, and
+    # the exponential's one; then sums of n terms
+    rel = (4 * float(w.abs().max()) * 2.0 ** -24 * math.log(2.0) + 1e-5)
+    p1, a1 = ctx.softmax_rows(src, 1e-3, bias)
+    _, a2 = ctx.softmax_rows(src, 1e-3, bias, want_prob=False)
+    stream = torch.cuda.current_stream().cuda_stream
+    def flat(prob, vec, argmax):
+        capi.check(ctx.lib.tsattn_softmax_rows(ctx._h, n_rows, n, vec.data_ptr(), 1, 0, n, 1e-3, bias.data_ptr(), prob, n, argmax.data_ptr(), stream))
+    p3, a3, a4, a5 = torch.empty_like(p1), torch.empty_like(a1), torch.empty_like(a1), torch.empty_like(a1)
+    flat(p3.data_ptr(), src, a3)
+    flat(None, src, a4)
+    over = src.clone()
+    flat(over.data_ptr(), over, a5)
+    for p in (p1, p3, over.view(torch.float32)):
+        assert ((p.double() - want).abs() <= rel * want + 1e-30).all()
+        assert (p.double().sum(1) - 1).abs().max() < 1e-5
+    first = (src.double() * float(np.float32(1e-3)) + bias.double()).argmax(1)
+    for a in (a1, a2, a3, a4, a5):
+        assert torch.equal(a, a1)
+    assert (w.gather(1, a1.long()[:, None]) - w.gather(1, first[:, None])).abs().max() < 1e-5   # (float logits may tie)
+    assert (a1[::2].long() == min(n - 1, n // 2, (n // 2 + 4096) % n)).all()
+    # the sampled choice, with and without scratch
+    c1 = ctx.sample_rows(p1, 0.9, seed=5, offset=17)
+    c2 = torch.empty_like(c1)
+    capi.check(ctx.lib.tsattn_sample_rows(ctx._h, n_rows, n, p1.data_ptr(), n, 0.9, None, 0, 5, 17, c2.data_ptr(), stream))
+    torch.cuda.synchronize()
+    assert torch.equal(c1, c2)
+
+
+def test_softmax_and_sampling_overlap_on_streams(ctx):
+    """One handle, four streams: nothing of a call stands in the handle, so what the calls return does not depend on others."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    src = [(torch.randn((5 + i, 20011), device="cuda", generator=g) * 3000).to(torch.int32) for i in range(4)]
+    def calls(x, seed):
+        prob, best = ctx.softmax_rows(x, 2e-3)
+        return prob, best, ctx.softmax_rows(x, 2e-3, want_prob=False)[1], ctx.sample_rows(prob, 0.8, seed=seed)
+    want = [calls(x, i) for i, x in enumerate(src)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in src]
+    got = []
+    for r in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got.append((i, calls(src[i], i)))
+    torch.cuda.synchronize()
+    for i, outs in got:
+        assert all(torch.equal(a, b) for a, b in zip(outs, want[i]))

@@ -215,6 +215,12 @@ class AttentionContext:
                                           _raw_stream()))
         return out
 
+    def _head_scratch(self, n):
+        """Scratch of one softmax or sampling call, from the current stream's allocator: calls on several streams may overlap."""
+        if n <= capi.HEAD_CHUNK:
+            return None, 0
+        return torch.empty_strided((capi.HEAD_SCRATCH_BYTES // 4,), (1,), dtype=torch.int32, device=self.device), capi.HEAD_SCRATCH_BYTES
+
     def softmax_rows(self, vec, scale, bias=None, want_prob=True, argmax=None):
         """The final SoftMax of ComputePrediction (cpu_infer.cpp:340-355, base 2) and the greedy choice: vec int32 [n_rows, n]
         or [planes, n_rows, n] (parts of a split-K product) -> (prob f32 [n_rows, n] or None, argmax int32 [n_rows])."""
@@ -224,7 +230,8 @@ class AttentionContext:
         prob = _new(n_rows, n, torch.float32, vec.device) if want_prob else None
         if argmax is None:
             argmax = torch.empty_strided((n_rows,), (1,), dtype=torch.int32, device=vec.device)
-        capi.check(capi.native.softmax_rows(self._h, n_rows, n, vec, planes, n_rows * n, n, float(scale), bias, prob, n, argmax, _raw_stream()))
+        capi.check(capi.native.softmax_rows(self._h, n_rows, n, vec, planes, n_rows * n, n, float(scale), bias, prob, n, argmax,
+                                              *self._head_scratch(n), _raw_stream()))
         return prob, argmax
 
     def sample_rows(self, prob, temperature, rnd=None, seed=0, offset=0, choice=None):
@@ -237,7 +244,7 @@ class AttentionContext:
         if choice is None:
             choice = torch.empty_strided((n_rows,), (1,), dtype=torch.int32, device=prob.device)
         capi.check(capi.native.sample_rows(self._h, n_rows, n, prob, prob.stride(0), float(temperature), rnd, rnd.stride(0) if rnd is not None else 0,
-                                           int(seed), int(offset), choice, _raw_stream()))
+                                           int(seed), int(offset), choice, *self._head_scratch(n), _raw_stream()))
         return choice
 
     def build_spans(self, seq_offset, n_tokens, window, doc_start_flag=None):

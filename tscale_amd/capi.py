@@ -17,6 +17,8 @@ SRC_F32, SRC_BF16, SRC_I32 = 0, 1, 2
 MM_I32, MM_F32, MM_ADD_SCALED, MM_I32_PLANES = 0, 1, 2, 3
 Q_8BIT, Q_BF16 = 0, 1
 SPAN_TILE_INTS = 32
+HEAD_SCRATCH_BYTES = 16384  # TSATTN_HEAD_SCRATCH_BYTES: what softmax and sampling of rows of more than TSATTN_HEAD_CHUNK values can use
+HEAD_CHUNK = 4096           # TSATTN_HEAD_CHUNK
 PREFILL_LONG_SPAN = 6144   # TSATTN_PREFILL_LONG_SPAN: span_len_hint from which tsattn_prefill uses a workspace
 
 STATUS_NAMES = {0: "OK", 1: "BAD_ARG", 2: "UNSUPPORTED", 3: "HIP", 4: "SCRATCH"}
@@ -137,7 +139,7 @@ class LayerArgs(_c.Structure):
 
 
 EXPORTS = ["tsattn_scratch_bytes", "tsattn_create", "tsattn_destroy", "tsattn_last_error", "tsattn_prefill", "tsattn_prefill_workspace_bytes",
-           "tsattn_decode", "tsattn_decode_static", "tsattn_cache_append", "tsattn_cache_fill", "tsattn_merge_lookups", "tsattn_span_tiles_count", "tsattn_build_span_tiles", "tsattn_rope_normalize_rows", "tsattn_fill_rope_table", "tsattn_kv_product", "tsattn_matmul_i8", "tsattn_layer_token_scratch_bytes", "tsattn_layer_token", "tsattn_embed_rows", "tsattn_softmax_rows", "tsattn_sample_rows", "tsattn_quantize_rows", "tsattn_build_spans", "tsattn_debug_read_counters", "tsattn_version"]
+           "tsattn_decode", "tsattn_decode_static", "tsattn_cache_append", "tsattn_cache_fill", "tsattn_merge_lookups", "tsattn_span_tiles_count", "tsattn_build_span_tiles", "tsattn_rope_normalize_rows", "tsattn_fill_rope_table", "tsattn_kv_product", "tsattn_matmul_i8", "tsattn_layer_token_scratch_bytes", "tsattn_layer_token", "tsattn_embed_rows", "tsattn_softmax_rows", "tsattn_softmax_rows_scratch", "tsattn_sample_rows", "tsattn_sample_rows_scratch", "tsattn_quantize_rows", "tsattn_build_spans", "tsattn_debug_read_counters", "tsattn_version"]
 
 _lib = None
 
@@ -198,9 +200,13 @@ def load():
         L.tsattn_softmax_rows.restype = _c.c_int
         L.tsattn_softmax_rows.argtypes = [_c.c_void_p, _c.c_int64, _c.c_int64, _c.c_void_p, _c.c_int, _c.c_int64, _c.c_int64, _c.c_float,
                                           _c.c_void_p, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_void_p]
+        L.tsattn_softmax_rows_scratch.restype = _c.c_int
+        L.tsattn_softmax_rows_scratch.argtypes = L.tsattn_softmax_rows.argtypes[:-1] + [_c.c_void_p, _c.c_int64, _c.c_void_p]
         L.tsattn_sample_rows.restype = _c.c_int
         L.tsattn_sample_rows.argtypes = [_c.c_void_p, _c.c_int64, _c.c_int64, _c.c_void_p, _c.c_int64, _c.c_float, _c.c_void_p, _c.c_int64,
                                          _c.c_uint64, _c.c_uint64, _c.c_void_p, _c.c_void_p]
+        L.tsattn_sample_rows_scratch.restype = _c.c_int
+        L.tsattn_sample_rows_scratch.argtypes = L.tsattn_sample_rows.argtypes[:-1] + [_c.c_void_p, _c.c_int64, _c.c_void_p]
         L.tsattn_quantize_rows.restype = _c.c_int
         L.tsattn_quantize_rows.argtypes = [_c.c_void_p, _c.c_int, _c.c_int, _c.c_void_p, _c.c_int64, _c.c_int64,
                                            _c.c_int, _c.c_int, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int64,
@@ -234,8 +240,8 @@ def _bind_native(L):
                       ("rope_normalize_rows", ProduceArgs), ("matmul_i8", MatmulArgs), ("layer_token", LayerArgs)):
         fields = b"".join(struct.pack("<HB", getattr(cls, f).offset, ord(kinds.get(t, "p"))) for f, t in cls._fields_)
         setattr(calls, name, _native.Call(address("tsattn_" + name), _c.sizeof(cls), fields))
-    _native.bind(*(address("tsattn_" + n) for n in ("quantize_rows", "build_spans", "build_span_tiles", "embed_rows", "softmax_rows", "sample_rows",
-                                                    "kv_product")))
+    _native.bind(*(address("tsattn_" + n) for n in ("quantize_rows", "build_spans", "build_span_tiles", "embed_rows", "softmax_rows_scratch",
+                                                    "sample_rows_scratch", "kv_product")))
     native = _native
 
 

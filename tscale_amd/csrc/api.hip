@@ -16,11 +16,10 @@
 struct tsattn_ctx {
     int device;
     int max_seqs, max_heads, max_head_dim, max_splits;
-    void *mem; // the handle's one allocation, in which:
+    void *mem; // the handle's one allocation (NULL: sizes of nothing), in which:
     float *part_acc;
     float *part_ml;
     int32_t *seq_done;
-    void *head; // records of the softmax and sampling launches
 };
 
 // Scratch of the entry point that allocates nothing (tsattn_decode_static): split partials [pair][split][d] f32, their
@@ -194,23 +193,21 @@ int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
     c->max_heads = cfg->max_heads;
     c->max_head_dim = cfg->max_head_dim;
     c->max_splits = cfg_splits(cfg);
-    // one allocation: row records, arrival counters of the single-split fused append (zero here, and left at zero by every
+    // one allocation: arrival counters of the single-split fused append (zero here, and left at zero by every
     // launch), split maxima and sums, split partials
     const size_t parts = c->max_head_dim > 0 ? (size_t)c->max_seqs * c->max_heads * c->max_splits : 0;
     const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t cnt_at = up(tsattn::HEAD_SCRATCH_BYTES), ml_at = cnt_at + up((size_t)c->max_seqs * sizeof(int32_t)),
-                 acc_at = ml_at + up(parts * 2 * sizeof(float)), total = acc_at + parts * c->max_head_dim * sizeof(float);
+    const size_t ml_at = up((size_t)c->max_seqs * sizeof(int32_t)), acc_at = ml_at + up(parts * 2 * sizeof(float)), total = acc_at + parts * c->max_head_dim * sizeof(float);
     uint8_t *mem = nullptr;
-    e = hipMalloc((void **)&mem, total);
-    if (e == hipSuccess && c->max_seqs > 0) e = hipMemset(mem + cnt_at, 0, (size_t)c->max_seqs * sizeof(int32_t));
+    if (total > 0) e = hipMalloc((void **)&mem, total);
+    if (e == hipSuccess && c->max_seqs > 0) e = hipMemset(mem, 0, (size_t)c->max_seqs * sizeof(int32_t));
     if (e != hipSuccess) {
         if (mem) (void)hipFree(mem);
         delete c;
         return hip_fail(e, "hipMalloc(handle scratch)");
     }
     c->mem = mem;
-    c->head = mem;
-    c->seq_done = (int32_t *)(mem + cnt_at);
+    c->seq_done = (int32_t *)mem;
     c->part_ml = (float *)(mem + ml_at);
     c->part_acc = (float *)(mem + acc_at);
     *out = c;
@@ -220,7 +217,7 @@ int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
 int tsattn_destroy(tsattn_handle_t h)
 {
     if (!h) return TSATTN_OK;
-    (void)hipFree(h->mem);
+    if (h->mem) (void)hipFree(h->mem);
     delete h;
     return TSATTN_OK;
 }
@@ -727,9 +724,16 @@ int tsattn_embed_rows(tsattn_handle_t h, int64_t n_rows, int dim, const int32_t 
     return TSATTN_OK;
 }
 
-int tsattn_softmax_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const int32_t *src, int src_planes, int64_t src_plane_stride,
-                        int64_t src_pitch, float scale, const float *bias, float *prob, int64_t prob_pitch, int32_t *argmax,
-                        void *stream)
+static int check_head_scratch(const char *who, const void *scratch, int64_t bytes)
+{
+    if (scratch && (uintptr_t)scratch % 4) return fail(TSATTN_ERR_BAD_ARG, "%s: scratch must be 4-byte aligned", who);
+    if (scratch && bytes < TSATTN_HEAD_SCRATCH_BYTES) return fail(TSATTN_ERR_SCRATCH, "%s: %lld bytes of scratch, %d needed", who, (long long)bytes, TSATTN_HEAD_SCRATCH_BYTES);
+    return TSATTN_OK;
+}
+
+int tsattn_softmax_rows_scratch(tsattn_handle_t h, int64_t n_rows, int64_t n, const int32_t *src, int src_planes, int64_t src_plane_stride,
+                                int64_t src_pitch, float scale, const float *bias, float *prob, int64_t prob_pitch, int32_t *argmax,
+                                void *scratch, int64_t scratch_bytes, void *stream)
 {
     if (!h) return fail(TSATTN_ERR_BAD_ARG, "tsattn_softmax_rows: null handle");
     if (n_rows < 0 || n < 0 || n > 0x7fffffff) return fail(TSATTN_ERR_BAD_ARG, "tsattn_softmax_rows: sizes");
@@ -738,17 +742,26 @@ int tsattn_softmax_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const int3
     if (src_pitch < n || (prob && prob_pitch < n)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_softmax_rows: pitches must cover a row");
     if (src_planes < 0 || src_planes > 16 || (src_planes > 1 && src_plane_stride < n_rows * src_pitch))
         return fail(TSATTN_ERR_BAD_ARG, "tsattn_softmax_rows: up to 16 source planes, at least n_rows * src_pitch elements apart");
+    if (const int rc = check_head_scratch("tsattn_softmax_rows", scratch, scratch_bytes)) return rc;
     tsattn::HeadParams p = {};
+    p.scratch = scratch;
     p.n_rows = n_rows; p.n = n; p.src = src; p.src_planes = src_planes > 1 ? src_planes : 1; p.src_plane_stride = src_plane_stride;
     p.src_pitch = src_pitch; p.scale = scale; p.bias = bias; p.prob = prob; p.prob_pitch = prob_pitch; p.argmax = argmax;
-    p.scratch = h->head;
     hipError_t e = tsattn::launch_softmax_rows(p, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "softmax launch");
     return TSATTN_OK;
 }
 
-int tsattn_sample_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const float *prob, int64_t prob_pitch, float temperature,
-                       const uint32_t *rnd, int64_t rnd_pitch, uint64_t seed, uint64_t offset, int32_t *choice, void *stream)
+int tsattn_softmax_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const int32_t *src, int src_planes, int64_t src_plane_stride,
+                        int64_t src_pitch, float scale, const float *bias, float *prob, int64_t prob_pitch, int32_t *argmax,
+                        void *stream)
+{
+    return tsattn_softmax_rows_scratch(h, n_rows, n, src, src_planes, src_plane_stride, src_pitch, scale, bias, prob, prob_pitch, argmax, nullptr, 0, stream);
+}
+
+int tsattn_sample_rows_scratch(tsattn_handle_t h, int64_t n_rows, int64_t n, const float *prob, int64_t prob_pitch, float temperature,
+                               const uint32_t *rnd, int64_t rnd_pitch, uint64_t seed, uint64_t offset, int32_t *choice, void *scratch,
+                               int64_t scratch_bytes, void *stream)
 {
     if (!h) return fail(TSATTN_ERR_BAD_ARG, "tsattn_sample_rows: null handle");
     if (n_rows < 0 || n <= 0 || n > 0x7fffffff) return fail(TSATTN_ERR_BAD_ARG, "tsattn_sample_rows: sizes");
@@ -756,13 +769,20 @@ int tsattn_sample_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const float
     if (!prob || !choice) return fail(TSATTN_ERR_BAD_ARG, "tsattn_sample_rows: null data pointer");
     if (prob_pitch < n || (rnd && rnd_pitch < n)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_sample_rows: pitches must cover a row");
     if (!(temperature > 0.0f)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_sample_rows: temperature %g must be positive", (double)temperature);
+    if (const int rc = check_head_scratch("tsattn_sample_rows", scratch, scratch_bytes)) return rc;
     tsattn::HeadParams p = {};
+    p.scratch = scratch;
     p.n_rows = n_rows; p.n = n; p.prob = const_cast<float *>(prob); p.prob_pitch = prob_pitch; p.temperature = temperature;
     p.rnd = rnd; p.rnd_pitch = rnd_pitch; p.seed = seed; p.offset = offset; p.argmax = choice;
-    p.scratch = h->head;
     hipError_t e = tsattn::launch_sample_rows(p, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "sampling launch");
     return TSATTN_OK;
+}
+
+int tsattn_sample_rows(tsattn_handle_t h, int64_t n_rows, int64_t n, const float *prob, int64_t prob_pitch, float temperature,
+                       const uint32_t *rnd, int64_t rnd_pitch, uint64_t seed, uint64_t offset, int32_t *choice, void *stream)
+{
+    return tsattn_sample_rows_scratch(h, n_rows, n, prob, prob_pitch, temperature, rnd, rnd_pitch, seed, offset, choice, nullptr, 0, stream);
 }
 
 void tsattn_fill_rope_table(int head_dim, int64_t max_len, float *table)

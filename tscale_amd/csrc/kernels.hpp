@@ -261,7 +261,6 @@ hipError_t prepare_gemm_mid(); // once per device
 hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out);
 hipError_t prepare_matmul_i8(); // once per device, before the first product
 
-constexpr int HEAD_SCRATCH_BYTES = 64 << 10;
 struct HeadParams {
     int64_t n_rows;
     // embedding
@@ -283,7 +282,8 @@ struct HeadParams {
     float *prob;
     int64_t prob_pitch;
     int32_t *argmax;
-    // scratch of the rows' chunks (HEAD_SCRATCH_BYTES), and what the launchers set: values per chunk, first row of a launch
+    // softmax and sampling: scratch the caller lends (TSATTN_HEAD_SCRATCH_BYTES) or NULL, and what the launchers set: values per
+    // chunk, first row of a launch
     void *scratch;
     int64_t chunk, row0;
     // sampling

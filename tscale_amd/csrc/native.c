@@ -206,8 +206,8 @@ static struct {
     __typeof__(tsattn_build_spans) *build_spans;
     __typeof__(tsattn_build_span_tiles) *build_span_tiles;
     __typeof__(tsattn_embed_rows) *embed_rows;
-    __typeof__(tsattn_softmax_rows) *softmax_rows;
-    __typeof__(tsattn_sample_rows) *sample_rows;
+    __typeof__(tsattn_softmax_rows_scratch) *softmax_rows;
+    __typeof__(tsattn_sample_rows_scratch) *sample_rows;
     __typeof__(tsattn_kv_product) *kv_product;
 } lib;
 
@@ -246,8 +246,8 @@ FLAT(quantize_rows, "piipqqiipqpqp", v[0].p, I(1), I(2), v[3].p, v[4].q, v[5].q,
 FLAT(build_spans, "pipqpqppp", v[0].p, I(1), v[2].p, v[3].q, v[4].p, v[5].q, v[6].p, v[7].p, v[8].p)
 FLAT(build_span_tiles, "pqpppp", v[0].p, v[1].q, v[2].p, v[3].p, v[4].p, v[5].p)
 FLAT(embed_rows, "pqipipqqfpqp", v[0].p, v[1].q, I(2), v[3].p, I(4), v[5].p, v[6].q, v[7].q, F(8), v[9].p, v[10].q, v[11].p)
-FLAT(softmax_rows, "pqqpiqqfppqpp", v[0].p, v[1].q, v[2].q, v[3].p, I(4), v[5].q, v[6].q, F(7), v[8].p, v[9].p, v[10].q, v[11].p, v[12].p)
-FLAT(sample_rows, "pqqpqfpquupp", v[0].p, v[1].q, v[2].q, v[3].p, v[4].q, F(5), v[6].p, v[7].q, (uint64_t)v[8].q, (uint64_t)v[9].q, v[10].p, v[11].p)
+FLAT(softmax_rows, "pqqpiqqfppqppqp", v[0].p, v[1].q, v[2].q, v[3].p, I(4), v[5].q, v[6].q, F(7), v[8].p, v[9].p, v[10].q, v[11].p, v[12].p, v[13].q, v[14].p)
+FLAT(sample_rows, "pqqpqfpquuppqp", v[0].p, v[1].q, v[2].q, v[3].p, v[4].q, F(5), v[6].p, v[7].q, (uint64_t)v[8].q, (uint64_t)v[9].q, v[10].p, v[11].p, v[12].q, v[13].p)
 FLAT(kv_product, "pqiiipqipqfpqp", v[0].p, v[1].q, I(2), I(3), I(4), v[5].p, v[6].q, I(7), v[8].p, v[9].q, F(10), v[11].p, v[12].q, v[13].p)
 
 static PyMethodDef methods[] = {
