@@ -48,3 +48,13 @@ def test_decode_splits(tmp_path):
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout[-2000:]
     assert r.stdout.startswith("OK")
+
+
+def test_stream_walk(tmp_path):
+    """tests/cpp/test_stream_walk.cpp: the requests of the streamed product, those past a wave's share included."""
+    import subprocess
+    exe = tmp_path / "test_stream_walk"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-o", str(exe), os.path.join(ROOT, "tests", "cpp", "test_stream_walk.cpp")], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout[-2000:]
+    assert r.stdout.startswith("OK")

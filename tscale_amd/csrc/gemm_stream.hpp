@@ -12,6 +12,7 @@
 #pragma once
 
 #include "gemm_few.hpp"
+#include "stream_walk.h"
 
 namespace tsattn {
 
@@ -55,18 +56,15 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(FewParams p)
     // row: row-per-lane reads then touch every bank once
     const int row = lane >> 3, chunk = (lane & 7) ^ (row >> 1);
     const int off0 = row * (int)p.w_pitch + chunk * 16, off1 = (row + 8) * (int)p.w_pitch + (chunk ^ 4) * 16;
-    int ask_blk = b0 + t0 / ns, ask_s = t0 % ns, ask_left = t1 - t0, ask_slot = 0;
+    StreamWalk walk = stream_walk(b0, t0, t1, ns);
+    int ask_slot = 0;
     auto ask = [&]() __attribute__((always_inline)) {
-        const int n0 = ask_blk * 16, rows = min(16, (int)p.n - n0);
-        // (past the share's end requests of nothing, so that one count holds for every stage)
-        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.w + (int64_t)n0 * p.w_pitch), 0,
-                                                                            ask_left > 0 ? (int)((rows - 1) * p.w_pitch + p.k) : 0, 0x00020000);
+        const StreamStage st = stream_next(walk, (int)p.n, k, (int)p.w_pitch);
+        const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.w + (int64_t)st.block * 16 * p.w_pitch), 0, st.size, 0x00020000);
         uint8_t *const d = ring + ask_slot * GS_STAGE_BYTES;
-        gs_request(wr, d, off0, ask_s * 128);
-        gs_request(wr, d + 1024, off1, ask_s * 128);
+        gs_request(wr, d, off0, st.scalar_off);
+        gs_request(wr, d + 1024, off1, st.scalar_off);
         ask_slot = ask_slot == GS_STAGES - 1 ? 0 : ask_slot + 1;
-        --ask_left;
-        if (++ask_s == ns) { ask_s = 0; ++ask_blk; }
     };
 
     // ---- the activations; what is asked for first arrives first, and they have the longer way
