@@ -74,3 +74,10 @@ def test_scratch_bytes_is_a_pure_host_function():
     cfg = capi.Config(0, 64, 16, 128, 32)
     n = lib.tsattn_scratch_bytes(ctypes.byref(cfg))
     assert n == 64 * 16 * 32 * (128 + 2) * 4 + 64 * 4   # split partials + per-sequence arrival counters
+
+
+@pytest.mark.parametrize("cfg,want", [((0, 4, 2, 0, 8), 4 * 4),              # no width: no partials are allocated, only counters
+                                      ((0, 3, 5, 64, 0), 3 * 5 * 32 * 66 * 4 + 3 * 4), ((0, 0, 0, 0, 0), 0), ((0, 0, 7, 128, 3), 0)])
+def test_scratch_bytes_is_what_a_handle_allocates(cfg, want):
+    """tsattn_create asks for this number of bytes and lays its parts out without gaps."""
+    assert capi.load().tsattn_scratch_bytes(ctypes.byref(capi.Config(*cfg))) == want

@@ -62,6 +62,22 @@ constexpr int DEFAULT_MAX_SPLITS = 32;
 
 int cfg_splits(const tsattn_config *cfg) { return cfg->max_splits > 0 ? cfg->max_splits : DEFAULT_MAX_SPLITS; }
 
+// The handle's one allocation: split partials [pair][split][d], their (max, sum) pairs, arrival counters.  Nothing between
+// them: a width is 64 or 128, so that every part begins where its type may stand.
+struct HandleScratch {
+    size_t ml_at, cnt_at, total;
+};
+
+HandleScratch handle_scratch(const tsattn_config *cfg)
+{
+    const size_t parts = cfg->max_head_dim > 0 ? (size_t)cfg->max_seqs * cfg->max_heads * cfg_splits(cfg) : 0;
+    HandleScratch s;
+    s.ml_at = parts * cfg->max_head_dim * sizeof(float);
+    s.cnt_at = s.ml_at + parts * 2 * sizeof(float);
+    s.total = s.cnt_at + (size_t)cfg->max_seqs * sizeof(int32_t);
+    return s;
+}
+
 bool head_dim_ok(int d) { return d == 64 || d == 128; }
 bool dtype_ok(int t) { return t == TSATTN_I8 || t == TSATTN_E4M3; }
 bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0; }
@@ -158,8 +174,7 @@ const char *tsattn_version(void) { return "tsattn 0.1 gfx950 (hip; mfma f8f6f4/i
 size_t tsattn_scratch_bytes(const tsattn_config *cfg)
 {
     if (!cfg || cfg->max_seqs < 0 || cfg->max_heads < 0 || cfg->max_head_dim < 0) return 0;
-    size_t parts = (size_t)cfg->max_seqs * cfg->max_heads * cfg_splits(cfg);
-    return parts * ((size_t)cfg->max_head_dim + 2) * sizeof(float) + (size_t)cfg->max_seqs * sizeof(int32_t);
+    return handle_scratch(cfg).total;
 }
 
 int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
@@ -193,23 +208,20 @@ int tsattn_create(const tsattn_config *cfg, tsattn_handle_t *out)
     c->max_heads = cfg->max_heads;
     c->max_head_dim = cfg->max_head_dim;
     c->max_splits = cfg_splits(cfg);
-    // one allocation: arrival counters of the single-split fused append (zero here, and left at zero by every
-    // launch), split maxima and sums, split partials
-    const size_t parts = c->max_head_dim > 0 ? (size_t)c->max_seqs * c->max_heads * c->max_splits : 0;
-    const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t ml_at = up((size_t)c->max_seqs * sizeof(int32_t)), acc_at = ml_at + up(parts * 2 * sizeof(float)), total = acc_at + parts * c->max_head_dim * sizeof(float);
+    const HandleScratch at = handle_scratch(cfg);
     uint8_t *mem = nullptr;
-    if (total > 0) e = hipMalloc((void **)&mem, total);
-    if (e == hipSuccess && c->max_seqs > 0) e = hipMemset(mem, 0, (size_t)c->max_seqs * sizeof(int32_t));
+    if (at.total > 0) e = hipMalloc((void **)&mem, at.total);
+    // (arrival counters of the single-split fused append: zero here, and left at zero by every launch)
+    if (e == hipSuccess && c->max_seqs > 0) e = hipMemset(mem + at.cnt_at, 0, (size_t)c->max_seqs * sizeof(int32_t));
     if (e != hipSuccess) {
         if (mem) (void)hipFree(mem);
         delete c;
         return hip_fail(e, "hipMalloc(handle scratch)");
     }
     c->mem = mem;
-    c->seq_done = (int32_t *)mem;
-    c->part_ml = (float *)(mem + ml_at);
-    c->part_acc = (float *)(mem + acc_at);
+    c->part_acc = (float *)mem;
+    c->part_ml = (float *)(mem + at.ml_at);
+    c->seq_done = (int32_t *)(mem + at.cnt_at);
     *out = c;
     return TSATTN_OK;
 }
