@@ -29,6 +29,22 @@ def test_layer_schedule_of_the_documented_models():
     assert [w for w, _ in sched].count(1) == 4 and [w for w, _ in sched].count(64) == 10 and len(sched) == 24
 
 
+def test_matrix_scales_of_every_form():
+    """A layer's scales: Python numbers, numpy scalars and arrays of one, tensors of one -- whose value at the time of the call counts."""
+    import torch
+    from tscale_amd.attention import VEC_SCALE, _product_scale
+    want = lambda x, n: float(np.float32(x) * np.float32(VEC_SCALE) * np.float32(np.sqrt(np.float32(1.0) / np.float32(n))))
+    for x in (0.3, 2, np.float32(0.3), np.float64(0.3), np.array(0.3), np.array(0.3, np.float32), torch.tensor(0.3), torch.tensor(0.3, dtype=torch.float64)):
+        assert _product_scale(x, 768) == want(float(x), 768) == _product_scale(x, 768)
+    t = torch.tensor(0.5)
+    assert _product_scale(t, 64) == want(0.5, 64)
+    t.fill_(0.25)
+    assert _product_scale(t, 64) == want(0.25, 64)
+    a = np.array(0.5)
+    a[...] = 0.75
+    assert _product_scale(a, 64) == want(0.75, 64)
+
+
 def test_prefill_workgroup_mapping_visits_every_head_and_tile_once(tmp_path):
     """tests/cpp/test_wg_map.cpp walks the launch mapping of tscale_amd/csrc/wg_map.h (the code the kernel runs) over
     ~1500 launch shapes on the CPU, divisors of 1 (one query tile, one sequence, one unit per group) included."""

@@ -406,11 +406,18 @@ STATE_NORM_TILE = 128     # gpt/model_params/model_dim.h:22
 COMBINER_REP = 4          # gpt/model_params/model_dim.h:12
 
 
-@functools.lru_cache(maxsize=4096)
-def _product_scale(scale, width):
-    """A matrix's scale times VEC_SCALE * CalcDotScale(width), in single precision as the reference multiplies it up."""
+def _product_scale_of(scale, width):
     f32 = np.float32
     return float(f32(scale) * f32(VEC_SCALE) * f32(np.sqrt(f32(1.0) / f32(width))))
+
+
+_product_scale_of_float = functools.lru_cache(maxsize=4096)(_product_scale_of)
+
+
+def _product_scale(scale, width):
+    """A matrix's scale times VEC_SCALE * CalcDotScale(width), in single precision as the reference multiplies it up.  The scale is
+    a number or an array or tensor of one; only a float's result is kept (a tensor may change in place)."""
+    return (_product_scale_of_float if type(scale) is float else _product_scale_of)(scale, width)
 
 
 def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratch=None, pending=None, defer=False):
