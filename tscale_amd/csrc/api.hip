@@ -143,7 +143,7 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
             return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: k_new/v_new must be 16-byte aligned with a pitch that covers a row");
         if ((a->k_scale_new && !a->k_scale) || (a->v_scale_new && !a->v_scale)) return fail(TSATTN_ERR_BAD_ARG, "tsattn_decode: new scales given without scale planes");
     }
-    if (lim.clear_counters && (a->k_new || front)) {
+    if (lim.clear_counters && a->k_new) {
         // the arrival counters of the single-split fused append start at zero: a launch leaves them so, but this scratch is
         // shared by every caller on the device (a fill kernel, not a memset: callers may be capturing a graph)
         hipError_t ez = tsattn::launch_zero_i32(lim.seq_done, a->n_seqs, (hipStream_t)stream);
