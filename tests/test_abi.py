@@ -22,6 +22,7 @@ STRUCTS = {
     "tsattn_produce_args": capi.ProduceArgs,
     "tsattn_matmul_args": capi.MatmulArgs,
     "tsattn_merge_args": capi.MergeArgs,
+    "tsattn_layer_args": capi.LayerArgs,
 }
 
 

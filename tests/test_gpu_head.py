@@ -163,3 +163,36 @@ def test_softmax_and_sampling_overlap_on_streams(ctx):
     torch.cuda.synchronize()
     for i, outs in got:
         assert all(torch.equal(a, b) for a, b in zip(outs, want[i]))
+
+def test_masked_and_infinite_logits(ctx):
+    """-inf masks a value out; +inf is the greedy choice (its row has no distribution); both in one row of several chunks and of one."""
+    for n in (1000, 20000):
+        src = torch.zeros((1, n), dtype=torch.int32, device="cuda")
+        src[0, 7], src[0, n - 2] = 3000, 9000
+        bias = torch.zeros(n, device="cuda")
+        bias[n - 2], bias[3:6] = -math.inf, -math.inf
+        prob, best = ctx.softmax_rows(src, 1e-3, bias)
+        w = src.double() * float(np.float32(1e-3)) + bias.double()
+        assert best.item() == 7 and (prob.double() - torch.softmax(w * math.log(2.0), 1)).abs().max() < 1e-6
+        assert (prob[0, 3:6] == 0).all() and prob[0, n - 2] == 0
+        assert ctx.sample_rows(prob, 1e-3, seed=1).item() == 7
+        bias[n // 2] = math.inf
+        for want_prob in (True, False):
+            assert ctx.softmax_rows(src, 1e-3, bias, want_prob=want_prob)[1].item() == n // 2
+
+
+@pytest.mark.parametrize("temperature", [0.05, 0.3])
+def test_sample_rows_at_low_temperatures(ctx, temperature):
+    """Where log(prob) / temperature is large, the single-precision score that picks the candidates has its largest error: all
+    probabilities within a few rounding steps of each other, so that only exact scores tell the winner."""
+    rng = np.random.default_rng(11)
+    n_rows, n = 6, 9001
+    prob = (np.float32(1e-4) * (1 + rng.integers(0, 8, (n_rows, n)) * np.float32(2.0 ** -22))).astype(np.float32)
+    prob[3:] = (np.exp(rng.standard_normal((3, n)) * 0.01) / n).astype(np.float32)
+    got = ctx.sample_rows(dev(prob), temperature, seed=21, offset=3).cpu().numpy()
+    want = orc.sample_rows(prob, temperature, seed=21, offset=3)
+    for i in np.nonzero(got != want)[0]: # (the two logf differ in their last bit: 2^-23 of log(prob) / temperature, both ways)
+        def score(k):
+            u = (float(orc.mix32(21, 3 + i * n + int(k))) + 0.5) / 2.0**32
+            return math.log(float(prob[i, k])) / temperature - math.log(-math.log(u))
+        assert abs(score(got[i]) - score(want[i])) <= 4 * 2.0 ** -23 * abs(math.log(float(prob[i, got[i]])) / temperature), (i, got[i], want[i])

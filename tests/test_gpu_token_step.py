@@ -22,11 +22,14 @@ def int8(g, *shape):
 
 
 @pytest.mark.parametrize("B,H,d,dim,relu,max_len", [
-    (1, 12, 64, 768, 64, 1400),       # splits of the cache; K in three groups per part
+    (1, 12, 64, 768, 64, 1400),       # K in three groups per part
+    (1, 12, 64, 768, 64, 4000),       # splits of the cache
+    (32, 16, 128, 2048, 128, 70),     # normalisations in launches of their own
     (3, 2, 128, 256, 128, 40), (16, 3, 64, 384, 128, 90), (17, 3, 64, 384, 64, 90), (33, 2, 128, 128, 128, 20), (128, 1, 64, 128, 64, 12)])
 def test_token_step_equals_the_chain(ctx, monkeypatch, B, H, d, dim, relu, max_len):
-    """Three layers (window 1, short window with a slope, all keys), two tokens: the cache bytes, scales and lengths of both
-    are equal, states and outputs equal up to int8 roundings of k * value that the order of the attention's sums flips."""
+    """Three layers (window 1, short window with a slope, all keys), two tokens: after every layer the caches (bytes, scales,
+    lengths), the attention's output, the product left for the next layer and the state are the chain's, bit for bit: the
+    launches make the same float operations in the same order."""
     g = torch.Generator(device="cuda").manual_seed(B * 1000 + d)
     qsum = H * d
     layers = [{"proj": int8(g, 4 * qsum, dim), "combiner": int8(g, dim, 4 * qsum), "expand": int8(g, H * relu, dim), "contract": int8(g, dim, H * relu),
@@ -37,33 +40,35 @@ def test_token_step_equals_the_chain(ctx, monkeypatch, B, H, d, dim, relu, max_l
     state0 = torch.randn((B, dim), device="cuda", generator=g)
     rope = ctx.fill_rope_table(d, max_len + 8)
 
+    fused = []
+    layer_token = attention._layer_token
+
     def steps(chain):
         with monkeypatch.context() as m:
-            if chain:
-                m.setattr(attention, "_layer_token", lambda *a: None)
+            m.setattr(attention, "_layer_token", (lambda *a: None) if chain else (lambda *a: fused.append(layer_token(*a)) or fused[-1]))
             caches = []
             for i in range(3):
                 c = KVCache(ctx, capi.I8, B, H, max_len, d)
                 c.k.copy_(k0[i]); c.v.copy_(v0[i]); c.k_scale.fill_(0.01); c.v_scale.fill_(attention.VEC_SCALE); c.cache_len.copy_(lens)
                 caches.append(c)
-            state, keep, outs = state0.clone(), {}, []
+            state, keep, seen = state0.clone(), {}, []
             for step in range(2):
                 pending = None
-                for layer, c in zip(layers, caches):
+                for i, (layer, c) in enumerate(zip(layers, caches)):
                     val, pending = attention.add_lookup_product(ctx, layer, c, lens + step, rope, state, scratch=keep, pending=pending, defer=True)
-                    outs.append(val.clone())
-                outs.append(attention.flush_state(ctx, pending, state))
+                    now = {"k": c.k, "v": c.v, "k_scale": c.k_scale, "v_scale": c.v_scale, "cache_len": c.cache_len, "output": val,
+                           "product": pending[0].sum(dim=0, dtype=torch.int32), "state": state}
+                    seen += [((step, i, name), x.clone()) for name, x in now.items()]
+                    assert pending[1] == attention._product_scale(layer["contract_scale"], H * relu)
+                seen += [((step, "norm"), attention.flush_state(ctx, pending, state).clone()), ((step, "state"), state.clone())]
             torch.cuda.synchronize()
-            return caches, state, outs
+            return seen
 
-    got_c, got_s, got_o = steps(False)
-    want_c, want_s, want_o = steps(True)
-    for c, w in zip(got_c, want_c):
-        assert torch.equal(c.cache_len, w.cache_len) and torch.equal(c.v_scale, w.v_scale)
-        assert (c.k != w.k).float().mean() < 1e-3 and (c.v != w.v).float().mean() < 1e-3
-    rms = want_s.square().mean().sqrt()
-    assert (got_s - want_s).abs().max() / rms < 2e-2
-    assert (got_o[0] - want_o[0]).abs().max() < 2e-5
+    got, want = steps(False), steps(True)
+    assert len(fused) == 6 and all(f is not None for f in fused)
+    for (what, x), (_, y) in zip(got, want):
+        assert torch.equal(x, y), what
+    assert not torch.equal(want[0][1], k0[0])   # (the step has written a row of keys)
 
 
 @pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 64, 65, 128])
