@@ -523,8 +523,8 @@ def model_ends(m, vocab, dim):
 
 def bench_token_step(ctx, steps):
     """One generated token per sequence through all 24 layers (per layer: state normalisation, four projections,
-    RoPE + per-head normalisation, cache append + attention over the cache with KVProduct, combiner, feed-forward; 9-10
-    library calls), B32 at cache length 2048+."""
+    RoPE + per-head normalisation, cache append + attention over the cache with KVProduct, combiner, feed-forward: one
+    library call of eight launches), B32 at cache length 2048+."""
     import torch
     from tscale_amd.attention import add_lookup_product, flush_state
     m = Int8Layers(ctx, cache_len=2048, seed=1313 + 9)
@@ -555,7 +555,7 @@ def bench_token_step(ctx, steps):
     n = m.prompt + 1 + reps // 2
     cache_bytes = sum(B * H * min(n - 1, w) * (2 * d + 8) for w, _ in m.sched)
     return {"config": "24 layers, B32, cache length ~2048+, model width 2048, 16 heads x 128, int8 weights and KV cache; "
-                      "9-10 library calls per layer in one HIP graph per token",
+                      "one library call (eight launches) per layer in one HIP graph per token",
             "ms_per_token_step": round(ms, 4), "tokens_per_s": round(B / ms * 1e3, 1),
             "weight_bytes": m.weight_bytes, "cache_bytes_per_step": cache_bytes,
             "GB/s": round((m.weight_bytes + cache_bytes) / ms / 1e6, 1),

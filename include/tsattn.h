@@ -385,9 +385,9 @@ typedef struct tsattn_matmul_args {
     float scale;
     void *out;
     int64_t out_pitch;
-    /* Optional scratch of the caller's (16-byte aligned): with at most 128 rows the weights are streamed once and K
-     * is split over more workgroups if there is room for the parts' sums (2 x 4 x m x n bytes or more; 16 x 4 x m x n
-     * is never exceeded).  The result is the same with and without it. */
+    /* Optional scratch of the caller's (16-byte aligned): a product of at most 128 rows by at most 496 columns (too few
+     * workgroups otherwise) splits K over more workgroups if there is room for the parts' sums (2 x 4 x m x n bytes or
+     * more; 16 x 4 x m x n is never exceeded).  Other products do not use it.  The result is the same with and without. */
     void *workspace;
     int64_t workspace_bytes;
     int *planes_out;           /* TSATTN_MM_I32_PLANES: host int that receives the number of planes */
@@ -396,9 +396,10 @@ typedef struct tsattn_matmul_args {
                                   src = out (its src, src_dtype, src_pitch, src_planes, src_plane_stride, n_rows and n_heads
                                   are taken from the product: n_heads = n / head_dim, which must divide n).  This is the
                                   reference's projection with its normalising epilogue (TStoreRowTileNormalizeRope,
-                                  gpt/compute/gpt_rope.cuh:4-66, lib/cuda/cuda_matmul.cuh:146-204).  Large products with an
-                                  int8 result do it in the product's own kernel and never write the int32 sums; otherwise
-                                  the library makes the two launches.  Either way `out` is scratch: what it holds after the
+                                  gpt/compute/gpt_rope.cuh:4-66, lib/cuda/cuda_matmul.cuh:146-204).  With an int8 result, heads
+                                  of 64 or 128 and not both a rotation and a residual, products of any size but a token
+                                  step's do it in the product's own kernel and never write the int32 sums; otherwise the
+                                  library makes the two launches.  Either way `out` is scratch: what it holds after the
                                   call is unspecified. */
 } tsattn_matmul_args;
 

@@ -196,7 +196,7 @@ class AttentionContext:
             assert mode != capi.MM_ADD_SCALED
             out = _new(m, n, torch.int32 if mode == capi.MM_I32 else torch.float32, a.device)
         assert out.stride(1) == 1 and out.dtype == (torch.int32 if mode == capi.MM_I32 else torch.float32)
-        # workspace: a uint8 tensor the caller keeps, room for split-K partial sums when m is small
+        # workspace: a uint8 tensor the caller keeps, room for split-K partial sums when the product is small both ways
         room = 0 if workspace is None else workspace.numel() * workspace.element_size()
         capi.check(capi.calls.matmul_i8(self._h, _raw_stream(), m, n, k, a, a.stride(0), w, w.stride(0), mode, float(scale), out, out.stride(0), workspace, room))
         return out
@@ -422,7 +422,8 @@ def _product_scale(scale, width):
 
 def add_lookup_product(ctx, layer, cache, t, rope, state, workspace=None, scratch=None, pending=None, defer=False):
     """One layer of the int8 inference path for one new token per sequence: AddLookupProduct,
-    gpt/train/cpu_infer.cpp:465-527, as a chain of 10-11 library calls (the C++ form is NTsAttn::TLayerComputer).
+    gpt/train/cpu_infer.cpp:465-527: one library call (tsattn_layer_token) where it serves the shape, else a chain of nine or
+    ten (as NTsAttn::TLayerComputer, the C++ form, makes them).
     layer: dict with uint8 (int8 bytes) matrices proj [4*H*d, dim] (the QK, QV, K and V matrices one after the other),
     combiner [dim, 4*H*d], expand [H*d, dim], contract [dim, H*d], floats qv_scale, combiner_scale, contract_scale, and
     width, slope.  cache: KVCache whose value scales are VEC_SCALE; t: int32 [B] positions; rope: table of

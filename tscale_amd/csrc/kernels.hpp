@@ -214,7 +214,7 @@ struct GemmParams {
     float scale;
     void *out;
     int64_t out_pitch;        // elements
-    void *workspace;          // optional room for split-K partial sums (few rows)
+    void *workspace;          // optional room for split-K partial sums (few rows, few columns)
     int64_t workspace_bytes;
     int64_t split_stride;     // set by the launcher: elements between the parts' planes
     // optional last step (ep_head_dim != 0): the producer applied to the int32 result, as launch_rope_normalize would
