@@ -385,9 +385,9 @@ typedef struct tsattn_matmul_args {
     float scale;
     void *out;
     int64_t out_pitch;
-    /* Optional scratch of the caller's (16-byte aligned): a product of at most 128 rows by at most 496 columns (too few
-     * workgroups otherwise) splits K over more workgroups if there is room for the parts' sums (2 x 4 x m x n bytes or
-     * more; 16 x 4 x m x n is never exceeded).  Other products do not use it.  The result is the same with and without. */
+    /* Optional scratch of the caller's (16-byte aligned): with at most 128 rows K is split over more workgroups where that
+     * is the faster way and there is room for the parts' sums (2 x 4 x m x n bytes or more; 16 x 4 x m x n is never
+     * exceeded).  The planes mode needs none.  The result is the same with and without it. */
     void *workspace;
     int64_t workspace_bytes;
     int *planes_out;           /* TSATTN_MM_I32_PLANES: host int that receives the number of planes */

@@ -68,3 +68,20 @@ def test_products_with_the_producer_at_tile_edges(ctx, m, heads, d, k, variant):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
     if variant == "resid":
         assert torch.equal(outs[0][2], outs[1][2])
+
+
+@pytest.mark.parametrize("m,n,k,split", [(32, 2048, 8192, True), (33, 513, 6144, True), (64, 768, 3072, True), (128, 132, 4096, True),
+                                         (8, 256, 1024, False), (32, 2048, 2048, False), (129, 256, 4096, False)])
+@pytest.mark.parametrize("mode", [capi.MM_I32, capi.MM_F32, capi.MM_ADD_SCALED])
+def test_product_through_a_lent_workspace(ctx, m, n, k, split, mode):
+    """Long products of few rows go through the workspace in parts, short ones and many rows do not touch it; the result is the
+    same with and without."""
+    g = torch.Generator(device="cuda").manual_seed(m * n)
+    a = torch.randint(-127, 128, (m, k), device="cuda", generator=g, dtype=torch.int32).to(torch.int8).view(torch.uint8)
+    w = torch.randint(-127, 128, (n, k), device="cuda", generator=g, dtype=torch.int32).to(torch.int8).view(torch.uint8)
+    room = torch.full((16 * m * n,), 0x7fedcba9, dtype=torch.int32, device="cuda")
+    state = torch.randn((m, n), device="cuda", generator=g) if mode == capi.MM_ADD_SCALED else None
+    outs = [ctx.matmul_i8(a, w, mode=mode, scale=1e-3, out=None if state is None else state.clone(), workspace=ws) for ws in (None, room)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    assert bool((room != 0x7fedcba9).any()) == split

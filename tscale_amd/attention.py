@@ -196,7 +196,7 @@ class AttentionContext:
             assert mode != capi.MM_ADD_SCALED
             out = _new(m, n, torch.int32 if mode == capi.MM_I32 else torch.float32, a.device)
         assert out.stride(1) == 1 and out.dtype == (torch.int32 if mode == capi.MM_I32 else torch.float32)
-        # workspace: a uint8 tensor the caller keeps, room for split-K partial sums when the product is small both ways
+        # workspace: a uint8 tensor the caller keeps, room for split-K partial sums when m is small
         room = 0 if workspace is None else workspace.numel() * workspace.element_size()
         capi.check(capi.calls.matmul_i8(self._h, _raw_stream(), m, n, k, a, a.stride(0), w, w.stride(0), mode, float(scale), out, out.stride(0), workspace, room))
         return out

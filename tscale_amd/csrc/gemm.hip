@@ -382,8 +382,23 @@ double rounds_us(int64_t tiles, double fixed, double per_stage, double full, int
 
 FewParams few_params(const GemmParams &p);
 
-Tiles choose_tiles(const GemmParams &p, bool wide_ok, bool normalised)
+// Parts of K through the caller's workspace and a second launch that adds them up, for results that cannot be left as planes: how
+// many (1: no room, or K cannot be cut) and about how many nanoseconds.  Rows and K beyond what a compute unit's LDS holds go in
+// parts (matrices from memory): 8192 -> 2048 under 32, 64 and 128 rows 12.0, 15.7 and 21.1 us, 16.3, 27.5 and 30.3 in one launch by
+// the better kernel; 3072 -> 768 under 64 rows 10.2 and 15.0.  Short products lose to the second launch: 1024 -> 256 under 8 rows
+// 7.2 and 5.4, 2048 -> 2048 under 32 rows 8.6 and 7.2.
+int workspace_parts(const GemmParams &p, double *ns)
 {
+    const int64_t room = p.workspace ? p.workspace_bytes / (p.m * p.n * 4) : 0;
+    int parts = 1;
+    if (room >= 2 && p.m <= FEW_ROWS) *ns = few_split(few_params(p), room >= 16 ? 16 : room >= 8 ? 8 : room >= 4 ? 4 : 2, &parts);
+    return parts;
+}
+
+// (*parts: of K through the workspace, 1 = one launch)
+Tiles choose_tiles(const GemmParams &p, bool wide_ok, bool normalised, int *parts)
+{
+    *parts = 1;
     const int64_t n256 = (p.n + 255) / 256, n128 = (p.n + 127) / 128;
     // no tiles faster than memory brings them the matrix (32 x 50257 x 2048: 26.5 us, 3.9 TB/s)
     const double memory = 4.0 + (double)p.n * p.k * 1e-6 / 4.6;
@@ -394,7 +409,15 @@ Tiles choose_tiles(const GemmParams &p, bool wide_ok, bool normalised)
     };
     consider(Tiles::ROWS64, std::max(memory, rounds_us(n128 * ((p.m + 63) / 64), 5.8, 0.25, 0.1, p.k)));
     if (wide_ok) consider(Tiles::WIDE, rounds_us(n256 * ((p.m + 255) / 256), 10.0, 0.87, 0.6, p.k));
-    if (p.m <= FEW_ROWS) consider(Tiles::FEW, few_ns(few_params(p), p.mode == TSATTN_MM_I32_PLANES ? 16 : 1) * 1e-3 + (normalised ? 5.0 : 0.0));
+    if (p.m <= FEW_ROWS) {
+        consider(Tiles::FEW, few_ns(few_params(p), p.mode == TSATTN_MM_I32_PLANES ? 16 : 1) * 1e-3 + (normalised ? 5.0 : 0.0));
+        if (p.mode != TSATTN_MM_I32_PLANES) {
+            double ns = 0.0;
+            *parts = workspace_parts(p, &ns);
+            if (*parts > 1 && ns * 1e-3 < best) tiles = Tiles::FEW;
+            else *parts = 1;
+        }
+    }
     return tiles;
 }
 
@@ -462,7 +485,8 @@ hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out
             // one operand besides the product: the old state, or cos and sin; wider groups than a head have a launch of their own
             fused = p.ep_dst_dtype == TSATTN_I8 && !(q.ep.resid && q.ep.pos) && (p.ep_head_dim == 64 || p.ep_head_dim == 128);
         }
-        const Tiles tiles = choose_tiles(p, offsets_fit || !fused, p.ep_head_dim != 0);
+        int parts;
+        const Tiles tiles = choose_tiles(p, offsets_fit || !fused, p.ep_head_dim != 0, &parts);
         *planes_out = 1;
         if (tiles != Tiles::FEW && fused) return launch_tiles<TSATTN_MM_I32>(q, tiles, p.ep_head_dim, st);
         hipError_t e;
@@ -479,16 +503,13 @@ hipError_t launch_matmul_i8(const GemmParams &p, hipStream_t st, int *planes_out
         if (e != hipSuccess || !p.ep_head_dim) return e;
         return launch_rope_normalize(q.ep, p.ep_dst_dtype, p.ep_head_dim, true, st);
     }
-    const Tiles tiles = choose_tiles(p, true, false);
+    int parts;
+    const Tiles tiles = choose_tiles(p, true, false, &parts);
     if (tiles == Tiles::FEW) {
         FewParams f = few_params(p);
-        // Parts through the caller's workspace and a second launch that adds them up: where the weights would otherwise
-        // come in through a few compute units only (an eighth of them).
-        const int64_t room = p.workspace ? p.workspace_bytes / (p.m * p.n * 4) : 0;
-        if (room < 2 || (p.n + 15) / 16 >= 32) return launch_gemm_few(f, st);
+        if (parts == 1) return launch_gemm_few(f, st);
         f.mode = TSATTN_MM_I32;
-        f.parts = few_parts(f, room >= 16 ? 16 : room >= 8 ? 8 : room >= 4 ? 4 : 2);
-        if (f.parts == 1) return launch_gemm_few(few_params(p), st);
+        f.parts = parts;
         f.out = p.workspace; f.out_pitch = p.n; f.out_stride = p.m * p.n;
         const hipError_t e = launch_gemm_few(f, st);
         if (e != hipSuccess) return e;

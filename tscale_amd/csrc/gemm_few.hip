@@ -159,6 +159,18 @@ double few_ns(const FewParams &p, int max_parts)
     return stream_fits(p) ? 4000 + (double)p.n * p.k / 6100 + p.m * (15 + (double)p.n * 4 / 4500) : few_best(p, 1, max_parts).ns;
 }
 
+double few_split(const FewParams &p, int max_parts, int *parts)
+{
+    double best = 0.0;
+    *parts = 1;
+    for (int n = 2; n <= max_parts && p.k / n >= 128; n *= 2) {
+        const FewPlan f = few_best(p, n, n);
+        const double ns = f.ns + 2700 + (double)(4 * n + 8) * (double)p.m * (double)p.n / 2200;
+        if (f.parts && (*parts == 1 || ns < best)) { best = ns; *parts = n; }
+    }
+    return best;
+}
+
 hipError_t launch_gemm_few(const FewParams &params, hipStream_t st)
 {
     FewParams p = params;

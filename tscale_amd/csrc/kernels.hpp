@@ -214,7 +214,7 @@ struct GemmParams {
     float scale;
     void *out;
     int64_t out_pitch;        // elements
-    void *workspace;          // optional room for split-K partial sums (few rows, few columns)
+    void *workspace;          // optional room for split-K partial sums (few rows)
     int64_t workspace_bytes;
     int64_t split_stride;     // set by the launcher: elements between the parts' planes
     // optional last step (ep_head_dim != 0): the producer applied to the int32 result, as launch_rope_normalize would
@@ -252,6 +252,8 @@ struct FewParams {
 bool few_source_ok(const FewParams &p);              // whether the kernel can normalise this source itself
 int few_parts(const FewParams &p, int max_parts);    // how many parts K is best cut into, at most max_parts
 double few_ns(const FewParams &p, int max_parts);    // about what the launch then takes, in nanoseconds
+// the same for two parts and more and the launch that adds them up; *parts: how many (1: K cannot be cut)
+double few_split(const FewParams &p, int max_parts, int *parts);
 hipError_t launch_gemm_few(const FewParams &p, hipStream_t st);
 hipError_t prepare_gemm_few(); // once per device
 
