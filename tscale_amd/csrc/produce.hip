@@ -19,7 +19,8 @@ namespace tsattn {
 // every float operation below is meant as written: no fused multiply-adds
 #pragma clang fp contract(off)
 
-template <int D, int DST, bool SRC_I32>
+// ROPE: with positions (a kernel of its own: without, their registers would cost the others 2 to 10 % of a large launch)
+template <int D, int DST, bool SRC_I32, bool ROPE>
 __global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
 {
     constexpr int LPP = D / 8, PAIRS = WAVE / LPP; // lanes per pair, pairs per wave
@@ -37,6 +38,16 @@ __global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
     v4f u0, u1, cs, sn;
     const int64_t e = row * p.src_pitch + (int64_t)head * D + x0;
     float *const resid = p.resid + row * p.resid_pitch + (int64_t)head * D + x0;
+    // The position is asked for first and the table's row as soon as it is there, behind the requests of the values: what is asked for
+    // first arrives first, and one wait covers both (33000 x 12 x 64, one int32 plane: 35.7 us with the position behind the values).
+    int t = ROPE ? p.pos[row] : 0;
+    const auto ask_rope = [&]() __attribute__((always_inline)) {
+        if (!ROPE) return;
+        t = t < 0 ? 0 : (t >= p.rope_len ? (int)p.rope_len - 1 : t);
+        const float *const rr = p.rope + (int64_t)t * D + x0;
+        cs = *(const v4f *)rr;
+        sn = *(const v4f *)(rr + 32);
+    };
     if (SRC_I32) {
         constexpr int PL = 4; // planes asked for together (those that are not there: the last one again)
         const int32_t *const src = (const int32_t *)p.src + e;
@@ -48,6 +59,7 @@ __global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
                 u0 = *(const v4f *)resid;
                 u1 = *(const v4f *)(resid + 32);
             }
+            ask_rope();
         }
         for (int p0 = 0; p0 < p.src_planes && p.src_planes > 1; p0 += PL) {
             v4i qa[PL], qb[PL];
@@ -61,6 +73,7 @@ __global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
                 u0 = *(const v4f *)resid;
                 u1 = *(const v4f *)(resid + 32);
             }
+            if (p0 == 0) ask_rope();
 #pragma unroll
             for (int i = 0; i < PL; ++i)
                 if (p0 + i < p.src_planes) { a += qa[i]; b += qb[i]; }
@@ -74,6 +87,7 @@ __global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
             u0 = *(const v4f *)resid;
             u1 = *(const v4f *)(resid + 32);
         }
+        ask_rope();
     }
     if (p.resid) {
         v0 = u0 + v0 * p.resid_scale;
@@ -83,12 +97,7 @@ __global__ __launch_bounds__(WAVE) void rope_normalize_kernel(ProduceParams p)
             *(v4f *)(resid + 32) = v1;
         }
     }
-    if (p.pos) {
-        int t = p.pos[row];
-        t = t < 0 ? 0 : (t >= p.rope_len ? (int)p.rope_len - 1 : t);
-        const float *const rr = p.rope + (int64_t)t * D + x0;
-        cs = *(const v4f *)rr;
-        sn = *(const v4f *)(rr + 32);
+    if (ROPE) {
         const bool turn = head < p.rope_heads; // (the other heads turn by the identity)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -162,25 +171,25 @@ hipError_t launch_rope_normalize(const ProduceParams &p, int dst_dtype, int head
     if (p.n_rows > 0xffffffffll / p.n_heads) return hipErrorInvalidValue; // (pairs are counted in 32 bits: 1 TB of values)
     const int per_wave = WAVE / (head_dim / 8); // (one group of 384 or 512 values)
     dim3 grid((unsigned)((n_pairs + per_wave - 1) / per_wave)), block(WAVE);
-#define TSATTN_PR(D_, DST_, I32_) hipLaunchKernelGGL((rope_normalize_kernel<D_, DST_, I32_>), grid, block, 0, st, p)
-    if (head_dim == 128 && dst_dtype == TSATTN_I8 && !src_i32) TSATTN_PR(128, TSATTN_I8, false);
-    else if (head_dim == 128 && dst_dtype == TSATTN_I8 && src_i32) TSATTN_PR(128, TSATTN_I8, true);
-    else if (head_dim == 128 && dst_dtype == TSATTN_E4M3 && !src_i32) TSATTN_PR(128, TSATTN_E4M3, false);
-    else if (head_dim == 128 && dst_dtype == TSATTN_E4M3 && src_i32) TSATTN_PR(128, TSATTN_E4M3, true);
-    else if (head_dim == 64 && dst_dtype == TSATTN_I8 && !src_i32) TSATTN_PR(64, TSATTN_I8, false);
-    else if (head_dim == 64 && dst_dtype == TSATTN_I8 && src_i32) TSATTN_PR(64, TSATTN_I8, true);
-    else if (head_dim == 64 && dst_dtype == TSATTN_E4M3 && !src_i32) TSATTN_PR(64, TSATTN_E4M3, false);
-    else if (head_dim == 64 && dst_dtype == TSATTN_E4M3 && src_i32) TSATTN_PR(64, TSATTN_E4M3, true);
-#define TSATTN_PR_WIDE(D_)                                                                               \
-    else if (head_dim == D_ && dst_dtype == TSATTN_I8 && !src_i32) TSATTN_PR(D_, TSATTN_I8, false);      \
-    else if (head_dim == D_ && dst_dtype == TSATTN_I8 && src_i32) TSATTN_PR(D_, TSATTN_I8, true);
+#define TSATTN_PR(D_, DST_, I32_, ROPE_)                                                             \
+    if (head_dim == D_ && dst_dtype == DST_ && src_i32 == I32_ && (p.pos != nullptr) == ROPE_) {          \
+        hipLaunchKernelGGL((rope_normalize_kernel<D_, DST_, I32_, ROPE_>), grid, block, 0, st, p);        \
+        return hipGetLastError();                                                                         \
+    }
+#define TSATTN_PR_HEAD(D_, DST_) \
+    TSATTN_PR(D_, DST_, false, false) TSATTN_PR(D_, DST_, false, true) TSATTN_PR(D_, DST_, true, false) TSATTN_PR(D_, DST_, true, true)
+#define TSATTN_PR_WIDE(D_) TSATTN_PR(D_, TSATTN_I8, false, false) TSATTN_PR(D_, TSATTN_I8, true, false)
+    TSATTN_PR_HEAD(64, TSATTN_I8)
+    TSATTN_PR_HEAD(64, TSATTN_E4M3)
+    TSATTN_PR_HEAD(128, TSATTN_I8)
+    TSATTN_PR_HEAD(128, TSATTN_E4M3)
     TSATTN_PR_WIDE(256)
     TSATTN_PR_WIDE(384)
     TSATTN_PR_WIDE(512)
 #undef TSATTN_PR_WIDE
-    else return hipErrorInvalidValue;
+#undef TSATTN_PR_HEAD
 #undef TSATTN_PR
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 // KVProduct, gpt/train/cpu_infer.cpp:320-337 (GPU form compute/gpt_combiner.cuh:13-37): the step after attention,
