@@ -265,18 +265,19 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     const float *vsb = p.vs ? p.vs + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
     v4i kreg[DEC_U], vreg[DEC_U];
     float ksr[DEC_U], vsr[DEC_U];
-    int row[DEC_U];
+    int row[DEC_U]; // (with the front, which has no registers for them, computed again where they are needed)
+    auto row_of = [&](int base, int u) __attribute__((always_inline)) { return FRONT ? base + u * KPL + g : row[u]; };
     auto request = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < DEC_U; ++u) {
-            row[u] = base + u * KPL + g;
-            const int rc = (row[u] < s1) ? row[u] : s1 - 1; // clamp the address, mask the logit below
+            if (!FRONT) row[u] = base + u * KPL + g;
+            const int r = row_of(base, u), rc = (r < s1) ? r : s1 - 1; // clamp the address, mask the logit below
             kreg[u] = __builtin_nontemporal_load((const v4i *)(kbase + (int64_t)rc * p.tok_stride));
             ksr[u] = ksb ? ksb[rc] : p.ks_const;
         }
 #pragma unroll
         for (int u = 0; u < DEC_U; ++u) {
-            const int rc = (row[u] < s1) ? row[u] : s1 - 1;
+            const int r = row_of(base, u), rc = (r < s1) ? r : s1 - 1;
             vreg[u] = __builtin_nontemporal_load((const v4i *)(vbase + (int64_t)rc * p.tok_stride));
             vsr[u] = vsb ? vsb[rc] : p.vs_const;
         }
@@ -416,12 +417,12 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             float bits = group_sum_bits<DTYPE, LPK>(qf.dot_partial_as_bits(kreg[u]));
             float accf = (DTYPE == TSATTN_I8) ? (float)__float_as_int(bits) : bits;
             if (DUMP) {
-                if (c == 0 && row[u] < s1) {
-                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + row[u]] = bits;
+                if (c == 0 && row_of(base, u) < s1) {
+                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + row_of(base, u)] = bits;
                 }
             }
-            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - row[u]);
-            s[u] = (row[u] < s1) ? dp : -INFINITY;
+            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - row_of(base, u));
+            s[u] = (row_of(base, u) < s1) ? dp : -INFINITY;
             m_new = fmaxf(m_new, s[u]);
         }
         float alpha = fast_exp2(m - m_new);

@@ -11,14 +11,17 @@ namespace tsattn {
 constexpr int decode_step_rows(int head_dim) { return 4 * 8 * (64 / (head_dim / 16)); }
 
 // The number of splits (at most max_splits, and at most 1024 workgroups) with the least time, in nanoseconds, by a fit of
-// launches of 12 to 240 pairs, 512 to 4096 rows and 1 to 16 splits:
-//   a workgroup walks its rows in whole steps at 33 bytes per nanosecond, workgroups that share a compute unit one after the other;
+// launches of 8 to 768 pairs, 512 to 4096 rows and 1 to 16 splits:
+//   a compute unit walks a workgroup's rows at 33 bytes per nanosecond in steps, of which the last is at least a third of a whole one;
+//   of several workgroups it walks all the rows;
 //   no launch is faster than memory delivers the rows, 6800 bytes per nanosecond;
-//   more than one split costs the merge launch, 2.8 us and 0.22 us per split.
-// What it chooses is within 0.5 % of the best number on average and 6 % at worst.  Without the steps (a workgroup's rows at 37 bytes
-// per nanosecond or its share of the memory's rate, the merge 3.5 us and 0.04 us per split) it was 2.2 % and 21 %: one sequence
-// of 12 heads of width 64 and 4096 rows in 15 splits 12.8 us, in 8 (one step each) 10.3; 4 of 16 heads of width 128 and 4096 rows in
-// 3 splits 20.5 us, in 4 18.4; 8 of them with 1500 rows in one 16.5 us, in 2 15.2.
+//   more than one split costs the merge launch, 2.0 us, 0.28 us per split and 3 ns per workgroup, and 0.2 us more where the number is no
+//   power of two (8 pairs of width 128 and 3100 rows: 12.6, 12.9, 11.8 us with 5, 6 and 8 splits).
+// What it chooses is within 0.7 % of the best number on average and 11 % at worst.  Without the steps (a workgroup's rows at 37 bytes
+// per nanosecond or its share of the memory's rate, the merge 3.5 us and 0.04 us per split) it was 2.2 % and 21 % up to 240 pairs: one
+// sequence of 12 heads of width 64 and 4096 rows in 15 splits 12.8 us, in 8 (one step each) 10.3; 4 of 16 heads of width 128 and
+// 4096 rows in 3 splits 20.5 us, in 4 18.4; 8 of them with 1500 rows in one 16.5 us, in 2 15.2; 17 with 4096 rows in one 63 us, in
+// 3 55 (a few compute units have two workgroups); 24 of 12 heads of width 64 and 1064 rows in one 13.8 us, in 3 15.1.
 inline int decode_choose_splits(int64_t rows, int head_dim, int64_t pairs, int max_splits)
 {
     const int step = decode_step_rows(head_dim), row_bytes = 2 * head_dim + 8;
@@ -26,11 +29,14 @@ inline int decode_choose_splits(int64_t rows, int head_dim, int64_t pairs, int m
     int best = 1;
     double best_ns = 0.0;
     for (int s = 1; s <= max_splits && (s == 1 || s * pairs <= 1024); ++s) {
-        const int64_t steps = ((rows + s - 1) / s + step - 1) / step;
-        const double walk = (double)(steps * step) * row_bytes / 33.0 * (double)((pairs * s + 255) / 256);
-        const double ns = (walk > memory ? walk : memory) + (s > 1 ? 2800.0 + 220.0 * s : 0.0);
+        const bool power = (s & (s - 1)) == 0;
+        const int64_t per = (rows + s - 1) / s, last = per % step, shared = (pairs * s + 255) / 256;
+        double walked = (double)(per - last) + (last ? (last > 0.3 * step ? (double)last : 0.3 * step) : 0.0);
+        if (walked < (double)(per * shared)) walked = (double)(per * shared);
+        const double walk = walked * row_bytes / 33.0;
+        const double ns = (walk > memory ? walk : memory) + (s > 1 ? 2000.0 + 280.0 * s + 3.0 * (double)(pairs * s) + (power ? 0.0 : 200.0) : 0.0);
         if (s == 1 || ns < best_ns) { best_ns = ns; best = s; }
-        if (steps <= 1) break; // (more splits shorten no workgroup's walk)
+        if (per <= step && power) break; // (more splits shorten no workgroup's walk)
     }
     return best;
 }

@@ -55,7 +55,7 @@ TSATTN_HD inline uint32_t wg_even(uint32_t i, uint32_t n)
 {
     // compute unit c; n % 32 of them hold one more than the others
     const uint32_t c = i & 31, first = (c - n) & (n < 32 ? 0u : 31u), few = n < 32 ? i : first;
-    const uint32_t later = (i < 64) & (n >= 64) ? 63 - first : n - 1 - c;
+    const uint32_t later = ((i < 64) & (n >= 64)) ? 63 - first : n - 1 - c;
     return i < 32 ? few : later;
 }
 
