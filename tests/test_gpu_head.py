@@ -196,3 +196,26 @@ def test_sample_rows_at_low_temperatures(ctx, temperature):
             u = (float(orc.mix32(21, 3 + i * n + int(k))) + 0.5) / 2.0**32
             return math.log(float(prob[i, k])) / temperature - math.log(-math.log(u))
         assert abs(score(got[i]) - score(want[i])) <= 4 * 2.0 ** -23 * abs(math.log(float(prob[i, got[i]])) / temperature), (i, got[i], want[i])
+
+
+def test_softmax_and_sampling_replay(ctx):
+    """Recorded once, replayed on other inputs with eager work between the replays: the eager results every time."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    src = torch.zeros((7, 20011), dtype=torch.int32, device="cuda")
+    calls = lambda: (lambda p: (*p, ctx.softmax_rows(src, 2e-3, want_prob=False)[1], ctx.sample_rows(p[0], 0.8, seed=4)))(ctx.softmax_rows(src, 2e-3))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        calls()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = calls()
+    for _ in range(4):
+        src.copy_((torch.randn(src.shape, device="cuda", generator=g) * 3000).to(torch.int32))
+        want = calls()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(recorded, want))
