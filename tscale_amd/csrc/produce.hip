@@ -7,7 +7,7 @@
 // One wave takes 64 / (D / 8) pairs: a lane holds eight values (four couples x, x + 32), squares go through the wave's LDS to
 // the lane that adds its pair's up in index order -- additions only, one instruction per value -- and the multiplier comes back
 // through a lane exchange: no barrier, no second pass over the values.  Bound by memory for large launches (65536 x 16 x 128 f32 ->
-// int8: 117 us, 5.8 TB/s; 121 us with workgroups of 32 pairs, 256 threads and three barriers), by its chain of waits for small
+// int8, no rotation: 124 us, 5.7 TB/s, as with workgroups of 32 pairs, 256 threads and three barriers), by its chain of waits for small
 // ones (531 x 16 x 128: 4.8 against 6.3 us; 32 x 16, two planes and the residual update: 4.5 against 5.6 us).
 #include <math.h>
 
