@@ -37,7 +37,7 @@ __device__ inline void store_out(const GemmParams &p, int64_t m, int64_t n, int 
     }
 }
 
-// Wide tiles for the largest products: 256 x 256 outputs by eight waves of 128 x 64, K in steps of 64 bytes, one
+// Wide tiles for the largest products: 256 x 256 outputs by eight waves, K in steps of 64 bytes, one
 // workgroup per compute unit; per MFMA cycle this moves a third less through LDS and the caches than 256 x 128 tiles.
 // Each SIMD holds two of the waves, one from each half of the workgroup, and the halves run half a step apart: while
 // one half issues the 16 MFMAs of its step, the other does its memory work (requests its share of the tile three
@@ -50,9 +50,19 @@ __device__ inline void store_out(const GemmParams &p, int64_t m, int64_t n, int 
 constexpr int GW_THREADS = 512, GW_BM = 256, GW_BN = 256, GW_BK = 64, GW_NBUF = 4;
 constexpr int GW_BUF = (GW_BM + GW_BN) * GW_BK;
 constexpr int GW_LDS_BYTES = GW_NBUF * GW_BUF;
-// with the producer as epilogue: the floats of 128 rows (row pitch head width + 4), a multiplier per (row, head), 256 positions
-constexpr int ep_lds_bytes(int head_dim) { return head_dim == 0 ? 0 : (128 * (GW_BN / head_dim) * (head_dim + 4) + 128 * (GW_BN / head_dim) + GW_BM) * 4; }
-constexpr int gw_lds_bytes(int head_dim) { return ep_lds_bytes(head_dim) > GW_LDS_BYTES ? ep_lds_bytes(head_dim) : GW_LDS_BYTES; }
+typedef int v4i_w __attribute__((ext_vector_type(4), aligned(4)));
+typedef float v4f_w __attribute__((ext_vector_type(4), aligned(4)));
+
+// four values of lanes 16..31 and 48..63 of lo change places with those of lanes 0..15 and 32..47 of hi
+__device__ __forceinline__ void swap16(float *lo, float *hi)
+{
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const auto y = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo[c]), __float_as_uint(hi[c]), false, false);
+        lo[c] = __uint_as_float(y[0]);
+        hi[c] = __uint_as_float(y[1]);
+    }
+}
 
 template <int MODE, int EP_D>
 __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
@@ -63,7 +73,13 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
     const int lane = tid & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int half = wave >> 2; // waves 0-3 and 4-7 land on SIMDs 0-3 each
-    const int wm = wave >> 2, wn = wave & 3;
+    // A wave's share is four blocks of 32 of the matrix instructions' first operand by two of the second.  For a plain result the
+    // activations come first: 128 rows x 64 columns, columns over lanes, so that it leaves in whole lines.  With the producer
+    // as epilogue the weights come first: 64 rows x 128 columns; lane li of acc[j][i] has row 32 i + li of the wave's rows and, four
+    // after four, the columns 32 j + 8 (r / 4) + 4 g + r % 4 -- a row's values lie in two lanes instead of over all of them.
+    // (The result of 65536 x 2048 -> 8192 as int32: 1240 us, 1328 with a row per lane.)
+    constexpr bool ROWS = EP_D != 0;
+    const int wm = ROWS ? wave & 3 : wave >> 2, wn = ROWS ? wave >> 2 : wave & 3;
     const int li = lane & 31, g = lane >> 5;
 
     // Which output tile.  The 8 XCDs take workgroups round-robin and each has its own L2; the workgroups an XCD runs at a
@@ -100,9 +116,9 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
     };
     // operands: row li of each 32-row block, chunk 2 * h + g of its 64 bytes (h: which 32 bytes of the step)
     const int f_perm = (li >> 2) & 3;
-    const int f_a = (wm * 128 + li) * GW_BK + ((g ^ f_perm) << 4);
-    const int f_w = (GW_BM + wn * 64 + li) * GW_BK + ((g ^ f_perm) << 4);
-    v4i fa[2][4], fw[2][2];
+    const int row_a = wm * (ROWS ? 64 : 128) + li, row_w = GW_BM + wn * (ROWS ? 128 : 64) + li;
+    const int at4 = (ROWS ? row_w : row_a) * GW_BK + ((g ^ f_perm) << 4), at2 = (ROWS ? row_a : row_w) * GW_BK + ((g ^ f_perm) << 4);
+    v4i f4[2][4], f2[2][2];
     v16i acc[4][2];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -118,11 +134,15 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
         asm volatile("" ::: "memory");                          \
     } while (0)
     const int n_steps = (int)(p.k / GW_BK);
-    // (with the producer as epilogue: the position of tile row tid, asked for now, so that the epilogue's rope rows do not
-    // wait for it)
-    int row_pos = 0;
+    // (with the producer as epilogue: the positions of this lane's rows, asked for now, so that the epilogue's rope rows do not
+    // wait for them)
+    int row_pos[2] = {0, 0};
     if constexpr (EP_D != 0) {
-        if (p.ep.pos && tid < GW_BM && m0 + tid < p.m) row_pos = p.ep.pos[m0 + tid];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int64_t m = m0 + wm * 64 + i * 32 + li;
+            if (p.ep.pos && m < p.m) row_pos[i] = p.ep.pos[m];
+        }
     }
     // requests past K fetch bytes that are never computed with (or zeros past the rows' end)
     request(0, gw_lds);
@@ -142,9 +162,9 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) fa[h][i] = *(const v4i *)(cur + ((f_a + i * 32 * GW_BK) ^ (h * 32)));
+            for (int j = 0; j < 4; ++j) f4[h][j] = *(const v4i *)(cur + ((at4 + j * 32 * GW_BK) ^ (h * 32)));
 #pragma unroll
-            for (int j = 0; j < 2; ++j) fw[h][j] = *(const v4i *)(cur + ((f_w + j * 32 * GW_BK) ^ (h * 32)));
+            for (int i = 0; i < 2; ++i) f2[h][i] = *(const v4i *)(cur + ((at2 + i * 32 * GW_BK) ^ (h * 32)));
         }
         GW_FENCE;
         asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
@@ -155,9 +175,9 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[h][i], fw[h][j], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < 2; ++i) acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f4[h][j], f2[h][i], acc[j][i], 0, 0, 0);
         __builtin_amdgcn_s_setprio(0);
         GW_FENCE;
         GW_BARRIER;
@@ -168,150 +188,145 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
 #undef GW_BARRIER
     if constexpr (EP_D != 0) {
         // The producer as the product's epilogue (the reference's projection kernels end the same way,
-        // TStoreRowTileNormalizeRope, gpt/compute/gpt_rope.cuh:4-66): the int32 sums never go to memory.  The tile's
-        // 256 columns are whole heads of EP_D; 128 of its rows at a time (blocks 2 s and 2 s + 1 of both row halves) go
-        // through LDS as floats -- after the residual update or the rotation, which are lane-local: a wave's 64 columns
-        // are one rotation block, x in acc[.][0] and x + 32 in acc[.][1] -- so that one thread per (row, head) can add up
-        // the squares in index order, as the producer kernel and the CPU path do (that chain of additions is the longest
-        // wait of the epilogue: the more pairs a step has, the more threads walk their chains side by side).  Every
-        // float operation as written there.  A residual update and a rotation in one call are left to the producer
-        // kernel by the launcher.
+        // TStoreRowTileNormalizeRope, gpt/compute/gpt_rope.cuh:4-66): the int32 sums never go to memory.  A wave's 128
+        // columns are whole heads.  Residual update and rotation are lane-local (x in acc[2 b][.] and x + 32 in
+        // acc[2 b + 1][.]); then one exchange between the wave's halves per two values gives every lane one row's 128
+        // values, whose squares it adds up in index order, as the producer kernel and the CPU path do, and converts them:
+        // no barrier, and only the bytes go through LDS (to leave as whole lines).  Every float operation as written there.
+        // A residual update and a rotation in one call are left to the producer kernel by the launcher.
+        // (With the waves' sums in the other layout, columns over lanes, the floats went through LDS 128 rows at a time for
+        // the ordered sums, three barriers each: 17.7 of a projection tile's 67 thousand cycles.  65536 rows, bytes alone /
+        // with a residual update: 2048 -> 8192 1179 / 1940 us, now 1120 / 1873; 2048 -> 2048 274 / 500, now 256 / 471.)
 #pragma clang fp contract(off)
-        constexpr int HEADS_T = GW_BN / EP_D;  // heads per tile
-        constexpr int PAIRS = 128 * HEADS_T;   // (row, head) pairs per step
-        constexpr int PITCH = EP_D + 4;        // rows 16 bytes aligned, 16 lanes' 16-byte reads on 64 different banks
-        static_assert(ep_lds_bytes(EP_D) == (PAIRS * PITCH + PAIRS + GW_BM) * 4 && PAIRS <= GW_THREADS, "the epilogue's LDS and threads");
-        float *const vals = (float *)gw_lds;
-        float *const mults = vals + PAIRS * PITCH;
-        int *const tile_pos = (int *)(mults + PAIRS); // positions of the tile's 256 rows
         const ProduceParams &e = p.ep;
-        const int head_t = (wn * 64) / EP_D, xbase = (wn * 64) % EP_D;
-        const int head = (int)(n0 / EP_D) + head_t;
-        const bool head_ok = head < e.n_heads;
-        const bool turn = head < e.rope_heads;
-        __syncthreads(); // every wave is done with the operand buffers
-        if (tid < GW_BM) tile_pos[tid] = row_pos < 0 ? 0 : (row_pos >= e.rope_len ? (int)e.rope_len - 1 : row_pos);
-        __syncthreads();
+        const int rows_here = (int)(p.m - m0 < GW_BM ? p.m - m0 : GW_BM);
+        constexpr int HEADS_W = 128 / EP_D; // heads per wave
+        const int head0 = (int)(n0 / EP_D) + wn * HEADS_W;
         // Addresses inside the tile are 32-bit offsets from a base that is the same for the whole wave (the launcher
         // checks that the pitches allow it): one add per access instead of a 64-bit multiply.
-        const int rows_here = (int)(p.m - m0 < GW_BM ? p.m - m0 : GW_BM);
-        const bool rotate = e.pos && turn;
-        const char *const rope_base = (const char *)(e.rope + xbase);
-        char *const resid_base = (char *)(e.resid + m0 * e.resid_pitch + (int64_t)head * EP_D + xbase);
+        char *const resid_base = (char *)(e.resid + m0 * e.resid_pitch + (n0 + wn * 128));
         const uint32_t resid_pitch_bytes = (uint32_t)e.resid_pitch * 4u;
-        // Everything a block of rows needs from memory is requested before any of it is used or stored (row by row, each
-        // row's stores would have to be waited for before the next row's loads, which they might overlap), and the next
-        // step's requests go out before this step's sums and conversion, which they pass under.  Per block two values
-        // per row and lane: the old state's, or cos and sin.
-        float xa[2][16], xb[2][16];
-        auto request = [&](int i, int set) __attribute__((always_inline)) {
+        float val[4][2][16];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) val[j][i][r] = (float)acc[j][i][r];
+        // Step s = (i, b): rows of block i, columns 64 b + ..63; what it needs from memory is requested two steps ahead.  State
+        // is read and written sixteen rows by 64 bytes at a time: the values of two groups of columns change places between
+        // the 16 lanes of the block's upper and lower rows (and back).
+        v4f x[2][8];
+        const int r16 = lane & 15, c16 = 8 * ((lane >> 4) & 1) + 4 * g;
+        auto resid_at = [&](int s, int k) __attribute__((always_inline)) { // k = (column half, 16 of its columns, 16 rows)
+            const int row = wm * 64 + (s >> 1) * 32 + (k & 1) * 16 + r16, col = (s & 1) * 64 + (k >> 1) * 16 + c16;
+            return resid_base + ((uint32_t)row * resid_pitch_bytes + (uint32_t)col * 4u);
+        };
+        auto resid_ok = [&](int s, int k) __attribute__((always_inline)) {
+            return wm * 64 + (s >> 1) * 32 + (k & 1) * 16 + r16 < rows_here && head0 + (s & 1) * 64 / EP_D < e.n_heads;
+        };
+        auto request = [&](int s) __attribute__((always_inline)) {
             if (e.resid) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = wm * 128 + i * 32 + 8 * (r / 4) + 4 * g + (r & 3);
-                    const bool ok = row < rows_here && head_ok;
-                    const float *const q0 = (const float *)(resid_base + ((uint32_t)row * resid_pitch_bytes + (uint32_t)li * 4u));
-                    xa[set][r] = ok ? q0[0] : 0.0f;
-                    xb[set][r] = ok ? q0[32] : 0.0f;
-                }
-            } else if (rotate) {
+                for (int k = 0; k < 8; ++k) x[s & 1][k] = resid_ok(s, k) ? *(const v4f_w *)resid_at(s, k) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            } else if (e.pos) {
+                const int i = s >> 1, t = row_pos[i] < 0 ? 0 : (row_pos[i] >= e.rope_len ? (int)e.rope_len - 1 : row_pos[i]);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t t = (uint32_t)tile_pos[wm * 128 + i * 32 + 8 * (r / 4) + 4 * g + (r & 3)];
-                    const float *const rope_row = (const float *)(rope_base + (t * (uint32_t)(EP_D * 4) + (uint32_t)li * 4u));
-                    xa[set][r] = rope_row[0];
-                    xb[set][r] = rope_row[32];
-                }
+                for (int k = 0; k < 8; ++k)
+                    x[s & 1][k] = *(const v4f_w *)((const char *)e.rope + ((uint32_t)t * (uint32_t)(EP_D * 4) + (uint32_t)((s & 1) * 64 % EP_D + 8 * k + 4 * g) * 4u));
             }
         };
-        request(0, 0);
-        request(1, 1);
-#pragma unroll // (the accumulators are registers: no run-time index into them)
-        for (int s = 0; s < 2; ++s) {
+        request(0);
+        request(1);
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int i = 2 * s + b;
+        for (int s = 0; s < 4; ++s) {
+            const int i = s >> 1, b = s & 1;
+            float *const v0 = val[2 * b][i], *const v1 = val[2 * b + 1][i];
+            if (e.resid) { // state += delta * scale, written back; the updated state is what gets normalised
+#pragma unroll
+                for (int k = 0; k < 8; k += 2) {
+                    float *const lo = (k < 4 ? v0 : v1) + (k & 2) * 4, *const hi = lo + 4;
+                    swap16(lo, hi);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        lo[c] = x[b][k][c] + lo[c] * e.resid_scale;
+                        hi[c] = x[b][k + 1][c] + hi[c] * e.resid_scale;
+                    }
+                    if (resid_ok(s, k)) *(v4f_w *)resid_at(s, k) = v4f{lo[0], lo[1], lo[2], lo[3]};
+                    if (resid_ok(s, k + 1)) *(v4f_w *)resid_at(s, k + 1) = v4f{hi[0], hi[1], hi[2], hi[3]};
+                    swap16(lo, hi);
+                }
+            } else if (e.pos && head0 + b * 64 / EP_D < e.rope_heads) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int rr = 8 * (r / 4) + 4 * g + (r & 3);
-                    const int row = wm * 128 + i * 32 + rr;
-                    float v0 = (float)acc[i][0][r], v1 = (float)acc[i][1][r];
-                    if (e.resid) { // state += delta * scale, written back; the updated state is what gets normalised
-                        v0 = xa[b][r] + v0 * e.resid_scale;
-                        v1 = xb[b][r] + v1 * e.resid_scale;
-                        if (row < rows_here && head_ok) {
-                            float *const q0 = (float *)(resid_base + ((uint32_t)row * resid_pitch_bytes + (uint32_t)li * 4u));
-                            q0[0] = v0;
-                            q0[32] = v1;
-                        }
-                    } else if (rotate) {
-                        const float cos_value = xa[b][r];
-                        const float sin_value = xb[b][r] * e.rotate_dir;
-                        const float r0 = v0 * cos_value - v1 * sin_value;
-                        const float r1 = v0 * sin_value + v1 * cos_value;
-                        v0 = r0;
-                        v1 = r1;
-                    } // (a head that is not rotated: cos 1 and sin 0 leave the values as they are)
-                    float *const dst = vals + ((b * 64 + wm * 32 + rr) * HEADS_T + head_t) * PITCH + xbase + li;
-                    dst[0] = v0;
-                    dst[32] = v1;
+                    const float cos_value = x[b][r / 4][r & 3], sin_value = x[b][4 + r / 4][r & 3] * e.rotate_dir;
+                    const float r0 = v0[r] * cos_value - v1[r] * sin_value;
+                    const float r1 = v0[r] * sin_value + v1[r] * cos_value;
+                    v0[r] = r0;
+                    v1[r] = r1;
                 }
-                if (s == 0) request(2 + b, b);
             }
-            __syncthreads();
-            if (tid < PAIRS) { // sum of squares in index order, scale
-                const int rc = tid / HEADS_T, ht = tid % HEADS_T;
-                const int64_t m = m0 + ((rc % 64) / 32) * 128 + (2 * s + rc / 64) * 32 + (rc % 32);
-                const int hd = (int)(n0 / EP_D) + ht;
-                const float *const v = vals + tid * PITCH;
-                float sum2 = 0.0f;
+            if (s < 2) request(s + 2);
+        }
+        // lane L gets row L of the wave's 64: [j][0] its columns 32 j + 8 q + ..3, [j][1] those 4 further on
 #pragma unroll
-                for (int x = 0; x < EP_D; x += 32) { // 32 values per round of LDS reads, added in index order
-                    v4f q[8];
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) q[c] = *(const v4f *)(v + x + 4 * c);
+            for (int r = 0; r < 16; ++r) {
+                const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(val[j][0][r]), __float_as_uint(val[j][1][r]), false, false);
+                val[j][0][r] = __uint_as_float(y[0]);
+                val[j][1][r] = __uint_as_float(y[1]);
+            }
+        const int row = wm * 64 + lane;
+        float mult[HEADS_W];
+#pragma unroll
+        for (int h = 0; h < HEADS_W; ++h) { // sum of squares in index order, scale
+            float sum2 = 0.0f;
+#pragma unroll
+            for (int j = h * EP_D / 32; j < (h + 1) * EP_D / 32; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
 #pragma unroll
                     for (int c = 0; c < 8; ++c) {
-                        sum2 = sum2 + q[c].x * q[c].x;
-                        sum2 = sum2 + q[c].y * q[c].y;
-                        sum2 = sum2 + q[c].z * q[c].z;
-                        sum2 = sum2 + q[c].w * q[c].w;
+                        const float y = val[j][c >> 2][4 * q + (c & 3)];
+                        sum2 = sum2 + y * y;
                     }
-                }
-                float discr = 0.0f, mult = 0.0f;
-                if (sum2 != 0.0f) {
-                    const float sko = (float)sqrt((double)(sum2 / (float)EP_D)); // correctly rounded (see the producer kernel)
-                    discr = sko * e.vec_scale;
-                    mult = 1.0f / discr;
-                }
-                mults[tid] = mult;
-                const int sh = hd - e.scale_head_begin;
-                if (e.scale && m < p.m && hd < e.n_heads && sh >= 0 && sh < e.scale_head_count)
-                    e.scale[sh * e.scale_pitch + m * e.scale_row_stride] = discr * e.scale_mult;
+            float discr = 0.0f;
+            mult[h] = 0.0f;
+            if (sum2 != 0.0f) {
+                const float sko = (float)sqrt((double)(sum2 / (float)EP_D)); // correctly rounded (see the producer kernel)
+                discr = sko * e.vec_scale;
+                mult[h] = 1.0f / discr;
             }
-            __syncthreads();
-            // Convert and store, 16 bytes per thread and step.  A head of zeros has mult 0: zero bytes.
-            constexpr int OUT_PER_PAIR = EP_D / 16;
-            static_assert((PAIRS * OUT_PER_PAIR) % GW_THREADS == 0, "whole steps of the workgroup");
-            const float low = e.relu ? 0.0f : -127.0f;
-            uint8_t *const dst_base = e.dst + m0 * e.dst_pitch + n0;
+            const int hd = head0 + h, sh = hd - e.scale_head_begin;
+            if (e.scale && row < rows_here && hd < e.n_heads && sh >= 0 && sh < e.scale_head_count)
+                e.scale[sh * e.scale_pitch + (m0 + row) * e.scale_row_stride] = discr * e.scale_mult;
+        }
+        // Convert; the wave's bytes go through 8 KiB of LDS of its own (16-byte chunk c of row r at c ^ r % 8) and leave as
+        // whole lines, eight rows per store.  A head of zeros has mult 0: zero bytes.
+        const float low = e.relu ? 0.0f : -127.0f;
+        __syncthreads(); // every wave is done with the operand buffers
+        uint8_t *const bytes = gw_lds + wave * 64 * 128;
 #pragma unroll
-            for (int j0 = 0; j0 < PAIRS * OUT_PER_PAIR; j0 += GW_THREADS) {
-                const int j = j0 + tid;
-                const int pr = j / OUT_PER_PAIR, x = (j % OUT_PER_PAIR) * 16;
-                const int rc = pr / HEADS_T, ht = pr % HEADS_T;
-                const int row = ((rc % 64) / 32) * 128 + (2 * s + rc / 64) * 32 + (rc % 32);
-                const float mult = mults[pr];
-                v4f q[4];
+        for (int c = 0; c < 8; ++c) {
+            const float m = mult[c * 16 / EP_D];
+            v4i w;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) q[k] = *(const v4f *)(vals + pr * PITCH + x + 4 * k);
-                uint32_t w[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) w[k] = pack_i8x4(q[k].x * mult, q[k].y * mult, q[k].z * mult, q[k].w * mult, low);
-                if (row < rows_here && (int)(n0 / EP_D) + ht < e.n_heads)
-                    *(v4i *)(dst_base + ((uint32_t)row * (uint32_t)e.dst_pitch + (uint32_t)(ht * EP_D + x))) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+            for (int k = 0; k < 4; ++k) {
+                const float *const y = &val[c >> 1][k & 1][4 * ((c & 1) * 2 + (k >> 1))];
+                w[k] = (int)pack_i8x4(y[0] * m, y[1] * m, y[2] * m, y[3] * m, low);
             }
-            __syncthreads(); // before the next step overwrites the values
+            *(v4i *)(bytes + lane * 128 + ((c ^ (lane & 7)) << 4)) = w;
+        }
+        asm volatile("" ::: "memory"); // (a wave's own bytes: LDS keeps its accesses in order)
+        uint8_t *const dst_base = e.dst + m0 * e.dst_pitch + n0 + wn * 128;
+        const int c = lane & 7;
+        const bool head_ok = head0 + c * 16 / EP_D < e.n_heads;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int r = k * 8 + (lane >> 3);
+            const v4i w = *(const v4i *)(bytes + r * 128 + ((c ^ (r & 7)) << 4));
+            if (wm * 64 + r < rows_here && head_ok) *(v4i *)(dst_base + ((uint32_t)(wm * 64 + r) * (uint32_t)e.dst_pitch + (uint32_t)c * 16u)) = w;
         }
     } else if constexpr (MODE == TSATTN_MM_ADD_SCALED) {
         // state += sum * scale: the 32 old values of a block of rows are requested together, then updated and stored
@@ -430,8 +445,8 @@ hipError_t launch_tiles(const GemmParams &p, Tiles tiles, int ep_d, hipStream_t 
         return launch_gemm_mid(q, tiles == Tiles::ROWS64 ? 64 : 128, ep_d, st);
     }
     const dim3 grid((unsigned)(((p.m + GW_BM - 1) / GW_BM) * ((p.n + GW_BN - 1) / GW_BN)));
-    if (ep_d == 128) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 128>), grid, dim3(GW_THREADS), gw_lds_bytes(128), st, p);
-    else if (ep_d == 64) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 64>), grid, dim3(GW_THREADS), gw_lds_bytes(64), st, p);
+    if (ep_d == 128) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 128>), grid, dim3(GW_THREADS), GW_LDS_BYTES, st, p);
+    else if (ep_d == 64) hipLaunchKernelGGL((gemm_wide_kernel<TSATTN_MM_I32, 64>), grid, dim3(GW_THREADS), GW_LDS_BYTES, st, p);
     else hipLaunchKernelGGL((gemm_wide_kernel<MODE, 0>), grid, dim3(GW_THREADS), GW_LDS_BYTES, st, p);
     return hipGetLastError();
 }
@@ -453,11 +468,11 @@ hipError_t prepare_matmul_i8()
     const struct {
         const void *kernel;
         int lds;
-    } kernels[] = {{(const void *)gemm_wide_kernel<TSATTN_MM_I32, 0>, gw_lds_bytes(0)},
-                   {(const void *)gemm_wide_kernel<TSATTN_MM_F32, 0>, gw_lds_bytes(0)},
-                   {(const void *)gemm_wide_kernel<TSATTN_MM_ADD_SCALED, 0>, gw_lds_bytes(0)},
-                   {(const void *)gemm_wide_kernel<TSATTN_MM_I32, 64>, gw_lds_bytes(64)},
-                   {(const void *)gemm_wide_kernel<TSATTN_MM_I32, 128>, gw_lds_bytes(128)}};
+    } kernels[] = {{(const void *)gemm_wide_kernel<TSATTN_MM_I32, 0>, GW_LDS_BYTES},
+                   {(const void *)gemm_wide_kernel<TSATTN_MM_F32, 0>, GW_LDS_BYTES},
+                   {(const void *)gemm_wide_kernel<TSATTN_MM_ADD_SCALED, 0>, GW_LDS_BYTES},
+                   {(const void *)gemm_wide_kernel<TSATTN_MM_I32, 64>, GW_LDS_BYTES},
+                   {(const void *)gemm_wide_kernel<TSATTN_MM_I32, 128>, GW_LDS_BYTES}};
     for (const auto &k : kernels) {
         const hipError_t e = hipFuncSetAttribute(k.kernel, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds);
         if (e != hipSuccess) return e;
