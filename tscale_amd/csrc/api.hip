@@ -643,7 +643,7 @@ int tsattn_layer_token(tsattn_handle_t h, const tsattn_layer_args *a, void *stre
     // w [n][k] times the rows that normalisation of `source` gives -- int32 planes, the state, or the state with the planes'
     // residual update -- which the product's launch makes itself (and leaves the state alone), or with more rows a launch
     // before it (which stores the updated state).
-    const bool own = B <= tsattn::FEW_NORM_ROWS;
+    const bool own = B <= tsattn::FEW_NORM_ROWS && a->state_pitch <= tsattn::UPDATE_MAX_PITCH;
     const auto norm_product = [&](const void *w, int64_t n, int64_t k, int32_t *out, int group, const int32_t *source, int planes, float *state, float scale,
                                   int relu, const tsattn::UpdateParams *update, int *parts) {
         tsattn::FewParams f = {};
@@ -673,7 +673,7 @@ int tsattn_layer_token(tsattn_handle_t h, const tsattn_layer_args *a, void *stre
         tsattn::UpdateParams u = {};
         if (own && src) {
             u.state = a->state; u.state_pitch = a->state_pitch; u.src = src; u.planes = planes; u.src_stride = B * a->dim;
-            u.rows = a->n_seqs; u.dim = (int)a->dim; u.scale = scale;
+            u.rows = a->n_seqs; u.dim = (int)a->dim; u.scale = scale; u.by_row = tsattn::wg_make_div((uint32_t)(a->dim / 4));
         }
         return u;
     };

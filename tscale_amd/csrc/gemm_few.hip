@@ -138,6 +138,8 @@ hipError_t launch_stream(FewParams p, hipStream_t st, bool prepare)
     const int mt = few_mt(p.m);
     const unsigned lds = (unsigned)gs_lds_bytes(mt, p.k);
     p.k_chunk = (int)gs_rows_bytes(mt, p.k);
+    p.blk_per = (int)((p.n + 15) / 16) / 256; p.blk_more = (int)((p.n + 15) / 16) % 256;
+    p.by_row = wg_make_div((uint32_t)p.k / 16);
     if (mt == 1) hipLaunchKernelGGL((gemm_stream_kernel<MODE, 1>), dim3(256), dim3(GS_THREADS), lds, st, p);
     else hipLaunchKernelGGL((gemm_stream_kernel<MODE, 2>), dim3(256), dim3(GS_THREADS), lds, st, p);
     return hipGetLastError();
@@ -148,7 +150,8 @@ hipError_t launch_stream(FewParams p, hipStream_t st, bool prepare)
 bool few_source_ok(const FewParams &p)
 {
     return p.m >= 1 && p.m <= FEW_NORM_ROWS && (p.group == 64 || p.group == 128) && p.k % p.group == 0 && p.k % 64 == 0 &&
-           (p.src_planes == 1 || p.src_planes == 2 || p.src_planes == 4 || (p.src_planes == 0 && p.state));
+           (p.src_planes == 1 || p.src_planes == 2 || p.src_planes == 4 || (p.src_planes == 0 && p.state)) && p.k <= (1 << 20) &&
+           p.state_pitch <= UPDATE_MAX_PITCH;
 }
 
 int few_parts(const FewParams &p, int max_parts) { return stream_fits(p) ? 1 : few_best(p, 1, max_parts).parts; }
@@ -187,6 +190,8 @@ hipError_t launch_gemm_few(const FewParams &params, hipStream_t st)
     p.wn_log = f.wn_log; p.wn = 1 << f.wn_log; p.wk = f.waves >> f.wn_log; p.wk_log = log2_of(p.wk); p.group_log = log2_of(p.group);
     p.k_part = f.k_part; p.k_chunk = f.k_chunk;
     p.groups = f.groups; p.walk = (int64_t)f.groups * 16 * p.wn < p.n;
+    p.blk_per = (int)((p.n + 15) / 16) / f.groups; p.blk_more = (int)((p.n + 15) / 16) % f.groups;
+    p.by_row = wg_make_div((uint32_t)p.k_chunk / (p.a ? 16 : 4));
     const int mt = few_mt(p.m);
     if (!p.a) return launch_norm(p, p.src_planes, p.state != nullptr, st, false);
     if (p.mode == TSATTN_MM_I32) return launch_rows<TSATTN_MM_I32>(p, mt, st, false);

@@ -8,11 +8,19 @@
 // LDS nor a barrier.  The activations of the workgroup's part of K stand in LDS.  Waves that share weight rows add up in
 // LDS; parts of K that go to different workgroups become planes of the result.
 //
+// A launch of a few microseconds is mostly the instructions before its first load: about one per 3 ns and wave.  So the start has
+// no division (runs of blocks and reciprocals come from the host; the two 64-bit divisions that gave a workgroup its run and the
+// eight that placed a thread's pieces were 700 instructions) and 32-bit offsets from scalar bases, and no weight request is behind a
+// branch, which would make the activations wait for the weights.  768 x 3072 under one row: activations in LDS 2.6 us after the
+// start, now 1.4; its normalising forms end after 4.1 instead of 5.6 us.
+//
 // The activations are int8 rows in memory, or they are made here: the rows a normalisation of the layer would have written
 // (state and the planes of the product before it in, RMS normalisation per group, int8 out), for the part of K this
 // workgroup multiplies.  Every workgroup repeats that for its columns, which costs it their bytes from L2, and a launch and
 // its memory round trip are gone from the chain that a token step is.
 #pragma once
+
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -31,6 +39,9 @@ inline int gf_lds_bytes(int waves, int mt, int64_t m, int64_t kc, int group)
     const int64_t sums = (int64_t)waves * mt * WAVE * 16;
     return (int)(b > sums ? b : sums);
 }
+
+template <int N>
+using Pieces = std::integral_constant<int, N>;
 
 // a barrier for LDS traffic only: requests to memory stay on their way over it
 __device__ __forceinline__ void gf_barrier()
@@ -57,8 +68,8 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_few_kernel(FewParams p)
     const int k_begin = (int)blockIdx.y * p.k_part, k_end = min((int)p.k, k_begin + p.k_part);
     // This wave's blocks of 16 weight rows: every wn-th of the workgroup's run of them (one, unless there are so many that
     // workgroups which stage the activations once and walk several blocks are the better cut).
-    const int blocks = ((int)p.n + 15) / 16;
-    const int blk0 = (int)((int64_t)blockIdx.x * blocks / gridDim.x) + wn, blk_end = (int)(((int64_t)blockIdx.x + 1) * blocks / gridDim.x);
+    const int begin = (int)blockIdx.x * p.blk_per + min((int)blockIdx.x, p.blk_more);
+    const int blk0 = begin + wn, blk_end = begin + p.blk_per + ((int)blockIdx.x < p.blk_more ? 1 : 0);
     const int w_off = r16 * (int)p.w_pitch + g * 16;
 
     const int pitch = p.k_chunk + 16;
@@ -109,9 +120,10 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_few_kernel(FewParams p)
         };
         auto after = [&](const Round &r) __attribute__((always_inline)) { return r.s + GF_U < s1 ? Round{r.blk, r.s + GF_U} : Round{r.blk + p.wn, s0}; };
         auto request = [&](v4i(&dst)[GF_U], const Round &r) __attribute__((always_inline)) {
-            const int n0 = r.blk * 16, rows = min(16, (int)p.n - n0); // (rows past n: zero bytes)
+            // (rows past n, and a round that is not there: zero bytes)
+            const int blk = r.blk < blk_end ? r.blk : blk_end - 1, n0 = blk * 16, rows = min(16, (int)p.n - n0);
             const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.w + (int64_t)n0 * p.w_pitch), 0,
-                                                                                (int)((rows - 1) * p.w_pitch + p.k), 0x00020000);
+                                                                                r.blk < blk_end ? (rows - 1) * (int)p.w_pitch + (int)p.k : 0, 0x00020000);
 #pragma unroll
             for (int u = 0; u < GF_U; ++u)
                 dst[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + kc + (r.s + u) * 64, 0, NT ? 2 : 0));
@@ -119,50 +131,63 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_few_kernel(FewParams p)
         Round r0 = Round{s0 < s1 ? blk0 : blk_end, s0}, r1 = after(r0);
         auto first_requests = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_sched_barrier(0);
-            if (r0.blk < blk_end) request(w[0], r0);
-            if (r1.blk < blk_end) request(w[1], r1);
+            request(w[0], r0);
+            request(w[1], r1);
             __builtin_amdgcn_sched_barrier(0);
         };
         if (kc != k_begin) gf_barrier(); // the chunk before has been multiplied
 
         // The activations' requests go out first: what is requested first arrives first, and they have the longer way
-        // to the multiplication.
+        // to the multiplication.  The weights' requests follow in the last round whatever there is to ask for: behind a branch they
+        // would have to be waited for together with the activations.
         if constexpr (SRC < 0) {
-            constexpr int QB = 8;
             const int per_row = len / 16, total = (int)p.m * per_row;
-            for (int base = 0; base < total; base += QB * GF_THREADS) {
+            const WgDiv by_row = len == p.k_chunk ? p.by_row : wg_make_div((uint32_t)per_row);
+            auto stage = [&](auto pieces, auto last, int base) __attribute__((always_inline)) { // pieces of every thread
+                constexpr int QB = decltype(pieces)::value;
                 v4i q[QB];
                 int dst[QB];
 #pragma unroll
                 for (int i = 0; i < QB; ++i) {
                     const int j = base + i * GF_THREADS + tid, jc = j < total ? j : total - 1;
-                    const int row = jc / per_row, c = jc - row * per_row;
+                    const int row = (int)wg_div_small((uint32_t)jc, by_row), c = jc - row * per_row;
                     dst[i] = row * pitch + c * 16;
-                    q[i] = *(const v4i *)(p.a + (int64_t)row * p.a_pitch + kc + c * 16);
+                    q[i] = *(const v4i *)(p.a + kc + (uint32_t)(row * (int)p.a_pitch + c * 16));
                 }
-                if (base + QB * GF_THREADS >= total) first_requests();
+                if constexpr (decltype(last)::value) first_requests();
 #pragma unroll
-                for (int i = 0; i < QB; ++i) *(v4i *)(a_lds + dst[i]) = q[i];
+                for (int i = 0; i < QB; ++i) {
+                    *(v4i *)(a_lds + dst[i]) = q[i];
+                }
+            };
+            if (total <= GF_THREADS) { // (one row: the rest of a round would be instructions for nothing)
+                stage(Pieces<1>(), std::true_type(), 0);
+            } else {
+                constexpr int QB = 8;
+                int base = 0;
+                for (; base + QB * GF_THREADS < total; base += QB * GF_THREADS) stage(Pieces<QB>(), std::false_type(), base);
+                stage(Pieces<QB>(), std::true_type(), base);
             }
             gf_barrier();
         } else {
             const int G = p.group, per_row = len / 4, total = (int)p.m * per_row, groups = len / G, pairs = (int)p.m * groups;
             float *const squares = vals + pairs * (G + 4), *const mults = squares + pairs * (G + 4);
-            constexpr int QB = SRC + (RESID ? 1 : 0) <= 3 ? 8 : 4;
-            for (int base = 0; base < total; base += QB * GF_THREADS) {
+            const WgDiv by_row = len == p.k_chunk ? p.by_row : wg_make_div((uint32_t)per_row);
+            auto stage = [&](auto pieces, auto last, int base) __attribute__((always_inline)) {
+                constexpr int QB = decltype(pieces)::value;
                 v4i sum[QB][SRC > 0 ? SRC : 1];
                 v4f st[QB];
                 int at[QB];
 #pragma unroll
                 for (int i = 0; i < QB; ++i) {
                     const int j = base + i * GF_THREADS + tid, jc = j < total ? j : total - 1;
-                    const int row = jc / per_row, x = (jc - row * per_row) * 4;
+                    const int row = (int)wg_div_small((uint32_t)jc, by_row), x = (jc - row * per_row) * 4;
                     at[i] = (row * groups + (x >> p.group_log)) * (G + 4) + (x & (G - 1));
 #pragma unroll
-                    for (int s = 0; s < SRC; ++s) sum[i][s] = *(const v4i *)(p.src + s * p.src_stride + (int64_t)row * p.k + kc + x);
-                    if (RESID) st[i] = *(const v4f *)(p.state + (int64_t)row * p.state_pitch + kc + x);
+                    for (int s = 0; s < SRC; ++s) sum[i][s] = *(const v4i *)((const char *)(p.src + s * p.src_stride + kc) + (uint32_t)(row * (int)p.k + x) * 4u);
+                    if (RESID) st[i] = *(const v4f *)((const char *)(p.state + kc) + (uint32_t)(row * (int)p.state_pitch + x) * 4u);
                 }
-                if (base + QB * GF_THREADS >= total) first_requests();
+                if constexpr (decltype(last)::value) first_requests();
 #pragma unroll
                 for (int i = 0; i < QB; ++i) {
                     v4f v;
@@ -181,6 +206,14 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_few_kernel(FewParams p)
                     *(v4f *)(vals + at[i]) = v;
                     *(v4f *)(squares + at[i]) = v4f{v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w};
                 }
+            };
+            if (total <= GF_THREADS) { // (one row: the rest of a round would be instructions for nothing)
+                stage(Pieces<1>(), std::true_type(), 0);
+            } else {
+                constexpr int QB = SRC + (RESID ? 1 : 0) <= 3 ? 8 : 4;
+                int base = 0;
+                for (; base + QB * GF_THREADS < total; base += QB * GF_THREADS) stage(Pieces<QB>(), std::false_type(), base);
+                stage(Pieces<QB>(), std::true_type(), base);
             }
             if constexpr (UPDATES) {
                 if (kc == k_begin) update.finish(p.upd);
@@ -189,26 +222,36 @@ __global__ __launch_bounds__(GF_THREADS) void gemm_few_kernel(FewParams p)
             for (int pr = tid; pr < pairs; pr += GF_THREADS) { // squares added in index order, as the producer does
                 const float *const v = squares + pr * (G + 4);
                 float sum2 = 0.0f;
-                for (int x = 0; x < G; x += 32) {
-                    v4f q[8];
+                v4f q0[4], q1[4]; // (sixteen on their way while sixteen are added)
+                auto read = [&](v4f(&q)[4], int x) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) q[c] = *(const v4f *)(v + x + 4 * c);
+                    for (int c = 0; c < 4; ++c) q[c] = *(const v4f *)(v + x + 4 * c);
+                };
+                auto add = [&](const v4f(&q)[4]) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) {
+                    for (int c = 0; c < 4; ++c) {
                         sum2 = sum2 + q[c].x;
                         sum2 = sum2 + q[c].y;
                         sum2 = sum2 + q[c].z;
                         sum2 = sum2 + q[c].w;
                     }
+                };
+                read(q0, 0);
+#pragma unroll 1
+                for (int x = 0; x < G; x += 32) {
+                    read(q1, x + 16);
+                    add(q0);
+                    read(q0, x + 32 < G ? x + 32 : 0);
+                    add(q1);
                 }
                 float mult = 0.0f;
-                if (sum2 != 0.0f) mult = 1.0f / ((float)sqrt((double)(sum2 / (float)G)) * p.vec_scale);
+                if (sum2 != 0.0f) mult = 1.0f / (sqrt_rounded(sum2 / (float)G) * p.vec_scale);
                 mults[pr] = mult;
             }
             gf_barrier();
             const float low = p.relu ? 0.0f : -127.0f;
             for (int j = tid; j < total; j += GF_THREADS) {
-                const int row = j / per_row, x = (j - row * per_row) * 4, pr = row * groups + (x >> p.group_log);
+                const int row = (int)wg_div_small((uint32_t)j, by_row), x = (j - row * per_row) * 4, pr = row * groups + (x >> p.group_log);
                 const v4f v = *(const v4f *)(vals + pr * (G + 4) + (x & (G - 1)));
                 const float mult = mults[pr]; // a group of zeros has 0: zero bytes
                 *(uint32_t *)(a_lds + row * pitch + x) = pack_i8x4(v.x * mult, v.y * mult, v.z * mult, v.w * mult, low);

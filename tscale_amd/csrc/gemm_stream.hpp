@@ -44,8 +44,7 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(FewParams p)
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r16 = lane & 15, g = lane >> 4;
     const int k = (int)p.k, pitch = k + 16, ns = (k + 127) / 128; // (the last stage may hold only half of its bytes)
-    const int blocks = ((int)p.n + 15) / 16;
-    const int b0 = (int)((int64_t)blockIdx.x * blocks / gridDim.x), b1 = (int)(((int64_t)blockIdx.x + 1) * blocks / gridDim.x);
+    const int b0 = (int)blockIdx.x * p.blk_per + min((int)blockIdx.x, p.blk_more), b1 = b0 + p.blk_per + ((int)blockIdx.x < p.blk_more ? 1 : 0);
     const int total = (b1 - b0) * ns;
     auto share = [&](int w) { return (int)((int64_t)w * total / GS_WAVES); }; // where wave w's stages begin
     const int t0 = share(wave), t1 = share(wave + 1);
@@ -77,9 +76,9 @@ __global__ __launch_bounds__(GS_THREADS) void gemm_stream_kernel(FewParams p)
 #pragma unroll
             for (int i = 0; i < QB; ++i) {
                 const int j = base + i * GS_THREADS + tid, jc = j < pieces ? j : pieces - 1;
-                const int m = jc / per_row, c = jc - m * per_row;
+                const int m = (int)wg_div_small((uint32_t)jc, p.by_row), c = jc - m * per_row;
                 dst[i] = m * pitch + c * 16;
-                q[i] = *(const v4i *)(p.a + (int64_t)m * p.a_pitch + c * 16);
+                q[i] = *(const v4i *)(p.a + (uint32_t)(m * (int)p.a_pitch + c * 16));
             }
             if (base + QB * GS_THREADS >= pieces) {
                 __builtin_amdgcn_sched_barrier(0);

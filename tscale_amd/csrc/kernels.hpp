@@ -17,7 +17,10 @@ struct UpdateParams {
     int64_t src_stride;
     int rows, dim;
     float scale;
+    WgDiv by_row; // dim / 4
 };
+// (with rows and pitches of few_source_ok: offsets of 32 bits)
+constexpr int64_t UPDATE_MAX_PITCH = 1 << 24;
 
 // The step that makes a token's attention operands, done by the attention launch itself: q, the new key and value rows
 // and the key of KVProduct are heads of the projections' int32 planes [n_seqs][4 n_heads d] (qk, qv, k, v one after the other)
@@ -248,6 +251,8 @@ struct FewParams {
     UpdateParams upd; // (sources of planes alone)
     int parts; // parts of K, one plane of the result each
     int wn, wn_log, wk, wk_log, k_part, k_chunk, groups, walk, group_log;
+    int blk_per, blk_more; // blocks of 16 weight rows per workgroup; the first blk_more take one more
+    WgDiv by_row;          // a chunk's row in the pieces that a thread stages: 16 bytes, or four values to normalise
 };
 bool few_source_ok(const FewParams &p);              // whether the kernel can normalise this source itself
 int few_parts(const FewParams &p, int max_parts);    // how many parts K is best cut into, at most max_parts

@@ -18,13 +18,13 @@ struct WgDiv {
     uint32_t d, m;
 };
 
-inline WgDiv wg_make_div(uint32_t d)
+TSATTN_HD inline WgDiv wg_make_div(uint32_t d)
 {
     WgDiv r;
     r.d = d ? d : 1;
     // ceil(2^32 / d) overestimates the quotient by at most one; it does not fit 32 bits for d = 1, where
     // 2^32 - 1 underestimates by exactly one instead
-    r.m = r.d == 1 ? 0xffffffffu : (uint32_t)(((1ull << 32) + r.d - 1) / r.d);
+    r.m = r.d == 1 ? 0xffffffffu : 0xffffffffu / r.d + 1;
     return r;
 }
 
@@ -36,6 +36,12 @@ TSATTN_HD inline uint32_t wg_divmod(uint32_t x, WgDiv by, uint32_t &rem)
     if (r >= (int32_t)by.d) { ++q; r -= (int32_t)by.d; }
     rem = (uint32_t)r;
     return q;
+}
+
+// x / d where d >= 2 and x * d < 2^32: the overestimate of the reciprocal does not reach the next whole number
+TSATTN_HD inline uint32_t wg_div_small(uint32_t x, WgDiv by)
+{
+    return (uint32_t)(((uint64_t)x * by.m) >> 32);
 }
 
 struct WgMap {
