@@ -104,6 +104,44 @@ __device__ inline int dpp_xor2(int v) { return dpp_mov<0x4E>(v); }        // qua
 __device__ inline int dpp_half_mirror(int v) { return dpp_mov<0x141>(v); } // lane i <-> 7-i in each 8
 __device__ inline int dpp_mirror(int v) { return dpp_mov<0x140>(v); }      // lane i <-> 15-i in each 16
 
+__device__ inline float lane_xor1(float v) { return __int_as_float(dpp_xor1(__float_as_int(v))); }
+__device__ inline float lane_xor2(float v) { return __int_as_float(dpp_xor2(__float_as_int(v))); }
+__device__ inline float lane_xor4(float v) { return __int_as_float(dpp_mov<0x1B>(dpp_half_mirror(__float_as_int(v)))); } // i ^ 7 ^ 3
+__device__ inline float lane_xor8(float v) { return __int_as_float(dpp_mov<0x128>(__float_as_int(v))); }                 // turned by 8 of 16
+// a's odd groups of 16 (its upper 32) lanes change places with b's even ones (its lower 32)
+__device__ inline void lane_swap16(float &a, float &b)
+{
+    const auto y = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(y[0]);
+    b = __uint_as_float(y[1]);
+}
+__device__ inline void lane_swap32(float &a, float &b)
+{
+    const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(y[0]);
+    b = __uint_as_float(y[1]);
+}
+// op over lane i and the lanes that differ from it in the bits FIRST, 2 FIRST, .. LAST of the lane number (1 to 32)
+template <int FIRST, int LAST, typename F>
+__device__ inline float lane_reduce(float v, F &&op)
+{
+    if (FIRST <= 1 && LAST >= 1) v = op(v, lane_xor1(v));
+    if (FIRST <= 2 && LAST >= 2) v = op(v, lane_xor2(v));
+    if (FIRST <= 4 && LAST >= 4) v = op(v, lane_xor4(v));
+    if (FIRST <= 8 && LAST >= 8) v = op(v, lane_xor8(v));
+    if (FIRST <= 16 && LAST >= 16) {
+        float w = v;
+        lane_swap16(v, w);
+        v = op(v, w);
+    }
+    if (FIRST <= 32 && LAST >= 32) {
+        float w = v;
+        lane_swap32(v, w);
+        v = op(v, w);
+    }
+    return v;
+}
+
 // A thread's share of a residual update: groups of four, `threads` apart; the first is requested before and stored after
 // whatever the kernel does in between.  delta * scale is rounded before it is added (two statements in the reference).
 struct ResidUpdate {

@@ -1,13 +1,13 @@
 // Single-token attention over a planar int8 / e4m3 KV cache: bandwidth-bound split-KV kernel plus
 // the cross-split merge.
 //
-// Work decomposition.  grid = (n_splits, n_heads, n_seqs), 256 threads.  A (sequence, head) pair owns
+// Work decomposition.  grid = (n_splits, n_heads, n_seqs), four or sixteen waves (decode_wide in decode_splits.h).  A (sequence, head) pair owns
 // two contiguous planes, K[L][d] and V[L][d]; a split owns a contiguous run of cache rows.  Inside
 // a wave, d/16 neighbouring lanes share one cache row and each lane reads 16 B of it, so one wave
 // load instruction covers 1 KiB of consecutive memory (8 rows at d=128, 16 rows at d=64).  Each lane
 // group keeps its own online-softmax state (running max, sum, 16 value accumulators) across all the
-// rows it visits; states are merged only once, at the end: across lane groups by wave shuffles,
-// across the four waves through LDS, across splits by merge_kernel.
+// rows it visits; states are merged only once, at the end: across lane groups by lane exchanges,
+// across the waves through LDS, across splits by merge_kernel.
 //
 // Semantics follow ComputeValLookup of gpt/train/cpu_infer.cpp:413-460: keys cur-1 ... cur-min(cur,W)
 // (cur itself when W == 0), a leading logit 0 of value zero (:444), logit =
@@ -20,9 +20,9 @@
 
 namespace tsattn {
 
-constexpr int DEC_THREADS = 256;
-constexpr int DEC_WAVES = DEC_THREADS / WAVE;
+constexpr int DEC_WAVES = 4, DEC_WIDE_WAVES = 16; // waves per workgroup (wide: few workgroups, which then have a compute unit each)
 constexpr int DEC_LONG = 8, DEC_SHORT = 2; // cache rows per lane group and step (short: ranges of one step of four waves)
+constexpr int DEC_WIDE_LONG = 4;           // the same with sixteen waves
 static_assert(decode_step_rows(64) == DEC_WAVES * DEC_LONG * (WAVE / (64 / 16)) && decode_step_rows(128) == DEC_WAVES * DEC_LONG * (WAVE / (128 / 16)), "the split rule's step");
 
 template <int DTYPE>
@@ -142,9 +142,12 @@ __device__ inline void kv_product_store(const uint8_t *kv_k, int64_t kv_k_pitch,
 // normalisation included -- is made by the first wave of every workgroup from the projections' planes of its own head, while
 // the other waves ask for their first cache rows (nothing is made twice but q by the splits of a head).  It saves a launch
 // of 5.7 us for 1.5 us; the bytes are those of rope_normalize_kernel, the same float operations in the same order.
-template <int DTYPE, int D, bool QBF16, bool DUMP, bool FRONT, int DEC_U>
-__global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams p)
+// GENERAL: any stride of the cache's tokens, and the raw dot products on request; the others address a step's rows with 24-bit
+// products from a scalar base (the launcher checks the stride): two 64-bit products per row were a third of the loop's instructions.
+template <int DTYPE, int D, bool QBF16, bool GENERAL, bool FRONT, int WAVES, int DEC_U>
+__device__ __forceinline__ void decode_split(const DecodeParams &p)
 {
+    constexpr int DEC_THREADS = WAVES * WAVE;
     constexpr int LPK = D / 16;      // lanes per cache row
     constexpr int KPL = WAVE / LPK;  // rows per wave load
     constexpr int ROWS_PER_STEP = DEC_U * KPL;
@@ -154,13 +157,13 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
     const int seq = blockIdx.z;
     const int tid = threadIdx.x;
     const int lane = tid & (WAVE - 1);
-    const int wave = tid / WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int c = lane % LPK;        // which 16-byte slice of the row
     const int g = lane / LPK;        // which row of a wave load
 
-    __shared__ float sm_m[DEC_WAVES];
-    __shared__ float sm_l[DEC_WAVES];
-    __shared__ float sm_acc[DEC_WAVES][D];
+    __shared__ float sm_m[WAVES];
+    __shared__ float sm_l[WAVES];
+    __shared__ float sm_acc[WAVES][D];
     __shared__ __attribute__((aligned(16))) float f_square[FRONT ? 4 * (D + 4) : 4];
     __shared__ __attribute__((aligned(16))) uint8_t f_row[FRONT ? 4 * D : 16]; // q, new key, key of KVProduct, new value
     __shared__ float f_key_scale;
@@ -259,27 +262,28 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         return;
     }
 
-    const uint8_t *kbase = p.k + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + c * 16;
-    const uint8_t *vbase = p.v + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride + c * 16;
-    const float *ksb = p.ks ? p.ks + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
-    const float *vsb = p.vs ? p.vs + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
+    const uint8_t *const kbase = p.k + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride;
+    const uint8_t *const vbase = p.v + (int64_t)seq * p.seq_stride + (int64_t)head * p.head_stride;
+    const float *const ksb = p.ks ? p.ks + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
+    const float *const vsb = p.vs ? p.vs + (int64_t)seq * p.s_seq_stride + (int64_t)head * p.s_head_stride : nullptr;
     v4i kreg[DEC_U], vreg[DEC_U];
     float ksr[DEC_U], vsr[DEC_U];
-    int row[DEC_U]; // (with the front, which has no registers for them, computed again where they are needed)
-    auto row_of = [&](int base, int u) __attribute__((always_inline)) { return FRONT ? base + u * KPL + g : row[u]; };
     auto request = [&](int base) __attribute__((always_inline)) {
+        const uint8_t *const kb = kbase + (int64_t)base * p.tok_stride, *const vb = vbase + (int64_t)base * p.tok_stride;
+        const int last = s1 - 1 - base; // clamp the address, mask the logit below
+        uint32_t row[DEC_U];
+        uint64_t at[DEC_U];
 #pragma unroll
         for (int u = 0; u < DEC_U; ++u) {
-            if (!FRONT) row[u] = base + u * KPL + g;
-            const int r = row_of(base, u), rc = (r < s1) ? r : s1 - 1; // clamp the address, mask the logit below
-            kreg[u] = __builtin_nontemporal_load((const v4i *)(kbase + (int64_t)rc * p.tok_stride));
-            ksr[u] = ksb ? ksb[rc] : p.ks_const;
+            row[u] = (uint32_t)min(u * KPL + g, last);
+            at[u] = GENERAL ? (uint64_t)row[u] * (uint64_t)p.tok_stride + c * 16 : __umul24(row[u], (uint32_t)p.tok_stride) + c * 16;
+            kreg[u] = __builtin_nontemporal_load((const v4i *)(kb + at[u]));
+            ksr[u] = ksb ? (ksb + base)[row[u]] : p.ks_const;
         }
 #pragma unroll
         for (int u = 0; u < DEC_U; ++u) {
-            const int r = row_of(base, u), rc = (r < s1) ? r : s1 - 1;
-            vreg[u] = __builtin_nontemporal_load((const v4i *)(vbase + (int64_t)rc * p.tok_stride));
-            vsr[u] = vsb ? vsb[rc] : p.vs_const;
+            vreg[u] = __builtin_nontemporal_load((const v4i *)(vb + at[u]));
+            vsr[u] = vsb ? (vsb + base)[row[u]] : p.vs_const;
         }
     };
     int base = s0 + wave * ROWS_PER_STEP;
@@ -331,7 +335,7 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
                     }
                 }
                 if (sum2 != 0.0f) {
-                    discr = (float)sqrt((double)(sum2 / (float)D)) * p.front.vec_scale;
+                    discr = sqrt_rounded(sum2 / (float)D) * p.front.vec_scale;
                     mult = 1.0f / discr;
                 }
                 if (lane == 1) f_key_scale = discr * p.front.key_mult;
@@ -394,13 +398,13 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         qf.set(qb);
     }
 
-    const float ads = att_dot_scale(D);
+    const float scale = att_dot_scale(D) * qs;
 
     float m = 0.0f, l = 0.0f;
     float acc[16];
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
 
-    for (; base < s1; base += DEC_WAVES * ROWS_PER_STEP) {
+    for (; base < s1; base += WAVES * ROWS_PER_STEP) {
         if constexpr (!FRONT) { // (with nothing to wait for but the query a second copy of the requests only makes the code longer: 4 % of a short launch)
             request(base);
             // Every request of the step before the first sum: left to itself the compiler moves the last value row's request
@@ -416,13 +420,14 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         for (int u = 0; u < DEC_U; ++u) {
             float bits = group_sum_bits<DTYPE, LPK>(qf.dot_partial_as_bits(kreg[u]));
             float accf = (DTYPE == TSATTN_I8) ? (float)__float_as_int(bits) : bits;
-            if (DUMP) {
-                if (c == 0 && row_of(base, u) < s1) {
-                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + row_of(base, u)] = bits;
+            const int row = base + u * KPL + g;
+            if (GENERAL) {
+                if (p.dbg && c == 0 && row < s1) {
+                    ((float *)p.dbg)[((int64_t)seq * p.n_heads + head) * p.dbg_pitch + row] = bits;
                 }
             }
-            float dp = accf * ksr[u] * ads * qs - p.slope * (float)(cur - row_of(base, u));
-            s[u] = (row_of(base, u) < s1) ? dp : -INFINITY;
+            float dp = accf * ksr[u] * scale - p.slope * (float)(cur - row);
+            s[u] = row < s1 ? dp : -INFINITY;
             m_new = fmaxf(m_new, s[u]);
         }
         float alpha = fast_exp2(m - m_new);
@@ -436,40 +441,51 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
             l += pu;
             accumulate_values<DTYPE>(pu * vsr[u], vreg[u], acc);
         }
-        if (FRONT && base + DEC_WAVES * ROWS_PER_STEP < s1) request(base + DEC_WAVES * ROWS_PER_STEP);
+        if (FRONT && base + WAVES * ROWS_PER_STEP < s1) request(base + WAVES * ROWS_PER_STEP);
     }
 
     // ---- merge the lane groups of this wave ---------------------------------------------------
+    // One maximum for all of them, then every exchange halves what a lane still adds up: 15 sums per lane instead of 64 (with all
+    // of them in every lane, through LDS, the merge took 1.1 of a short launch's 6 us).  A lane ends with the columns
+    // 16 c + e .. of its c, e the bits of its group number from the top.
+    const auto largest = [](float x, float y) __attribute__((always_inline)) { return fmaxf(x, y); };
+    const auto sum = [](float x, float y) __attribute__((always_inline)) { return x + y; };
+    const float m_wave = lane_reduce<LPK, 32>(m, largest), f_lane = fast_exp2(m - m_wave);
+    l = lane_reduce<LPK, 32>(l * f_lane, sum);
 #pragma unroll
-    for (int o = LPK; o < WAVE; o <<= 1) {
-        float m_o = __shfl_xor(m, o, WAVE);
-        float l_o = __shfl_xor(l, o, WAVE);
-        float m_n = fmaxf(m, m_o);
-        float a = fast_exp2(m - m_n), b = fast_exp2(m_o - m_n);
-        l = l * a + l_o * b;
+    for (int i = 0; i < 16; ++i) acc[i] *= f_lane;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float acc_o = __shfl_xor(acc[i], o, WAVE);
-            acc[i] = acc[i] * a + acc_o * b;
-        }
-        m = m_n;
+    for (int i = 0; i < 8; ++i) {
+        lane_swap32(acc[i], acc[i + 8]);
+        acc[i] += acc[i + 8];
     }
-    if (g == 0) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sm_acc[wave][c * 16 + i] = acc[i];
-        if (c == 0) { sm_m[wave] = m; sm_l[wave] = l; }
+    for (int i = 0; i < 4; ++i) {
+        lane_swap16(acc[i], acc[i + 4]);
+        acc[i] += acc[i + 4];
     }
+    const bool high8 = lane & 8, high4 = lane & 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float keep = high8 ? acc[i + 2] : acc[i], give = high8 ? acc[i] : acc[i + 2];
+        acc[i] = keep + lane_xor8(give);
+    }
+    const int e = (lane >> 5) * 8 + ((lane >> 4) & 1) * 4 + (high8 ? 2 : 0);
+    if (LPK == 4) {
+        const float keep = high4 ? acc[1] : acc[0], give = high4 ? acc[0] : acc[1];
+        sm_acc[wave][c * 16 + e + (high4 ? 1 : 0)] = keep + lane_xor4(give);
+    } else {
+        *(v2f *)&sm_acc[wave][c * 16 + e] = v2f{acc[0], acc[1]};
+    }
+    if (lane == 0) { sm_m[wave] = m_wave; sm_l[wave] = l; }
     __syncthreads();
     // ---- merge the waves, write this split's partial --------------------------------------------
     if (tid < D) {
-        float M = sm_m[0];
-        for (int w = 1; w < DEC_WAVES; ++w) M = fmaxf(M, sm_m[w]);
-        float o = 0, L = 0;
-        for (int w = 0; w < DEC_WAVES; ++w) {
-            float f = fast_exp2(sm_m[w] - M);
-            o += sm_acc[w][tid] * f;
-            L += sm_l[w] * f;
-        }
+        const float m_w = sm_m[lane % WAVES], M = lane_reduce<1, WAVES / 2>(m_w, largest); // (lane i: wave i % WAVES)
+        const float f_w = fast_exp2(m_w - M), L = lane_reduce<1, WAVES / 2>(sm_l[lane % WAVES] * f_w, sum);
+        float o = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) o += sm_acc[w][tid] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f_w), w));
         if (direct) {
             // the only split: add the zero vector's weight 2^-M (M >= 0 by construction) and normalise here
             const float res = o / (L + fast_exp2(-M));
@@ -482,6 +498,19 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_split_kernel(DecodeParams 
         }
     }
     if (count_row) report_done(); // after the barrier above: every thread has read the old length
+}
+
+template <int DTYPE, int D, bool QBF16, bool GENERAL, bool FRONT, int DEC_U>
+__global__ __launch_bounds__(DEC_WAVES * WAVE) void decode_split_kernel(DecodeParams p)
+{
+    decode_split<DTYPE, D, QBF16, GENERAL, FRONT, DEC_WAVES, DEC_U>(p);
+}
+
+// Sixteen waves per workgroup
+template <int DTYPE, int D, bool QBF16, bool FRONT, int DEC_U>
+__global__ __launch_bounds__(DEC_WIDE_WAVES * WAVE) void decode_wide_kernel(DecodeParams p)
+{
+    decode_split<DTYPE, D, QBF16, false, FRONT, DEC_WIDE_WAVES, DEC_U>(p);
 }
 
 // out = sum_s acc_s 2^(m_s - M) / (2^-M + sum_s l_s 2^(m_s - M)),  M = max(0, max_s m_s)
@@ -515,20 +544,41 @@ __global__ __launch_bounds__(D) void decode_merge_kernel(const float *part_acc, 
 template <int DTYPE, int D, int U>
 static hipError_t launch_decode_u(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
 {
-    const bool dump = p.dbg != nullptr;
+    const dim3 block(DEC_WAVES * WAVE);
+    const bool general = p.dbg != nullptr || p.tok_stride >= (1 << 24);
     if (p.front.src) {
         if constexpr (DTYPE == TSATTN_I8) {
-            if (qbf16 || dump || !p.kv_out) return hipErrorInvalidValue;
-            hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, false, true, U>), grid, dim3(DEC_THREADS), 0, st, p);
+            if (qbf16 || p.dbg || !p.kv_out) return hipErrorInvalidValue;
+            if (general) hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, true, true, DEC_LONG>), grid, block, 0, st, p);
+            else hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, false, true, U>), grid, block, 0, st, p);
         } else {
             return hipErrorInvalidValue;
         }
     } else if (qbf16) {
-        if (dump) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, true, false, DEC_LONG>), grid, dim3(DEC_THREADS), 0, st, p);
-        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, false, false, U>), grid, dim3(DEC_THREADS), 0, st, p);
+        if (general) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, true, false, DEC_LONG>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, false, false, U>), grid, block, 0, st, p);
     } else {
-        if (dump) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, true, false, DEC_LONG>), grid, dim3(DEC_THREADS), 0, st, p);
-        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, false, false, U>), grid, dim3(DEC_THREADS), 0, st, p);
+        if (general) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, true, false, DEC_LONG>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, false, false, U>), grid, block, 0, st, p);
+    }
+    return hipGetLastError();
+}
+
+template <int DTYPE, int D, int U>
+static hipError_t launch_decode_wide(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
+{
+    const dim3 block(DEC_WIDE_WAVES * WAVE);
+    if (p.front.src) {
+        if constexpr (DTYPE == TSATTN_I8) {
+            if (qbf16 || !p.kv_out) return hipErrorInvalidValue;
+            hipLaunchKernelGGL((decode_wide_kernel<TSATTN_I8, D, false, true, U>), grid, block, 0, st, p);
+        } else {
+            return hipErrorInvalidValue;
+        }
+    } else if (qbf16) {
+        hipLaunchKernelGGL((decode_wide_kernel<DTYPE, D, true, false, U>), grid, block, 0, st, p);
+    } else {
+        hipLaunchKernelGGL((decode_wide_kernel<DTYPE, D, false, false, U>), grid, block, 0, st, p);
     }
     return hipGetLastError();
 }
@@ -536,11 +586,16 @@ static hipError_t launch_decode_u(const DecodeParams &p, bool qbf16, dim3 grid, 
 template <int DTYPE, int D>
 static hipError_t launch_decode_dd(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
 {
+    constexpr int64_t KPL = WAVE / (D / 16);
     // A range that four waves cover in one step of two rows per lane group (a 64-key window) is shared out in such steps:
     // with steps of eight the first wave alone would compute all of it (W = 64, d = 128: 1.8 us of its instructions).
     int64_t rows = p.max_len < p.window ? p.max_len : p.window;
     rows = (rows + p.n_splits - 1) / p.n_splits;
-    if (rows <= (int64_t)DEC_WAVES * DEC_SHORT * (WAVE / (D / 16))) return launch_decode_u<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st);
+    if (rows <= DEC_WAVES * DEC_SHORT * KPL) return launch_decode_u<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st);
+    if (p.wide && !p.dbg && p.tok_stride < (1 << 24)) {
+        if (rows <= DEC_WIDE_WAVES * DEC_SHORT * KPL) return launch_decode_wide<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st);
+        return launch_decode_wide<DTYPE, D, DEC_WIDE_LONG>(p, qbf16, grid, st);
+    }
     return launch_decode_u<DTYPE, D, DEC_LONG>(p, qbf16, grid, st);
 }
 

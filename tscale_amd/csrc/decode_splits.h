@@ -41,4 +41,17 @@ inline int decode_choose_splits(int64_t rows, int head_dim, int64_t pairs, int m
     return best;
 }
 
+// Whether a launch of `groups` workgroups with `rows` cache rows each takes sixteen waves per workgroup (decode_wide_kernel)
+// instead of four.  Where a workgroup has a compute unit to itself, four waves are one per SIMD, which issues an instruction every
+// 7.6 cycles where two and more get one in every 3.8; sixteen walk the rows at 1.05 to 1.16 us per step of the four, which take 1.3
+// us for each step begun, and cost 0.7 us more to start and to merge.  Microseconds with four and sixteen, one launch, width 64: 12 pairs
+// of 300 rows 4.5 and 4.9, 701 5.9 and 5.5, 1500 7.1 and 7.3, 4096 13.6 and 12.6; 156 of 4096 19.7 and 17.5, e4m3 20.4 and 18.0; width
+// 128: 16 of 300 6.1 and 5.5, of 4096 24.6 and 22.7; 128 of 4096 in two splits 26.9 and 25.0.  With more workgroups than compute units
+// the four are the better share: 288 of width 64, 1500 rows 12.9 and 15.7.
+inline bool decode_wide(int64_t rows, int head_dim, int64_t groups)
+{
+    const double steps = (double)rows / decode_step_rows(head_dim);
+    return groups <= 256 && 0.7 + 1.12 * steps < 1.3 * (double)(int64_t)(steps + 0.999);
+}
+
 } // namespace tsattn

@@ -51,6 +51,7 @@ struct DecodeParams {
     float slope;
     int n_heads;
     int n_splits;
+    bool wide; // sixteen waves per workgroup instead of four
     float *part_acc; // [seq][head][split][d]
     float *part_ml;  // [seq][head][split][2] = running max, sum
     void *dbg;
