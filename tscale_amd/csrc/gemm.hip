@@ -144,10 +144,10 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
             if (p.ep.pos && m < p.m) row_pos[i] = p.ep.pos[m];
         }
     }
-    // requests past K fetch bytes that are never computed with (or zeros past the rows' end)
+    const int k_bytes = (int)p.k;
     request(0, gw_lds);
-    request(GW_BK, gw_lds + GW_BUF);
-    request(2 * GW_BK, gw_lds + 2 * GW_BUF);
+    request(wide_k_offset(1, GW_BK, k_bytes), gw_lds + GW_BUF);
+    request(wide_k_offset(2, GW_BK, k_bytes), gw_lds + 2 * GW_BUF);
     asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); // this wave's share of the first tile has landed
     GW_BARRIER;
     if (half == 1) GW_BARRIER; // the second half of the workgroup runs half a step behind the first
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(GW_THREADS, 1) void gemm_wide_kernel(GemmParams p)
         // memory half: request the tile of step s + 3 into the buffer step s - 1 was read from, read this step's
         // operands, make sure this wave's share of the tile of step s + 1 has landed before the barrier
         GW_FENCE;
-        request((s + 3) * GW_BK, gw_lds + ((s + 3) & 3) * GW_BUF);
+        request(wide_k_offset(s + 3, GW_BK, k_bytes), gw_lds + ((s + 3) & 3) * GW_BUF);
         GW_FENCE;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {

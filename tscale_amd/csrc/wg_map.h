@@ -44,6 +44,15 @@ TSATTN_HD inline uint32_t wg_div_small(uint32_t x, WgDiv by)
     return (uint32_t)(((uint64_t)x * by.m) >> 32);
 }
 
+// Where in K the wide product's request number `step` begins, tiles of `tile` bytes: three requests are ahead of the step that is
+// multiplied, and those past the last step ask for the last tile again (never multiplied): a scalar offset past the rows' end is not
+// what a descriptor's bounds check is sure to cover.
+TSATTN_HD inline int wide_k_offset(int step, int tile, int k)
+{
+    const int at = step * tile, last = k - tile;
+    return at < last ? at : last;
+}
+
 struct WgMap {
     int period_tiles;  // T: query tiles per period of equal span structure, 0 = unknown
     int period_group;  // G: units per group of the period-aware order, 0 = that order is not used
