@@ -11,6 +11,7 @@
 #include "../../include/tsattn.h"
 #include "../../include/tsattn_test_hooks.h"
 #include "decode_splits.h"
+#include "few_offsets.h"
 #include "kernels.hpp"
 
 struct tsattn_ctx {
@@ -642,7 +643,7 @@ int tsattn_layer_token(tsattn_handle_t h, const tsattn_layer_args *a, void *stre
     // w [n][k] times the rows that normalisation of `source` gives -- int32 planes, the state, or the state with the planes'
     // residual update -- which the product's launch makes itself (and leaves the state alone), or with more rows a launch
     // before it (which stores the updated state).
-    const bool own = B <= tsattn::FEW_NORM_ROWS && a->state_pitch <= tsattn::UPDATE_MAX_PITCH;
+    const bool own = B <= tsattn::FEW_NORM_ROWS && tsattn::few_offsets_fit(B, std::max(a->dim, a->relu_dim), a->state_pitch);
     const auto norm_product = [&](const void *w, int64_t n, int64_t k, int32_t *out, int group, const int32_t *source, int planes, float *state, float scale,
                                   int relu, const tsattn::UpdateParams *update, int *parts) {
         tsattn::FewParams f = {};

@@ -1,4 +1,5 @@
 // The int8 product with few activation rows (one token per sequence): plan and launches.  The kernel: gemm_few.hpp.
+#include "few_offsets.h"
 #include "gemm_stream.hpp"
 
 namespace tsattn {
@@ -150,8 +151,8 @@ hipError_t launch_stream(FewParams p, hipStream_t st, bool prepare)
 bool few_source_ok(const FewParams &p)
 {
     return p.m >= 1 && p.m <= FEW_NORM_ROWS && (p.group == 64 || p.group == 128) && p.k % p.group == 0 && p.k % 64 == 0 &&
-           (p.src_planes == 1 || p.src_planes == 2 || p.src_planes == 4 || (p.src_planes == 0 && p.state)) && p.k <= (1 << 20) &&
-           p.state_pitch <= UPDATE_MAX_PITCH;
+           (p.src_planes == 1 || p.src_planes == 2 || p.src_planes == 4 || (p.src_planes == 0 && p.state)) &&
+           few_offsets_fit(p.m, p.k, p.state_pitch);
 }
 
 int few_parts(const FewParams &p, int max_parts) { return stream_fits(p) ? 1 : few_best(p, 1, max_parts).parts; }

@@ -19,8 +19,7 @@ struct UpdateParams {
     float scale;
     WgDiv by_row; // dim / 4
 };
-// (with rows and pitches of few_source_ok: offsets of 32 bits)
-constexpr int64_t UPDATE_MAX_PITCH = 1 << 24;
+// (rows, dim and state_pitch as few_offsets_fit takes them: offsets of 32 bits)
 
 // The step that makes a token's attention operands, done by the attention launch itself: q, the new key and value rows
 // and the key of KVProduct are heads of the projections' int32 planes [n_seqs][4 n_heads d] (qk, qv, k, v one after the other)
