@@ -17,7 +17,9 @@ constexpr int decode_step_rows(int head_dim) { return 4 * 8 * (64 / (head_dim / 
 //   no launch is faster than memory delivers the rows, 6800 bytes per nanosecond;
 //   more than one split costs the merge launch, 2.0 us, 0.28 us per split and 3 ns per workgroup, and 0.2 us more where the number is no
 //   power of two (8 pairs of width 128 and 3100 rows: 12.6, 12.9, 11.8 us with 5, 6 and 8 splits).
-// What it chooses is within 0.7 % of the best number on average and 11 % at worst.  Without the steps (a workgroup's rows at 37 bytes
+// What it chooses is within 0.7 % of the best number on average and 11 % at worst.  (Times of the kernel before its merge by halving
+// exchanges and 24-bit offsets; the present one walks at 54 to 66 bytes per nanosecond, a launch takes 1 to 2 us less, and the choice is 1.0 % off
+// the best number on average.)  Without the steps (a workgroup's rows at 37 bytes
 // per nanosecond or its share of the memory's rate, the merge 3.5 us and 0.04 us per split) it was 2.2 % and 21 % up to 240 pairs: one
 // sequence of 12 heads of width 64 and 4096 rows in 15 splits 12.8 us, in 8 (one step each) 10.3; 4 of 16 heads of width 128 and
 // 4096 rows in 3 splits 20.5 us, in 4 18.4; 8 of them with 1500 rows in one 16.5 us, in 2 15.2; 17 with 4096 rows in one 63 us, in

@@ -21,7 +21,8 @@ int log2_of(int x)
 }
 
 // What a launch with this cut would take, in nanoseconds; what matters is the order of the cuts.  From launches of
-// 768 x 768 to 8192 x 2048 matrices under 1 and 32 rows, each with every cut: 3.3 us for a launch whatever it does, the
+// 768 x 768 to 8192 x 2048 matrices under 1 and 32 rows, each with every cut (before the kernel's start became 1.2 us shorter, which
+// is the same for all of them): 3.3 us for a launch whatever it does, the
 // matrix at 6 TB/s, what a wave's steps add one after the other, the activations of a compute unit's workgroups (int8 rows,
 // or what they are normalised from) at 45 bytes per nanosecond, and workgroups beyond one or two per compute unit, which
 // cost their start: 8192 x 2048 under one row takes 6.3 us with 512 workgroups of four waves, 9.9 us with 1024.
