@@ -117,7 +117,8 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     p.ks_const = a->k_scale_const; p.vs_const = a->v_scale_const;
     p.cache_len = a->cache_len; p.window = a->window; p.slope = a->alibi_slope;
     p.n_heads = a->n_heads; p.n_splits = splits;
-    p.wide = tsattn::decode_wide((rows + splits - 1) / splits, a->head_dim, (int64_t)a->n_seqs * a->n_heads * splits);
+    const tsattn::DecodeKind kind = a->dtype == TSATTN_E4M3 ? tsattn::DECODE_E4M3 : front || a->k_new ? tsattn::DECODE_I8_APPEND : tsattn::DECODE_I8;
+    p.wide = tsattn::decode_wide((rows + splits - 1) / splits, a->head_dim, (int64_t)a->n_seqs * a->n_heads * splits, kind);
     p.part_acc = lim.part_acc; p.part_ml = lim.part_ml;
     p.dbg = a->debug_qk_acc; p.dbg_pitch = a->debug_pitch;
     p.out = a->out;

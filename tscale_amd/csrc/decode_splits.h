@@ -43,17 +43,30 @@ inline int decode_choose_splits(int64_t rows, int head_dim, int64_t pairs, int m
     return best;
 }
 
+// What a decode launch has to do.  An int8 launch that also adds the new row is one kind whether its rows come from a launch before it or from
+// its own front: a layer's one call and the chain of calls that it stands for add up in the same order.
+enum DecodeKind { DECODE_I8, DECODE_E4M3, DECODE_I8_APPEND };
+
+constexpr int DECODE_WIDE_GROUPS = 256; // compute units
+
 // Whether a launch of `groups` workgroups with `rows` cache rows each takes sixteen waves per workgroup (decode_wide_kernel)
 // instead of four.  Where a workgroup has a compute unit to itself, four waves are one per SIMD, which issues an instruction every
-// 7.6 cycles where two and more get one in every 3.8; sixteen walk the rows at 1.05 to 1.16 us per step of the four, which take 1.3
-// us for each step begun, and cost 0.7 us more to start and to merge.  Microseconds with four and sixteen, one launch, width 64: 12 pairs
-// of 300 rows 4.5 and 4.9, 701 5.9 and 5.5, 1500 7.1 and 7.3, 4096 13.6 and 12.6; 156 of 4096 19.7 and 17.5, e4m3 20.4 and 18.0; width
-// 128: 16 of 300 6.1 and 5.5, of 4096 24.6 and 22.7; 128 of 4096 in two splits 26.9 and 25.0.  With more workgroups than compute units
-// the four are the better share: 288 of width 64, 1500 rows 12.9 and 15.7.
-inline bool decode_wide(int64_t rows, int head_dim, int64_t groups)
+// 7.6 cycles where two and more get one in every 3.8, and have a quarter of the requests on their way; sixteen cost 0.3 to 0.4 us
+// more to start and to merge.  The step of the four decides: below it sixteen only shorten a wave's share of it, from one row on past
+// it the four begin another.  Microseconds by which sixteen are faster (a minus: slower), averages of launches of 8 to 256 workgroups in
+// one to twelve splits in a replayed graph, by rows per workgroup in steps of the four, each launch on a cache of its own / all on one:
+//                   1/4 - 1/2      1/2 - 3/4       3/4 - 1      1 - 1 1/2    1 1/2 - 2      2 - 3        more
+//   int8          -0.01 / -0.16   -0.22 / -0.47   -1.0 / -1.1   0.8 / 0.5   0.04 / -0.1   0.9 / 0.3    2.5 / 1.6
+//   e4m3           0.15 / -0.02   -0.24 / -0.68   -1.0 / -1.2   0.9 / 0.4   0.12 / 0.0    1.1 / 0.4    3.0 / 2.4
+//   with a front   0.31            0.22            0.03         0.7        -0.04          0.7          2.6
+// (up to a quarter of a step both take the four's short steps).  With sixteen waves the other fifteen ask for their rows while the first makes
+// the front, so that shorter ranges gain, too; above half a step an appending launch without one loses more than it gains.  With more
+// workgroups than compute units the four are the better share: 288 of width 64, 1500 rows 12.9 and 15.7 us; 96 pairs of 1024 rows in
+// three splits 9.5 and 11.9.
+inline bool decode_wide(int64_t rows, int head_dim, int64_t groups, DecodeKind kind = DECODE_I8)
 {
-    const double steps = (double)rows / decode_step_rows(head_dim);
-    return groups <= 256 && 0.7 + 1.12 * steps < 1.3 * (double)(int64_t)(steps + 0.999);
+    const int step = decode_step_rows(head_dim);
+    return groups <= DECODE_WIDE_GROUPS && (rows > step || (kind != DECODE_I8 && rows <= step / 2));
 }
 
 } // namespace tsattn
