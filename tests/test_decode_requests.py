@@ -32,7 +32,7 @@ def test_no_wait_between_a_steps_requests(tmp_path):
         elif "global_load_dwordx4" in line and line.rstrip().endswith(" nt"):  # a cache row
             assert not waited, kernel
             requests[kernel] += 1
-    assert len(requests) == 24  # two types, two widths; with and without bf16 queries: long and short steps, the dump
+    assert len(requests) == 32  # two types, two widths; with and without bf16 queries, any stride: long and short steps
     for kernel, n in requests.items():
         rows = int(re.search(r"ELi(\d+)EEEv", kernel).group(1))
         assert n == 2 * rows, (kernel, n)

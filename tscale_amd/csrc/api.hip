@@ -10,7 +10,6 @@
 
 #include "../../include/tsattn.h"
 #include "../../include/tsattn_test_hooks.h"
-#include "decode_splits.h"
 #include "few_offsets.h"
 #include "kernels.hpp"
 
@@ -108,7 +107,7 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     const int64_t rows = a->window < a->max_len ? std::max<int64_t>(a->window, 1) : a->max_len; // rows one query can see
     int splits = a->n_splits;
     if (splits < 0 || splits > max_splits) return fail(TSATTN_ERR_SCRATCH, "tsattn_decode: n_splits %d exceeds the scratch's %d for this batch", splits, max_splits);
-    const tsattn::DecodeKind kind = a->dtype == TSATTN_E4M3 ? tsattn::DECODE_E4M3 : front || a->k_new ? tsattn::DECODE_I8_APPEND : tsattn::DECODE_I8;
+    const tsattn::DecodeKind kind = tsattn::decode_kind(a->dtype == TSATTN_E4M3, front || a->k_new, a->tok_stride, a->debug_qk_acc != nullptr);
     if (splits == 0) splits = tsattn::decode_choose_splits(rows, a->head_dim, (int64_t)a->n_seqs * a->n_heads, max_splits, kind);
     tsattn::DecodeParams p = {};
     p.q = (const uint8_t *)a->q; p.q_pitch = a->q_pitch; p.q_scale = a->q_scale; p.q_scale_const = a->q_scale_const;
@@ -118,7 +117,7 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     p.ks_const = a->k_scale_const; p.vs_const = a->v_scale_const;
     p.cache_len = a->cache_len; p.window = a->window; p.slope = a->alibi_slope;
     p.n_heads = a->n_heads; p.n_splits = splits;
-    p.wide = tsattn::decode_wide((rows + splits - 1) / splits, a->head_dim, (int64_t)a->n_seqs * a->n_heads * splits, kind);
+    p.form = tsattn::decode_form((rows + splits - 1) / splits, a->head_dim, (int64_t)a->n_seqs * a->n_heads * splits, kind);
     p.part_acc = lim.part_acc; p.part_ml = lim.part_ml;
     p.dbg = a->debug_qk_acc; p.dbg_pitch = a->debug_pitch;
     p.out = a->out;

@@ -1,7 +1,7 @@
 // Single-token attention over a planar int8 / e4m3 KV cache: bandwidth-bound split-KV kernel plus
 // the cross-split merge.
 //
-// Work decomposition.  grid = (n_splits, n_heads, n_seqs), four or sixteen waves (decode_wide in decode_splits.h).  A (sequence, head) pair owns
+// Work decomposition.  grid = (n_splits, n_heads, n_seqs), four or sixteen waves (decode_form in decode_splits.h).  A (sequence, head) pair owns
 // two contiguous planes, K[L][d] and V[L][d]; a split owns a contiguous run of cache rows.  Inside
 // a wave, d/16 neighbouring lanes share one cache row and each lane reads 16 B of it, so one wave
 // load instruction covers 1 KiB of consecutive memory (8 rows at d=128, 16 rows at d=64).  Each lane
@@ -15,15 +15,9 @@
 // scale (:454).  The running max starts at 0 in every split, which is what the zero logit makes it
 // in the reference anyway, so no split ever needs a -inf state.
 #include "common.hpp"
-#include "decode_splits.h"
 #include "kernels.hpp"
 
 namespace tsattn {
-
-constexpr int DEC_WAVES = 4, DEC_WIDE_WAVES = 16; // waves per workgroup (wide: few workgroups, which then have a compute unit each)
-constexpr int DEC_LONG = 8, DEC_SHORT = 2; // cache rows per lane group and step (short: ranges of one step of four waves)
-constexpr int DEC_WIDE_LONG = 4;           // the same with sixteen waves
-static_assert(decode_step_rows(64) == DEC_WAVES * DEC_LONG * (WAVE / (64 / 16)) && decode_step_rows(128) == DEC_WAVES * DEC_LONG * (WAVE / (128 / 16)), "the split rule's step");
 
 template <int DTYPE>
 struct QFrag;
@@ -545,20 +539,20 @@ template <int DTYPE, int D, int U>
 static hipError_t launch_decode_u(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
 {
     const dim3 block(DEC_WAVES * WAVE);
-    const bool general = p.dbg != nullptr || p.tok_stride >= (1 << 24);
+    const bool general = p.form.general;
     if (p.front.src) {
         if constexpr (DTYPE == TSATTN_I8) {
             if (qbf16 || p.dbg || !p.kv_out) return hipErrorInvalidValue;
-            if (general) hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, true, true, DEC_LONG>), grid, block, 0, st, p);
+            if (general) hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, true, true, U>), grid, block, 0, st, p);
             else hipLaunchKernelGGL((decode_split_kernel<TSATTN_I8, D, false, false, true, U>), grid, block, 0, st, p);
         } else {
             return hipErrorInvalidValue;
         }
     } else if (qbf16) {
-        if (general) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, true, false, DEC_LONG>), grid, block, 0, st, p);
+        if (general) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, true, false, U>), grid, block, 0, st, p);
         else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, true, false, false, U>), grid, block, 0, st, p);
     } else {
-        if (general) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, true, false, DEC_LONG>), grid, block, 0, st, p);
+        if (general) hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, true, false, U>), grid, block, 0, st, p);
         else hipLaunchKernelGGL((decode_split_kernel<DTYPE, D, false, false, false, U>), grid, block, 0, st, p);
     }
     return hipGetLastError();
@@ -586,21 +580,15 @@ static hipError_t launch_decode_wide(const DecodeParams &p, bool qbf16, dim3 gri
 template <int DTYPE, int D>
 static hipError_t launch_decode_dd(const DecodeParams &p, bool qbf16, dim3 grid, hipStream_t st)
 {
-    constexpr int64_t KPL = WAVE / (D / 16);
-    // A range that four waves cover in one step of two rows per lane group (a 64-key window) is shared out in such steps:
-    // with steps of eight the first wave alone would compute all of it (W = 64, d = 128: 1.8 us of its instructions).
-    int64_t rows = p.max_len < p.window ? p.max_len : p.window;
-    rows = (rows + p.n_splits - 1) / p.n_splits;
-    if (rows <= DEC_WAVES * DEC_SHORT * KPL) return launch_decode_u<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st);
-    if (p.wide && !p.dbg && p.tok_stride < (1 << 24)) {
-        if (rows <= DEC_WIDE_WAVES * DEC_SHORT * KPL) return launch_decode_wide<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st);
-        return launch_decode_wide<DTYPE, D, DEC_WIDE_LONG>(p, qbf16, grid, st);
+    if (p.form.waves == DEC_WIDE_WAVES) {
+        return p.form.rows == DEC_SHORT ? launch_decode_wide<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st) : launch_decode_wide<DTYPE, D, DEC_WIDE_LONG>(p, qbf16, grid, st);
     }
-    return launch_decode_u<DTYPE, D, DEC_LONG>(p, qbf16, grid, st);
+    return p.form.rows == DEC_SHORT ? launch_decode_u<DTYPE, D, DEC_SHORT>(p, qbf16, grid, st) : launch_decode_u<DTYPE, D, DEC_LONG>(p, qbf16, grid, st);
 }
 
 hipError_t launch_decode(const DecodeParams &p, int dtype, int head_dim, bool qbf16, int n_seqs, float *out, hipStream_t st)
 {
+    if (p.form.general ? p.form.waves != DEC_WAVES : p.dbg != nullptr || p.tok_stride >= DECODE_NEAR) return hipErrorInvalidValue;
     dim3 grid(p.n_splits, p.n_heads, n_seqs);
     hipError_t e;
     if (dtype == TSATTN_I8 && head_dim == 128) e = launch_decode_dd<TSATTN_I8, 128>(p, qbf16, grid, st);

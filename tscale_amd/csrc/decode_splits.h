@@ -1,18 +1,29 @@
-// How many workgroups share a (sequence, head) pair's cache rows in a decode launch.  Plain C++: no device code, so that the
-// rule can be tested without a GPU.
+// How many workgroups share a (sequence, head) pair's cache rows in a decode launch, and in which form they walk them.  Plain C++: no
+// device code, so that the rules can be tested without a GPU.
 #pragma once
 
 #include <stdint.h>
 
 namespace tsattn {
 
-// cache rows that a workgroup of decode_split_kernel takes per step: four waves, eight rows per lane group, head_dim / 16 lanes
-// per row
-constexpr int decode_step_rows(int head_dim) { return 4 * 8 * (64 / (head_dim / 16)); }
+constexpr int DEC_WAVES = 4, DEC_WIDE_WAVES = 16; // waves per workgroup (wide: few workgroups, which then have a compute unit each)
+constexpr int DEC_LONG = 8, DEC_SHORT = 2; // cache rows per lane group and step (short: ranges of one step of the waves)
+constexpr int DEC_WIDE_LONG = 4;           // the same with sixteen waves
+
+// cache rows that a workgroup of four waves takes per step of DEC_LONG: head_dim / 16 lanes per row
+constexpr int decode_step_rows(int head_dim) { return DEC_WAVES * DEC_LONG * (64 / (head_dim / 16)); }
 
 // What a decode launch has to do.  An int8 launch that also adds the new row is one kind whether its rows come from a launch before it or from
 // its own front: a layer's one call and the chain of calls that it stands for add up in the same order.
-enum DecodeKind { DECODE_I8, DECODE_E4M3, DECODE_I8_APPEND };
+// DECODE_GENERAL: the kernels for any stride of the cache's tokens and for the dump of raw dot products, which exist with four waves.
+enum DecodeKind { DECODE_I8, DECODE_E4M3, DECODE_I8_APPEND, DECODE_GENERAL };
+
+constexpr int64_t DECODE_NEAR = 1 << 24; // token strides from here on are general: the other kernels multiply them in 24 bits
+
+constexpr DecodeKind decode_kind(bool e4m3, bool append, int64_t tok_stride, bool dump)
+{
+    return dump || tok_stride >= DECODE_NEAR ? DECODE_GENERAL : e4m3 ? DECODE_E4M3 : append ? DECODE_I8_APPEND : DECODE_I8;
+}
 
 constexpr int DECODE_WIDE_GROUPS = 256; // compute units
 
@@ -33,7 +44,23 @@ constexpr int DECODE_WIDE_GROUPS = 256; // compute units
 inline bool decode_wide(int64_t rows, int head_dim, int64_t groups, DecodeKind kind = DECODE_I8)
 {
     const int step = decode_step_rows(head_dim);
-    return groups <= DECODE_WIDE_GROUPS && (rows > step || (kind != DECODE_I8 && rows > step / 4 && rows <= step / 2));
+    return kind != DECODE_GENERAL && groups <= DECODE_WIDE_GROUPS && (rows > step || (kind != DECODE_I8 && rows > step / 4 && rows <= step / 2));
+}
+
+// The form of a launch of `groups` workgroups with `rows` cache rows each.  A range that the waves cover in one step of two rows per lane
+// group (a 64-key window) is shared out in such steps, whatever the stride: with steps of eight the first wave alone would compute
+// all of it (window 64, width 128: 1.8 us of its instructions).
+struct DecodeForm {
+    int waves, rows; // per workgroup; per lane group and step
+    bool general;
+};
+
+inline DecodeForm decode_form(int64_t rows, int head_dim, int64_t groups, DecodeKind kind)
+{
+    const bool wide = decode_wide(rows, head_dim, groups, kind);
+    const int waves = wide ? DEC_WIDE_WAVES : DEC_WAVES;
+    const bool one = rows <= waves * DEC_SHORT * (64 / (head_dim / 16));
+    return {waves, one ? DEC_SHORT : wide ? DEC_WIDE_LONG : DEC_LONG, kind == DECODE_GENERAL};
 }
 
 constexpr double DECODE_START_NS = 3550.0, DECODE_MERGE_NS = 2000.0, DECODE_SPLIT_NS = 305.0;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "decode_splits.h"
 #include "wg_map.h"
 
 namespace tsattn {
@@ -50,7 +51,7 @@ struct DecodeParams {
     float slope;
     int n_heads;
     int n_splits;
-    bool wide; // sixteen waves per workgroup instead of four
+    DecodeForm form;
     float *part_acc; // [seq][head][split][d]
     float *part_ml;  // [seq][head][split][2] = running max, sum
     void *dbg;
