@@ -30,6 +30,23 @@ int main()
                                 if (rows <= 64) want(f.waves == DEC_WAVES && f.rows == DEC_SHORT, "a window of 64", d, rows);
                             }
                     }
+    // what tests/test_gpu_decode_wide.py and tests/test_gpu_token_step.py are about takes the forms they name
+    const struct { DecodeKind kind; int pairs, head_dim, rows, splits, per_group; } SIXTEEN[] = { // splits 0: chosen
+        {DECODE_I8, 12, 64, 513, 1, DEC_WIDE_LONG}, {DECODE_I8, 12, 64, 1023, 1, DEC_WIDE_LONG}, {DECODE_E4M3, 12, 64, 1025, 2, DEC_WIDE_LONG},
+        {DECODE_E4M3, 12, 64, 2100, 2, DEC_WIDE_LONG}, {DECODE_I8, 12, 128, 257, 1, DEC_WIDE_LONG}, {DECODE_E4M3, 12, 128, 511, 1, DEC_WIDE_LONG},
+        {DECODE_I8, 12, 128, 513, 2, DEC_WIDE_LONG}, {DECODE_I8, 12, 128, 1100, 2, DEC_WIDE_LONG}, {DECODE_E4M3, 12, 64, 129, 1, DEC_SHORT},
+        {DECODE_E4M3, 12, 64, 256, 1, DEC_SHORT}, {DECODE_E4M3, 12, 128, 65, 1, DEC_SHORT}, {DECODE_E4M3, 12, 128, 128, 1, DEC_SHORT},
+        {DECODE_I8_APPEND, 6, 64, 200, 0, DEC_SHORT}, {DECODE_I8_APPEND, 6, 128, 100, 0, DEC_SHORT}, {DECODE_I8_APPEND, 6, 64, 700, 0, DEC_WIDE_LONG},
+        {DECODE_I8_APPEND, 6, 128, 400, 0, DEC_WIDE_LONG}, {DECODE_I8_APPEND, 156, 64, 1025, 0, DEC_WIDE_LONG}, {DECODE_I8_APPEND, 6, 64, 4500, 0, DEC_WIDE_LONG},
+        {DECODE_I8_APPEND, 6, 128, 2300, 0, DEC_WIDE_LONG}};
+    int several = 0;
+    for (const auto &l : SIXTEEN) {
+        const int s = l.splits ? l.splits : decode_choose_splits(l.rows, l.head_dim, l.pairs, 32, l.kind);
+        const DecodeForm f = decode_form((l.rows + s - 1) / s, l.head_dim, (int64_t)l.pairs * s, l.kind);
+        want(f.waves == DEC_WIDE_WAVES && f.rows == l.per_group, "sixteen waves", l.head_dim, l.rows);
+        several += l.splits == 0 && s > 1;
+    }
+    want(several == 2, "several splits", 0, several);
     if (ok) printf("OK\n");
     return ok ? 0 : 1;
 }
