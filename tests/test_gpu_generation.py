@@ -85,13 +85,14 @@ def test_prompt_then_generate(ctx, dtype, window, slope):
 
 @pytest.mark.parametrize("dtype", [capi.I8, capi.E4M3])
 @pytest.mark.parametrize("window,slope,splits", [(10 ** 6, 0.0, 0), (64, 0.5, 1), (1, 0.0, 1), (10 ** 6, 0.1, 3)])
-def test_fused_append_equals_append_then_decode(ctx, dtype, window, slope, splits):
+@pytest.mark.parametrize("L", [40, 100, 200, 700])   # short steps; sixteen waves in one short step; long steps; sixteen waves
+def test_fused_append_equals_append_then_decode(ctx, dtype, window, slope, splits, L):
     """tsattn_decode with k_new/v_new does what tsattn_cache_append + tsattn_decode do (cpu_infer.cpp:506-509):
     same cache contents, same lengths, bit-identical outputs, step after step; a full cache drops the row in
     both."""
     from tscale_amd import KVCache
-    B, H, d, L = 4, 3, 128, 40
-    start = [0, 17, 38, 5]          # sequence 2 fills up after two steps
+    B, H, d = 4, 3, 128
+    start = [0, 17, L - 2, L // 8]  # sequence 2 fills up after two steps
     rng = np.random.default_rng(3)
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
     caches = []

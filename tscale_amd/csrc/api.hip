@@ -107,8 +107,8 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     const int64_t rows = a->window < a->max_len ? std::max<int64_t>(a->window, 1) : a->max_len; // rows one query can see
     int splits = a->n_splits;
     if (splits < 0 || splits > max_splits) return fail(TSATTN_ERR_SCRATCH, "tsattn_decode: n_splits %d exceeds the scratch's %d for this batch", splits, max_splits);
-    const tsattn::DecodeKind kind = tsattn::decode_kind(a->dtype == TSATTN_E4M3, front || a->k_new, a->tok_stride, a->debug_qk_acc != nullptr);
-    if (splits == 0) splits = tsattn::decode_choose_splits(rows, a->head_dim, (int64_t)a->n_seqs * a->n_heads, max_splits, kind);
+    const bool general = tsattn::decode_general(a->tok_stride, a->debug_qk_acc != nullptr);
+    if (splits == 0) splits = tsattn::decode_choose_splits(rows, a->head_dim, (int64_t)a->n_seqs * a->n_heads, max_splits, general);
     tsattn::DecodeParams p = {};
     p.q = (const uint8_t *)a->q; p.q_pitch = a->q_pitch; p.q_scale = a->q_scale; p.q_scale_const = a->q_scale_const;
     p.k = (const uint8_t *)a->k_cache; p.v = (const uint8_t *)a->v_cache;
@@ -117,7 +117,7 @@ static int decode_with_scratch(const DecodeScratch &lim, const tsattn_decode_arg
     p.ks_const = a->k_scale_const; p.vs_const = a->v_scale_const;
     p.cache_len = a->cache_len; p.window = a->window; p.slope = a->alibi_slope;
     p.n_heads = a->n_heads; p.n_splits = splits;
-    p.form = tsattn::decode_form((rows + splits - 1) / splits, a->head_dim, (int64_t)a->n_seqs * a->n_heads * splits, kind);
+    p.form = tsattn::decode_form((rows + splits - 1) / splits, a->head_dim, (int64_t)a->n_seqs * a->n_heads * splits, general);
     p.part_acc = lim.part_acc; p.part_ml = lim.part_ml;
     p.dbg = a->debug_qk_acc; p.dbg_pitch = a->debug_pitch;
     p.out = a->out;

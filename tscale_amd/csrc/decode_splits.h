@@ -13,19 +13,12 @@ constexpr int DEC_WIDE_LONG = 4;           // the same with sixteen waves
 // cache rows that a workgroup of four waves takes per step of DEC_LONG: head_dim / 16 lanes per row
 constexpr int decode_step_rows(int head_dim) { return DEC_WAVES * DEC_LONG * (64 / (head_dim / 16)); }
 
-// What a decode launch has to do.  An int8 launch that also adds the new row is one kind whether its rows come from a launch before it or from
-// its own front: a layer's one call and the chain of calls that it stands for add up in the same order.
-// DECODE_GENERAL: the kernels for any stride of the cache's tokens and for the dump of raw dot products, which exist with four waves.
-enum DecodeKind { DECODE_I8, DECODE_E4M3, DECODE_I8_APPEND, DECODE_GENERAL };
-
-constexpr int64_t DECODE_NEAR = 1 << 24; // token strides from here on are general: the other kernels multiply them in 24 bits
-
-constexpr DecodeKind decode_kind(bool e4m3, bool append, int64_t tok_stride, bool dump)
-{
-    return dump || tok_stride >= DECODE_NEAR ? DECODE_GENERAL : e4m3 ? DECODE_E4M3 : append ? DECODE_I8_APPEND : DECODE_I8;
-}
-
 constexpr int DECODE_WIDE_GROUPS = 256; // compute units
+
+// Whether a launch takes the general kernels, which exist with four waves: any stride of the cache's tokens (the others multiply it in 24 bits)
+// and the dump of raw dot products.
+constexpr int64_t DECODE_NEAR = 1 << 24;
+constexpr bool decode_general(int64_t tok_stride, bool dump) { return dump || tok_stride >= DECODE_NEAR; }
 
 // Whether a launch of `groups` workgroups with `rows` cache rows each takes sixteen waves per workgroup (decode_wide_kernel)
 // instead of four.  Where a workgroup has a compute unit to itself, four waves are one per SIMD, which issues an instruction every
@@ -37,14 +30,15 @@ constexpr int DECODE_WIDE_GROUPS = 256; // compute units
 //   int8          -0.01 / -0.16   -0.22 / -0.47   -1.0 / -1.1   0.8 / 0.5   0.04 / -0.1   0.9 / 0.3    2.5 / 1.6
 //   e4m3           0.15 / -0.02   -0.24 / -0.68   -1.0 / -1.2   0.9 / 0.4   0.12 / 0.0    1.1 / 0.4    3.0 / 2.4
 //   with a front   0.31            0.22            0.03         0.7        -0.04          0.7          2.6
-// (up to a quarter of a step the four take short steps and are 0.4 us faster in every kind).  With sixteen waves the other fifteen ask for their rows while the first makes
-// the front, so that shorter ranges gain, too; above half a step an appending launch without one loses more than it gains.  With more
-// workgroups than compute units the four are the better share: 288 of width 64, 1500 rows 12.9 and 15.7 us; 96 pairs of 1024 rows in
-// three splits 9.5 and 11.9.
-inline bool decode_wide(int64_t rows, int head_dim, int64_t groups, DecodeKind kind = DECODE_I8)
+// (up to a quarter of a step the four take short steps and are 0.4 us faster throughout).  A cache of its own is what a model's layer has; one
+// cache for all launches stays in the L2s.  With sixteen waves the other fifteen ask for their rows while the first makes the front, so
+// that a front gains at shorter ranges, too; the rule is one for all, so that an append in the launch, one before it and a layer's one
+// call add up in the same order.  With more workgroups than compute units the four are the better share: 288 of width 64, 1500 rows 12.9
+// and 15.7 us; 96 pairs of 1024 rows in three splits 9.5 and 11.9.
+inline bool decode_wide(int64_t rows, int head_dim, int64_t groups, bool general = false)
 {
     const int step = decode_step_rows(head_dim);
-    return kind != DECODE_GENERAL && groups <= DECODE_WIDE_GROUPS && (rows > step || (kind != DECODE_I8 && rows > step / 4 && rows <= step / 2));
+    return !general && groups <= DECODE_WIDE_GROUPS && (rows > step || (rows > step / 4 && rows <= step / 2));
 }
 
 // The form of a launch of `groups` workgroups with `rows` cache rows each.  A range that the waves cover in one step of two rows per lane
@@ -55,12 +49,12 @@ struct DecodeForm {
     bool general;
 };
 
-inline DecodeForm decode_form(int64_t rows, int head_dim, int64_t groups, DecodeKind kind)
+inline DecodeForm decode_form(int64_t rows, int head_dim, int64_t groups, bool general)
 {
-    const bool wide = decode_wide(rows, head_dim, groups, kind);
+    const bool wide = decode_wide(rows, head_dim, groups, general);
     const int waves = wide ? DEC_WIDE_WAVES : DEC_WAVES;
     const bool one = rows <= waves * DEC_SHORT * (64 / (head_dim / 16));
-    return {waves, one ? DEC_SHORT : wide ? DEC_WIDE_LONG : DEC_LONG, kind == DECODE_GENERAL};
+    return {waves, one ? DEC_SHORT : wide ? DEC_WIDE_LONG : DEC_LONG, general};
 }
 
 constexpr double DECODE_START_NS = 3550.0, DECODE_MERGE_NS = 2000.0, DECODE_SPLIT_NS = 305.0;
@@ -73,14 +67,14 @@ constexpr double DECODE_START_NS = 3550.0, DECODE_MERGE_NS = 2000.0, DECODE_SPLI
 //   no launch is faster than memory delivers the rows, 8000 bytes per nanosecond;
 //   more than one split costs the merge launch, 2.0 us, 0.3 us per split and 1.7 ns per workgroup, and 0.15 us more where the number is no
 //   power of two.
-inline double decode_time(int64_t rows, int head_dim, int64_t pairs, int splits, DecodeKind kind)
+inline double decode_time(int64_t rows, int head_dim, int64_t pairs, int splits, bool general)
 {
     const int step = decode_step_rows(head_dim), row_bytes = 2 * head_dim + 8;
     const int64_t per = (rows + splits - 1) / splits, groups = pairs * splits, shared = (groups + DECODE_WIDE_GROUPS - 1) / DECODE_WIDE_GROUPS;
     double ns;
     if (4 * per <= step) {
         ns = DECODE_START_NS;
-    } else if (decode_wide(per, head_dim, groups, kind)) {
+    } else if (decode_wide(per, head_dim, groups, general)) {
         const int half = step / 2;
         ns = 3780.0 + (double)((per + half - 1) / half * half) * row_bytes / 47.5;
     } else {
@@ -98,18 +92,18 @@ inline double decode_time(int64_t rows, int head_dim, int64_t pairs, int splits,
 }
 
 // The number of splits (1, 2, 3, 4, 6, 8, 12 and so on; at most max_splits, and at most 1024 workgroups) with the least such time.  Together
-// with the form that decode_wide gives it it is 0.14 % off the best of both forms and all numbers on average, 6.5 % at worst (on one cache
-// 0.5 % and 8 %).  Chosen by a fit of the four waves alone and the form after it, it was 0.8 and 13 %: 64 pairs of width 64, 1500 rows on one cache in 3
+// with the form that decode_wide gives it it is 0.2 % off the best of both forms and all numbers on average, 6.5 % at worst (on one cache
+// 0.6 % and 8 %).  Chosen by a fit of the four waves alone and the form after it, it was 0.8 and 13 %: 64 pairs of width 64, 1500 rows on one cache in 3
 // splits and two launches 8.2 us where one launch of sixteen waves takes 7.4 to 7.9; 156 pairs of width 128, 2500 rows in 3 splits 23.6, in one
 // launch of sixteen 21.4.
-inline int decode_choose_splits(int64_t rows, int head_dim, int64_t pairs, int max_splits, DecodeKind kind = DECODE_I8)
+inline int decode_choose_splits(int64_t rows, int head_dim, int64_t pairs, int max_splits, bool general = false)
 {
     int best = 1;
-    double best_ns = decode_time(rows, head_dim, pairs, 1, kind);
+    double best_ns = decode_time(rows, head_dim, pairs, 1, general);
     for (int s = 1; (rows + s - 1) / s * 4 > decode_step_rows(head_dim);) { // (more splits shorten no workgroup's walk)
         s = s == 1 ? 2 : (s & (s - 1)) == 0 ? s + s / 2 : s / 3 * 4;
         if (s > max_splits || s * pairs > 1024 || DECODE_START_NS + DECODE_MERGE_NS + DECODE_SPLIT_NS * s >= best_ns) break; // (nor can more be less)
-        const double ns = decode_time(rows, head_dim, pairs, s, kind);
+        const double ns = decode_time(rows, head_dim, pairs, s, general);
         if (ns < best_ns) { best_ns = ns; best = s; }
     }
     return best;
