@@ -1,6 +1,6 @@
 // CPU test of the choice between four and sixteen waves per workgroup of a decode launch.  The times are microseconds of launches in a
 // replayed graph (MI355X, int8 cache, bf16 queries) with four and with sixteen; the rule has to choose one that is at most 7 % slower
-// than the other (5 % is the worst of these lines as measured), and four from one workgroup more than there are compute units.  Built
+// than the other (3 % is the worst of these lines, all launches on one cache), and four from one workgroup more than there are compute units.  Built
 // with g++ (no GPU needed).
 #include <cstdio>
 
